@@ -27,6 +27,27 @@ constexpr int kWin = 128;      // window length of the reference sweeps (arrsize
 constexpr int kReal = kWin - 2 * kNpad;  // interior cells per window (realarr)
 constexpr int kWaveSize = 64;
 
+// FP64 path: per-slot constants of the radial and theta sweeps, entry-major (entry e of slot s at
+// tab[e*tstride + s], each rounded from the reference's own expression), so that a lane's two
+// consecutive cells are one 16-byte load and no cell divides by its geometry:
+//   radius of the cell centre, left edge, width, volume, reciprocals of radius, width and volume,
+//   -1/r/r at the centre, -1/x/x and 1/x at the left edge, r_cyl and its reciprocal, paraset's
+//   c0..c4 (parabola.cu:138-176) of the Eulerian grid, nu, c_s^2;
+//   2-D, per step: cos / sin of dt (vrot - v_y) / 2, the planet's turn against the slot in half a
+//   step (3-D, per step: vrot = res_v / r_cyl);
+//   3-D: sin, cos of theta and theta at the centre; the theta grid's left edge, width,
+//   volume and their reciprocals, sin / cos at the left edge and its paraset.
+// The stride leaves kT64Overhang slots past the last one (copies of it) for a window's tail.
+enum Tab64 {
+  kT64Rad, kT64Xa, kT64Dx, kT64Vol, kT64Irad, kT64Idx, kT64Ivol, kT64Star, kT64Fst, kT64Ixa,
+  kT64Rc, kT64Irc, kT64P0, kT64P4 = kT64P0 + 4, kT64Nu, kT64Cs2, kT64RotC, kT64RotS,
+  kT64Entries2d,
+  kT64Sp = kT64Entries2d, kT64Cp, kT64Pol, kT64Vrot,
+  kT64Za, kT64Dz, kT64Volz, kT64Idz, kT64Ivolz, kT64Spl, kT64Cpl, kT64P0z, kT64P4z = kT64P0z + 4,
+  kT64Entries3d
+};
+constexpr int kT64Overhang = 128;   // a radial or theta window's length
+
 enum Field { FR = 0, FP = 1, FU = 2, FV = 3, FW = 4, kNField = 5 };
 
 struct DevGrid {
@@ -42,6 +63,14 @@ struct DevGrid {
   int *rot_j, *inc_j;
   const double *y, *dy, *yc, *yvol;
   const pn_symdisk* val;
+  // FP64 contexts (null on the FP32 path): the slot table, in 3-D its theta-major copy (slot
+  // (ir, kz) at kz + sk ir, so that a theta pencil's slots are consecutive), per column cos / sin
+  // of the angle from the planet, and paraset of a uniform azimuthal grid
+  double *tab, *tabz;
+  double2* ptrig;
+  long tstride;
+  int uniform_phi;
+  double p0y[5];
 };
 
 struct DevParams {

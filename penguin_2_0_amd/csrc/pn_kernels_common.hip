@@ -210,6 +210,7 @@ __global__ __launch_bounds__(256) void k_reduce(DevGrid g, DevParams prm, const 
   __shared__ double sh[4];
   const long ncell = (long)g.imax * g.kmax * g.jmax;
   const Planet pl{ss->planet.m, ss->planet.x, ss->planet.y, ss->planet.vx, ss->planet.vy, ss->planet.rs, prm.bary};
+  const Grav G(pl, false);
   double acc = 0.0;
   for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < ncell; t += (long)gridDim.x * blockDim.x) {
     const int j = (int)(t % g.jmax);
@@ -228,10 +229,10 @@ __global__ __launch_bounds__(256) void k_reduce(DevGrid g, DevParams prm, const 
       if (dd > exclude * exclude) {
         const double bg = pow(g.xc[s], -prm.p_alpha);
         if (mode == 8) {
-          tmp = -grav_rad_cyl<double>(pl, rad, phi, 0.0, 0.0);
+          tmp = -grav_rad_cyl(G, rad, cos(phi - pl.y));
           tmp *= (r - bg) * g.xvol[s] * g.yvol[j0];
         } else {
-          tmp = -grav_azi_cyl<double>(pl, rad, phi, 0.0, 0.0);
+          tmp = -grav_azi_cyl(G, rad, cos(phi - pl.y), sin(phi - pl.y));
           tmp *= rad * (r - bg) * g.xvol[s] * g.yvol[j0];
         }
       }
@@ -461,6 +462,21 @@ __device__ __forceinline__ void rot_rows_slot(const DevGrid& g, double vy, float
   }
 }
 
+// the per-step rows of the FP64 table: in 2-D cos / sin of dt (res_v / r_cyl - v_y) / 2, in 3-D
+// vrot = res_v / r_cyl (ghost slots keep res_v = 0)
+__device__ __forceinline__ void turn_rows_slot(const DevGrid& g, double vy, double dt, int s) {
+  const double vrot = g.res_v[s] / g.radc[s];
+  if (g.tabz) {
+    g.tab[kT64Vrot * g.tstride + s] = vrot;
+    g.tabz[kT64Vrot * g.tstride + s / g.sr + (long)g.sk * (s % g.sr)] = vrot;
+    return;
+  }
+  double sn, cs;
+  sincos(0.5 * dt * (vrot - vy), &sn, &cs);
+  g.tab[kT64RotC * g.tstride + s] = cs;
+  g.tab[kT64RotS * g.tstride + s] = sn;
+}
+
 // Index_Shift of the ring in slot s (if s holds one) with its vrot row, then the slot's
 // rotation rows: everything per slot reads and writes that slot only
 __device__ __forceinline__ void ring_slot(DevGrid& g, const DevParams& prm, double dt, double fr, double vy,
@@ -471,6 +487,7 @@ __device__ __forceinline__ void ring_slot(DevGrid& g, const DevParams& prm, doub
     if (tab) tab[(long)kTabVrot * tstride + s] = (float)(g.res_v[s] / g.radc[s]);
   }
   if (tab) rot_rows_slot(g, vy, tab, tabz, tstride, dt, s);
+  if (g.tab) turn_rows_slot(g, vy, dt, s);
 }
 
 // Everything of a step before the sweeps, in one workgroup (main.cu:345-370): dt from ncfl
@@ -498,7 +515,7 @@ __device__ __forceinline__ void pre_step_body(DevGrid g, const DevParams& prm, S
     ss->fr_shift = s_fr;
     s_py = ss->planet.y;   // the half kick below changes velocities only
     // the trig table depends on the planet's azimuth alone: refresh it when that moved
-    s_trig = (trig != nullptr) && !(ss->trig_ok && ss->trig_y == s_py);
+    s_trig = (trig != nullptr || g.ptrig != nullptr) && !(ss->trig_ok && ss->trig_y == s_py);
     if (s_trig) {
       ss->trig_ok = 1;
       ss->trig_y = s_py;
@@ -519,8 +536,14 @@ __device__ __forceinline__ void pre_step_body(DevGrid g, const DevParams& prm, S
   if (s_trig) {
     const double py = s_py;
     for (int j = threadIdx.x; j < g.jmax; j += blockDim.x) {
-      const double a = 0.5 * (g.yc[j] - py);
-      trig[j] = make_float2((float)sin(a), (float)cos(a));
+      if (trig) {
+        const double a = 0.5 * (g.yc[j] - py);
+        trig[j] = make_float2((float)sin(a), (float)cos(a));
+      } else {
+        double sn, cs;
+        sincos(g.yc[j] - py, &sn, &cs);
+        g.ptrig[j] = make_double2(cs, sn);
+      }
     }
   }
   __syncthreads();
@@ -532,11 +555,14 @@ __device__ __forceinline__ void pre_step_body(DevGrid g, const DevParams& prm, S
     ss->FrRot = (prm.frrot == 1) ? b.vy : 0.0;
     b.vy -= ss->FrRot;
   }
-  if (tab && rings) {
+  if ((tab || g.tab) && rings) {
     __syncthreads();
     const double vy = ss->planet.vy;
     // one workgroup per disk (the batched pre-step runs one per disk of the grid)
-    for (int s = threadIdx.x; s < g.sr * g.sk; s += blockDim.x) rot_rows_slot(g, vy, tab, tabz, tstride, dt, s);
+    for (int s = threadIdx.x; s < g.sr * g.sk; s += blockDim.x) {
+      if (tab) rot_rows_slot(g, vy, tab, tabz, tstride, dt, s);
+      else turn_rows_slot(g, vy, dt, s);
+    }
   }
 }
 
@@ -653,6 +679,45 @@ int red_blocks(const DevGrid& g) {
 hipError_t launch_index_shift(const LaunchCtx& c) {
   int n = c.g.imax * c.g.kmax;
   k_index_shift<<<(n + 255) / 256, 256, 0, c.stream>>>(c.g, c.p, c.ss);
+  return hipGetLastError();
+}
+
+namespace {
+__global__ __launch_bounds__(256) void k_prep64(DevGrid g, const StepScalars* __restrict__ ss, int nslot) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < g.jmax) {
+    double sn, cs;
+    sincos(g.yc[t] - ss->planet.y, &sn, &cs);
+    g.ptrig[t] = make_double2(cs, sn);
+  }
+  if (t < nslot) turn_rows_slot(g, ss->planet.vy, ss->dt, t);
+}
+// sin / cos of theta in the 3-D slot table and its theta-major copy, by the functions the theta
+// sweep itself takes of a moved edge: its area factor (cos x0 - cos x) / (x - x0) of an edge that
+// hardly moves keeps nothing but the last bits of both cosines
+__global__ __launch_bounds__(256) void k_tab64_theta(DevGrid g, int nslot) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= nslot) return;
+  const long sz = s / g.sr + (long)g.sk * (s % g.sr);
+  const double v[4] = {sin(g.zc[s]), cos(g.zc[s]), sin(g.z[s]), cos(g.z[s])};
+  const int e[4] = {kT64Sp, kT64Cp, kT64Spl, kT64Cpl};
+  for (int q = 0; q < 4; ++q) {
+    g.tab[e[q] * g.tstride + s] = v[q];
+    g.tabz[e[q] * g.tstride + sz] = v[q];
+  }
+}
+}  // namespace
+
+hipError_t fp64_tab_theta(const LaunchCtx& c) {
+  const int nslot = c.g.sr * c.g.sk;
+  k_tab64_theta<<<(nslot + 255) / 256, 256, 0, c.stream>>>(c.g, nslot);
+  return hipGetLastError();
+}
+
+hipError_t fp64_prep(const LaunchCtx& c) {
+  const int nslot = c.g.sr * c.g.sk;
+  const int n = nslot > c.g.jmax ? nslot : c.g.jmax;
+  k_prep64<<<(n + 255) / 256, 256, 0, c.stream>>>(c.g, c.ss, nslot);
   return hipGetLastError();
 }
 

@@ -692,6 +692,7 @@ __global__ __launch_bounds__(256) void k_reduce_f32(DevGrid g, DevF32 f, DevPara
   __shared__ double sh[4];
   const long ncell = (long)g.imax * g.kmax * g.jmax;
   const Planet pl{ss->planet.m, ss->planet.x, ss->planet.y, ss->planet.vx, ss->planet.vy, ss->planet.rs, prm.bary};
+  const Grav G(pl, false);
   double acc = 0.0;
   for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < ncell; t += (long)gridDim.x * blockDim.x) {
     const int j = (int)(t % g.jmax);
@@ -708,8 +709,8 @@ __global__ __launch_bounds__(256) void k_reduce_f32(DevGrid g, DevF32 f, DevPara
       const double dd = (rad - pl.x) * (rad - pl.x) + rad * rad * (phi - pl.y) * (phi - pl.y);
       if (dd > exclude * exclude) {
         const double bg = pow(g.xc[s], -prm.p_alpha);
-        if (mode == 8) tmp = -grav_rad_cyl<double>(pl, rad, phi, 0.0, 0.0) * (r - bg) * g.xvol[s] * g.yvol[j0];
-        else tmp = -grav_azi_cyl<double>(pl, rad, phi, 0.0, 0.0) * (rad * (r - bg) * g.xvol[s] * g.yvol[j0]);
+        if (mode == 8) tmp = -grav_rad_cyl(G, rad, cos(phi - pl.y)) * (r - bg) * g.xvol[s] * g.yvol[j0];
+        else tmp = -grav_azi_cyl(G, rad, cos(phi - pl.y), sin(phi - pl.y)) * (rad * (r - bg) * g.xvol[s] * g.yvol[j0]);
       }
     }
     acc += tmp;

@@ -33,6 +33,11 @@ struct DiskDev {
   int tstride;
 };
 
+// per-step tables of the FP64 sweeps from ss (planet, dt) and the rings' res_v: a caller of a
+// single sweep runs it first; a step's pre-step does the same
+hipError_t fp64_prep(const LaunchCtx& c);
+// sin / cos of theta in the 3-D FP64 slot table, from the uploaded grid
+hipError_t fp64_tab_theta(const LaunchCtx& c);
 // FP64 path (pn_kernels_fp64.hip); each returns hipSuccess or the launch error
 hipError_t fp64_sweep_x(const LaunchCtx& c, int src);
 hipError_t fp64_sweep_y(const LaunchCtx& c, int src);

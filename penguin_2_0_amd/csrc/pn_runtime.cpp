@@ -149,7 +149,7 @@ int launch_cfl_any(pn_ctx* c, int src) {   // partial maxima, then dt
 }
 
 // sweeps of one step; the state returns to cur in 2-D and moves to the other buffer in 3-D.
-// prep: refresh the FP32 per-step tables first; roll: the integer roll after the sweeps.
+// prep: refresh the per-step tables first; roll: the integer roll after the sweeps.
 int launch_sweeps(pn_ctx* c, int& cur, int do_cfl, bool prep, bool roll) {
   LaunchCtx L = lctx(c);
   if (is_f32(c)) {
@@ -164,6 +164,7 @@ int launch_sweeps(pn_ctx* c, int& cur, int do_cfl, bool prep, bool roll) {
       PN_LAUNCH(c, "sweep_y", f32_sweep_y(L, c->df, c->var_y, cur ^ 1, do_cfl));
     }
   } else {
+    if (prep) PN_LAUNCH(c, "prep", fp64_prep(L));
     PN_LAUNCH(c, "ghosts", launch_fill_ghosts(L, cur));
     PN_LAUNCH(c, "sweep_x", fp64_sweep_x(L, cur));
     PN_LAUNCH(c, "sweep_y", fp64_sweep_y(L, cur ^ 1));
@@ -202,6 +203,95 @@ int launch_step(pn_ctx* c, int& cur) {
 
 }  // namespace rt
 }  // namespace pn
+
+namespace {
+
+// paraset (parabola.cu:138-176) of cell t on widths w(t), operation for operation
+template <class W>
+void paraset_host(const W& w, long t, double* c) {
+  auto an = [&](long i) { return w(i) + w(i + 1); };
+  auto bn = [&](long i) { return an(i) + w(i); };
+  auto cc = [&](long i) { return an(i) + w(i + 1); };
+  const double d = 1.0 / (an(t - 1) + an(t + 1));
+  const double ain = 1.0 / an(t), bi = 1.0 / bn(t), ci = 1.0 / cc(t);
+  c[0] = w(t) * ain * (1.0 + 2.0 * d * w(t + 1) * (an(t - 1) * bi - an(t + 1) * ci));
+  c[1] = -d * w(t) * an(t - 1) * bi;
+  c[2] = d * w(t + 1) * an(t + 1) * ci;
+  const double e = w(t) / (an(t - 1) + w(t + 1));
+  c[3] = e * bn(t - 1) * ain;
+  c[4] = e * cc(t) * (1.0 / an(t - 1));
+}
+
+// the FP64 sweeps' slot table (Tab64) from the per-slot geometry kept in c, and the azimuthal
+// grid's paraset when every width is the same.  Enqueues the upload from tab, which the caller
+// keeps until it has synchronised.
+int upload_tab64(pn_ctx* c, const std::vector<double>& radc, const std::vector<double>& cs2,
+                 const std::vector<double>& nu, std::vector<double>& tab) {
+  DevGrid& d = c->dg;
+  const bool d3 = c->P.ndim == 3;
+  const long nslot = static_cast<long>(d.sr) * d.sk, ts = d.tstride, sr = d.sr;
+  const int ne = d3 ? kT64Entries3d : kT64Entries2d;
+  const size_t n1 = static_cast<size_t>(ne) * ts, nt = d3 ? 2 * n1 : n1;
+  tab.resize(nt + 2 * static_cast<size_t>(d.jmax));
+  for (long s = 0; s < nslot; ++s) {
+    const long row = s / sr * sr;
+    double q[kT64Entries3d];
+    const double rad = c->h_xc[s], x = c->h_x[s];
+    q[kT64Rad] = rad;
+    q[kT64Xa] = x;
+    q[kT64Dx] = c->h_dx[s];
+    q[kT64Vol] = c->h_xvol[s];
+    q[kT64Irad] = 1.0 / rad;
+    q[kT64Idx] = 1.0 / c->h_dx[s];
+    q[kT64Ivol] = 1.0 / c->h_xvol[s];
+    q[kT64Star] = -1.0 / rad / rad;
+    q[kT64Fst] = -1.0 / x / x;
+    q[kT64Ixa] = 1.0 / x;
+    q[kT64Rc] = radc[s];
+    q[kT64Irc] = 1.0 / radc[s];
+    // widths past a row's ends repeat its end widths (no kept parabola reads those coefficients)
+    paraset_host([&](long t) { return c->h_dx[std::min(std::max(t, row), row + sr - 1)]; }, s, &q[kT64P0]);
+    q[kT64Nu] = nu[s];
+    q[kT64Cs2] = cs2[s];
+    q[kT64RotC] = 1.0;   // no turn until the first step
+    q[kT64RotS] = 0.0;
+    if (d3) {
+      const double th = c->h_zc[s], za = c->h_z[s], vz = c->h_zvol[s] * rad;
+      q[kT64Pol] = th;
+      q[kT64Vrot] = 0.0;   // until the first step
+      q[kT64Za] = za;
+      q[kT64Dz] = c->h_dz[s];
+      q[kT64Volz] = vz;
+      q[kT64Idz] = 1.0 / c->h_dz[s];
+      q[kT64Ivolz] = 1.0 / vz;
+      q[kT64Sp] = q[kT64Cp] = q[kT64Spl] = q[kT64Cpl] = 0.0;   // fp64_tab_theta
+      const long ir = s % sr, last = d.sk - 1;
+      paraset_host([&](long k) { return c->h_dz[ir + sr * std::min(std::max(k, 0L), last)]; }, s / sr, &q[kT64P0z]);
+    }
+    for (int e = 0; e < ne; ++e) tab[e * ts + s] = q[e];
+  }
+  for (int e = 0; e < ne; ++e)
+    for (long o = nslot; o < ts; ++o) tab[e * ts + o] = tab[e * ts + nslot - 1];
+  if (d3) {   // theta-major: slot s = ir + sr kz goes to kz + sk ir
+    double* z = tab.data() + n1;
+    for (int e = 0; e < ne; ++e) {
+      for (long s = 0; s < nslot; ++s) z[e * ts + s / sr + d.sk * (s % sr)] = tab[e * ts + s];
+      for (long o = nslot; o < ts; ++o) z[e * ts + o] = tab[e * ts + nslot - 1];
+    }
+  }
+  for (int j = 0; j < d.jmax; ++j) {   // the planet's angles, until the first step
+    tab[nt + 2 * j] = 1.0;
+    tab[nt + 2 * j + 1] = 0.0;
+  }
+  PN_HIP(c, hipMemcpyAsync(d.tab, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  d.uniform_phi = 1;
+  for (int j = 1; j < d.jmax; ++j)
+    if (c->h_dy[j] != c->h_dy[0]) d.uniform_phi = 0;
+  paraset_host([&](long) { return c->h_dy[0]; }, 0, d.p0y);
+  return PN_OK;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -287,6 +377,17 @@ int pn_create(const pn_grid* g, const pn_params* p, int precision, pn_ctx** out)
       if (p->ndim == 3) c->ncflp = std::max(c->ncflp, f32_cfl_partials_z(d, v));
     }
   if (r2 == PN_OK) r2 = dalloc(c, &c->cflp, c->ncflp);
+  if (precision == PN_FP64) {
+    // one allocation: the slot table, its theta-major copy (3-D), then the planet's angles
+    const size_t ne = p->ndim == 3 ? kT64Entries3d : kT64Entries2d;
+    d.tstride = (nslot + kT64Overhang + 1) / 2 * 2;
+    const size_t n1 = ne * d.tstride, nt = p->ndim == 3 ? 2 * n1 : n1;
+    if (r2 == PN_OK) r2 = dalloc(c, &d.tab, nt + 2 * static_cast<size_t>(g->jmax));
+    if (r2 == PN_OK) {
+      if (p->ndim == 3) d.tabz = d.tab + n1;
+      d.ptrig = reinterpret_cast<double2*>(d.tab + nt);
+    }
+  }
   if (precision == PN_FP32) {
     float *fdy, *fyvol;
     double *rbg, *vbg;
@@ -460,11 +561,13 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
   c->h_cs2 = scs2;
 
   hipStream_t st = c->stream;
+  std::vector<double> tab64;   // outlives its upload
   const size_t cells = static_cast<size_t>(nslot) * J;
   if (!is_f32(c)) {
     for (int b = 0; b < 2; ++b)
       for (int f = 0; f < kNField; ++f)
         PN_HIP(c, hipMemcpyAsync(d.f[b][f], F[f].data(), cells * sizeof(double), hipMemcpyHostToDevice, st));
+    if ((rc = upload_tab64(c, sradc, scs2, snu, tab64)) != PN_OK) return rc;
   } else {
     const bool d3 = (c->P.ndim == 3);
     const bool adia = (c->P.eos == 3);
@@ -727,6 +830,7 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
   PN_HIP(c, up(d.val, val, nring * sizeof(pn_symdisk)));
   rc = sync(c);
   if (rc != PN_OK) return rc;
+  if (d.tabz) PN_LAUNCH(c, "theta table", fp64_tab_theta(lctx(c)));
   if (lft != c->h_lft.data()) {
     c->h_lft.assign(static_cast<const char*>(lft), static_cast<const char*>(lft) + lr_bytes);
     c->h_rgh.assign(static_cast<const char*>(rgh), static_cast<const char*>(rgh) + lr_bytes);
@@ -883,6 +987,7 @@ int pn_sweep_axis(pn_ctx* c, int axis, double dt, const pn_body* planet, double 
     else if (axis == 1) PN_LAUNCH(c, "sweep_y", f32_sweep_y(L, c->df, c->var_y, c->cur, 0));
     else PN_LAUNCH(c, "sweep_z", f32_sweep_z(L, c->df, c->var_z, c->cur, 0));
   } else {
+    PN_LAUNCH(c, "prep", fp64_prep(L));
     if (axis == 0) PN_LAUNCH(c, "ghosts", launch_fill_ghosts(L, c->cur));
     hipError_t e = (axis == 0) ? fp64_sweep_x(L, c->cur) : (axis == 1) ? fp64_sweep_y(L, c->cur) : fp64_sweep_z(L, c->cur);
     if (e != hipSuccess) return fail(c, PN_ERR_HIP, "sweep %d: %s", axis, hipGetErrorString(e));

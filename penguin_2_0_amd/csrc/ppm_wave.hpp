@@ -110,23 +110,15 @@ __device__ __forceinline__ int cell_of(int K, int h) { return K * (int)(threadId
 template <int SL>
 __device__ __forceinline__ int cell_in(int K, int h) { return K * (int)((threadIdx.x & 63) % SL) + h; }
 
-template <typename T>
-__device__ __forceinline__ T min3(T A, T B, T Cc) {   // simple_func.cu:2-14
-  if (A < B) return (Cc < A) ? Cc : A;
-  return (Cc < B) ? Cc : B;
-}
-
 // the limited slope of parabola.cu:87-96: sign(t1) min(|t1|, 2 |da_l|, 2 |da_r|), zero at an
-// extremum.  FP64 keeps the reference's compare chain (min3) operation for operation; FP32 takes
-// the same minimum with one v_min3 and the sign by copysign (the values are the same: a
-// minimum and a sign change round nothing).
+// extremum: a minimum of magnitudes and the sign by copysign, the values of the reference's
+// compare chain (a minimum and a sign change round nothing, doubling is exact)
 template <typename T>
 __device__ __forceinline__ T limited_slope(T t1, T da_l, T da_r) {
   if constexpr (sizeof(T) == 4) {
     t1 = copysignf(fminf(fminf(fabsf(t1), 2.0f * fabsf(da_l)), 2.0f * fabsf(da_r)), t1);
   } else {
-    if (t1 < T(0.0)) t1 = -min3(-t1, T(2.0) * fabs(da_l), T(2.0) * fabs(da_r));
-    else t1 = min3(t1, T(2.0) * fabs(da_l), T(2.0) * fabs(da_r));
+    t1 = copysign(fmin(fabs(t1), T(2.0) * fmin(fabs(da_l), fabs(da_r))), t1);
   }
   if (da_l * da_r < T(0.0)) t1 = T(0.0);
   return t1;
@@ -136,6 +128,71 @@ __device__ __forceinline__ T max3(T A, T B, T Cc) {   // simple_func.cu:16-28
   if (A > B) return (Cc > A) ? Cc : A;
   return (Cc > B) ? Cc : B;
 }
+
+// ---------------------------------------------------------------------------------------
+// FP64 divisions, roots, exp and log of the windows.  A sweep divides by the same few numbers
+// over and over (a radius three times in a row, a cell's density, the Lagrangian volume), and
+// the compiler's division is 11 instructions each time.  Here a reciprocal is formed once and
+// each quotient by it takes three: q = a y, r = a - q b (exact in an FMA), q + r y, which is the
+// correctly rounded a / b for any y within an ulp of 1 / b (Markstein 1990), so the result
+// keeps the bits of the division.  For finite, normal operands; a zero or non-finite divisor
+// gives NaN where a division gives an infinity.
+
+// 1 / b to an ulp: the hardware estimate (2^-24 or better) and one cubic step
+__device__ __forceinline__ double rcp64(double b) {
+  const double y = __builtin_amdgcn_rcp(b);
+  const double e = __builtin_fma(-b, y, 1.0);
+  return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
+// 1 / b correctly rounded, from y = rcp64(b)
+__device__ __forceinline__ double rcp64_rn(double b) {
+  const double y = rcp64(b);
+  return __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+}
+// a / b correctly rounded, y = 1 / b to an ulp
+__device__ __forceinline__ double div64(double a, double b, double y) {
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-q, b, a), y, q);
+}
+// 1 / sqrt(x), x > 0, to 1.5 ulp
+__device__ __forceinline__ double rsq64(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+}
+// sqrt(x) correctly rounded, x > 0 and normal
+__device__ __forceinline__ double sqrt64_rn(double x) {
+  const double y = rsq64(x);
+  const double g = x * y;
+  return __builtin_fma(__builtin_fma(-g, g, x), 0.5 * y, g);
+}
+// exp(t) for |t| < 1/8: 1 + (t + t^2 / 2 + ... + t^10 / 10!); the one rounding that matters is
+// the last addition's
+__device__ __forceinline__ double exp_small(double t) {
+  double q = __builtin_fma(t, 1.0 / 3628800.0, 1.0 / 362880.0);
+  q = __builtin_fma(t, q, 1.0 / 40320.0);
+  q = __builtin_fma(t, q, 1.0 / 5040.0);
+  q = __builtin_fma(t, q, 1.0 / 720.0);
+  q = __builtin_fma(t, q, 1.0 / 120.0);
+  q = __builtin_fma(t, q, 1.0 / 24.0);
+  q = __builtin_fma(t, q, 1.0 / 6.0);
+  q = __builtin_fma(t, q, 0.5);
+  return 1.0 + __builtin_fma(t * t, q, t);
+}
+// atanh(x) for |x| < 1/8: the odd series to x^17; 2 atanh((a - b) / (a + b)) = log(a / b)
+__device__ __forceinline__ double atanh_small(double x) {
+  const double z = x * x;
+  double q = __builtin_fma(z, 1.0 / 17.0, 1.0 / 15.0);
+  q = __builtin_fma(z, q, 1.0 / 13.0);
+  q = __builtin_fma(z, q, 1.0 / 11.0);
+  q = __builtin_fma(z, q, 1.0 / 9.0);
+  q = __builtin_fma(z, q, 1.0 / 7.0);
+  q = __builtin_fma(z, q, 1.0 / 5.0);
+  q = __builtin_fma(z, q, 1.0 / 3.0);
+  return __builtin_fma(x * z, q, x);
+}
+// true in every lane when the condition holds in any lane of the wavefront (wave-uniform)
+__device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
 
 // ---------------------------------------------------------------------------------------
 // planet + star gravity (forces.cu:4-182).  Without bary: the star at the origin (its -1/r^2
@@ -148,123 +205,107 @@ struct Planet {
   int bary;
 };
 
-template <typename T>
-struct BaryPos {   // stm, plm and the two bodies' distances from the barycentre
-  T stm, plm, plx, stx;
-  __device__ __forceinline__ BaryPos(const Planet& p) {
-    stm = T(1.0) / (T(1.0) + (T)p.m);
-    plm = (T)p.m * stm;
-    plx = (T)p.x * stm;
-    stx = (T)p.x * plm;
+// the planet and star as the force forms take them: plm, plx the planet's mass and distance
+// (about the star: m, x, the spherical forms with the reduced mass m/(1+m); barycentric: m/(1+m)
+// and x/(1+m)), stm, stx the star's mass 1/(1+m) and distance from the barycentre, ix2 = 1/x^2
+// of the indirect term.  Formed once per wavefront.
+struct Grav {
+  double plm, plx, rs2, ix2, stm, stx, iplx, plx2, iplx2;
+  bool bary;
+  __device__ __forceinline__ Grav(const Planet& p, bool sph) {
+    stm = 1.0 / (1.0 + p.m);
+    bary = p.bary != 0;
+    plm = (bary || sph) ? p.m * stm : p.m;
+    plx = bary ? p.x * stm : p.x;
+    stx = p.x * (p.m * stm);
+    ix2 = 1.0 / (p.x * p.x);
+    rs2 = p.rs * p.rs;
+    iplx = rcp64(plx);
+    plx2 = plx * plx;
+    iplx2 = rcp64(plx2);
   }
 };
 
-template <typename T>
-__device__ __forceinline__ T grav_rad_cyl(const Planet& p, T rad, T azi, T z, T dt) {   // forces.cu:112-134
-  T cosfac = cos(azi - ((T)p.y + dt * (T)p.vy));
-  T rs = (T)p.rs;
-  if (p.bary) {
-    const BaryPos<T> b(p);
-    T Rp = sqrt(rad * rad + b.plx * b.plx - T(2.0) * b.plx * rad * cosfac + z * z + rs * rs);
-    T Rs = sqrt(rad * rad + b.stx * b.stx + T(2.0) * b.stx * rad * cosfac + z * z);
-    return -b.plm * (rad - b.plx * cosfac) / (Rp * Rp * Rp) - b.stm * (rad + b.stx * cosfac) / (Rs * Rs * Rs);
-  }
-  T plm = (T)p.m, plx = (T)p.x;
-  T Rp = sqrt(rad * rad + plx * plx - T(2.0) * plx * rad * cosfac + z * z + rs * rs);
-  return -plm * (rad - plx * cosfac) / (Rp * Rp * Rp) - plm * cosfac / (plx * plx);
+// The forces take the angle to the planet as its cosine and sine (and in 3-D the cell's sin and
+// cos theta): a sweep forms those once per column and turns them by small angles, instead of
+// a library cos and sin of every cell at each of three times.  The planet's 1/R^3 comes from a
+// reciprocal root (the cylindrical forms; the spherical ones below round as written).
+__device__ __forceinline__ double cube(double x) { return x * x * x; }
+// a / R^3, R = sqrt(R2), rounded as written: the star's pull, which the disk's rotation nearly
+// cancels, so its last bit is seen
+__device__ __forceinline__ double over_cube(double a, double R2) {
+  const double R = sqrt64_rn(R2), R3 = R * R * R;
+  return div64(a, R3, rcp64(R3));
 }
-template <typename T>
-__device__ __forceinline__ T grav_azi_cyl(const Planet& p, T rad, T azi, T z, T dt) {   // forces.cu:136-159
-  T ph = azi - ((T)p.y + dt * (T)p.vy);
-  T cosfac = cos(ph);
-  T sinfac = sin(ph);
-  T rs = (T)p.rs;
-  if (p.bary) {
-    const BaryPos<T> b(p);
-    T Rp = sqrt(rad * rad + b.plx * b.plx - T(2.0) * b.plx * rad * cosfac + z * z + rs * rs);
-    T Rs = sqrt(rad * rad + b.stx * b.stx + T(2.0) * b.stx * rad * cosfac + z * z);
-    return -b.plm * b.plx * sinfac / (Rp * Rp * Rp) + b.stm * b.stx * sinfac / (Rs * Rs * Rs);
-  }
-  T plm = (T)p.m, plx = (T)p.x;
-  T Rp = sqrt(rad * rad + plx * plx - T(2.0) * plx * rad * cosfac + z * z + rs * rs);
-  return -plm * plx * sinfac / (Rp * Rp * Rp) + plm * sinfac / plx / plx;
+__device__ __forceinline__ double grav_rad_cyl(const Grav& g, double rad, double cosfac) {   // forces.cu:112-134
+  const double ri3 = cube(rsq64(rad * rad + g.plx * g.plx - 2.0 * g.plx * rad * cosfac + g.rs2));
+  const double f = -g.plm * (rad - g.plx * cosfac) * ri3;
+  if (!g.bary) return f - g.plm * cosfac * g.ix2;
+  return f - over_cube(g.stm * (rad + g.stx * cosfac), rad * rad + g.stx * g.stx + 2.0 * g.stx * rad * cosfac);
 }
-template <typename T>
-__device__ __forceinline__ T grav_pol_cyl(const Planet& p, T rad, T azi, T z, T dt) {   // forces.cu:161-182
-  T cosfac = cos(azi - ((T)p.y + dt * (T)p.vy));
-  T rs = (T)p.rs;
-  if (p.bary) {
-    const BaryPos<T> b(p);
-    T Rp = sqrt(rad * rad + b.plx * b.plx - T(2.0) * b.plx * rad * cosfac + z * z + rs * rs);
-    T Rs = sqrt(rad * rad + b.stx * b.stx + T(2.0) * b.stx * rad * cosfac + z * z);
-    return -b.plm * z / (Rp * Rp * Rp) - b.stm * z / (Rs * Rs * Rs);
-  }
-  T plm = (T)p.m, plx = (T)p.x;
-  T Rp = sqrt(rad * rad + plx * plx - T(2.0) * plx * rad * cosfac + z * z + rs * rs);
-  return -plm * z / (Rp * Rp * Rp);
+__device__ __forceinline__ double grav_azi_cyl(const Grav& g, double rad, double cosfac, double sinfac) {   // forces.cu:136-159
+  const double ri3 = cube(rsq64(rad * rad + g.plx * g.plx - 2.0 * g.plx * rad * cosfac + g.rs2));
+  const double f = -g.plm * g.plx * sinfac * ri3;
+  if (!g.bary) return f + g.plm * sinfac * g.ix2;
+  return f + over_cube(g.stm * g.stx * sinfac, rad * rad + g.stx * g.stx + 2.0 * g.stx * rad * cosfac);
 }
-template <typename T>
-__device__ __forceinline__ T grav_rad_sph(const Planet& p, T rad, T azi, T pol, T dt) {   // forces.cu:23-50
-  T cosfac = cos(azi - ((T)p.y + dt * (T)p.vy));
-  T sinpol = sin(pol);
-  T rs = (T)p.rs;
-  if (p.bary) {
-    const BaryPos<T> b(p);
-    T Rp = rad * rad + b.plx * b.plx - T(2.0) * b.plx * rad * cosfac * sinpol;
-    Rp = sqrt(Rp + rs * rs);
-    T Rs = sqrt(rad * rad + b.stx * b.stx + T(2.0) * b.stx * rad * cosfac * sinpol);
-    return -b.plm * (rad - b.plx * cosfac * sinpol) / (Rp * Rp * Rp) -
-           b.stm * (rad + b.stx * cosfac * sinpol) / (Rs * Rs * Rs);
-  }
-  T stm = T(1.0) / (T(1.0) + (T)p.m);
-  T plm = (T)p.m * stm;
-  T plx = (T)p.x;
-  T Rp = rad * rad + plx * plx - T(2.0) * plx * rad * cosfac * sinpol;
-  Rp = sqrt(Rp + rs * rs);
-  return -plm * (rad - plx * cosfac * sinpol) / (Rp * Rp * Rp) - stm / (rad * rad) -
-         plm * sinpol * cosfac / (plx * plx);
+// The spherical forms round every operation as written.  The theta sweep's area factor
+// (cos x0 - cos x) / (x - x0) of an edge that hardly moves turns a last-bit change of x into a
+// relative 1e-9 of the pressure force on v_theta, so a 3-D disk follows the reference's run only
+// as long as its rounding is followed everywhere.  star2 = stm / rad^2, which the caller forms (not
+// used in the barycentric frame).
+__device__ __forceinline__ double grav_rad_sph(const Grav& g, double rad, double cosfac, double sinpol, double star2) {   // forces.cu:23-50
+  const double f = over_cube(-g.plm * (rad - g.plx * cosfac * sinpol),
+                             rad * rad + g.plx * g.plx - 2.0 * g.plx * rad * cosfac * sinpol + g.rs2);
+  if (!g.bary) return f - star2 - div64(g.plm * sinpol * cosfac, g.plx2, g.iplx2);
+  return f - over_cube(g.stm * (rad + g.stx * cosfac * sinpol),
+                       rad * rad + g.stx * g.stx + 2.0 * g.stx * rad * cosfac * sinpol);
 }
-template <typename T>
-__device__ __forceinline__ T grav_azi_sph(const Planet& p, T rad, T azi, T pol, T dt) {   // forces.cu:52-81
-  T ph = azi - ((T)p.y + dt * (T)p.vy);
-  T cosfac = cos(ph);
-  T sinfac = sin(ph);
-  T sinpol = sin(pol);
-  rad /= sinpol;
-  T rs = (T)p.rs;
-  if (p.bary) {
-    const BaryPos<T> b(p);
-    T Rp = rad * rad + b.plx * b.plx - T(2.0) * b.plx * rad * cosfac * sinpol;
-    Rp = sqrt(Rp + rs * rs);
-    T Rs = sqrt(rad * rad + b.stx * b.stx + T(2.0) * b.stx * rad * cosfac * sinpol);
-    return -b.plm * b.plx * sinfac / (Rp * Rp * Rp) + b.stm * b.stx * sinfac / (Rs * Rs * Rs);
-  }
-  T stm = T(1.0) / (T(1.0) + (T)p.m);
-  T plm = (T)p.m * stm;
-  T plx = (T)p.x;
-  T Rp = rad * rad + plx * plx - T(2.0) * plx * rad * cosfac * sinpol;
-  Rp = sqrt(Rp + rs * rs);
-  return -plm * plx * sinfac / (Rp * Rp * Rp) + plm * sinpol * sinfac / plx / plx;
+// rad: the spherical radius
+__device__ __forceinline__ double grav_azi_sph(const Grav& g, double rad, double cosfac, double sinfac, double sinpol) {   // forces.cu:52-81
+  const double f = over_cube(-g.plm * g.plx * sinfac,
+                             rad * rad + g.plx * g.plx - 2.0 * g.plx * rad * cosfac * sinpol + g.rs2);
+  if (!g.bary) return f + div64(div64(g.plm * sinpol * sinfac, g.plx, g.iplx), g.plx, g.iplx);
+  return f + over_cube(g.stm * g.stx * sinfac, rad * rad + g.stx * g.stx + 2.0 * g.stx * rad * cosfac * sinpol);
 }
-template <typename T>
-__device__ __forceinline__ T grav_pol_sph(const Planet& p, T rad, T azi, T pol, T dt) {   // forces.cu:83-110
-  T cosfac = cos(azi - ((T)p.y + dt * (T)p.vy));
-  T cospol = cos(pol);
-  T sinpol = sin(pol);
-  T rs = (T)p.rs;
-  if (p.bary) {
-    const BaryPos<T> b(p);
-    T Rp = rad * rad + b.plx * b.plx - T(2.0) * b.plx * rad * cosfac * sinpol;
-    Rp = sqrt(Rp + rs * rs);
-    T Rs = sqrt(rad * rad + b.stx * b.stx + T(2.0) * b.stx * rad * cosfac * sinpol);
-    return b.plm * b.plx * cosfac * cospol / (Rp * Rp * Rp) - b.stm * b.stx * cosfac * cospol / (Rs * Rs * Rs);
+__device__ __forceinline__ double grav_pol_sph(const Grav& g, double rad, double cosfac, double sinpol, double cospol) {   // forces.cu:83-110
+  const double f = over_cube(g.plm * g.plx * cosfac * cospol,
+                             rad * rad + g.plx * g.plx - 2.0 * g.plx * rad * cosfac * sinpol + g.rs2);
+  if (!g.bary) {
+    const double d = sinpol * g.plx * g.plx;
+    return f - div64(g.plm * cosfac * cospol, d, rcp64(d));
   }
-  T stm = T(1.0) / (T(1.0) + (T)p.m);
-  T plm = (T)p.m * stm;
-  T plx = (T)p.x;
-  T Rp = rad * rad + plx * plx - T(2.0) * plx * rad * cosfac * sinpol;
-  Rp = sqrt(Rp + rs * rs);
-  return plm * plx * cosfac * cospol / (Rp * Rp * Rp) - plm * cosfac * cospol / (sinpol * plx * plx);
+  return f - over_cube(g.stm * g.stx * cosfac * cospol, rad * rad + g.stx * g.stx + 2.0 * g.stx * rad * cosfac * sinpol);
+}
+// sin and cos of e: Taylor series for |e| < 1/2, past it (a coarse ring's shift over a long
+// step) the library functions, in wavefronts that need them
+__device__ __forceinline__ void sincos_small(double e, double& s, double& c) {
+  const double z = e * e;
+  double q = __builtin_fma(z, 1.0 / 6227020800.0, -1.0 / 39916800.0);
+  q = __builtin_fma(z, q, 1.0 / 362880.0);
+  q = __builtin_fma(z, q, -1.0 / 5040.0);
+  q = __builtin_fma(z, q, 1.0 / 120.0);
+  q = __builtin_fma(z, q, -1.0 / 6.0);
+  s = __builtin_fma(e * z, q, e);
+  double w = __builtin_fma(z, -1.0 / 87178291200.0, 1.0 / 479001600.0);
+  w = __builtin_fma(z, w, -1.0 / 3628800.0);
+  w = __builtin_fma(z, w, 1.0 / 40320.0);
+  w = __builtin_fma(z, w, -1.0 / 720.0);
+  w = __builtin_fma(z, w, 1.0 / 24.0);
+  w = __builtin_fma(z, w, -0.5);
+  c = __builtin_fma(z, w, 1.0);
+  const bool big = !(fabs(e) < 0.5);
+  if (wave_any(big)) {
+    double sb, cb;
+    sincos(e, &sb, &cb);
+    s = big ? sb : s;
+    c = big ? cb : c;
+  }
+}
+// cos and sin of (a + b) from those of a and b
+__device__ __forceinline__ void turn(double ca, double sa, double cb, double sb, double& c, double& s) {
+  c = ca * cb - sa * sb;
+  s = sa * cb + ca * sb;
 }
 template <typename T>
 __device__ __forceinline__ T potential(bool planet_on, const Planet& p, T rad, T azi, T z) {   // forces.cu:4-21
@@ -289,6 +330,22 @@ __device__ __forceinline__ T potential(bool planet_on, const Planet& p, T rad, T
 template <int AXIS_, int GX_, int GY_, int GZ_, int EOS_, int VISC_>
 struct Cfg {
   static constexpr int AXIS = AXIS_, GX = GX_, GY = GY_, GZ = GZ_, EOS = EOS_, VISC = VISC_;
+};
+
+// the FP64 slot table's entries of this lane's two cells: one 16-byte load per entry, the
+// entry's address in scalar registers and the lane's byte offset in a vector one
+typedef double f64x2_t __attribute__((ext_vector_type(2), aligned(8)));
+struct TabLane64 {
+  const double* tab;
+  long stride;     // doubles per entry
+  unsigned voff;   // byte offset of the slot of this lane's first cell
+  __device__ __forceinline__ C<double, 2> get(int e) const {
+    const f64x2_t v = *reinterpret_cast<const f64x2_t*>(reinterpret_cast<const char*>(tab + e * stride) + voff);
+    C<double, 2> o;
+    o[0] = v.x;
+    o[1] = v.y;
+    return o;
+  }
 };
 
 // the energy a cell carries into the Lagrangian step from the window's p, rho, u and first
@@ -350,52 +407,104 @@ __device__ __forceinline__ Para<T, K> paraset(int nmin, int nmaxp, const C<T, K>
   return P;
 }
 
+// paraset of the Lagrangian grid, FP64.  Its coefficients multiply differences of neighbouring
+// cells, which enter the edge values far below their last bit, so 2-D sweeps share reciprocals
+// (one estimate for 1/an, 1/bn, 1/cc, one for both sums); with EX every quotient rounds as
+// written.  Coefficients are formed in every cell; those outside the reference's index ranges
+// (parabola.cu:138-176) reach no parabola that a kept cell reads.
+template <int K, bool EX>
+__device__ __forceinline__ Para<double, K> paraset64(const C<double, K>& dx) {
+  Para<double, K> P;
+  C<double, K> dxp = next1(dx);
+  C<double, K> an, ain, bn, bi, cc, ci;
+#pragma unroll
+  for (int h = 0; h < K; ++h) {
+    an[h] = dx[h] + dxp[h];
+    bn[h] = an[h] + dx[h];
+    cc[h] = an[h] + dxp[h];
+    if constexpr (EX) {
+      ain[h] = rcp64_rn(an[h]);
+      bi[h] = rcp64_rn(bn[h]);
+      ci[h] = rcp64_rn(cc[h]);
+    } else {
+      const double ab = an[h] * bn[h];
+      const double t = rcp64(ab * cc[h]), tc = t * cc[h];
+      ain[h] = tc * bn[h];
+      bi[h] = tc * an[h];
+      ci[h] = t * ab;
+    }
+  }
+  C<double, K> anm = prev1(an), anp = next1(an), bnm = prev1(bn), ainm = prev1(ain);
+#pragma unroll
+  for (int h = 0; h < K; ++h) {
+    const double s1 = anm[h] + anp[h], s2 = anm[h] + dxp[h];
+    double e;
+    if constexpr (EX) {
+      const double d = rcp64_rn(s1);
+      P.c0[h] = dx[h] * ain[h] * (1.0 + 2.0 * d * dxp[h] * (anm[h] * bi[h] - anp[h] * ci[h]));
+      P.c1[h] = -d * dx[h] * anm[h] * bi[h];
+      P.c2[h] = d * dxp[h] * anp[h] * ci[h];
+      e = div64(dx[h], s2, rcp64(s2));
+    } else {
+      const double t = rcp64(s1 * s2), d = t * s2;
+      const double wb = d * anm[h] * bi[h], wc = d * anp[h] * ci[h];
+      P.c0[h] = dx[h] * ain[h] * __builtin_fma(2.0 * dxp[h], wb - wc, 1.0);
+      P.c1[h] = -dx[h] * wb;
+      P.c2[h] = dxp[h] * wc;
+      e = dx[h] * (t * s1);
+    }
+    P.c3[h] = e * bnm[h] * ain[h];
+    P.c4[h] = e * cc[h] * ainm[h];
+  }
+  return P;
+}
+
 template <typename T, int K>
 struct Parab {
   C<T, K> al, da, a6;   // left value, jump, curvature; valid on [nmin+2, nmaxp-2)
 };
 
-// parabola (parabola.cu:70-136) on [nmin, nmaxp)
-template <typename T, int K, int SL = 64>
-__device__ __forceinline__ Parab<T, K> parabola(int nmin, int nmaxp, const C<T, K>& flat, const C<T, K>& val,
-                                                const Para<T, K>& P) {
-  C<T, K> vm = prev1(val), vp = next1(val);
-  C<T, K> slope, dar;
+// parabola (parabola.cu:70-136), valid on [nmin+2, nmaxp-2) for coefficients valid on the
+// reference's ranges of [nmin, nmaxp); outside it holds values no kept cell reads.  omf = 1 -
+// flat.  The differences come once per interface (da_l of a cell is da_r of the one before it,
+// the same subtraction); everything else is the reference's, operation for operation.
+template <int K>
+__device__ __forceinline__ Parab<double, K> parabola(const C<double, K>& flat, const C<double, K>& omf,
+                                                     const C<double, K>& val, const Para<double, K>& P) {
+  C<double, K> vp = next1(val);
+  C<double, K> slope, dar;
+#pragma unroll
+  for (int h = 0; h < K; ++h) dar[h] = vp[h] - val[h];
+  C<double, K> dal = prev1(dar);
+#pragma unroll
+  for (int h = 0; h < K; ++h)
+    slope[h] = limited_slope<double>(P.c3[h] * dar[h] + P.c4[h] * dal[h], dal[h], dar[h]);
+  C<double, K> slp = next1(slope);
+  C<double, K> ar;
+#pragma unroll
+  for (int h = 0; h < K; ++h)
+    ar[h] = val[h] + P.c0[h] * dar[h] + P.c1[h] * slp[h] + P.c2[h] * slope[h];
+  C<double, K> alv = prev1(ar);
+  Parab<double, K> o;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    T a = val[h];
-    T da_r = vp[h] - a;
-    T da_l = a - vm[h];
-    slope[h] = limited_slope<T>(P.c3[h] * da_r + P.c4[h] * da_l, da_l, da_r);
-    dar[h] = da_r;
-  }
-  C<T, K> slp = next1(slope);
-  C<T, K> ar;
-#pragma unroll
-  for (int h = 0; h < K; ++h) ar[h] = val[h] + P.c0[h] * dar[h] + P.c1[h] * slp[h] + P.c2[h] * slope[h];
-  C<T, K> alv = prev1(ar);
-  Parab<T, K> o;
-#pragma unroll
-  for (int h = 0; h < K; ++h) {
-    const int c = cell_in<SL>(K, h);
-    T a = val[h];
-    T t1 = flat[h] * a;
-    T t2 = T(1.0) - flat[h];
-    T arr = t1 + t2 * ar[h];
-    T la = t1 + t2 * alv[h];
+    const double a = val[h];
+    double t1 = flat[h] * a;
+    double arr = __builtin_fma(omf[h], ar[h], t1);
+    double la = __builtin_fma(omf[h], alv[h], t1);
     t1 = arr - la;
-    t2 = t1 * t1;
-    t1 = t1 * (T(6.0) * (a - T(0.5) * (arr + la)));
-    if ((arr - a) * (a - la) <= T(0.0)) {
+    const double t2 = t1 * t1;
+    t1 = t1 * (6.0 * (a - 0.5 * (arr + la)));
+    if ((arr - a) * (a - la) <= 0.0) {
       arr = a;
       la = a;
     }
-    if (t2 < t1) la = T(3.0) * a - T(2.0) * arr;
-    if (t2 < -t1) arr = T(3.0) * a - T(2.0) * la;
-    bool in = (c >= nmin + 2 && c < nmaxp - 2);
-    o.da[h] = in ? arr - la : T(0);
-    o.a6[h] = in ? T(6.0) * (a - T(0.5) * (arr + la)) : T(0);
-    o.al[h] = in ? la : T(0);
+    const double a3 = 3.0 * a;
+    if (t2 < t1) la = a3 - 2.0 * arr;
+    if (t2 < -t1) arr = a3 - 2.0 * la;
+    o.da[h] = arr - la;
+    o.a6[h] = 6.0 * (a - 0.5 * (arr + la));
+    o.al[h] = la;
   }
   return o;
 }
@@ -415,86 +524,42 @@ __device__ __forceinline__ void derivs(T xm, T x0, T xp, T um, T u0, T up, T& fi
 }
 
 // Window state and per-cell geometry.
-template <typename T, int K>
+template <int K>
 struct Win {
-  C<T, K> r, p, u, v, w, e;
-  C<T, K> xa0, dx0, dvol0, rad, azi, pol, vrot;
+  C<double, K> r, p, u, v, w, e;
+  C<double, K> xa0, dx0, dvol0, rad;   // left edge, width, volume, radius of the sweep's forces
+  C<double, K> azi;                    // azimuth of the cell centre
+  C<double, K> ca, sa;                 // cos, sin of its angle from the planet before the step
 };
 
-// interface / centre force of one axis (forces.cu:185-372)
-template <typename T, class CF>
-__device__ __forceinline__ T force_x(const RunFlags& rf, const Planet& pl, bool bound, T dt, T rad, T azi, T pol,
-                                     T vc, T vm, T wc, T wm) {
-  T grav, ftot;
-  if constexpr (CF::GX == 1) {
-    if (rf.planet) {
-      grav = grav_rad_cyl<T>(pl, rad, azi, pol, dt);
-      if (!pl.bary) grav += T(-1.0) / rad / rad;
-    } else {
-      T dis = sqrt(rad * rad + pol * pol);
-      grav = -rad / dis / dis / dis;
-    }
-    ftot = grav;
-    if (bound) {
-      T l = T(0.5) * (vc + vm);
-      ftot += l * l / rad / rad / rad;
-    } else {
-      ftot += vc * vc / rad / rad / rad;
-    }
-  } else if constexpr (CF::GX == 2) {
-    grav = rf.planet ? grav_rad_sph<T>(pl, rad, azi, pol, dt) : T(-1.0) / rad / rad;
-    ftot = grav;
-    T sp = rad * sin(pol);
-    if (bound) {
-      T lw = T(0.5) * (wc + wm);
-      T lv = T(0.5) * (vc + vm);
-      ftot += lw * lw / rad / rad / rad;
-      ftot += lv * lv / rad / (sp * sp);
-    } else {
-      ftot += wc * wc / rad / rad / rad;
-      ftot += vc * vc / rad / (sp * sp);
-    }
-  } else {
-    ftot = T(0.0);
-  }
-  return ftot;
-}
+// What a sweep reads beside the window: tx (radial and theta sweeps, the slot table at this
+// lane's cells) or the ring's numbers (azimuthal sweep: vrot, 1 / rad rounded, sin theta, theta,
+// the spherical radius, and p0, the uniform grid's interpolation coefficients, null on a grid that is not uniform)
+struct Ring64 {
+  double vrot, irad, sinpol, pol, rsph;
+  const double* p0;
+};
 
-template <typename T, class CF>
-__device__ __forceinline__ T force_y(const RunFlags& rf, const Planet& pl, T dt, T rad, T azi, T pol) {
-  if constexpr (CF::GY == 3) return rf.planet ? grav_azi_cyl<T>(pl, rad, azi, pol, dt) : T(0.0);
-  else if constexpr (CF::GY == 4) return rf.planet ? grav_azi_sph<T>(pl, rad, azi, pol, dt) : T(0.0);
-  else return T(0.0);
-}
-
-template <typename T, class CF>
-__device__ __forceinline__ T force_z(const RunFlags& rf, const Planet& pl, bool bound, T dt, T rad, T azi, T pol,
-                                     T wc, T wm) {
-  if constexpr (CF::GZ == 0) {
-    if (rf.planet) return grav_pol_cyl<T>(pl, rad, azi, pol, dt);
-    T dis = sqrt(rad * rad + pol * pol);
-    return -pol / dis / dis / dis;
-  } else if constexpr (CF::GZ == 5) {
-    T grav = rf.planet ? grav_pol_sph<T>(pl, rad, azi, pol, dt) : T(0.0);
-    T rc = rad * sin(pol);
-    T l = bound ? T(0.5) * (wc + wm) : wc;
-    return grav + (l * l * cos(pol)) / rc / rc / rc;
-  } else {
-    return T(0.0);
-  }
-}
-
-// One PPMLR update of the window (ppmlr.cu:2-56).  nmax = window length.  On return the
-// cells [6, nmax-6) hold the updated r, u, v, w (and p for EOS 1, 2).
-template <typename T, int K, class CF>
-__device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot, const Planet& pl,
-                                           const RunFlags& rf, T gam) {
+// One PPMLR update of the window (ppmlr.cu:2-56).  c0 = this lane's first cell, nmax = window
+// length, drift = vrot - v_y (azimuthal sweep).  On return the cells [6, nmax-6) hold the
+// updated r, u, v, w (and p for EOS 1, 2).  What is kept of the reference's arithmetic bit for
+// bit and what is not: in 3-D everything.  In 2-D every value that a stored field is built from
+// rounds as the reference's does; the planet's pull, the logarithm and exponential of the
+// interface and the Lagrangian interpolation coefficients carry an ulp of their own.
+template <int K, class CF>
+__device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const Ring64& ring, int c0, int nmax,
+                                           double dt, double FrRot, const Planet& pl, const RunFlags& rf, double gam) {
+  using T = double;
   constexpr int AX = CF::AXIS;
   const T hdt = T(0.5) * dt;
   const T smallp = T(1.0e-15), smallr = T(1.0e-15);
   const T fourthd = T(1.3333333333333333333333333);
   const T third = T(0.3333333333333333333333333);
   const T gamm = gam - T(1.0);
+  constexpr bool EX = CF::GX == 2;   // 3-D: every operation rounds as the reference's
+  const Grav G(pl, CF::GX == 2);
+  // 3-D: cos and sin of the angle to the planet a time t into the step (forces.cu:25, 55-57)
+  auto angle = [&](T azi, T vrot, T t) { return azi + t * vrot - (pl.y + t * pl.vy); };
 
   // ---- flatten (flatten.cu:7-40)
   C<T, K> flat = splat<T, K>(T(0));
@@ -504,14 +569,14 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     C<T, K> steep;
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_of(K, h);
+      const int c = c0 + h;
       T s = T(0.0);
       if (c >= 2 && c < nmax - 2) {
         T dp1 = pp1[h] - pm1[h];
         T dp2 = pp2[h] - pm2[h];
         if (fabs(dp2) < smallp) dp2 = smallp;
-        T ddp = fabs(dp1) / fmin(pp1[h], pm1[h]);
-        bool shock = ddp > T(0.33);
+        const T lo = fmin(pp1[h], pm1[h]);
+        bool shock = div64(fabs(dp1), lo, rcp64(lo)) > T(0.33);
         if (um1[h] < up1[h]) shock = false;
         if (shock) s = fmax(T(0.0), (dp1 / dp2 - T(0.75)) * T(5.0));
       }
@@ -520,54 +585,132 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     C<T, K> sm = prev1(steep), sp = next1(steep);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_of(K, h);
+      const int c = c0 + h;
       flat[h] = (c >= 2 && c < nmax - 2) ? fmin(T(0.5), max3(sm[h], steep[h], sp[h])) : T(0.0);
     }
   }
 
   // ---- states (states.cu:3-73)
-  Para<T, K> P0 = paraset(0, nmax, W.dx0);
-  C<T, K> ftot_s;
-  {
-    C<T, K> vm = prev1(W.v);
-    C<T, K> wm;
-    if constexpr (CF::GX == 2 || CF::GZ == 5) wm = prev1(W.w);
+  Para<T, K> P0;
+  C<T, K> irad, idx, idvol;   // rounded reciprocals
+  C<T, K> hc, hs, vrot;       // the turn of the angle to the planet in half a step; 3-D: vrot
+  if constexpr (AX == 1) {
+    if (ring.p0) {
+      P0.c0 = splat<T, K>(ring.p0[0]);
+      P0.c1 = splat<T, K>(ring.p0[1]);
+      P0.c2 = splat<T, K>(ring.p0[2]);
+      P0.c3 = splat<T, K>(ring.p0[3]);
+      P0.c4 = splat<T, K>(ring.p0[4]);
+    } else {
+      P0 = paraset<T, K>(0, nmax, W.dx0);
+    }
+    irad = splat<T, K>(ring.irad);
+#pragma unroll
+    for (int h = 0; h < K; ++h) {
+      idx[h] = rcp64_rn(W.dx0[h]);
+      idvol[h] = rcp64_rn(W.dvol0[h]);
+    }
+  } else {
+    constexpr int b = AX == 0 ? kT64P0 : kT64P0z;
+    P0.c0 = tx.get(b);
+    P0.c1 = tx.get(b + 1);
+    P0.c2 = tx.get(b + 2);
+    P0.c3 = tx.get(b + 3);
+    P0.c4 = tx.get(b + 4);
+    irad = tx.get(kT64Irad);
+    idx = tx.get(AX == 0 ? kT64Idx : kT64Idz);
+    if constexpr (EX) {
+      vrot = tx.get(kT64Vrot);
+    } else if (rf.planet) {
+      hc = tx.get(kT64RotC);
+      hs = tx.get(kT64RotS);
+    }
+  }
+  // half a step of the force at the left edge (forces.cu:185-372).  Star and centrifugal force
+  // nearly cancel, and their sum moves the interface through u*, so both round as written
+  C<T, K> fh;
+  if constexpr (AX == 0) {
+    C<T, K> vm = prev1(W.v), wm, spol;
+    const C<T, K> fst = tx.get(kT64Fst), ixa = tx.get(kT64Ixa);   // -1/x/x, 1/x
+    if constexpr (CF::GX == 2) {
+      wm = prev1(W.w);
+      spol = tx.get(kT64Sp);
+    }
+#pragma unroll
+    for (int h = 0; h < K; ++h) {
+      const T lv = T(0.5) * (W.v[h] + vm[h]);
+      const T x = W.xa0[h], y = ixa[h];
+      T f = fst[h], c = T(0), s;
+      if constexpr (CF::GX == 1) {
+        if (rf.planet) turn(W.ca[h], W.sa[h], hc[h], hs[h], c, s);
+        if (rf.planet) f = grav_rad_cyl(G, x, c) + (G.bary ? T(0) : f);
+        f += div64(div64(div64(lv * lv, x, y), x, y), x, y);
+      } else {
+        const T lw = T(0.5) * (W.w[h] + wm[h]);
+        const T x2 = x * x, sp = x * spol[h], sp2 = sp * sp;
+        if (rf.planet) c = cos(angle(W.azi[h], vrot[h], hdt));
+        if (rf.planet) f = grav_rad_sph(G, x, c, spol[h], div64(G.stm, x2, rcp64(x2)));
+        f += div64(div64(div64(lw * lw, x, y), x, y), x, y);
+        f += div64(div64(lv * lv, x, y), sp2, rcp64(sp2));
+      }
+      fh[h] = hdt * f;
+    }
+  } else if constexpr (AX == 1) {
+    const T drift = ring.vrot - pl.vy;
+    T c1 = T(1), s1 = T(0);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       T f = T(0);
-      if constexpr (AX == 0) {
-        T wmh = (CF::GX == 2) ? wm[h] : T(0);
-        f = force_x<T, CF>(rf, pl, true, hdt, W.xa0[h], W.azi[h] + hdt * W.vrot[h], W.pol[h], W.v[h], vm[h], W.w[h],
-                           wmh);
-      } else if constexpr (AX == 1) {
-        f = force_y<T, CF>(rf, pl, hdt, W.rad[h], W.xa0[h] + hdt * W.vrot[h], W.pol[h]);
-      } else {
-        T wmh = (CF::GZ == 5) ? wm[h] : T(0);
-        f = force_z<T, CF>(rf, pl, true, hdt, W.rad[h], W.azi[h] + hdt * W.vrot[h], W.xa0[h], W.w[h], wmh);
+      if (rf.planet) {
+        if constexpr (EX) {
+          const T ph = angle(W.xa0[h], ring.vrot, hdt);
+          f = grav_azi_sph(G, ring.rsph, cos(ph), sin(ph), ring.sinpol);
+        } else {
+          // from the cell's left edge; on a uniform grid the same turn in every cell
+          if (h == 0 || !ring.p0) sincos_small(hdt * drift - T(0.5) * W.dx0[h], s1, c1);
+          T c, s;
+          turn(W.ca[h], W.sa[h], c1, s1, c, s);
+          f = grav_azi_cyl(G, W.rad[h], c, s);
+        }
       }
-      ftot_s[h] = f;
+      fh[h] = hdt * f;
+    }
+  } else {
+    C<T, K> wm = prev1(W.w);
+    const C<T, K> spl = tx.get(kT64Spl), cpl = tx.get(kT64Cpl);
+#pragma unroll
+    for (int h = 0; h < K; ++h) {
+      const T l = T(0.5) * (W.w[h] + wm[h]);
+      const T rc = W.rad[h] * spl[h], y = rcp64(rc);
+      T f = T(0);
+      if (rf.planet) f = grav_pol_sph(G, W.rad[h], cos(angle(W.azi[h], vrot[h], hdt)), spl[h], cpl[h]);
+      f += div64(div64(div64(l * l * cpl[h], rc, y), rc, y), rc, y);
+      fh[h] = hdt * f;
     }
   }
-  C<T, K> cs, csfac;
+  C<T, K> cs, csfac, omf;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    T s = hdt * sqrt(gam * W.p[h] / W.r[h]) / W.dx0[h];
-    if constexpr (AX == 1) s /= W.rad[h];
-    if constexpr (AX == 2 && CF::GZ == 5) s /= W.rad[h];
+    const T c2 = div64(gam * W.p[h], W.r[h], rcp64(W.r[h]));
+    T s = div64(hdt * sqrt64_rn(c2), W.dx0[h], idx[h]);
+    if constexpr (AX == 1 || (AX == 2 && CF::GZ == 5)) s = div64(s, W.rad[h], irad[h]);
     cs[h] = s;
     csfac[h] = T(1.0) - fourthd * s;
+    omf[h] = T(1.0) - flat[h];
   }
-  // left state at interface c = right-edge average of cell c-1; right state = left-edge
-  // average of cell c (states.cu:45-68)
-  C<T, K> Spl, Spr, Srl, Srr, Sul, Sur;
-  {
-    Parab<T, K> q = parabola(0, nmax, flat, W.p, P0);
-    C<T, K> re, le;
+  auto traced = [&](const Parab<T, K>& q, C<T, K>& re, C<T, K>& le) {
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       re[h] = q.al[h] + q.da[h] - cs[h] * (q.da[h] - csfac[h] * q.a6[h]);
       le[h] = q.al[h] + cs[h] * (q.da[h] + csfac[h] * q.a6[h]);
     }
+  };
+  // left state at interface c = right-edge average of cell c-1; right state = left-edge
+  // average of cell c (states.cu:45-68)
+  C<T, K> Spl, Spr, Srl, Srr, Sul, Sur;
+  {
+    C<T, K> re, le;
+    traced(parabola(flat, omf, W.p, P0), re, le);
     C<T, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -576,13 +719,8 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     }
   }
   {
-    Parab<T, K> q = parabola(0, nmax, flat, W.r, P0);
     C<T, K> re, le;
-#pragma unroll
-    for (int h = 0; h < K; ++h) {
-      re[h] = q.al[h] + q.da[h] - cs[h] * (q.da[h] - csfac[h] * q.a6[h]);
-      le[h] = q.al[h] + cs[h] * (q.da[h] + csfac[h] * q.a6[h]);
-    }
+    traced(parabola(flat, omf, W.r, P0), re, le);
     C<T, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -591,18 +729,13 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     }
   }
   {
-    Parab<T, K> q = parabola(0, nmax, flat, W.u, P0);
     C<T, K> re, le;
-#pragma unroll
-    for (int h = 0; h < K; ++h) {
-      re[h] = q.al[h] + q.da[h] - cs[h] * (q.da[h] - csfac[h] * q.a6[h]);
-      le[h] = q.al[h] + cs[h] * (q.da[h] + csfac[h] * q.a6[h]);
-    }
+    traced(parabola(flat, omf, W.u, P0), re, le);
     C<T, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      Sul[h] = rem[h] + hdt * ftot_s[h];
-      Sur[h] = le[h] + hdt * ftot_s[h];
+      Sul[h] = rem[h] + fh[h];
+      Sur[h] = le[h] + fh[h];
     }
   }
 
@@ -613,10 +746,32 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     T pl_ = Spl[h], rl = Srl[h], ul = Sul[h], pr = Spr[h], rr = Srr[h], ur = Sur[h];
     T um, pm;
     if constexpr (CF::EOS == 0) {
-      T t1 = T(0.5) * (sqrt(pl_ / rl) + sqrt(pr / rr));
-      T t2 = T(-0.5) * (ur - ul) / t1;
-      pm = sqrt(pl_ * pr) * exp(t2);
-      um = ul - t1 * log(pm / pl_);
+      // t1 = (sqrt(pl/rl) + sqrt(pr/rr))/2, t2 = -(ur-ul)/(2 t1), p* = sqrt(pl pr) exp(t2),
+      // u* = ul - t1 log(p*/pl).  t1 scales small differences, so its roots are taken as
+      // pl rsq(pl rl); p* and the ratio under the logarithm keep the roundings of the closed form.
+      // Jumps past the series (a Mach or pressure jump of 1/8 between two cells) take the library
+      // functions, in wavefronts that hold one in a cell whose interface is used.
+      if constexpr (EX) {
+        const T t1 = T(0.5) * (sqrt64_rn(div64(pl_, rl, rcp64(rl))) + sqrt64_rn(div64(pr, rr, rcp64(rr))));
+        const T t2 = div64(T(-0.5) * (ur - ul), t1, rcp64(t1));
+        pm = sqrt64_rn(pl_ * pr) * exp(t2);
+        um = ul - t1 * log(div64(pm, pl_, rcp64(pl_)));
+      } else {
+        const T t1 = T(0.5) * __builtin_fma(pl_, rsq64(pl_ * rl), pr * rsq64(pr * rr));
+        const T t2 = T(-0.5) * (ur - ul) * rcp64(t1);
+        pm = sqrt64_rn(pl_ * pr) * exp_small(t2);
+        const T ratio = div64(pm, pl_, rcp64(pl_));
+        const T x = (ratio - T(1.0)) * rcp64(ratio + T(1.0));   // log(ratio) = 2 atanh(x)
+        um = ul - t1 * (T(2.0) * atanh_small(x));
+        const int c = c0 + h;
+        const bool big = c >= 3 && c < nmax - 2 && !(fabs(t2) < 0.125 && fabs(x) < 0.125);
+        if (wave_any(big)) {
+          const T pb = sqrt(pl_ * pr) * exp(t2);
+          const T ub = ul - t1 * log(pb / pl_);
+          pm = big ? pb : pm;
+          um = big ? ub : um;
+        }
+      }
     } else if constexpr (CF::EOS == 2 || CF::EOS == 3) {
       const T gamfac2 = gam + T(1.0), gamz = gamm / gam / T(2.0);
       T cs_l = sqrt(gam * pl_ / rl);
@@ -667,18 +822,18 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
   C<T, K> dtdm, vf, xa, dxl, dvol;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_of(K, h);
+    const int c = c0 + h;
     T delx;
     if constexpr (AX == 0) {
       delx = dt * umid[h];
     } else if constexpr (AX == 1) {
-      if constexpr (CF::GY > 2) delx = dt * (umid[h] / W.rad[h] - W.vrot[h] - FrRot);
+      if constexpr (CF::GY > 2) delx = dt * (div64(umid[h], W.rad[h], irad[h]) - ring.vrot - FrRot);
       else delx = dt * umid[h];
     } else {
-      if constexpr (CF::GZ == 5) delx = dt * umid[h] / W.rad[h];
-      else delx = dt * umid[h];
+      delx = div64(dt * umid[h], W.rad[h], irad[h]);
     }
-    dtdm[h] = dt / (W.r[h] * W.dvol0[h]);
+    const T m = W.r[h] * W.dvol0[h];
+    dtdm[h] = div64(dt, m, rcp64(m));
     bool in = (c >= 3 && c < nmax - 2);
     vf[h] = in ? W.xa0[h] + delx : W.xa0[h] + T(0.5) * W.dx0[h];
   }
@@ -686,29 +841,87 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     C<T, K> vfp = next1(vf);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_of(K, h);
+      const int c = c0 + h;
       bool in = (c >= 3 && c < nmax - 3);
       dxl[h] = in ? vfp[h] - vf[h] : W.dx0[h];
       xa[h] = in ? vf[h] : W.xa0[h];
     }
   }
   C<T, K> fto1, fto2, xcl;
+  C<T, K> spol, cpol, star, irc, rcyl;
+  if constexpr (AX == 0) star = tx.get(kT64Star);
+  if constexpr (AX == 0 && CF::GX == 2) spol = tx.get(kT64Sp);
+  if constexpr (AX == 2) {
+    spol = tx.get(kT64Sp);
+    cpol = tx.get(kT64Cp);
+    rcyl = tx.get(kT64Rc);
+    irc = tx.get(kT64Irc);
+  }
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    T xc_ = xa[h] + T(0.5) * dxl[h];
+    const T xc_ = xa[h] + T(0.5) * dxl[h];
     xcl[h] = xc_;
+    T f1 = T(0), f2 = T(0);
     if constexpr (AX == 0) {
-      fto1[h] = force_x<T, CF>(rf, pl, false, T(0.0), W.rad[h], W.azi[h], W.pol[h], W.v[h], T(0), W.w[h], T(0));
-      fto2[h] = force_x<T, CF>(rf, pl, false, dt, xc_, W.azi[h] + dt * W.vrot[h], W.pol[h], W.v[h], T(0), W.w[h], T(0));
+      // at the cell centre before and at the moved centre after the step (forces.cu:185-232)
+      const T rad = W.rad[h], y2 = rcp64_rn(xc_);
+      f1 = star[h];                    // -1 / rad / rad
+      f2 = -div64(y2, xc_, y2);
+      T c2 = T(0), s2;
+      if constexpr (CF::GX == 1) {
+        if (rf.planet) {
+          turn(W.ca[h], W.sa[h], T(1.0) - T(2.0) * hs[h] * hs[h], T(2.0) * hs[h] * hc[h], c2, s2);
+          f1 = grav_rad_cyl(G, rad, W.ca[h]) + (G.bary ? T(0) : f1);
+          f2 = grav_rad_cyl(G, xc_, c2) + (G.bary ? T(0) : f2);
+        }
+        const T l2 = W.v[h] * W.v[h];
+        f1 += div64(div64(div64(l2, rad, irad[h]), rad, irad[h]), rad, irad[h]);
+        f2 += div64(div64(div64(l2, xc_, y2), xc_, y2), xc_, y2);
+      } else {
+        if (rf.planet) {
+          const T a = rad * rad, b = xc_ * xc_;
+          c2 = cos(angle(W.azi[h], vrot[h], dt));
+          f1 = grav_rad_sph(G, rad, cos(angle(W.azi[h], T(0), T(0))), spol[h], div64(G.stm, a, rcp64(a)));
+          f2 = grav_rad_sph(G, xc_, c2, spol[h], div64(G.stm, b, rcp64(b)));
+        }
+        const T w2 = W.w[h] * W.w[h], v2 = W.v[h] * W.v[h];
+        const T p1 = rad * spol[h], p2 = xc_ * spol[h], q1 = p1 * p1, q2 = p2 * p2;
+        f1 += div64(div64(div64(w2, rad, irad[h]), rad, irad[h]), rad, irad[h]);
+        f1 += div64(div64(v2, rad, irad[h]), q1, rcp64(q1));
+        f2 += div64(div64(div64(w2, xc_, y2), xc_, y2), xc_, y2);
+        f2 += div64(div64(v2, xc_, y2), q2, rcp64(q2));
+      }
     } else if constexpr (AX == 1) {
-      fto1[h] = force_y<T, CF>(rf, pl, T(0.0), W.rad[h], W.azi[h], W.pol[h]);
-      fto2[h] = force_y<T, CF>(rf, pl, dt, W.rad[h], xc_ + dt * W.vrot[h], W.pol[h]);
+      if (rf.planet) {
+        if constexpr (EX) {
+          const T p1 = angle(W.azi[h], T(0), T(0)), p2 = angle(xc_, ring.vrot, dt);
+          f1 = grav_azi_sph(G, ring.rsph, cos(p1), sin(p1), ring.sinpol);
+          f2 = grav_azi_sph(G, ring.rsph, cos(p2), sin(p2), ring.sinpol);
+        } else {
+          T c, s, ce, se;
+          sincos_small((xc_ - W.azi[h]) + dt * (ring.vrot - pl.vy), se, ce);
+          turn(W.ca[h], W.sa[h], ce, se, c, s);
+          f1 = grav_azi_cyl(G, W.rad[h], W.ca[h], W.sa[h]);
+          f2 = grav_azi_cyl(G, W.rad[h], c, s);
+        }
+      }
     } else {
-      fto1[h] = force_z<T, CF>(rf, pl, false, T(0.0), W.rad[h], W.azi[h], W.pol[h], W.w[h], T(0));
-      fto2[h] = force_z<T, CF>(rf, pl, false, dt, W.rad[h], W.azi[h] + dt * W.vrot[h], xc_, W.w[h], T(0));
+      const T l2 = W.w[h] * W.w[h];
+      T sx, cx;
+      sincos(xc_, &sx, &cx);
+      const T rc2 = W.rad[h] * sx, y2 = rcp64(rc2);
+      if (rf.planet) {
+        f1 = grav_pol_sph(G, W.rad[h], cos(angle(W.azi[h], T(0), T(0))), spol[h], cpol[h]);
+        f2 = grav_pol_sph(G, W.rad[h], cos(angle(W.azi[h], vrot[h], dt)), sx, cx);
+      }
+      f1 += div64(div64(div64(l2 * cpol[h], rcyl[h], irc[h]), rcyl[h], irc[h]), rcyl[h], irc[h]);
+      f2 += div64(div64(div64(l2 * cx, rc2, y2), rc2, y2), rc2, y2);
     }
+    fto1[h] = f1;
+    fto2[h] = f2;
   }
-  C<T, K> umidp;
+  C<T, K> umidp, cxa, cx0;   // theta: cos of the moved and of the unmoved left edge
+  if constexpr (AX == 2) cx0 = tx.get(kT64Cpl);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     const T x_ = xa[h], x0 = W.xa0[h], d_ = dxl[h];
@@ -722,13 +935,10 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
       if constexpr (CF::GY == 0) { dv = d_; vv = T(1.0); }
       else { dv = d_ * W.rad[h]; vv = T(1.0); }
     } else {
-      if constexpr (CF::GZ == 0) { dv = d_; vv = T(1.0); }
-      else {
-        T delx = x_ - x0;
-        T dum = cos(x_);
-        dv = (dum - cos(x_ + d_)) * W.rad[h];
-        vv = (delx == T(0.0)) ? sin(x_) : (cos(x0) - dum) / delx;
-      }
+      const T delx = x_ - x0;
+      cxa[h] = cos(x_);
+      dv = (cxa[h] - cos(x_ + d_)) * W.rad[h];
+      vv = (delx == T(0.0)) ? sin(x_) : (cx0[h] - cxa[h]) / delx;
     }
     dvol[h] = dv;
     vf[h] = vv;   // area factor at the left face
@@ -738,22 +948,24 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     C<T, K> pmp = next1(pmid), vfp = next1(vf), ump = next1(umidp);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_of(K, h);
+      const int c = c0 + h;
       bool in = (c >= 3 && c < nmax - 3);
       T qh = T(0);
       if constexpr (CF::EOS == 0) qh = W.p[h] / W.r[h];
       else if constexpr (CF::EOS == 1) qh = W.p[h] / pow(W.r[h], gam);
-      T rn = fmax(W.r[h] * (W.dvol0[h] / dvol[h]), smallr);
+      T rn = fmax(W.r[h] * div64(W.dvol0[h], dvol[h], rcp64(dvol[h])), smallr);
       T delx = T(0.5) * dt * (fto1[h] + fto2[h]);
       delx += -dtdm[h] * (pmp[h] - pmid[h]) * T(0.5) * (vfp[h] + vf[h]);
       T un = W.u[h] + delx;
       if constexpr (CF::EOS == 2) {
         T ef = W.e[h] - dtdm[h] * (vfp[h] * ump[h] - vf[h] * umidp[h]);
         T x_ = xcl[h];
+        T pol = T(0);   // theta of the cell in 3-D (the 2-D table does not hold it)
+        if constexpr (AX == 0 && CF::GX == 2) pol = tx.get(kT64Pol)[h];
         if constexpr (AX == 0)
-          qh = ef - T(0.5) * ((un * un) + (W.v[h] * W.v[h] / x_ / x_)) - potential<T>(rf.planet, pl, x_, W.azi[h], W.pol[h]);
+          qh = ef - T(0.5) * ((un * un) + (W.v[h] * W.v[h] / x_ / x_)) - potential<T>(rf.planet, pl, x_, W.azi[h], pol);
         else if constexpr (AX == 1)
-          qh = ef - T(0.5) * (un * un) - potential<T>(rf.planet, pl, W.rad[h], x_, W.pol[h]);
+          qh = ef - T(0.5) * (un * un) - potential<T>(rf.planet, pl, W.rad[h], x_, ring.pol);
         else
           qh = ef - T(0.5) * (un * un) - potential<T>(rf.planet, pl, W.rad[h], W.azi[h], x_);
         qh = fmax(gamm * qh, smallp);
@@ -774,8 +986,10 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
   }
 
   // ---- remap (remap.cu:14-226)
-  Para<T, K> P1 = paraset(3, nmax - 3, dxl);
-  C<T, K> dxf, dxf2, fr, delC;
+  if constexpr (AX != 1) idvol = tx.get(AX == 0 ? kT64Ivol : kT64Ivolz);
+  Para<T, K> P1 = paraset64<K, EX>(dxl);
+  C<T, K> dxf, dxf2, fr;
+  C<bool, K> delC;
   C<T, K> dxm = prev1(dxl);
   C<T, K> lvol;
 #pragma unroll
@@ -790,33 +1004,36 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
       if constexpr (CF::GY == 0) lv = x_ - x0;
       else lv = (x_ - x0) * W.rad[h];
     } else {
-      if constexpr (CF::GZ == 0) lv = x_ - x0;
-      else lv = (cos(x0) - cos(x_)) * W.rad[h];
+      lv = (cx0[h] - cxa[h]) * W.rad[h];
     }
     lvol[h] = lv;
-    T d = x_ - x0;
-    delC[h] = (d >= T(0.0)) ? T(1) : T(0);
-    if (d >= T(0.0)) {
-      d = T(0.5) * d / dxm[h];
-      dxf2[h] = T(1.0) - fourthd * d;
-    } else {
-      d = T(0.5) * d / dxl[h];
-      dxf2[h] = T(1.0) + fourthd * d;
-    }
-    dxf[h] = d;
+    const T d = x_ - x0;
+    delC[h] = d >= T(0.0);
+    // 1 - (4/3) d' for a face moving up, 1 + (4/3) d' for one moving down, d' < 0
+    const T den = d >= T(0.0) ? dxm[h] : dxl[h];
+    const T e = EX ? div64(T(0.5) * d, den, rcp64(den)) : T(0.5) * d * rcp64(den);
+    dxf[h] = e;
+    dxf2[h] = T(1.0) - fourthd * fabs(e);
   }
   // face average of a parabola swept through the face (remap.cu:59-90, get_flux :1-10)
   auto face = [&](const Parab<T, K>& Q, C<T, K>& out) {
     C<T, K> alm = prev1(Q.al), dam = prev1(Q.da), a6m = prev1(Q.a6);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      if (delC[h] != T(0)) out[h] = alm[h] + dam[h] - dxf[h] * (dam[h] - dxf2[h] * a6m[h]);
-      else out[h] = Q.al[h] - dxf[h] * (Q.da[h] + dxf2[h] * Q.a6[h]);
+      T up, dn;
+      if constexpr (EX) {
+        up = alm[h] + dam[h] - dxf[h] * (dam[h] - dxf2[h] * a6m[h]);
+        dn = Q.al[h] - dxf[h] * (Q.da[h] + dxf2[h] * Q.a6[h]);
+      } else {
+        up = __builtin_fma(-dxf[h], __builtin_fma(-dxf2[h], a6m[h], dam[h]), alm[h] + dam[h]);
+        dn = __builtin_fma(-dxf[h], __builtin_fma(dxf2[h], Q.a6[h], Q.da[h]), Q.al[h]);
+      }
+      out[h] = delC[h] ? up : dn;
     }
   };
   C<T, K> mass, invm;
   {
-    Parab<T, K> Q = parabola(3, nmax - 3, flat, W.r, P1);
+    Parab<T, K> Q = parabola(flat, omf, W.r, P1);
     C<T, K> fv;
     face(Q, fv);
 #pragma unroll
@@ -824,16 +1041,16 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     C<T, K> frp = next1(fr);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_of(K, h);
+      const int c = c0 + h;
       T m = W.r[h] * dvol[h];
-      T rn = fmax(smallr, (m + fr[h] - frp[h]) / W.dvol0[h]);
+      T rn = fmax(smallr, div64(m + fr[h] - frp[h], W.dvol0[h], idvol[h]));
       mass[h] = m;
-      invm[h] = T(1.0) / (rn * W.dvol0[h]);
+      invm[h] = rcp64_rn(rn * W.dvol0[h]);
       if (c >= 6 && c < nmax - 6) W.r[h] = rn;
     }
   }
   auto remap_field = [&](C<T, K>& X) {
-    Parab<T, K> Q = parabola(3, nmax - 3, flat, X, P1);
+    Parab<T, K> Q = parabola(flat, omf, X, P1);
     C<T, K> fl;
     face(Q, fl);
 #pragma unroll
@@ -841,7 +1058,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     C<T, K> flp = next1(fl);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_of(K, h);
+      const int c = c0 + h;
       if (c >= 6 && c < nmax - 6) X[h] = (X[h] * mass[h] + (fl[h] - flp[h])) * invm[h];
     }
   };
@@ -852,7 +1069,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
     remap_field(q);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_of(K, h);
+      const int c = c0 + h;
       if (c >= 6 && c < nmax - 6) {
         if constexpr (CF::EOS == 1) W.p[h] = fmax(smallp, pow(W.r[h], gam) * q[h]);
         else W.p[h] = fmax(smallp, W.r[h] * q[h]);
@@ -861,41 +1078,68 @@ __device__ __forceinline__ void ppmlr_wave(Win<T, K>& W, int nmax, T dt, T FrRot
   }
 }
 
+// derivs (viscosity.cu:2-19) with the divisions by its three coordinate differences shared by
+// every field of a cell.  quot<EX>: a / b from y = 1 / b to an ulp; the viscous update is a small
+// increment, so in 2-D its quotients need not round as divisions do
+template <bool EX>
+__device__ __forceinline__ double quot(double a, double b, double y) {
+  if constexpr (EX) return div64(a, b, y);
+  else return a * y;
+}
+template <bool EX>
+struct Fit64 {
+  double x2, x3, i2, i3, i32;
+  __device__ __forceinline__ Fit64(double xm, double x0, double xp) {
+    x2 = x0 - xm;
+    x3 = xp - xm;
+    i2 = rcp64(x2);
+    i3 = rcp64(x3);
+    i32 = rcp64(x3 - x2);
+  }
+  __device__ __forceinline__ void operator()(double um, double u0, double up, double& first, double& second) const {
+    const double h2 = quot<EX>(u0 - um, x2, i2), h3 = quot<EX>(up - um, x3, i3), x32 = x3 - x2;
+    second = 2.0 * quot<EX>(h3 - h2, x32, i32);
+    first = second * x2 + quot<EX>(x3 * h2 - x2 * h3, x32, i32);
+  }
+};
+
 // device_viscosity_r (viscosity.cu:370-421); R = cylindrical radius per cell, x = left edges
-template <typename T, int K>
-__device__ __forceinline__ void visc_r(Win<T, K>& W, int lim, T dt, const C<T, K>& R, const C<T, K>& nu, bool do_w) {
-  C<T, K> nr, vv;
+template <int K, bool EX>
+__device__ __forceinline__ void visc_r(Win<K>& W, int c0, int lim, double dt, const C<double, K>& R, const C<double, K>& nu, bool do_w) {
+  C<double, K> nr, vv;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     nr[h] = nu[h] * W.r[h];
-    vv[h] = W.v[h] / (R[h] * R[h]);
+    const double R2 = R[h] * R[h];
+    vv[h] = div64(W.v[h], R2, rcp64(R2));
   }
-  C<T, K> xm = prev1(W.xa0), xp = next1(W.xa0);
-  C<T, K> nm = prev1(nr), np = next1(nr);
-  C<T, K> um = prev1(W.u), up = next1(W.u);
-  C<T, K> vm = prev1(vv), vp = next1(vv);
-  C<T, K> wm, wp;
+  C<double, K> xm = prev1(W.xa0), xp = next1(W.xa0);
+  C<double, K> nm = prev1(nr), np = next1(nr);
+  C<double, K> um = prev1(W.u), up = next1(W.u);
+  C<double, K> vm = prev1(vv), vp = next1(vv);
+  C<double, K> wm, wp;
   if (do_w) {
     wm = prev1(W.w);
     wp = next1(W.w);
   }
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_of(K, h);
-    T rho = W.r[h], n = nr[h], Ri = R[h];
-    T dn, d1, d2;
-    derivs<T>(xm[h], W.xa0[h], xp[h], nm[h], n, np[h], dn, d2);
-    derivs<T>(xm[h], W.xa0[h], xp[h], um[h], W.u[h], up[h], d1, d2);
-    T ddu = T(2.0) * n * d2 + T(2.0) * dn * d1 + T(2.0) * n * d1 / Ri - T(2.0) * n * W.u[h] / Ri / Ri;
-    ddu = W.u[h] + dt * ddu / rho;
-    derivs<T>(xm[h], W.xa0[h], xp[h], vm[h], vv[h], vp[h], d1, d2);
-    T ddv = Ri * n * d2 + Ri * dn * d1 + T(3.0) * n * d1;
-    ddv = vv[h] * Ri + dt * ddv / rho;
-    T ddw = W.w[h];
+    const int c = c0 + h;
+    const double rho = W.r[h], n = nr[h], Ri = R[h], iR = rcp64(Ri), irho = rcp64(rho);
+    double dn, d1, d2;
+    const Fit64<EX> D(xm[h], W.xa0[h], xp[h]);
+    D(nm[h], n, np[h], dn, d2);
+    D(um[h], W.u[h], up[h], d1, d2);
+    double ddu = 2.0 * n * d2 + 2.0 * dn * d1 + quot<EX>(2.0 * n * d1, Ri, iR) - quot<EX>(quot<EX>(2.0 * n * W.u[h], Ri, iR), Ri, iR);
+    ddu = W.u[h] + quot<EX>(dt * ddu, rho, irho);
+    D(vm[h], vv[h], vp[h], d1, d2);
+    double ddv = Ri * n * d2 + Ri * dn * d1 + 3.0 * n * d1;
+    ddv = vv[h] * Ri + quot<EX>(dt * ddv, rho, irho);
+    double ddw = W.w[h];
     if (do_w) {
-      derivs<T>(xm[h], W.xa0[h], xp[h], wm[h], W.w[h], wp[h], d1, d2);
-      T t = n * d2 + dn * d1 + n * d1 / Ri;
-      ddw = W.w[h] + dt * t / rho;
+      D(wm[h], W.w[h], wp[h], d1, d2);
+      double t = n * d2 + dn * d1 + quot<EX>(n * d1, Ri, iR);
+      ddw = W.w[h] + quot<EX>(dt * t, rho, irho);
     }
     if (c >= kNpad && c < lim - kNpad) {
       W.u[h] = ddu;
@@ -907,41 +1151,42 @@ __device__ __forceinline__ void visc_r(Win<T, K>& W, int lim, T dt, const C<T, K
 
 // device_viscosity_p (viscosity.cu:423-472), called with (u, v, w) = (u_r, v_phi, w) of the
 // azimuthal sweep, i.e. sweep fields (w, u, v); x = left edges times R
-template <typename T, int K>
-__device__ __forceinline__ void visc_p(Win<T, K>& W, int lim, T dt, T R, T nu, const C<T, K>& x, bool do_w) {
-  C<T, K> nr;
+template <int K, bool EX>
+__device__ __forceinline__ void visc_p(Win<K>& W, int c0, int lim, double dt, double R, double nu, const C<double, K>& x, bool do_w) {
+  C<double, K> nr;
 #pragma unroll
   for (int h = 0; h < K; ++h) nr[h] = nu * W.r[h];
-  C<T, K> xm = prev1(x), xp = next1(x);
-  C<T, K> nm = prev1(nr), np = next1(nr);
+  C<double, K> xm = prev1(x), xp = next1(x);
+  C<double, K> nm = prev1(nr), np = next1(nr);
   // parameter v of the reference = sweep u (v_phi); parameter u = sweep w (u_r);
   // parameter w = sweep v
-  C<T, K> pvm = prev1(W.u), pvp = next1(W.u);
-  C<T, K> pum = prev1(W.w), pup = next1(W.w);
-  C<T, K> pwm, pwp;
+  C<double, K> pvm = prev1(W.u), pvp = next1(W.u);
+  C<double, K> pum = prev1(W.w), pup = next1(W.w);
+  C<double, K> pwm, pwp;
   if (do_w) {
     pwm = prev1(W.v);
     pwp = next1(W.v);
   }
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_of(K, h);
-    T rho = W.r[h], n = nr[h];
-    T dn, d1, d2;
-    derivs<T>(xm[h], x[h], xp[h], nm[h], n, np[h], dn, d2);
-    derivs<T>(xm[h], x[h], xp[h], pvm[h], W.u[h], pvp[h], d1, d2);
-    T ddv = T(2.0) * n * d2 + T(2.0) * dn * d1;
-    T ddu = T(0.0);
-    ddv = W.u[h] + dt * ddv / rho;
-    T ddw = W.v[h];
+    const int c = c0 + h;
+    const double rho = W.r[h], n = nr[h], irho = rcp64(rho);
+    double dn, d1, d2;
+    const Fit64<EX> D(xm[h], x[h], xp[h]);
+    D(nm[h], n, np[h], dn, d2);
+    D(pvm[h], W.u[h], pvp[h], d1, d2);
+    double ddv = 2.0 * n * d2 + 2.0 * dn * d1;
+    double ddu = 0.0;
+    ddv = W.u[h] + quot<EX>(dt * ddv, rho, irho);
+    double ddw = W.v[h];
     if (do_w) {
-      derivs<T>(xm[h], x[h], xp[h], pwm[h], W.v[h], pwp[h], d1, d2);
-      T t = n * d2 + dn * d1;
-      ddw = W.v[h] + dt * t / rho;
+      D(pwm[h], W.v[h], pwp[h], d1, d2);
+      double t = n * d2 + dn * d1;
+      ddw = W.v[h] + quot<EX>(dt * t, rho, irho);
     }
-    derivs<T>(xm[h], x[h], xp[h], pum[h], W.w[h], pup[h], d1, d2);
+    D(pum[h], W.w[h], pup[h], d1, d2);
     ddu += n * d2 + dn * d1;
-    ddu = W.w[h] + dt * ddu / rho;
+    ddu = W.w[h] + quot<EX>(dt * ddu, rho, irho);
     if (c >= kNpad && c < lim - kNpad) {
       W.u[h] = ddv;
       if (do_w) W.v[h] = ddw;
@@ -954,32 +1199,33 @@ __device__ __forceinline__ void visc_p(Win<T, K>& W, int lim, T dt, T R, T nu, c
 // along the pencil (the reference's w) taking 2 nu rho d2 + 2 dn d1 and the transverse ones
 // nu rho d2 + dn d1, no curvature terms.  The theta sweep passes (u, v, w) = (v_r, v_phi,
 // v_theta) and x = r times the theta left edges.
-template <typename T, int K>
-__device__ __forceinline__ void visc_z(const C<T, K>& rho, int lim, T dt, T nu, const C<T, K>& x, C<T, K>& u,
-                                       C<T, K>& v, C<T, K>& w) {
-  C<T, K> nr;
+template <int K, bool EX>
+__device__ __forceinline__ void visc_z(const C<double, K>& rho, int c0, int lim, double dt, double nu, const C<double, K>& x, C<double, K>& u,
+                                       C<double, K>& v, C<double, K>& w) {
+  C<double, K> nr;
 #pragma unroll
   for (int h = 0; h < K; ++h) nr[h] = nu * rho[h];
-  C<T, K> xm = prev1(x), xp = next1(x);
-  C<T, K> nm = prev1(nr), np = next1(nr);
-  C<T, K> um = prev1(u), up = next1(u);
-  C<T, K> vm = prev1(v), vp = next1(v);
-  C<T, K> wm = prev1(w), wp = next1(w);
+  C<double, K> xm = prev1(x), xp = next1(x);
+  C<double, K> nm = prev1(nr), np = next1(nr);
+  C<double, K> um = prev1(u), up = next1(u);
+  C<double, K> vm = prev1(v), vp = next1(v);
+  C<double, K> wm = prev1(w), wp = next1(w);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_of(K, h);
-    T n = nr[h], rh = rho[h];
-    T dn, d1, d2;
-    derivs<T>(xm[h], x[h], xp[h], nm[h], n, np[h], dn, d2);
-    derivs<T>(xm[h], x[h], xp[h], wm[h], w[h], wp[h], d1, d2);
-    T ddw = T(2.0) * n * d2 + T(2.0) * dn * d1;
-    derivs<T>(xm[h], x[h], xp[h], um[h], u[h], up[h], d1, d2);
-    T ddu = n * d2 + dn * d1;
-    derivs<T>(xm[h], x[h], xp[h], vm[h], v[h], vp[h], d1, d2);
-    T ddv = n * d2 + dn * d1;
-    ddw = w[h] + dt * ddw / rh;
-    ddu = u[h] + dt * ddu / rh;
-    ddv = v[h] + dt * ddv / rh;
+    const int c = c0 + h;
+    const double n = nr[h], rh = rho[h], irho = rcp64(rh);
+    double dn, d1, d2;
+    const Fit64<EX> D(xm[h], x[h], xp[h]);
+    D(nm[h], n, np[h], dn, d2);
+    D(wm[h], w[h], wp[h], d1, d2);
+    double ddw = 2.0 * n * d2 + 2.0 * dn * d1;
+    D(um[h], u[h], up[h], d1, d2);
+    double ddu = n * d2 + dn * d1;
+    D(vm[h], v[h], vp[h], d1, d2);
+    double ddv = n * d2 + dn * d1;
+    ddw = w[h] + quot<EX>(dt * ddw, rh, irho);
+    ddu = u[h] + quot<EX>(dt * ddu, rh, irho);
+    ddv = v[h] + quot<EX>(dt * ddv, rh, irho);
     if (c >= kNpad && c < lim - kNpad) {
       w[h] = ddw;
       u[h] = ddu;

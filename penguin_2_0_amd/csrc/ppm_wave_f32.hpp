@@ -156,9 +156,6 @@ __device__ __forceinline__ float planet_fth_sph(const PlanetF& p, float r, float
   return f;
 }
 
-// true in every lane when the condition holds in any lane of the wavefront (wave-uniform)
-__device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
-
 // log(1 + x): 2 atanh(x / (2 + x)) as an odd series for |x| < 1/4, else the library log.
 // Deviations that large are rare (next to a planet), so the library branch is taken only by
 // wavefronts that hold one; elsewhere it costs a compare and a scalar branch.
