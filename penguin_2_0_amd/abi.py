@@ -297,7 +297,7 @@ class Context:
                                          len(disk.val)), "pn_load_rings")
 
     def store(self) -> np.ndarray:
-        out = np.zeros(self.grid.imax * self.grid.kmax, ring_dtype(self.grid.jmax))
+        out = np.empty(self.grid.imax * self.grid.kmax, ring_dtype(self.grid.jmax))   # every byte is written
         self._chk(self.lib.pn_store_rings(self.h, _ptr(out), out.nbytes), "pn_store_rings")
         return out
 

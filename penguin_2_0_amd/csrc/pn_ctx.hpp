@@ -31,6 +31,11 @@ struct pn_ctx {
   double* ringbuf = nullptr;        // device, one double per interior ring (ring means)
   hipStream_t stream = nullptr;
   std::vector<void*> allocs;
+  // pinned staging of pn_store_rings: two pieces of the fields and the FARGO state (made on the
+  // first picture, at most 8 MiB or two rings beside 24 bytes a slot)
+  void* stage = nullptr;
+  bool stage_pinned = false;
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
   int cur = 0;                      // buffer holding the state
   bool loaded = false;
   // host copies of the per-ring values the device never changes (for packing)

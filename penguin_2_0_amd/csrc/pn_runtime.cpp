@@ -4,10 +4,13 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -15,6 +18,7 @@
 #include "pn_f32.hpp"
 #include "pn_host.hpp"
 #include "pn_launch.hpp"
+#include "pn_crew.hpp"
 #include "pn_ctx.hpp"
 
 using namespace pn;
@@ -291,6 +295,194 @@ int upload_tab64(pn_ctx* c, const std::vector<double>& radc, const std::vector<d
   return PN_OK;
 }
 
+// bytes of one half of a context's pinned staging buffer: fields come down in pieces of this
+// size, one piece copied while the other is packed.  Larger pieces gain nothing (the copy engine
+// is at its rate from about 1 MB), and a batch holds one buffer per disk.
+constexpr size_t kStageBytes = size_t(4) << 20;
+// output bytes that pay for one more packing thread (a thread starts in ~20 us and writes
+// new pages at a few GB/s), and the most threads a call starts
+constexpr size_t kBytesPerThread = size_t(4) << 20;
+constexpr int kMaxThreads = 16;
+
+// how the fields travel: nf of them in pieces of at most per slots, each field of a piece at
+// field_bytes of its half of the staging buffer
+struct Staging {
+  char* base;
+  size_t es, half, field_bytes;
+  long per;
+};
+
+int open_staging(pn_ctx* c, Staging& st) {
+  const DevGrid& d = c->dg;
+  const long nslot = static_cast<long>(d.sr) * d.sk;
+  // FP64: w may come and go with the state loaded
+  const int nmax = is_f32(c) ? (c->P.ndim == 3 || c->P.eos == 3 ? 4 : 3) : kNField;
+  st.es = is_f32(c) ? sizeof(float) : sizeof(double);
+  const size_t row = st.es * static_cast<size_t>(d.jmax) * nmax;
+  st.per = std::max<long>(1, static_cast<long>(std::min<size_t>(kStageBytes / row, nslot)));
+  st.half = row * st.per;
+  st.field_bytes = st.half / nmax;
+  for (hipEvent_t& e : c->stage_ev)
+    if (!e) PN_HIP(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  if (!c->stage) {
+    const size_t n = 2 * st.half + 24 * static_cast<size_t>(nslot);   // and the FARGO state
+    c->stage_pinned = hipHostMalloc(&c->stage, n, hipHostMallocDefault) == hipSuccess;
+    if (!c->stage_pinned) {   // no pinned memory to be had: the copies then go through the driver's own
+      (void)hipGetLastError();
+      c->stage = std::malloc(n);
+      if (!c->stage) return fail(c, PN_ERR_HIP, "no host memory for %zu staging bytes", n);
+    }
+  }
+  st.base = static_cast<char*>(c->stage);
+  return PN_OK;
+}
+
+int crew_size(size_t bytes) {
+  const int hw = std::max(1, static_cast<int>(std::thread::hardware_concurrency()));
+  return static_cast<int>(std::min<size_t>(std::min(kMaxThreads, hw), std::max<size_t>(1, bytes / kBytesPerThread)));
+}
+
+char* field_ptr(pn_ctx* c, int buf, int f) {
+  return is_f32(c) ? reinterpret_cast<char*>(c->df.f[buf][f]) : reinterpret_cast<char*>(c->dg.f[buf][f]);
+}
+
+// nf fields of every slot into buffer 0, fill(slot, dst) writing the slot's rows (row f at
+// dst + f * stride bytes) on the crew's threads, one piece filled while the one before is on its
+// way; then buffer 0 into buffer 1 on the device
+template <class Fill>
+int send_fields(pn_ctx* c, Crew& crew, int nf, const Fill& fill) {
+  Staging S;
+  int rc = open_staging(c, S);
+  if (rc != PN_OK) return rc;
+  const DevGrid& d = c->dg;
+  const long nslot = static_cast<long>(d.sr) * d.sk;
+  const size_t rowb = S.es * static_cast<size_t>(d.jmax);
+  int h = 0;
+  for (long s0 = 0, n = 0; s0 < nslot; s0 += S.per, ++n, h ^= 1) {
+    const long ns = std::min(S.per, nslot - s0);
+    if (n >= 2) PN_HIP(c, hipEventSynchronize(c->stage_ev[h]));
+    char* const st = S.base + h * S.half;
+    crew.run(ns, [&](long b, long e) {
+      for (long t = b; t < e; ++t) fill(s0 + t, st + t * rowb, S.field_bytes);
+    });
+    for (int f = 0; f < nf; ++f)
+      PN_HIP(c, hipMemcpyAsync(field_ptr(c, 0, f) + s0 * rowb, st + f * S.field_bytes, ns * rowb, hipMemcpyHostToDevice, c->stream));
+    PN_HIP(c, hipEventRecord(c->stage_ev[h], c->stream));
+  }
+  for (int f = 0; f < nf; ++f)
+    PN_HIP(c, hipMemcpyAsync(field_ptr(c, 1, f), field_ptr(c, 0, f), nslot * rowb, hipMemcpyDeviceToDevice, c->stream));
+  return PN_OK;
+}
+
+// The interior rings of the current state as hydr_ring records into out (imax kmax records, every
+// byte written).  72 bytes a cell leave the host whatever the state's precision, so the bound is
+// the host's rate of filling new pages: the fields come down in pieces into pinned memory, and
+// several threads write the records of one piece (phi geometry and, in 2-D, the zero w filled in
+// on the host) while the next is on its way.  1024 x 3072, one thread and pageable copies of whole
+// fields before: 43 ms (FP64), 54 ms (FP32).
+int fetch_rings(pn_ctx* c, char* out) {
+  const DevGrid& d = c->dg;
+  const int I = c->g.imax, J = c->g.jmax, K = c->g.kmax;
+  const long nslot = static_cast<long>(d.sr) * d.sk, nring = static_cast<long>(I) * K;
+  const bool f32 = is_f32(c), d3 = c->P.ndim == 3, adia = c->P.eos == 3;
+  const int nf = f32 ? (d3 || adia ? 4 : 3) : (c->dp.has_w ? 5 : 4);
+  // a piece spans whole slots, the ghost slots between two theta rows included
+  Staging S;
+  int rc = open_staging(c, S);
+  if (rc != PN_OK) return rc;
+  const size_t es = S.es, half = S.half, field_bytes = S.field_bytes;
+  const long per = S.per;
+  char* const stage = S.base;
+  const double* const rot = reinterpret_cast<const double*>(stage + 2 * half);
+  PN_HIP(c, hipMemcpyAsync(stage + 2 * half, d.rot_v, 24 * static_cast<size_t>(nslot), hipMemcpyDeviceToHost, c->stream));
+  auto slot = [&](long m) { return static_cast<long>(slot_of(d, static_cast<int>(m % I), static_cast<int>(m / I))); };
+  // the piece from ring m: its rings are m .. end - 1
+  auto piece_end = [&](long m) {
+    const long s0 = slot(m);
+    long e = m;
+    while (e < nring && slot(e) - s0 < per) e = std::min(nring, std::min((e / I + 1) * I, e + (s0 + per - slot(e))));
+    return e;
+  };
+  auto copy = [&](long m, long e, int h) -> int {
+    const long s0 = slot(m), ns = slot(e - 1) + 1 - s0;
+    for (int f = 0; f < nf; ++f)
+      PN_HIP(c, hipMemcpyAsync(stage + h * half + f * field_bytes, field_ptr(c, c->cur, f) + s0 * J * es, ns * J * es,
+                               hipMemcpyDeviceToHost, c->stream));
+    PN_HIP(c, hipEventRecord(c->stage_ev[h], c->stream));
+    return PN_OK;
+  };
+  const size_t rb = pn_ring_bytes(J), jb = 8 * static_cast<size_t>(J);
+  const double* const res = rot + nslot;
+  const int32_t* const rj = reinterpret_cast<const int32_t*>(res + nslot);
+  auto pack = [&](long m, long s0, const char* st) {
+    const long s = slot(m);
+    RingView R = ring_view(out, J, m);
+    auto field = [&](int f) { return st + f * field_bytes + (s - s0) * J * es; };
+    if (f32) {
+      const float* g0 = reinterpret_cast<const float*>(field(0));
+      const float* g1 = reinterpret_cast<const float*>(field(1));
+      const float* g2 = reinterpret_cast<const float*>(field(2));
+      const float* g3 = nf == 4 ? reinterpret_cast<const float*>(field(3)) : nullptr;
+      const double rb_ = c->h_rbg[s], vb = c->h_vbg[s], qb = c->h_qbg[s], cs2 = c->h_cs2[s];
+      for (int j = 0; j < J; ++j) R.r[j] = rb_ + static_cast<double>(g0[j]);
+      // isothermal closure (ppm.cu:139); EOS 3 carries q = p / Sigma
+      if (adia)
+        for (int j = 0; j < J; ++j) R.p[j] = R.r[j] * (qb + static_cast<double>(g3[j]));
+      else
+        for (int j = 0; j < J; ++j) R.p[j] = R.r[j] * cs2;
+      for (int j = 0; j < J; ++j) R.u[j] = static_cast<double>(g1[j]);
+      for (int j = 0; j < J; ++j) R.v[j] = vb + static_cast<double>(g2[j]);
+      if (d3)
+        for (int j = 0; j < J; ++j) R.w[j] = static_cast<double>(g3[j]);
+      else
+        std::memset(R.w, 0, jb);
+    } else {
+      std::memcpy(R.r, field(FR), jb);
+      std::memcpy(R.p, field(FP), jb);
+      std::memcpy(R.u, field(FU), jb);
+      std::memcpy(R.v, field(FV), jb);
+      if (nf == 5) std::memcpy(R.w, field(FW), jb);
+      else std::memset(R.w, 0, jb);
+    }
+    *R.x = c->h_x[s]; *R.dx = c->h_dx[s]; *R.xvol = c->h_xvol[s]; *R.xc = c->h_xc[s];
+    std::memcpy(R.y, c->h_y.data(), jb);
+    std::memcpy(R.dy, c->h_dy.data(), jb);
+    std::memcpy(R.yvol, c->h_yvol.data(), jb);
+    std::memcpy(R.yc, c->h_yc.data(), jb);
+    *R.z = c->h_z[s]; *R.dz = c->h_dz[s]; *R.zvol = c->h_zvol[s]; *R.zc = c->h_zc[s];
+    *R.i = static_cast<int32_t>(m % I);
+    *R.k = static_cast<int32_t>(m / I);
+    *R.rot_v = rot[s];
+    *R.res_v = res[s];
+    *R.rot_j = rj[s];
+    *R.inc_j = rj[nslot + s];
+  };
+  Crew crew(crew_size(rb * nring));
+  long m = 0, e = piece_end(0);
+  int h = 0;
+  rc = copy(m, e, h);
+  while (rc == PN_OK) {
+    const long m1 = e, e1 = m1 < nring ? piece_end(m1) : m1;
+    if (m1 < nring && (rc = copy(m1, e1, h ^ 1)) != PN_OK) break;
+    const hipError_t he = hipEventSynchronize(c->stage_ev[h]);
+    if (he != hipSuccess) {
+      rc = fail(c, PN_ERR_HIP, "fetching the state: %s", hipGetErrorString(he));
+      break;
+    }
+    const long s0 = slot(m);
+    const char* st = stage + h * half;
+    crew.run(e - m, [&](long b, long t) {
+      for (long n = b; n < t; ++n) pack(m + n, s0, st);
+    });
+    if (m1 >= nring) break;
+    m = m1;
+    e = e1;
+    h ^= 1;
+  }
+  const int rs = sync(c);   // nothing is left in flight into the staging buffer, also after a failure
+  return rc != PN_OK ? rc : rs;
+}
+
 }  // namespace
 
 extern "C" {
@@ -355,11 +547,16 @@ int pn_create(const pn_grid* g, const pn_params* p, int precision, pn_ctx** out)
   }
   double *x, *dx, *xc, *xvol, *z, *dz, *zc, *zvol, *radc, *cs2, *nu, *y, *dy, *yc, *yvol;
   pn_symdisk* val;
-  double** slot_tabs[] = {&x, &dx, &xc, &xvol, &z, &dz, &zc, &zvol, &radc, &cs2, &nu, &d.rot_v, &d.res_v};
+  double** slot_tabs[] = {&x, &dx, &xc, &xvol, &z, &dz, &zc, &zvol, &radc, &cs2, &nu};
   for (double** t : slot_tabs)
     if (r2 == PN_OK) r2 = dalloc(c, t, nslot);
-  if (r2 == PN_OK) r2 = dalloc(c, &d.rot_j, nslot);
-  if (r2 == PN_OK) r2 = dalloc(c, &d.inc_j, nslot);
+  // the FARGO state of every slot in one block, so that a picture fetches it with one copy
+  if (r2 == PN_OK) r2 = dalloc(c, &d.rot_v, 3 * nslot);
+  if (r2 == PN_OK) {
+    d.res_v = d.rot_v + nslot;
+    d.rot_j = reinterpret_cast<int*>(d.res_v + nslot);
+    d.inc_j = d.rot_j + nslot;
+  }
   double** col_tabs[] = {&y, &dy, &yc, &yvol};
   for (double** t : col_tabs)
     if (r2 == PN_OK) r2 = dalloc(c, t, g->jmax);
@@ -453,6 +650,10 @@ int pn_destroy(pn_ctx* c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   if (c->gexec) hipGraphExecDestroy(c->gexec);
   for (void* q : c->allocs) hipFree(q);
+  if (c->stage && c->stage_pinned) hipHostFree(c->stage);
+  else std::free(c->stage);
+  for (hipEvent_t e : c->stage_ev)
+    if (e) hipEventDestroy(e);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
   return PN_OK;
@@ -473,19 +674,17 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
 
   const DevGrid& d = c->dg;
   const long nslot = static_cast<long>(d.sr) * d.sk;
-  std::vector<double> F[kNField];
-  for (int f = 0; f < kNField; ++f) F[f].assign(static_cast<size_t>(nslot) * J, 0.0);
   std::vector<double> sx(nslot, 0.0), sdx(nslot, 1.0), sxc(nslot, 1.0), sxvol(nslot, 1.0), sz(nslot, 0.0),
       sdz(nslot, 1.0), szc(nslot, 0.0), szvol(nslot, 1.0), srot_v(nslot, 0.0), sres_v(nslot, 0.0), svbg(nslot, 0.0);
   std::vector<int32_t> srot_j(nslot, 0), sinc_j(nslot, 0);
-  // field values are copied as bytes so that signed zeros and NaN payloads survive
+  // the record each slot takes its fields from (null for the corner slots of a 3-D grid, whose
+  // fields are zero), and the record's number in its array for messages
+  std::vector<const void*> rec(nslot, nullptr);
+  std::vector<long> rec_no(nslot, 0);
   auto take = [&](const void* base, long idx, int slot, bool interior) -> int {
     RingView R = ring_view(const_cast<void*>(base), J, idx);
-    std::memcpy(&F[FR][static_cast<size_t>(slot) * J], R.r, 8 * J);
-    std::memcpy(&F[FP][static_cast<size_t>(slot) * J], R.p, 8 * J);
-    std::memcpy(&F[FU][static_cast<size_t>(slot) * J], R.u, 8 * J);
-    std::memcpy(&F[FV][static_cast<size_t>(slot) * J], R.v, 8 * J);
-    std::memcpy(&F[FW][static_cast<size_t>(slot) * J], R.w, 8 * J);
+    rec[slot] = R.r;
+    rec_no[slot] = idx;
     sx[slot] = *R.x; sdx[slot] = *R.dx; sxc[slot] = *R.xc; sxvol[slot] = *R.xvol;
     sz[slot] = *R.z; sdz[slot] = *R.dz; szc[slot] = *R.zc; szvol[slot] = *R.zvol;
     srot_v[slot] = *R.rot_v;
@@ -496,11 +695,6 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
       sinc_j[slot] = *R.inc_j;
       if (*R.rot_j < 0 || *R.rot_j >= J) return fail(c, PN_ERR_LAYOUT, "ring %ld: rot_j %d outside [0, %d)", idx, *R.rot_j, J);
     }
-    // every ring must carry the phi geometry of ring 0 (init.cpp:201-206, 316-319)
-    RingView R0 = ring_view(const_cast<void*>(rings), J, 0);
-    if (std::memcmp(R.y, R0.y, 8 * J) || std::memcmp(R.dy, R0.dy, 8 * J) || std::memcmp(R.yc, R0.yc, 8 * J) ||
-        std::memcmp(R.yvol, R0.yvol, 8 * J))
-      return fail(c, PN_ERR_LAYOUT, "ring %ld: phi geometry differs from ring 0", idx);
     return PN_OK;
   };
   int rc;
@@ -525,15 +719,35 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
         if ((rc = take(udr, kk + PN_NPAD * i, slot_of(d, i, kk - PN_NPAD), false)) != PN_OK) return rc;
         if ((rc = take(top, kk + PN_NPAD * i, slot_of(d, i, K + kk), false)) != PN_OK) return rc;
       }
-  // is w carried?  It is identically zero in a 2-D state built by the reference's init; a
-  // non-zero w is advected passively like any other field
-  int has_w = (c->P.ndim == 3) ? 1 : 0;
-  if (!has_w)
-    for (double wv : F[FW])
-      if (wv != 0.0 || std::signbit(wv)) {
-        has_w = 1;
-        break;
+  // every ring must carry the phi geometry of ring 0 (init.cpp:201-206, 316-319).  Is w carried?
+  // It is identically zero in a 2-D state built by the reference's init; a non-zero w is advected
+  // passively like any other field
+  Crew crew(crew_size(rings_bytes));
+  std::atomic<long> odd_slot{nslot};   // the first slot whose geometry differs
+  std::atomic<int> any_w{c->P.ndim == 3 ? 1 : 0};
+  const RingView Rg = ring_view(const_cast<void*>(rings), J, 0);
+  crew.run(nslot, [&](long b, long e) {
+    for (long s = b; s < e; ++s) {
+      if (!rec[s]) continue;
+      const RingView R = ring_view(const_cast<void*>(rec[s]), J, 0);
+      if (std::memcmp(R.y, Rg.y, 8 * J) || std::memcmp(R.dy, Rg.dy, 8 * J) || std::memcmp(R.yc, Rg.yc, 8 * J) ||
+          std::memcmp(R.yvol, Rg.yvol, 8 * J)) {
+        long at = odd_slot.load();
+        while (s < at && !odd_slot.compare_exchange_weak(at, s)) {
+        }
+        return;
       }
+      if (any_w.load(std::memory_order_relaxed) == 0)
+        for (int j = 0; j < J; ++j)
+          if (R.w[j] != 0.0 || std::signbit(R.w[j])) {
+            any_w.store(1, std::memory_order_relaxed);
+            break;
+          }
+    }
+  });
+  if (odd_slot.load() < nslot)
+    return fail(c, PN_ERR_LAYOUT, "ring %ld: phi geometry differs from ring 0", rec_no[odd_slot.load()]);
+  const int has_w = any_w.load();
   if (is_f32(c) && has_w && c->P.ndim == 2)
     return fail(c, PN_ERR_UNSUPPORTED, "the 2-D FP32 path carries no w (2-D disk with w = 0)");
   c->dp.has_w = has_w;
@@ -564,9 +778,20 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
   std::vector<double> tab64;   // outlives its upload
   const size_t cells = static_cast<size_t>(nslot) * J;
   if (!is_f32(c)) {
-    for (int b = 0; b < 2; ++b)
-      for (int f = 0; f < kNField; ++f)
-        PN_HIP(c, hipMemcpyAsync(d.f[b][f], F[f].data(), cells * sizeof(double), hipMemcpyHostToDevice, st));
+    // field values travel as bytes, so signed zeros and NaN payloads survive
+    const size_t jb = 8 * static_cast<size_t>(J);
+    const int nf = has_w ? 5 : 4;
+    rc = send_fields(c, crew, nf, [&](long s, char* dst, size_t stride) {
+      const RingView R = ring_view(const_cast<void*>(rec[s]), J, 0);
+      const double* const src[kNField] = {R.r, R.p, R.u, R.v, R.w};
+      for (int f = 0; f < nf; ++f) {
+        if (rec[s]) std::memcpy(dst + f * stride, src[f], jb);
+        else std::memset(dst + f * stride, 0, jb);
+      }
+    });
+    if (rc != PN_OK) return rc;
+    if (!has_w)
+      for (int b = 0; b < 2; ++b) PN_HIP(c, hipMemsetAsync(d.f[b][FW], 0, cells * sizeof(double), st));
     if ((rc = upload_tab64(c, sradc, scs2, snu, tab64)) != PN_OK) return rc;
   } else {
     const bool d3 = (c->P.ndim == 3);
@@ -574,12 +799,15 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
     const int nf = (d3 || adia) ? 4 : 3;
     // backgrounds: the SymDisk record of an interior ring, a ghost ring's own (uniform) values
     std::vector<double> rbg(nslot);
-    for (long s = 0; s < nslot; ++s) rbg[s] = F[FR][static_cast<size_t>(s) * J];
+    auto first = [&](long s, int f) {   // the record's first value of field f (0 for a corner slot)
+      return rec[s] ? static_cast<const double*>(rec[s])[static_cast<size_t>(f) * J] : 0.0;
+    };
+    for (long s = 0; s < nslot; ++s) rbg[s] = first(s, FR);
     for (int k = 0; k < K; ++k)
       for (int i = 0; i < I; ++i) rbg[slot_of(d, i, k)] = val[i + static_cast<long>(I) * k].r;
     // EOS 3: the background pressure of the same records, and q_b = p_b / Sigma_b
     std::vector<double> pbg(nslot), qbg(nslot);
-    for (long s = 0; s < nslot; ++s) pbg[s] = adia ? F[FP][static_cast<size_t>(s) * J] : scs2[s] * rbg[s];
+    for (long s = 0; s < nslot; ++s) pbg[s] = adia ? first(s, FP) : scs2[s] * rbg[s];
     if (adia)
       for (int k = 0; k < K; ++k)
         for (int i = 0; i < I; ++i) pbg[slot_of(d, i, k)] = val[i + static_cast<long>(I) * k].p;
@@ -605,20 +833,25 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
     for (long s = 0; s < nslot; ++s) qbg[s] = pbg[s] / rbg[s];
     c->h_qbg = qbg;
     // Sigma - Sigma_b, v_r, v_phi - v_bg and (3-D) v_theta, rounded once
-    std::vector<float> G[4];
-    for (int f = 0; f < nf; ++f) G[f].resize(cells);
-    for (long s = 0; s < nslot; ++s)
-      for (int j = 0; j < J; ++j) {
-        const size_t a = static_cast<size_t>(s) * J + j;
-        G[0][a] = static_cast<float>(F[FR][a] - rbg[s]);
-        G[1][a] = static_cast<float>(F[FU][a]);
-        G[2][a] = static_cast<float>(F[FV][a] - bvbg[s]);
-        if (d3) G[3][a] = static_cast<float>(F[FW][a]);
-        if (adia) G[3][a] = static_cast<float>(F[FP][a] / F[FR][a] - qbg[s]);
+    rc = send_fields(c, crew, nf, [&](long s, char* dst, size_t stride) {
+      float* const g0 = reinterpret_cast<float*>(dst);
+      float* const g1 = reinterpret_cast<float*>(dst + stride);
+      float* const g2 = reinterpret_cast<float*>(dst + 2 * stride);
+      float* const g3 = reinterpret_cast<float*>(dst + 3 * stride);
+      if (!rec[s]) {   // a corner slot: fields and backgrounds zero
+        for (int f = 0; f < nf; ++f) std::memset(dst + f * stride, 0, sizeof(float) * J);
+        return;
       }
-    for (int b = 0; b < 2; ++b)
-      for (int f = 0; f < nf; ++f)
-        PN_HIP(c, hipMemcpyAsync(c->df.f[b][f], G[f].data(), cells * sizeof(float), hipMemcpyHostToDevice, st));
+      const RingView R = ring_view(const_cast<void*>(rec[s]), J, 0);
+      for (int j = 0; j < J; ++j) g0[j] = static_cast<float>(R.r[j] - rbg[s]);
+      for (int j = 0; j < J; ++j) g1[j] = static_cast<float>(R.u[j]);
+      for (int j = 0; j < J; ++j) g2[j] = static_cast<float>(R.v[j] - bvbg[s]);
+      if (d3)
+        for (int j = 0; j < J; ++j) g3[j] = static_cast<float>(R.w[j]);
+      if (adia)
+        for (int j = 0; j < J; ++j) g3[j] = static_cast<float>(R.p[j] / R.r[j] - qbg[s]);
+    });
+    if (rc != PN_OK) return rc;
     // the per-slot table, entry-major, every entry evaluated in FP64 and rounded once; the
     // overhang past the last slot repeats it.  Radial neighbours are slots s +- 1 of the same
     // theta row, theta neighbours s +- sr.
@@ -855,67 +1088,7 @@ int pn_store_rings(pn_ctx* c, void* rings, size_t rings_bytes) {
   const int I = c->g.imax, J = c->g.jmax, K = c->g.kmax;
   const size_t rb = pn_ring_bytes(J);
   if (!rings || rings_bytes != rb * I * K) return fail(c, PN_ERR_ARG, "rings: %zu bytes, expected %zu", rings_bytes, rb * I * K);
-  const DevGrid& d = c->dg;
-  const long nslot = static_cast<long>(d.sr) * d.sk;
-  const size_t cells = static_cast<size_t>(nslot) * J;
-  std::vector<double> F[kNField];
-  for (int f = 0; f < kNField; ++f) F[f].assign(cells, 0.0);
-  std::vector<float> G[4];
-  const int nf = (c->P.ndim == 3 || c->P.eos == 3) ? 4 : 3;
-  if (!is_f32(c)) {
-    for (int f = 0; f < kNField; ++f)
-      PN_HIP(c, hipMemcpyAsync(F[f].data(), d.f[c->cur][f], cells * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  } else {
-    for (int f = 0; f < nf; ++f) {
-      G[f].resize(cells);
-      PN_HIP(c, hipMemcpyAsync(G[f].data(), c->df.f[c->cur][f], cells * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    }
-  }
-  std::vector<double> rot_v(nslot), res_v(nslot);
-  std::vector<int32_t> rot_j(nslot), inc_j(nslot);
-  PN_HIP(c, hipMemcpyAsync(rot_v.data(), d.rot_v, nslot * 8, hipMemcpyDeviceToHost, c->stream));
-  PN_HIP(c, hipMemcpyAsync(res_v.data(), d.res_v, nslot * 8, hipMemcpyDeviceToHost, c->stream));
-  PN_HIP(c, hipMemcpyAsync(rot_j.data(), d.rot_j, nslot * 4, hipMemcpyDeviceToHost, c->stream));
-  PN_HIP(c, hipMemcpyAsync(inc_j.data(), d.inc_j, nslot * 4, hipMemcpyDeviceToHost, c->stream));
-  int rc = sync(c);
-  if (rc != PN_OK) return rc;
-  if (is_f32(c))
-    for (long s = 0; s < nslot; ++s)
-      for (int j = 0; j < J; ++j) {
-        const size_t a = static_cast<size_t>(s) * J + j;
-        const double r = c->h_rbg[s] + static_cast<double>(G[0][a]);
-        F[FR][a] = r;
-        // isothermal closure (ppm.cu:139); EOS 3 carries q = p / Sigma
-        F[FP][a] = (c->P.eos == 3) ? r * (c->h_qbg[s] + static_cast<double>(G[3][a])) : r * c->h_cs2[s];
-        F[FU][a] = static_cast<double>(G[1][a]);
-        F[FV][a] = c->h_vbg[s] + static_cast<double>(G[2][a]);
-        if (c->P.ndim == 3) F[FW][a] = static_cast<double>(G[3][a]);
-      }
-  std::memset(rings, 0, rb * I * K);
-  for (int k = 0; k < K; ++k)
-    for (int i = 0; i < I; ++i) {
-      const long m = i + static_cast<long>(I) * k;
-      const int s = slot_of(d, i, k);
-      RingView R = ring_view(rings, J, m);
-      std::memcpy(R.r, &F[FR][static_cast<size_t>(s) * J], 8 * J);
-      std::memcpy(R.p, &F[FP][static_cast<size_t>(s) * J], 8 * J);
-      std::memcpy(R.u, &F[FU][static_cast<size_t>(s) * J], 8 * J);
-      std::memcpy(R.v, &F[FV][static_cast<size_t>(s) * J], 8 * J);
-      std::memcpy(R.w, &F[FW][static_cast<size_t>(s) * J], 8 * J);
-      *R.x = c->h_x[s]; *R.dx = c->h_dx[s]; *R.xvol = c->h_xvol[s]; *R.xc = c->h_xc[s];
-      std::memcpy(R.y, c->h_y.data(), 8 * J);
-      std::memcpy(R.dy, c->h_dy.data(), 8 * J);
-      std::memcpy(R.yvol, c->h_yvol.data(), 8 * J);
-      std::memcpy(R.yc, c->h_yc.data(), 8 * J);
-      *R.z = c->h_z[s]; *R.dz = c->h_dz[s]; *R.zvol = c->h_zvol[s]; *R.zc = c->h_zc[s];
-      *R.i = i;
-      *R.k = k;
-      *R.rot_v = rot_v[s];
-      *R.res_v = res_v[s];
-      *R.rot_j = rot_j[s];
-      *R.inc_j = inc_j[s];
-    }
-  return PN_OK;
+  return fetch_rings(c, static_cast<char*>(rings));
 }
 
 int pn_get_dt(pn_ctx* c, double dt_prev, double FrRot, double* dt) {
@@ -1434,12 +1607,12 @@ int pn_run(pn_ctx* c, int nsteps, int graph, pn_run_state* st) {
 int pn_save_snapshot(pn_ctx* c, const char* path) {
   if (!c || !path) return PN_ERR_ARG;
   const size_t n = pn_ring_bytes(c->g.jmax) * c->g.imax * c->g.kmax;
-  std::vector<char> buf(n);
-  int rc = pn_store_rings(c, buf.data(), n);
+  std::unique_ptr<char[]> buf(new char[n]);   // every byte is written
+  int rc = pn_store_rings(c, buf.get(), n);
   if (rc != PN_OK) return rc;
   FILE* f = std::fopen(path, "wb");
   if (!f) return fail(c, PN_ERR_IO, "cannot open %s for writing", path);
-  size_t w = std::fwrite(buf.data(), 1, n, f);
+  size_t w = std::fwrite(buf.get(), 1, n, f);
   int cl = std::fclose(f);
   if (w != n || cl != 0) return fail(c, PN_ERR_IO, "short write to %s", path);
   return PN_OK;
