@@ -9,17 +9,10 @@
 // geometry's reciprocals, the Eulerian paraset and the star's pull at fixed radii come from a
 // per-slot table instead of ~60 divisions a cell, the rest share reciprocals (div64), and in 2-D
 // the angle to the planet is turned from a per-column cosine and sine instead of taken anew at
-// three times.  1024 x 3072, inviscid: radial sweep 208 -> 149 us (5347 -> 2516 static VALU
-// instructions a pass; what is left waits on its gathers), azimuthal 189 -> 115 us; the spherical
-// sweeps of a 96 x 288 x 32 disk, which keep every bit, 110 / 83 / 345 -> 78 / 62 / 190 us
-// (r / phi / theta).
-//
-// Work decomposition: one wavefront per (pencil, window).  Windows are the reference's
-// (ppm.cu:34-48, 169-196): 128 cells starting every 116, with 6 halo cells per side, the
-// last one shortened to the pencil's remainder (a remainder of zero gets a full window
-// instead of being skipped).  Four waves per 256-thread workgroup; workgroup ids are
-// remapped so that consecutive logical workgroups land on the same XCD (ids are dealt
-// round-robin to the 8 XCDs) and neighbouring columns share that XCD's L2.
+// three times: 1024 x 3072, inviscid, 5347 -> 2516 static VALU instructions a radial pass.  With the
+// radial and theta sweeps staged through LDS and short windows packed two to a wavefront (below):
+//   1024 x 3072 radial 208 -> 125 us, azimuthal 189 -> 108 us; 256 x 768 radial 30.6 -> 13.5 us;
+//   96 x 288 x 32, whose sweeps keep every bit, r / phi / theta 110 / 83 / 345 -> 68 / 61 / 97 us.
 #include "pn_launch.hpp"
 #include "ppm_wave.hpp"
 
@@ -60,101 +53,202 @@ __device__ __forceinline__ Planet load_planet(const StepScalars* ss, int bary) {
   return p;
 }
 
-// Waves per SIMD the radial sweep asks for: the inviscid isothermal cylindrical sweep needs
-// 172 VGPRs, two waves; at 168 it holds three with no spill and runs 1024 x 3072 in 0.248
-// instead of 0.274 ms.  Every other form spills at 168 (the viscous one four accesses, the
-// other closures and the 3-D sweeps tens), so they keep what the allocator gives.
+// Waves per SIMD asked for.  The isothermal sweeps settle at 166-190 VGPRs, two waves; at 168 they
+// hold three for at most nine spilled registers a pass (1024 x 3072 azimuthal 115 -> 108 us, theta
+// sweep of 96 x 288 x 32 190 -> 176 us).  The other closures need 210 and more: two waves.
 template <class CF>
-constexpr int x_waves() {
-  return (CF::EOS == 0 && CF::GX == 1 && CF::VISC == 0) ? 3 : 1;
+constexpr int waves64() {
+  return CF::EOS == 0 ? 3 : 1;
 }
 
 // ---------------------------------------------------------------------------------------
-// radial sweep (sweepx, ppm.cu:26-160): pencil = lab column j0 of theta layer k
-template <class CF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(x_waves<CF>(), 8))) void k_sweep_x(DevGrid g, DevParams prm, const StepScalars* __restrict__ ss,
-                                                 int src) {
-  const int lane = threadIdx.x & 63;
-  const int gw = xcd_swizzle(blockIdx.x, gridDim.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  const int jmax = g.jmax;
-  const int j0 = gw % jmax;
-  const int rest = gw / jmax;
-  const int l = rest % g.nwin_x;
-  const int k = rest / g.nwin_x;
-  if (k >= g.kmax) return;   // wave-uniform; the kernel has no barriers
+// radial and theta sweeps (sweepx, ppm.cu:26-160; the reference has no caller for the theta sweep,
+// main.cu:376: it is assembled from the theta pieces it holds, forces.cu:298-372,
+// states.cu:29-39, evolve.cu:26-29, 63-67, 110-124, remap.cu:50-54, init.cpp:415-541).
+//
+// A pencil crosses rings, so its cells lie jmax apart in HBM and a wavefront's load of one field
+// touched 128 lines; the cells of neighbouring lab columns are contiguous.  A workgroup of four
+// waves therefore takes one window of four consecutive columns, stages its fields in LDS with
+// loads contiguous along phi, runs a pencil per wave from LDS, puts the results back in place and
+// stores them contiguously (1024 x 3072 radial: 148 -> 125 us; two columns a wave, for 64-byte
+// rows, lost more to the registers its loop holds: 192 us).  A window of at most 64 cells (a short
+// last window, a short theta pencil) takes eight columns instead, two per wavefront, one in each
+// half: every stage indexes cells within its own window, so a stencil across the seam sees what it
+// sees past a window's end, and no kept cell depends on it.
+template <int NF>
+struct Tile64 {
+  // [field][column][cell]: 4 columns of 130 or 8 of 66 (even strides: two-cell reads aligned)
+  static constexpr int kField = 528;
+  double f[NF][kField];
+  int srot[kWin];   // rot_j of the window's slots
+};
 
+// columns of a workgroup's window of lim cells
+__host__ __device__ inline int tile_columns(int lim) { return lim <= kWin / 2 ? 2 * kWavesPerBlock : kWavesPerBlock; }
+
+template <class CF>
+__device__ __forceinline__ void pencil64(const DevGrid& g, const DevParams& prm, const StepScalars* __restrict__ ss,
+                                         int src, int grp, int l, int row, Tile64<CF::GX == 2 ? 5 : 4>& T) {
+  constexpr bool TH = CF::AXIS == 2;
+  constexpr int NF = CF::GX == 2 ? 5 : 4, TPB = 64 * kWavesPerBlock, NIT = 2;
+  const int jmax = g.jmax;
+  const int lim = TH ? win_len(g.kmax, g.nwin_z, l) : win_len(g.imax, g.nwin_x, l);
+  const int s0 = TH ? slot_of(g, row, kReal * l - kNpad) : slot_of(g, kReal * l - kNpad, row);
+  const int step = TH ? g.sr : 1;
+  const bool two = lim <= kWin / 2;   // workgroup-uniform: two columns per wavefront
+  const int sh = two ? 3 : 2, nc = 1 << sh, ld = two ? kWin / 2 + 2 : kWin + 2;
+  const int jb = grp * nc;
+  static_assert(kWavesPerBlock == 4, "columns of a workgroup");
+  // staging: this thread moves cells cs and cs + cstep of column qs; columns past jmax read column
+  // jmax - 1, which is not stored
+  const int cstep = TPB >> sh, qs = threadIdx.x & (nc - 1), cs = threadIdx.x >> sh;
+  const int jl = jb + qs, jlc = jl < jmax ? jl : jmax - 1;
+  for (int c = threadIdx.x; c < kWin; c += TPB) T.srot[c] = g.rot_j[s0 + step * (c < lim ? c : lim - 1)];
+  __syncthreads();
+  double v[NIT][NF];
+#pragma unroll
+  for (int it = 0; it < NIT; ++it) {
+    const int c = cs + cstep * it;
+    const long a = (long)(s0 + step * (c < lim ? c : lim - 1)) * jmax + wrapj(jlc - T.srot[c], jmax);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) v[it][f] = g.f[src][f][a];
+  }
+#pragma unroll
+  for (int it = 0; it < NIT; ++it)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) T.f[f][qs * ld + cs + cstep * it] = v[it][f];
+  __syncthreads();
+
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double dt = ss->dt, FrRot = ss->FrRot;
   const Planet pl = load_planet(ss, prm.bary);
-  RunFlags rf{prm.flat, prm.plnt > 0, 1, 1, prm.ndim};
-  const int lim = win_len(g.imax, g.nwin_x, l);
-  rf.remap_v = 1;
-  rf.remap_w = prm.has_w;
-  const double* __restrict__ fr = g.f[src][FR];
-  const double* __restrict__ fp = g.f[src][FP];
-  const double* __restrict__ fu = g.f[src][FU];
-  const double* __restrict__ fv = g.f[src][FV];
-  const double* __restrict__ fw = g.f[src][FW];
-
-  // cells past the window read the overhang of the table (finite values no kept cell depends on)
-  const int s0 = slot_of(g, kReal * l - kNpad, k);
-  const TabLane64 tx{g.tab, g.tstride, 8u * (unsigned)(s0 + kK * lane)};
-  Win<kK> W;
-  const C<double, kK> radc = tx.get(kT64Rc);
-  long addr[kK];
-  W.rad = tx.get(kT64Rad);
-  W.xa0 = tx.get(kT64Xa);
-  W.dx0 = tx.get(kT64Dx);
-  W.dvol0 = tx.get(kT64Vol);
-  W.azi = splat<double, kK>(g.yc[j0]);
-  const double2 tr = g.ptrig[j0];
-  W.ca = splat<double, kK>(tr.x);
-  W.sa = splat<double, kK>(tr.y);
+  const RunFlags rf{prm.flat, prm.plnt > 0, 1, prm.has_w, prm.ndim};
+  const int ll = two ? lane % 32 : lane, c0 = kK * ll;
+  const int q = two ? 2 * wv + lane / 32 : wv;   // this lane's column
+  if (jb + (two ? 2 * wv : wv) < jmax) {         // wave-uniform; the barriers below are outside
+    const int j0 = jb + q < jmax ? jb + q : jmax - 1;
+    // cells past the window read the table's next slots or its overhang (finite values no kept
+    // cell depends on)
+    const TabLane64 tx{TH ? g.tabz : g.tab, g.tstride,
+                       8u * (unsigned)((TH ? kReal * l - kNpad + g.k0 + g.sk * (row + kNpad) : s0) + c0)};
+    double* const tf = &T.f[0][q * ld + c0];   // this lane's cells of field 0
+    constexpr int fs = Tile64<NF>::kField;
+    Win<kK> W;
+    const C<double, kK> radc = tx.get(kT64Rc);
+    W.rad = tx.get(kT64Rad);
+    W.xa0 = tx.get(TH ? kT64Za : kT64Xa);
+    W.dx0 = tx.get(TH ? kT64Dz : kT64Dx);
+    W.dvol0 = tx.get(TH ? kT64Volz : kT64Vol);
+    W.azi = splat<double, kK>(g.yc[j0]);
+    const double2 tr = g.ptrig[j0];
+    W.ca = splat<double, kK>(tr.x);
+    W.sa = splat<double, kK>(tr.y);
+    long aw[kK];   // 2-D: w, carried only by a state that has one, comes straight from HBM
 #pragma unroll
-  for (int h = 0; h < kK; ++h) {
-    const int c = kK * lane + h;
-    const int s = s0 + (c < lim ? c : lim - 1);   // keep loads in bounds; results unused
-    const long a = (long)s * jmax + wrapj(j0 - g.rot_j[s], jmax);
-    addr[h] = a;
-    double r = fr[a], p = fp[a], u = fu[a], v = fv[a];
-    double w = prm.has_w ? fw[a] : 0.0;
-    if (CF::GY > 2) v *= radc[h];
-    if (CF::GZ == 5) w *= W.rad[h];
-    W.r[h] = r; W.p[h] = p; W.u[h] = u; W.v[h] = v; W.w[h] = w;
-    W.e[h] = energy_of<CF>(p, r, u, v, prm.gam);
-  }
+    for (int h = 0; h < kK; ++h) {
+      const int c = c0 + h;
+      const double r = tf[FR * fs + h], p = tf[FP * fs + h], fu = tf[FU * fs + h], fv = tf[FV * fs + h];
+      double u, vv, w;
+      if constexpr (TH) {   // sweep components: v_theta, v_r, angular momentum
+        u = tf[FW * fs + h];
+        vv = fu;
+        w = fv * radc[h];
+      } else {
+        u = fu;
+        vv = fv * radc[h];
+        if constexpr (CF::GX == 2) {
+          w = tf[FW * fs + h] * W.rad[h];
+        } else {
+          w = 0.0;
+          if (prm.has_w) {
+            const int cc = c < lim ? c : lim - 1;
+            aw[h] = (long)(s0 + cc) * jmax + wrapj(j0 - T.srot[cc], jmax);
+            w = g.f[src][FW][aw[h]];
+          }
+        }
+      }
+      W.r[h] = r; W.p[h] = p; W.u[h] = u; W.v[h] = vv; W.w[h] = w;
+      W.e[h] = energy_of<CF>(p, r, u, vv, prm.gam);
+    }
 
-  ppmlr_wave<kK, CF>(W, tx, Ring64{}, kK * lane, lim, dt, FrRot, pl, rf, prm.gam);
-  if constexpr (CF::VISC) visc_r<kK, CF::GX == 2>(W, kK * lane, lim, dt, radc, tx.get(kT64Nu), prm.ndim == 3);
-
-  const C<double, kK> irc = tx.get(kT64Irc), cs2 = tx.get(kT64Cs2);
-  double* __restrict__ dr = g.f[src ^ 1][FR];
-  double* __restrict__ dp = g.f[src ^ 1][FP];
-  double* __restrict__ du = g.f[src ^ 1][FU];
-  double* __restrict__ dv = g.f[src ^ 1][FV];
-  double* __restrict__ dw = g.f[src ^ 1][FW];
+    ppmlr_wave<kK, CF>(W, tx, Ring64{}, c0, lim, dt, FrRot, pl, rf, prm.gam);
+    const C<double, kK> irc = tx.get(kT64Irc), cs2 = tx.get(kT64Cs2);
+    C<double, kK> vphi;
+    if constexpr (TH) {
+      // v_phi from the angular momentum the sweep carried; then device_viscosity_z
+      // (viscosity.cu:474-518) on (v_r, v_phi, v_theta)
 #pragma unroll
-  for (int h = 0; h < kK; ++h) {
-    const int c = kK * lane + h;
-    if (c >= kNpad && c < lim - kNpad) {
-      const long a = addr[h];
-      const double r = W.r[h];
-      double p;
-      if constexpr (CF::EOS == 0) p = r * cs2[h];
-      else if constexpr (CF::EOS == 1) p = cs2[h] * pow(r, prm.gam) / prm.gam;
-      else p = W.p[h];
-      dr[a] = r;
-      dp[a] = p;
-      du[a] = W.u[h];
-      dv[a] = (CF::GY > 2) ? div64(W.v[h], radc[h], irc[h]) : W.v[h];
-      if (prm.has_w) dw[a] = (CF::GZ == 5) ? W.w[h] / W.rad[h] : W.w[h];
+      for (int h = 0; h < kK; ++h) vphi[h] = div64(W.w[h], radc[h], irc[h]);
+      if constexpr (CF::VISC) {
+        C<double, kK> x;
+#pragma unroll
+        for (int h = 0; h < kK; ++h) x[h] = W.xa0[h] * W.rad[h];
+        visc_z<kK, true>(W.r, c0, lim, dt, prm.vis_nu, x, W.v, vphi, W.u);
+      }
+    } else {
+      if constexpr (CF::VISC) visc_r<kK, CF::GX == 2>(W, c0, lim, dt, radc, tx.get(kT64Nu), prm.ndim == 3);
+#pragma unroll
+      for (int h = 0; h < kK; ++h) vphi[h] = div64(W.v[h], radc[h], irc[h]);
+    }
+#pragma unroll
+    for (int h = 0; h < kK; ++h) {
+      const int c = c0 + h;
+      if (c >= kNpad && c < lim - kNpad) {   // only this half's lanes hold column q
+        const double r = W.r[h];
+        double p;
+        if constexpr (CF::EOS == 0) p = r * cs2[h];
+        else if constexpr (CF::EOS == 1) p = cs2[h] * pow(r, prm.gam) / prm.gam;
+        else p = W.p[h];
+        tf[FR * fs + h] = r;
+        tf[FP * fs + h] = p;
+        tf[FU * fs + h] = TH ? W.v[h] : W.u[h];
+        tf[FV * fs + h] = vphi[h];
+        if constexpr (TH) tf[FW * fs + h] = W.u[h];
+        else if constexpr (CF::GX == 2) tf[FW * fs + h] = W.w[h] / W.rad[h];
+        else if (prm.has_w && jb + q < jmax) g.f[src ^ 1][FW][aw[h]] = W.w[h];
+      }
     }
   }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < NIT; ++it) {
+    const int c = cs + cstep * it;
+    if (jl < jmax && c >= kNpad && c < lim - kNpad) {
+      const long a = (long)(s0 + step * c) * jmax + wrapj(jl - T.srot[c], jmax);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) g.f[src ^ 1][f][a] = T.f[f][qs * ld + c];
+    }
+  }
+}
+
+// workgroups of one row's windows: every window but the last is full
+__host__ __device__ inline int row_groups(int len, int nwin, int jmax, int* last) {
+  const int nc = tile_columns(len - kReal * (nwin - 1) + 2 * kNpad);
+  *last = (jmax + nc - 1) / nc;
+  return (nwin - 1) * ((jmax + kWavesPerBlock - 1) / kWavesPerBlock) + *last;
+}
+
+// items: column group x window x row (radial: theta layer k; theta: ring i), column groups fastest,
+// so that workgroups of one XCD share the lines of neighbouring columns
+template <class CF>
+__global__ __launch_bounds__(64 * kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(waves64<CF>(), 8))) void k_pencil64(
+    DevGrid g, DevParams prm, const StepScalars* __restrict__ ss, int src) {
+  __shared__ Tile64<CF::GX == 2 ? 5 : 4> T;
+  const int nwin = CF::AXIS == 2 ? g.nwin_z : g.nwin_x, len = CF::AXIS == 2 ? g.kmax : g.imax;
+  const int full = (g.jmax + kWavesPerBlock - 1) / kWavesPerBlock;
+  int last;
+  const int per = row_groups(len, nwin, g.jmax, &last);
+  const int bid = xcd_swizzle(blockIdx.x, gridDim.x);
+  const int row = bid / per, r = bid % per;
+  const int l = r < (nwin - 1) * full ? r / full : nwin - 1;
+  pencil64<CF>(g, prm, ss, src, r - l * full, l, row, T);
 }
 
 // ---------------------------------------------------------------------------------------
 // azimuthal sweep (sweepy, ppm.cu:162-307): pencil = one periodic ring
 template <class CF>
-__global__ __launch_bounds__(256) void k_sweep_y(DevGrid g, DevParams prm, const StepScalars* __restrict__ ss,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves64<CF>(), 8))) void k_sweep_y(DevGrid g, DevParams prm, const StepScalars* __restrict__ ss,
                                                  int src) {
   const int lane = threadIdx.x & 63;
   const int gw = xcd_swizzle(blockIdx.x, gridDim.x) * kWavesPerBlock + (threadIdx.x >> 6);
@@ -244,103 +338,25 @@ __global__ __launch_bounds__(256) void k_sweep_y(DevGrid g, DevParams prm, const
   }
 }
 
-// ---------------------------------------------------------------------------------------
-// theta sweep (3-D): pencil = (ring i, lab column j0) over theta layers.  The reference has
-// no caller for it (main.cu:376); it is assembled from the theta pieces it holds
-// (forces.cu:298-372, states.cu:29-39, evolve.cu:26-29, 63-67, 110-124, remap.cu:50-54,
-// init.cpp:415-541).  Sweep components: u <- v_theta (w), v <- v_r (u),
-// w <- v_phi * r sin(theta) (the angular momentum get_fz's centrifugal term expects).  With
-// viscosity the window then takes device_viscosity_z (viscosity.cu:474-518) on
-// (v_r, v_phi, v_theta).
-template <class CF>
-__global__ __launch_bounds__(256) void k_sweep_z(DevGrid g, DevParams prm, const StepScalars* __restrict__ ss,
-                                                 int src) {
-  const int lane = threadIdx.x & 63;
-  const int gw = xcd_swizzle(blockIdx.x, gridDim.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  const int jmax = g.jmax;
-  const int j0 = gw % jmax;
-  const int rest = gw / jmax;
-  const int l = rest % g.nwin_z;
-  const int i = rest / g.nwin_z;
-  if (i >= g.imax) return;
-
-  const double dt = ss->dt, FrRot = ss->FrRot;
-  const Planet pl = load_planet(ss, prm.bary);
-  RunFlags rf{prm.flat, prm.plnt > 0, 1, 1, prm.ndim};
-  const int lim = win_len(g.kmax, g.nwin_z, l);
-
-  // the theta-major table: slots run along the pencil; cells past the window read the next
-  // ring's slots or the overhang (finite values no kept cell depends on)
-  const TabLane64 tx{g.tabz, g.tstride, 8u * (unsigned)(kReal * l - kNpad + g.k0 + g.sk * (i + kNpad) + kK * lane)};
-  Win<kK> W;
-  const C<double, kK> radc = tx.get(kT64Rc);
-  long addr[kK];
-  W.rad = tx.get(kT64Rad);
-  W.xa0 = tx.get(kT64Za);
-  W.dx0 = tx.get(kT64Dz);
-  W.dvol0 = tx.get(kT64Volz);
-  W.azi = splat<double, kK>(g.yc[j0]);
-  const double2 tr = g.ptrig[j0];
-  W.ca = splat<double, kK>(tr.x);
-  W.sa = splat<double, kK>(tr.y);
-#pragma unroll
-  for (int h = 0; h < kK; ++h) {
-    const int c = kK * lane + h;
-    const int s = slot_of(g, i, kReal * l - kNpad + (c < lim ? c : lim - 1));
-    const long a = (long)s * jmax + wrapj(j0 - g.rot_j[s], jmax);
-    addr[h] = a;
-    const double r = g.f[src][FR][a], p = g.f[src][FP][a];
-    const double u = g.f[src][FW][a], v = g.f[src][FU][a];
-    W.r[h] = r; W.p[h] = p; W.u[h] = u; W.v[h] = v;
-    W.w[h] = g.f[src][FV][a] * radc[h];
-    W.e[h] = energy_of<CF>(p, r, u, v, prm.gam);
-  }
-
-  ppmlr_wave<kK, CF>(W, tx, Ring64{}, kK * lane, lim, dt, FrRot, pl, rf, prm.gam);
-  // v_phi from the angular momentum the sweep carried
-  const C<double, kK> irc = tx.get(kT64Irc), cs2 = tx.get(kT64Cs2);
-  C<double, kK> vphi;
-#pragma unroll
-  for (int h = 0; h < kK; ++h) vphi[h] = div64(W.w[h], radc[h], irc[h]);
-  if constexpr (CF::VISC) {
-    C<double, kK> x;
-#pragma unroll
-    for (int h = 0; h < kK; ++h) x[h] = W.xa0[h] * W.rad[h];
-    visc_z<kK, true>(W.r, kK * lane, lim, dt, prm.vis_nu, x, W.v, vphi, W.u);
-  }
-
-#pragma unroll
-  for (int h = 0; h < kK; ++h) {
-    const int c = kK * lane + h;
-    if (c >= kNpad && c < lim - kNpad) {
-      const long a = addr[h];
-      const double r = W.r[h];
-      double p;
-      if constexpr (CF::EOS == 0) p = r * cs2[h];
-      else if constexpr (CF::EOS == 1) p = cs2[h] * pow(r, prm.gam) / prm.gam;
-      else p = W.p[h];
-      g.f[src ^ 1][FR][a] = r;
-      g.f[src ^ 1][FP][a] = p;
-      g.f[src ^ 1][FW][a] = W.u[h];
-      g.f[src ^ 1][FU][a] = W.v[h];
-      g.f[src ^ 1][FV][a] = vphi[h];
-    }
-  }
-}
-
 template <int AX, class CF>
-void launch_one(dim3 grid, dim3 block, const LaunchCtx& c, int src) {
-  if constexpr (AX == 0) k_sweep_x<CF><<<grid, block, 0, c.stream>>>(c.g, c.p, c.ss, src);
-  else if constexpr (AX == 1) k_sweep_y<CF><<<grid, block, 0, c.stream>>>(c.g, c.p, c.ss, src);
-  else k_sweep_z<CF><<<grid, block, 0, c.stream>>>(c.g, c.p, c.ss, src);
+void launch_one(const LaunchCtx& c, int src) {
+  if constexpr (AX == 1) {
+    const long waves = (long)c.g.nwin_y * c.g.imax * c.g.kmax;
+    k_sweep_y<CF><<<(unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock), 64 * kWavesPerBlock, 0, c.stream>>>(
+        c.g, c.p, c.ss, src);
+  } else {
+    int last;
+    const long per = AX == 0 ? row_groups(c.g.imax, c.g.nwin_x, c.g.jmax, &last)
+                             : row_groups(c.g.kmax, c.g.nwin_z, c.g.jmax, &last);
+    const long rows = AX == 0 ? c.g.kmax : c.g.imax;
+    k_pencil64<CF><<<(unsigned)(per * rows), 64 * kWavesPerBlock, 0, c.stream>>>(c.g, c.p, c.ss, src);
+  }
 }
 
 template <int AX>
-hipError_t dispatch(const LaunchCtx& c, int src, long waves) {
-  const int blocks = (int)((waves + kWavesPerBlock - 1) / kWavesPerBlock);
+hipError_t dispatch(const LaunchCtx& c, int src) {
   const DevParams& p = c.p;
-  dim3 grid(blocks), block(64 * kWavesPerBlock);
-#define PN_LAUNCH(GX, GY, GZ, EOS, VISC) launch_one<AX, Cfg<AX, GX, GY, GZ, EOS, VISC>>(grid, block, c, src)
+#define PN_LAUNCH(GX, GY, GZ, EOS, VISC) launch_one<AX, Cfg<AX, GX, GY, GZ, EOS, VISC>>(c, src)
   if constexpr (AX == 2) {   // only spherical disks have a theta sweep
     if (p.ngeomx == 1) return hipErrorInvalidValue;
   }
@@ -373,14 +389,8 @@ hipError_t dispatch(const LaunchCtx& c, int src, long waves) {
 
 }  // namespace
 
-hipError_t fp64_sweep_x(const LaunchCtx& c, int src) {
-  return dispatch<0>(c, src, (long)c.g.jmax * c.g.nwin_x * c.g.kmax);
-}
-hipError_t fp64_sweep_y(const LaunchCtx& c, int src) {
-  return dispatch<1>(c, src, (long)c.g.nwin_y * c.g.imax * c.g.kmax);
-}
-hipError_t fp64_sweep_z(const LaunchCtx& c, int src) {
-  return dispatch<2>(c, src, (long)c.g.jmax * c.g.nwin_z * c.g.imax);
-}
+hipError_t fp64_sweep_x(const LaunchCtx& c, int src) { return dispatch<0>(c, src); }
+hipError_t fp64_sweep_y(const LaunchCtx& c, int src) { return dispatch<1>(c, src); }
+hipError_t fp64_sweep_z(const LaunchCtx& c, int src) { return dispatch<2>(c, src); }
 
 }  // namespace pn
