@@ -61,6 +61,24 @@ constexpr int waves64() {
   return CF::EOS == 0 ? 3 : 1;
 }
 
+// CFL term of one direction, (|v| + c_s) / width (timestep.cu:48-73), y = 1 / width: the rounded
+// quotient, and infinity for an infinite speed (which div64 alone would lose)
+__device__ __forceinline__ double cfl_term(double v, double cs, double width, double y) {
+  const double a = fabs(v) + cs;
+  return fmax(div64(a, width, y), 0.5 * (a * y));
+}
+// sqrt(gam p / r) of the CFL, rounded as written; zero and infinity as the library functions have them
+__device__ __forceinline__ double cfl_sound(double gp, double r) {
+  const double y = rcp64(r);
+  const double c2 = fmax(div64(gp, r, y), 0.5 * (gp * y));
+  const double s = sqrt64_rn(c2);
+  return c2 > 0.0 && c2 < 1.0e300 ? s : c2;
+}
+__device__ __forceinline__ double wave_max(double v) {
+  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
+  return v;
+}
+
 // ---------------------------------------------------------------------------------------
 // radial and theta sweeps (sweepx, ppm.cu:26-160; the reference has no caller for the theta sweep,
 // main.cu:376: it is assembled from the theta pieces it holds, forces.cu:298-372,
@@ -81,14 +99,18 @@ struct Tile64 {
   static constexpr int kField = 528;
   double f[NF][kField];
   int srot[kWin];   // rot_j of the window's slots
+  double red[kWavesPerBlock];
 };
 
 // columns of a workgroup's window of lim cells
 __host__ __device__ inline int tile_columns(int lim) { return lim <= kWin / 2 ? 2 * kWavesPerBlock : kWavesPerBlock; }
 
+// With do_cfl (the theta sweep, a 3-D step's last) every thread returns the largest CFL term of the
+// cells it stored.
 template <class CF>
-__device__ __forceinline__ void pencil64(const DevGrid& g, const DevParams& prm, const StepScalars* __restrict__ ss,
-                                         int src, int grp, int l, int row, Tile64<CF::GX == 2 ? 5 : 4>& T) {
+__device__ __forceinline__ double pencil64(const DevGrid& g, const DevParams& prm, const StepScalars* __restrict__ ss,
+                                           int src, int grp, int l, int row, int do_cfl,
+                                           Tile64<CF::GX == 2 ? 5 : 4>& T) {
   constexpr bool TH = CF::AXIS == 2;
   constexpr int NF = CF::GX == 2 ? 5 : 4, TPB = 64 * kWavesPerBlock, NIT = 2;
   const int jmax = g.jmax;
@@ -211,15 +233,41 @@ __device__ __forceinline__ void pencil64(const DevGrid& g, const DevParams& prm,
     }
   }
   __syncthreads();
+  double m = 0.0;
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int c = cs + cstep * it;
     if (jl < jmax && c >= kNpad && c < lim - kNpad) {
-      const long a = (long)(s0 + step * c) * jmax + wrapj(jl - T.srot[c], jmax);
+      const int s = s0 + step * c, j = wrapj(jl - T.srot[c], jmax);
+      const long a = (long)s * jmax + j;
+      double x[NF];
 #pragma unroll
-      for (int f = 0; f < NF; ++f) g.f[src ^ 1][f][a] = T.f[f][qs * ld + c];
+      for (int f = 0; f < NF; ++f) {
+        x[f] = T.f[f][qs * ld + c];
+        g.f[src ^ 1][f][a] = x[f];
+      }
+      if constexpr (TH) {
+        if (do_cfl) {   // k_cfl's terms of this cell
+          const double* t = g.tab + s;
+          const long ts = g.tstride;
+          const double rc = t[kT64Rc * ts], snd = cfl_sound(prm.gam * x[FP], x[FR]);
+          const double wy = g.dy[j] * rc, wz = t[kT64Dz * ts] * t[kT64Rad * ts];
+          m = fmax(m, cfl_term(x[FU], snd, t[kT64Dx * ts], t[kT64Idx * ts]));
+          m = fmax(m, cfl_term(x[FV] - g.rot_v[s] - FrRot * rc, snd, wy, rcp64(wy)));
+          m = fmax(m, cfl_term(x[FW], snd, wz, rcp64(wz)));
+        }
+      }
     }
   }
+  return m;
+}
+
+// the largest of a workgroup's values to *out; red: one double per wave
+__device__ __forceinline__ void block_cfl(double m, double* red, double* out) {
+  m = wave_max(m);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) *out = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
 }
 
 // workgroups of one row's windows: every window but the last is full
@@ -233,7 +281,7 @@ __host__ __device__ inline int row_groups(int len, int nwin, int jmax, int* last
 // so that workgroups of one XCD share the lines of neighbouring columns
 template <class CF>
 __global__ __launch_bounds__(64 * kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(waves64<CF>(), 8))) void k_pencil64(
-    DevGrid g, DevParams prm, const StepScalars* __restrict__ ss, int src) {
+    DevGrid g, DevParams prm, const StepScalars* __restrict__ ss, double* __restrict__ cflp, int src, int do_cfl) {
   __shared__ Tile64<CF::GX == 2 ? 5 : 4> T;
   const int nwin = CF::AXIS == 2 ? g.nwin_z : g.nwin_x, len = CF::AXIS == 2 ? g.kmax : g.imax;
   const int full = (g.jmax + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -242,19 +290,24 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) __attribute__((amdgpu_waves_pe
   const int bid = xcd_swizzle(blockIdx.x, gridDim.x);
   const int row = bid / per, r = bid % per;
   const int l = r < (nwin - 1) * full ? r / full : nwin - 1;
-  pencil64<CF>(g, prm, ss, src, r - l * full, l, row, T);
+  const double m = pencil64<CF>(g, prm, ss, src, r - l * full, l, row, do_cfl, T);
+  if constexpr (CF::AXIS == 2) {
+    if (do_cfl) block_cfl(m, T.red, &cflp[blockIdx.x]);   // kernel-uniform
+  }
 }
 
 // ---------------------------------------------------------------------------------------
 // azimuthal sweep (sweepy, ppm.cu:162-307): pencil = one periodic ring
 template <class CF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves64<CF>(), 8))) void k_sweep_y(DevGrid g, DevParams prm, const StepScalars* __restrict__ ss,
-                                                 int src) {
+                                                 double* __restrict__ cflp, int src, int do_cfl) {
+  __shared__ double red[kWavesPerBlock];
+  double m = 0.0;
   const int lane = threadIdx.x & 63;
   const int gw = xcd_swizzle(blockIdx.x, gridDim.x) * kWavesPerBlock + (threadIdx.x >> 6);
   const int l = gw % g.nwin_y;
   const int n = gw / g.nwin_y;
-  if (n >= g.imax * g.kmax) return;
+  if (n < g.imax * g.kmax) {   // wave-uniform; the barrier is outside
   const int i = n % g.imax, k = n / g.imax;
   const int s = slot_of(g, i, k);
   const int jmax = g.jmax;
@@ -334,29 +387,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves64<CF>
       du[j] = W.w[h];
       dv[j] = W.u[h];
       if (prm.has_w) dw[j] = W.v[h];
+      if constexpr (CF::GY == 3) {
+        if (do_cfl) {   // the next step's CFL terms of this cell, as k_cfl takes them (2-D)
+          const double snd = cfl_sound(prm.gam * p, r), wy = g.dy[j] * rc;
+          m = fmax(m, cfl_term(W.w[h], snd, g.tab[kT64Dx * g.tstride + s], g.tab[kT64Idx * g.tstride + s]));
+          m = fmax(m, cfl_term(W.u[h] - g.rot_v[s] - FrRot * rc, snd, wy, rcp64(wy)));
+        }
+      }
     }
+  }
+  }
+  if constexpr (CF::GY == 3) {
+    if (do_cfl) block_cfl(m, red, &cflp[blockIdx.x]);   // kernel-uniform
   }
 }
 
 template <int AX, class CF>
-void launch_one(const LaunchCtx& c, int src) {
+void launch_one(const LaunchCtx& c, int src, int do_cfl) {
   if constexpr (AX == 1) {
     const long waves = (long)c.g.nwin_y * c.g.imax * c.g.kmax;
     k_sweep_y<CF><<<(unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock), 64 * kWavesPerBlock, 0, c.stream>>>(
-        c.g, c.p, c.ss, src);
+        c.g, c.p, c.ss, c.cflp, src, do_cfl);
   } else {
     int last;
     const long per = AX == 0 ? row_groups(c.g.imax, c.g.nwin_x, c.g.jmax, &last)
                              : row_groups(c.g.kmax, c.g.nwin_z, c.g.jmax, &last);
     const long rows = AX == 0 ? c.g.kmax : c.g.imax;
-    k_pencil64<CF><<<(unsigned)(per * rows), 64 * kWavesPerBlock, 0, c.stream>>>(c.g, c.p, c.ss, src);
+    k_pencil64<CF><<<(unsigned)(per * rows), 64 * kWavesPerBlock, 0, c.stream>>>(c.g, c.p, c.ss, c.cflp, src, do_cfl);
   }
 }
 
 template <int AX>
-hipError_t dispatch(const LaunchCtx& c, int src) {
+hipError_t dispatch(const LaunchCtx& c, int src, int do_cfl) {
+  if (do_cfl && (AX != (c.p.ndim == 3 ? 2 : 1) || fp64_cfl_partials(c.g) > c.ncflp)) return hipErrorInvalidValue;
   const DevParams& p = c.p;
-#define PN_LAUNCH(GX, GY, GZ, EOS, VISC) launch_one<AX, Cfg<AX, GX, GY, GZ, EOS, VISC>>(c, src)
+#define PN_LAUNCH(GX, GY, GZ, EOS, VISC) launch_one<AX, Cfg<AX, GX, GY, GZ, EOS, VISC>>(c, src, do_cfl)
   if constexpr (AX == 2) {   // only spherical disks have a theta sweep
     if (p.ngeomx == 1) return hipErrorInvalidValue;
   }
@@ -389,8 +454,16 @@ hipError_t dispatch(const LaunchCtx& c, int src) {
 
 }  // namespace
 
-hipError_t fp64_sweep_x(const LaunchCtx& c, int src) { return dispatch<0>(c, src); }
-hipError_t fp64_sweep_y(const LaunchCtx& c, int src) { return dispatch<1>(c, src); }
-hipError_t fp64_sweep_z(const LaunchCtx& c, int src) { return dispatch<2>(c, src); }
+int fp64_cfl_partials(const DevGrid& g) {
+  if (g.ndim == 3) {
+    int last;
+    return row_groups(g.kmax, g.nwin_z, g.jmax, &last) * g.imax;
+  }
+  return (g.nwin_y * g.imax + kWavesPerBlock - 1) / kWavesPerBlock;
+}
+
+hipError_t fp64_sweep_x(const LaunchCtx& c, int src) { return dispatch<0>(c, src, 0); }
+hipError_t fp64_sweep_y(const LaunchCtx& c, int src, int do_cfl) { return dispatch<1>(c, src, do_cfl); }
+hipError_t fp64_sweep_z(const LaunchCtx& c, int src, int do_cfl) { return dispatch<2>(c, src, do_cfl); }
 
 }  // namespace pn

@@ -40,8 +40,11 @@ hipError_t fp64_prep(const LaunchCtx& c);
 hipError_t fp64_tab_theta(const LaunchCtx& c);
 // FP64 path (pn_kernels_fp64.hip); each returns hipSuccess or the launch error
 hipError_t fp64_sweep_x(const LaunchCtx& c, int src);
-hipError_t fp64_sweep_y(const LaunchCtx& c, int src);
-hipError_t fp64_sweep_z(const LaunchCtx& c, int src);
+// do_cfl (the step's last sweep: azimuthal in 2-D, theta in 3-D): each workgroup's CFL maximum of
+// the state it stores to c.cflp[workgroup], fp64_cfl_partials of them
+hipError_t fp64_sweep_y(const LaunchCtx& c, int src, int do_cfl);
+hipError_t fp64_sweep_z(const LaunchCtx& c, int src, int do_cfl);
+int fp64_cfl_partials(const DevGrid& g);
 
 // common small kernels (pn_kernels_common.hip)
 hipError_t launch_index_shift(const LaunchCtx& c);

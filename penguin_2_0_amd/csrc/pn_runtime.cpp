@@ -80,19 +80,19 @@ int nwin(int len) { return (len + kReal - 1) / kReal; }
 
 bool is_f32(const pn_ctx* c) { return c->precision == PN_FP32; }
 
-// the next step's CFL maximum can be taken in the last sweep's epilogue when FrRot cannot
-// change inside a step, i.e. unless the planet moves under the disk's torque
-// the next dt from the last sweep's epilogue: FP32, no work after the sweeps that changes the
-// state the CFL reads (a moving planet's update reads the sweeps' result; damping changes it)
-bool fused_cfl(const pn_ctx* c) { return is_f32(c) && c->P.plnt_flag < 2 && !c->P.kill_flag; }
+// the next dt from the last sweep's epilogue: FrRot cannot change inside a step (it does when the
+// planet moves under the disk's torque) and nothing after the sweeps changes the state the CFL
+// reads (damping does)
+bool fused_cfl(const pn_ctx* c) { return c->P.plnt_flag < 2 && !c->P.kill_flag; }
 
 // the FP32 radial sweep of the context's geometry
 hipError_t f32_x(const pn_ctx* c, const LaunchCtx& L, int variant, int src) {
   return (c->P.ndim == 3) ? f32_sweep_x3(L, c->df, variant, src) : f32_sweep_x(L, c->df, variant, src);
 }
 
-// CFL partials the step's last FP32 sweep writes
-int f32_fused_partials(const pn_ctx* c) {
+// CFL partials the step's last sweep writes
+int fused_partials(const pn_ctx* c) {
+  if (!is_f32(c)) return fp64_cfl_partials(c->dg);
   return (c->P.ndim == 3) ? f32_cfl_partials_z(c->dg, c->var_z) : f32_cfl_partials_y(c->dg, c->var_y);
 }
 
@@ -171,9 +171,9 @@ int launch_sweeps(pn_ctx* c, int& cur, int do_cfl, bool prep, bool roll) {
     if (prep) PN_LAUNCH(c, "prep", fp64_prep(L));
     PN_LAUNCH(c, "ghosts", launch_fill_ghosts(L, cur));
     PN_LAUNCH(c, "sweep_x", fp64_sweep_x(L, cur));
-    PN_LAUNCH(c, "sweep_y", fp64_sweep_y(L, cur ^ 1));
+    PN_LAUNCH(c, "sweep_y", fp64_sweep_y(L, cur ^ 1, c->P.ndim == 2 ? do_cfl : 0));
     if (c->P.ndim == 3) {
-      PN_LAUNCH(c, "sweep_z", fp64_sweep_z(L, cur));
+      PN_LAUNCH(c, "sweep_z", fp64_sweep_z(L, cur, do_cfl));
       cur ^= 1;
     }
   }
@@ -200,7 +200,7 @@ int launch_step(pn_ctx* c, int& cur) {
   if ((rc = launch_sweeps(c, cur, fused ? 1 : 0, false, !post)) != PN_OK) return rc;
   // damping zones: ring-uniform relaxation, which commutes with the integer roll
   if (c->P.kill_flag) PN_LAUNCH(c, "damp", is_f32(c) ? f32_damp(L, c->df, cur) : launch_damp(L, cur));
-  if (post) PN_LAUNCH(c, "post step", launch_post_step(L, fused ? f32_fused_partials(c) : 0));
+  if (post) PN_LAUNCH(c, "post step", launch_post_step(L, fused ? fused_partials(c) : 0));
   else PN_LAUNCH(c, "planet update", launch_planet_after_sweep(L, cur, is_f32(c) ? &c->df : nullptr));
   return PN_OK;
 }
@@ -566,8 +566,8 @@ int pn_create(const pn_grid* g, const pn_params* p, int precision, pn_ctx** out)
   if (r2 == PN_OK) r2 = dalloc(c, &c->out2, 2);
   if (r2 == PN_OK) r2 = dalloc(c, &c->ringbuf, static_cast<size_t>(g->imax) * g->kmax);
   // CFL partials: one per block of the grid-stride CFL kernels (at most 2048) or one per
-  // workgroup of the FP32 sweep that takes the CFL in its epilogue, in any variant
-  c->ncflp = 2048;
+  // workgroup of the sweep that takes the CFL in its epilogue (FP32: in any variant)
+  c->ncflp = precision == PN_FP64 ? std::max(2048, fp64_cfl_partials(d)) : 2048;
   if (precision == PN_FP32)
     for (int v = 0; v < kNumF32VariantsZ; ++v) {
       if (v < kNumF32Variants) c->ncflp = std::max(c->ncflp, f32_cfl_partials_y(d, v));
@@ -1162,7 +1162,7 @@ int pn_sweep_axis(pn_ctx* c, int axis, double dt, const pn_body* planet, double 
   } else {
     PN_LAUNCH(c, "prep", fp64_prep(L));
     if (axis == 0) PN_LAUNCH(c, "ghosts", launch_fill_ghosts(L, c->cur));
-    hipError_t e = (axis == 0) ? fp64_sweep_x(L, c->cur) : (axis == 1) ? fp64_sweep_y(L, c->cur) : fp64_sweep_z(L, c->cur);
+    hipError_t e = (axis == 0) ? fp64_sweep_x(L, c->cur) : (axis == 1) ? fp64_sweep_y(L, c->cur, 0) : fp64_sweep_z(L, c->cur, 0);
     if (e != hipSuccess) return fail(c, PN_ERR_HIP, "sweep %d: %s", axis, hipGetErrorString(e));
   }
   if ((rc = sync(c)) != PN_OK) return rc;
@@ -1197,11 +1197,11 @@ int pn_time_kernels(pn_ctx* c, int nrep, double* ms6) {
           c->cur ^= 1;
           break;
         case 3:
-          e = is_f32(c) ? f32_sweep_y(L, c->df, c->var_y, c->cur, c->P.ndim == 2) : fp64_sweep_y(L, c->cur);
+          e = is_f32(c) ? f32_sweep_y(L, c->df, c->var_y, c->cur, c->P.ndim == 2) : fp64_sweep_y(L, c->cur, c->P.ndim == 2);
           c->cur ^= 1;
           break;
         case 4:
-          e = is_f32(c) ? f32_sweep_z(L, c->df, c->var_z, c->cur, 1) : fp64_sweep_z(L, c->cur);
+          e = is_f32(c) ? f32_sweep_z(L, c->df, c->var_z, c->cur, 1) : fp64_sweep_z(L, c->cur, 1);
           c->cur ^= 1;
           break;
         case 5: e = launch_rotate(L); break;
