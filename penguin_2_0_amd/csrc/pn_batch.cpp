@@ -191,21 +191,31 @@ LaunchCtx on_batch(pn_batch* b, pn_ctx* c) {
   return L;
 }
 
+// every disk's dt comes from its last sweep: consecutive steps then share a launch (k_mid_step_batch)
+bool all_fused(const pn_batch* b) {
+  for (const pn_ctx* c : b->disks)
+    if (cfl_before_step(c)) return false;
+  return true;
+}
+
 // one step of every disk: the CFL pass of each disk whose planet moves or which has damping
 // zones, the batched pre-step, each disk's radial ghost copies, the batched sweeps, each
 // damped disk's damping, the batched post-step,
 // then each moving planet's time, drift, disk forces (modes 8 / 9 from its FP32 state) and
 // closing kick -- the order pn_run gives a single disk (damping is ring-uniform, so it commutes
-// with the roll that the post-step does for a moving planet's disk)
-int launch_batch_step(pn_batch* b, int cur) {
+// with the roll that the post-step does for a moving planet's disk).  With every CFL fused, a step
+// that is not its run's first starts from the tables its predecessor left and one that is not its
+// last ends in the mid-step (post-step and next pre-step).
+int launch_batch_step(pn_batch* b, int cur, bool first, bool last) {
   const int n = ndisk(b);
+  const bool fused = all_fused(b);
   hipError_t e = hipSuccess;
   for (pn_ctx* c : b->disks) {
     if (!cfl_before_step(c) || e != hipSuccess) continue;
     int ncfl = 0;
     e = f32_cfl(on_batch(b, c), c->df, cur, &ncfl);
   }
-  if (e == hipSuccess) e = launch_pre_step_batch(b->stream, b->dd, n);
+  if (e == hipSuccess && (!fused || first)) e = launch_pre_step_batch(b->stream, b->dd, n);
   for (pn_ctx* c : b->disks) {   // radial boundary codes other than 3 (launches nothing for 3)
     if (e != hipSuccess) break;
     e = f32_fill_ghosts(on_batch(b, c), c->df, cur);
@@ -216,7 +226,10 @@ int launch_batch_step(pn_batch* b, int cur) {
     if (!c->P.kill_flag || e != hipSuccess) continue;
     e = f32_damp(on_batch(b, c), c->df, cur);
   }
-  if (e == hipSuccess) e = launch_post_step_batch(b->stream, b->dd, n);
+  if (e == hipSuccess) {
+    if (fused && !last) e = launch_mid_step_batch(b->stream, b->dd, n);
+    else e = launch_post_step_batch(b->stream, b->dd, n);
+  }
   for (pn_ctx* c : b->disks) {
     if (c->P.plnt_flag != 2 || e != hipSuccess) continue;
     e = launch_planet_after_sweep(on_batch(b, c), cur, &c->df);
@@ -225,18 +238,21 @@ int launch_batch_step(pn_batch* b, int cur) {
   return PN_OK;
 }
 
-// n steps of every disk from buffer cur (a 2-D step returns there): replays of the step
-// captured as a graph from that buffer, or direct launches
+// n steps of every disk from buffer cur (a 2-D step returns there): replays of a middle step
+// captured as a graph from that buffer (with every CFL fused: sweeps and mid-step, between the
+// first pre-step and a last step launched directly), or direct launches
 int batch_steps(pn_batch* b, int cur, int nsteps, int graph) {
+  const bool fused = all_fused(b);
   int done = 0, rc;
-  if (graph && nsteps > 0) {
+  const bool replay = graph && nsteps > 1;
+  if (replay) {
     // the captured step names its buffer; a disk moved to the other one since (for example by
     // pn_sweep_axis on pn_batch_disk) needs a step captured from there
     if (b->gexec && b->gexec_cur != cur) drop_graph(b);
     if (!b->gexec) {
       hipGraph_t gr;
       PB_HIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-      rc = launch_batch_step(b, cur);
+      rc = launch_batch_step(b, cur, false, false);
       hipError_t e = hipStreamEndCapture(b->stream, &gr);
       if (rc != PN_OK) return rc;
       if (e != hipSuccess) return bfail(b, PN_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
@@ -245,10 +261,11 @@ int batch_steps(pn_batch* b, int cur, int nsteps, int graph) {
       if (e != hipSuccess) return bfail(b, PN_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
       b->gexec_cur = cur;
     }
-    for (; done < nsteps; ++done) PB_HIP(b, hipGraphLaunch(b->gexec, b->stream));
+    if (fused) PB_HIP(b, launch_pre_step_batch(b->stream, b->dd, ndisk(b)));
+    for (; done < (fused ? nsteps - 1 : nsteps); ++done) PB_HIP(b, hipGraphLaunch(b->gexec, b->stream));
   }
-  for (; done < nsteps; ++done)
-    if ((rc = launch_batch_step(b, cur)) != PN_OK) return rc;
+  for (bool first = !(replay && fused); done < nsteps; ++done, first = false)
+    if ((rc = launch_batch_step(b, cur, first, done == nsteps - 1)) != PN_OK) return rc;
   return PN_OK;
 }
 

@@ -41,8 +41,8 @@ struct pn_ctx {
   // host copies of the per-ring values the device never changes (for packing)
   std::vector<double> h_x, h_dx, h_xc, h_xvol, h_z, h_dz, h_zc, h_zvol, h_vbg, h_rbg, h_cs2, h_qbg;
   std::vector<double> h_y, h_dy, h_yc, h_yvol;
-  // graph of one step (2-D) or two steps (3-D, the buffers alternate)
-  hipGraphExec_t gexec = nullptr;
+  // graphs of one unit of steps (2-D: one; 3-D: two, the buffers alternate) and of several
+  hipGraphExec_t gexec[2] = {nullptr, nullptr};
   int gexec_cur = 0;   // the buffer the captured steps start from (and, whole, end on)
   // host copies of the fixed inputs, so a snapshot can be re-entered (restart)
   std::vector<char> h_lft, h_rgh, h_udr, h_top;
@@ -60,6 +60,7 @@ int upload_scalars(pn_ctx* c, const StepScalars& h);
 int download_scalars(pn_ctx* c, StepScalars* h);
 int sync(pn_ctx* c);
 int launch_cfl_any(pn_ctx* c, int src);
+void drop_graphs(pn_ctx* c);
 // steps from dt0 that cannot reach a landing room away (dt grows by at most 1.1 per step)
 int steps_before_landing(double dt0, double room, int cap);
 

@@ -403,8 +403,7 @@ __device__ double block_max_partials(const double* __restrict__ cflp, int n, dou
   m = wave_max(m);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0)
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) m = fmax(m, sh[w]);
+  if (threadIdx.x < 64) m = wave_max(threadIdx.x < (int)(blockDim.x >> 6) ? sh[threadIdx.x] : 0.0);
   return m;
 }
 
@@ -610,7 +609,7 @@ __device__ __forceinline__ void post_step_body(DevGrid g, const DevParams& prm, 
   if (roll && prm.fargo > 0) roll_rings(g);
   double mx = 0.0;
   if (ncfl > 0) mx = block_max_partials(cflp, ncfl, sh);
-  if (threadIdx.x != 0) return;
+  if (threadIdx.x != 0) return;   // the caller's next barrier, if it has one, is every thread's
   const double dt = ss->dt;
   ss->simtime += dt;
   ss->ncycle += 1;
@@ -641,10 +640,41 @@ __global__ __launch_bounds__(kStepThreads) void k_post_step(DevGrid g, DevParams
   post_step_body(g, prm, ss, cflp, ncfl, roll != 0);
 }
 
+// The end of one step and the beginning of the next in one workgroup, for a step whose dt comes
+// from its last sweep's CFL: between two steps a disk then launches this alone, where the two
+// bodies apart cost two launches (128 x 384, FP32: 29.6 -> 23.0 us a step with the longer graphs).
+// Every thread rolls and shifts the same rings in both bodies, so between them only thread 0's
+// scalars have to be seen.
+__global__ __launch_bounds__(kStepThreads) void k_mid_step(DevGrid g, DevParams prm, StepScalars* ss,
+                                                           const double* __restrict__ cflp, int ncfl, float2* trig,
+                                                           float* tab, float* tabz, int tstride, int rings) {
+  post_step_body(g, prm, ss, cflp, ncfl, rings != 0);
+  __syncthreads();
+  pre_step_body(g, prm, ss, nullptr, 0, trig, tab, tabz, tstride, rings != 0);
+}
+
+// the per-slot part of both over the whole grid, one thread per slot, after k_mid_step with rings
+// 0: the roll of the step that ended, then k_pre_rings' work
+__global__ __launch_bounds__(256) void k_mid_rings(DevGrid g, DevParams prm, const StepScalars* ss, float* tab,
+                                                   float* tabz, int tstride) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= g.sr * g.sk) return;
+  if (prm.fargo > 0) {
+    const int i = s % g.sr - kNpad, k = s / g.sr - g.k0;
+    if (i >= 0 && i < g.imax && k >= 0 && k < g.kmax) {
+      int j = g.rot_j[s] + g.inc_j[s];
+      if (j < 0) j += g.jmax;
+      if (j >= g.jmax) j -= g.jmax;
+      g.rot_j[s] = j;
+    }
+  }
+  ring_slot(g, prm, ss->dt, ss->fr_shift, ss->planet.vy, tab, tabz, tstride, s);
+}
+
 // the largest of n CFL partials per workgroup, grid-strided: a disk whose fused CFL leaves
 // more partials than kSplitPartials has them folded into kCflChunks maxima first, so the
 // single-workgroup post-step reads few
-constexpr int kSplitPartials = 4096, kCflChunks = 256;
+constexpr int kSplitPartials = 8192, kCflChunks = 256;
 __global__ __launch_bounds__(256) void k_max_chunks(const double* __restrict__ in, int n, double* __restrict__ out) {
   __shared__ double sh[4];
   double m = 0.0;
@@ -664,6 +694,14 @@ __global__ __launch_bounds__(kStepThreads) void k_post_step_batch(const DiskDev*
     return;
   }
   post_step_body(D.g, D.p, D.ss, D.cflp, D.ncfl_post, true);
+}
+
+// one workgroup per disk of a batch whose every dt comes from its last sweep: k_mid_step
+__global__ __launch_bounds__(kStepThreads) void k_mid_step_batch(const DiskDev* __restrict__ dd) {
+  const DiskDev& D = dd[blockIdx.x];
+  post_step_body(D.g, D.p, D.ss, D.cflp, D.ncfl_post, true);
+  __syncthreads();
+  pre_step_body(D.g, D.p, D.ss, nullptr, 0, D.trig, D.tab, nullptr, D.tstride, true);
 }
 
 int red_blocks(const DevGrid& g) {
@@ -780,6 +818,37 @@ hipError_t launch_pre_step(const LaunchCtx& c, int ncfl, float2* trig, float* ta
   return hipGetLastError();
 }
 
+namespace {
+// the CFL partials a single workgroup reads: folded first when there are many (the reduction
+// scratch is free while a step runs)
+const double* fold_partials(const LaunchCtx& c, int ncfl, int* np) {
+  *np = ncfl;
+  if (ncfl <= kSplitPartials) return c.cflp;
+  k_max_chunks<<<kCflChunks, 256, 0, c.stream>>>(c.cflp, ncfl, c.partials);
+  *np = kCflChunks;
+  return c.partials;
+}
+}  // namespace
+
+hipError_t launch_mid_step(const LaunchCtx& c, int ncfl, float2* trig, float* tab, float* tabz, int tstride) {
+  if (ncfl < 1 || ncfl > c.ncflp || c.p.plnt == 2) return hipErrorInvalidValue;
+  const bool split = split_rings(c.g);
+  int np;
+  const double* parts = fold_partials(c, ncfl, &np);
+  k_mid_step<<<1, kStepThreads, 0, c.stream>>>(c.g, c.p, c.ss, parts, np, trig, tab, tabz, tstride, split ? 0 : 1);
+  if (split) {
+    const int n = c.g.sr * c.g.sk;
+    k_mid_rings<<<(n + 255) / 256, 256, 0, c.stream>>>(c.g, c.p, c.ss, tab, tabz, tstride);
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_mid_step_batch(hipStream_t s, const DiskDev* dd, int ndisk) {
+  if (ndisk < 1) return hipErrorInvalidValue;
+  k_mid_step_batch<<<ndisk, kStepThreads, 0, s>>>(dd);
+  return hipGetLastError();
+}
+
 hipError_t launch_post_step(const LaunchCtx& c, int ncfl) {
   if (ncfl < 0 || ncfl > c.ncflp || c.p.plnt == 2) return hipErrorInvalidValue;
   const bool split = split_rings(c.g);
@@ -787,13 +856,8 @@ hipError_t launch_post_step(const LaunchCtx& c, int ncfl) {
     const int n = c.g.imax * c.g.kmax;
     k_rotate<<<(n + 255) / 256, 256, 0, c.stream>>>(c.g);
   }
-  const double* parts = c.cflp;
-  int np = ncfl;
-  if (ncfl > kSplitPartials) {   // the reduction scratch is free while a step runs
-    k_max_chunks<<<kCflChunks, 256, 0, c.stream>>>(c.cflp, ncfl, c.partials);
-    parts = c.partials;
-    np = kCflChunks;
-  }
+  int np;
+  const double* parts = fold_partials(c, ncfl, &np);
   k_post_step<<<1, kStepThreads, 0, c.stream>>>(c.g, c.p, c.ss, parts, np, split ? 0 : 1);
   return hipGetLastError();
 }

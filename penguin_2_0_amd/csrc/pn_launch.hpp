@@ -81,9 +81,13 @@ hipError_t launch_pre_step(const LaunchCtx& c, int ncfl, float2* trig, float* ta
 // from ncfl partials when ncfl > 0 (disks of many slots: the roll from a grid-wide kernel;
 // many partials: folded first by a grid-wide kernel into the reduction scratch)
 hipError_t launch_post_step(const LaunchCtx& c, int ncfl);
+// launch_post_step of one step and launch_pre_step (ncfl 0) of the next in one workgroup; ncfl >= 1,
+// plnt_flag < 2
+hipError_t launch_mid_step(const LaunchCtx& c, int ncfl, float2* trig, float* tab, float* tabz, int tstride);
 // the same for every disk of a batch, one workgroup per disk (pre-step with ncfl 0; post-step
 // with each disk's ncfl_post)
 hipError_t launch_pre_step_batch(hipStream_t s, const DiskDev* dd, int ndisk);
 hipError_t launch_post_step_batch(hipStream_t s, const DiskDev* dd, int ndisk);
+hipError_t launch_mid_step_batch(hipStream_t s, const DiskDev* dd, int ndisk);
 
 }  // namespace pn

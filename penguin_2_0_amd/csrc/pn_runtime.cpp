@@ -64,6 +64,13 @@ int dalloc(pn_ctx* c, T** p, size_t n) {
   return PN_OK;
 }
 
+void drop_graphs(pn_ctx* c) {
+  for (hipGraphExec_t& g : c->gexec) {
+    if (g) hipGraphExecDestroy(g);
+    g = nullptr;
+  }
+}
+
 LaunchCtx lctx(pn_ctx* c) {
   LaunchCtx L;
   L.g = c->dg;
@@ -182,9 +189,12 @@ int launch_sweeps(pn_ctx* c, int& cur, int do_cfl, bool prep, bool roll) {
 }
 
 // one full step of main.cu:345-387 on the device, reading and writing c->ss:
-//   [CFL partials] pre-step (dt, Index_Shift, half kick, FP32 tables) -> sweeps -> post-step
-// (roll, planet, time, and the next dt when the CFL is fused into the last sweep)
-int launch_step(pn_ctx* c, int& cur) {
+//   [CFL partials] pre-step (dt, Index_Shift, half kick, per-step tables) -> sweeps -> post-step
+// (roll, planet, time, and the next dt when the CFL is fused into the last sweep).  With a fused CFL
+// consecutive steps share a launch: a step that is not the first of its run starts from the tables
+// its predecessor left (first = false), one that is not the last ends in the mid-step (last =
+// false), post-step and next pre-step in one.
+int launch_step(pn_ctx* c, int& cur, bool first, bool last) {
   LaunchCtx L = lctx(c);
   const bool fused = fused_cfl(c);
   int ncfl = 0, rc;
@@ -195,9 +205,13 @@ int launch_step(pn_ctx* c, int& cur) {
   float2* trig = is_f32(c) ? c->df.trig : nullptr;
   float* tab = is_f32(c) ? c->df.tab : nullptr;
   float* tabz = is_f32(c) ? c->df.tabz : nullptr;
-  PN_LAUNCH(c, "pre step", launch_pre_step(L, ncfl, trig, tab, tabz, c->df.tstride));
+  if (!fused || first) PN_LAUNCH(c, "pre step", launch_pre_step(L, ncfl, trig, tab, tabz, c->df.tstride));
   const bool post = c->P.plnt_flag < 2;
   if ((rc = launch_sweeps(c, cur, fused ? 1 : 0, false, !post)) != PN_OK) return rc;
+  if (fused && !last) {
+    PN_LAUNCH(c, "mid step", launch_mid_step(L, fused_partials(c), trig, tab, tabz, c->df.tstride));
+    return PN_OK;
+  }
   // damping zones: ring-uniform relaxation, which commutes with the integer roll
   if (c->P.kill_flag) PN_LAUNCH(c, "damp", is_f32(c) ? f32_damp(L, c->df, cur) : launch_damp(L, cur));
   if (post) PN_LAUNCH(c, "post step", launch_post_step(L, fused ? fused_partials(c) : 0));
@@ -648,7 +662,7 @@ int pn_destroy(pn_ctx* c) {
   if (!c) return PN_OK;
   // drain first: no replay of the graph, and no kernel reading these buffers, may still run
   if (c->stream) hipStreamSynchronize(c->stream);
-  if (c->gexec) hipGraphExecDestroy(c->gexec);
+  drop_graphs(c);
   for (void* q : c->allocs) hipFree(q);
   if (c->stage && c->stage_pinned) hipHostFree(c->stage);
   else std::free(c->stage);
@@ -1075,10 +1089,7 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
   }
   c->cur = 0;
   c->loaded = true;
-  if (c->gexec) {
-    hipGraphExecDestroy(c->gexec);
-    c->gexec = nullptr;
-  }
+  drop_graphs(c);
   return PN_OK;
 }
 
@@ -1295,10 +1306,7 @@ int pn_tune(pn_ctx* c, int nrep, int* var_x, int* var_y) {
   c->df.nwin_y = f32_windows(c->g.jmax, kF32VariantsY[by][0]);
   c->df.nwin_z = f32_windows(c->g.kmax, kF32VariantsZ[bz][0]);
   c->tuned = true;
-  if (c->gexec) {
-    hipGraphExecDestroy(c->gexec);
-    c->gexec = nullptr;
-  }
+  drop_graphs(c);
   if (var_x) *var_x = bx;
   if (var_y) *var_y = by;
   return PN_OK;
@@ -1321,10 +1329,7 @@ int pn_set_variant_z(pn_ctx* c, int var_z) {
   c->var_z = var_z;
   c->df.nwin_z = f32_windows(c->g.kmax, kF32VariantsZ[var_z][0]);
   c->tuned = true;
-  if (c->gexec) {
-    hipGraphExecDestroy(c->gexec);
-    c->gexec = nullptr;
-  }
+  drop_graphs(c);
   return PN_OK;
 }
 
@@ -1338,10 +1343,7 @@ int pn_set_packing(pn_ctx* c, int on) {
   if (!c || (on != 0 && on != 1)) return PN_ERR_ARG;
   c->pack_tails = on;
   c->df.pack_tails = on;
-  if (c->gexec) {   // the captured launches carry the old flag
-    hipGraphExecDestroy(c->gexec);
-    c->gexec = nullptr;
-  }
+  drop_graphs(c);   // the captured launches carry the old flag
   return PN_OK;
 }
 
@@ -1359,10 +1361,7 @@ int pn_set_variants(pn_ctx* c, int var_x, int var_y) {
   c->df.nwin_y = f32_windows(c->g.jmax, kF32VariantsY[var_y][0]);
   c->df.nwin_z = f32_windows(c->g.kmax, kF32VariantsZ[var_x][0]);
   c->tuned = true;
-  if (c->gexec) {
-    hipGraphExecDestroy(c->gexec);
-    c->gexec = nullptr;
-  }
+  drop_graphs(c);
   return PN_OK;
 }
 
@@ -1493,41 +1492,52 @@ namespace pn {
 namespace rt {
 namespace {
 
-// n steps from the current buffer: captured-graph replays for whole units of per_graph steps
-// (a 3-D step flips the buffer, so its graph holds two), the rest launched directly.  A
-// graph is captured from the buffer the state is in and captured again when an odd number of
-// direct 3-D steps has moved the state to the other one.
+// n steps from the current buffer: replays of captured steps, the rest launched directly.  The
+// captured steps are middle ones (with a fused CFL: sweeps and mid-step), so they need the first
+// pre-step before them and a last step after them.  Two graphs are kept: one unit (a 3-D step flips
+// the buffer, so its unit is two steps), and kGraphUnits of them for long runs, whose replays leave
+// about 3 us fewer between steps.  A graph is captured from the buffer the state is in and
+// captured again when the state has moved to the other one.
+constexpr int kGraphUnits = 8;
+
 int run_steps(pn_ctx* c, int nsteps, int graph) {
-  const int per_graph = (c->P.ndim == 3) ? 2 : 1;
+  const int unit = (c->P.ndim == 3) ? 2 : 1;
+  const bool fused = fused_cfl(c);
   int done = 0, rc;
-  if (graph && nsteps >= per_graph) {
-    if (c->gexec && c->gexec_cur != c->cur) {
-      hipGraphExecDestroy(c->gexec);
-      c->gexec = nullptr;
+  if (graph && nsteps > unit) {
+    if (c->gexec_cur != c->cur) drop_graphs(c);
+    // with a fused CFL the first step's pre-step stands alone and the last step is a direct one
+    const int room = fused ? nsteps - 1 : nsteps;
+    if (fused) {
+      PN_LAUNCH(c, "pre step", launch_pre_step(lctx(c), 0, is_f32(c) ? c->df.trig : nullptr, is_f32(c) ? c->df.tab : nullptr,
+                                               is_f32(c) ? c->df.tabz : nullptr, c->df.tstride));
     }
-    if (!c->gexec) {
-      hipGraph_t gr;
-      PN_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      int cur = c->cur;
-      rc = PN_OK;
-      for (int s = 0; s < per_graph && rc == PN_OK; ++s) rc = launch_step(c, cur);
-      hipError_t e = hipStreamEndCapture(c->stream, &gr);
-      if (rc != PN_OK) return rc;
-      if (e != hipSuccess) return fail(c, PN_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
-      if (cur != c->cur) return fail(c, PN_ERR_STATE, "captured steps do not return to their buffer");
-      e = hipGraphInstantiate(&c->gexec, gr, nullptr, nullptr, 0);
-      hipGraphDestroy(gr);
-      if (e != hipSuccess) return fail(c, PN_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
-      c->gexec_cur = c->cur;
-    }
-    while (nsteps - done >= per_graph) {
-      PN_HIP(c, hipGraphLaunch(c->gexec, c->stream));
-      done += per_graph;
+    for (int size = 1; size >= 0; --size) {
+      const int per = size ? kGraphUnits * unit : unit;
+      // the long graph pays for its capture over a few replays
+      if (size ? room < 3 * per : room - done < per) continue;
+      if (!c->gexec[size]) {
+        hipGraph_t gr;
+        PN_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+        int cur = c->cur;
+        rc = PN_OK;
+        for (int s = 0; s < per && rc == PN_OK; ++s) rc = launch_step(c, cur, false, false);
+        hipError_t e = hipStreamEndCapture(c->stream, &gr);
+        if (rc != PN_OK) return rc;
+        if (e != hipSuccess) return fail(c, PN_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
+        if (cur != c->cur) return fail(c, PN_ERR_STATE, "captured steps do not return to their buffer");
+        e = hipGraphInstantiate(&c->gexec[size], gr, nullptr, nullptr, 0);
+        hipGraphDestroy(gr);
+        if (e != hipSuccess) return fail(c, PN_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
+        c->gexec_cur = c->cur;
+      }
+      for (; room - done >= per; done += per) PN_HIP(c, hipGraphLaunch(c->gexec[size], c->stream));
     }
   }
   int cur = c->cur;
-  for (; done < nsteps; ++done)
-    if ((rc = launch_step(c, cur)) != PN_OK) return rc;
+  const bool primed = fused && graph && nsteps > unit;   // the pre-step of the next step has run
+  for (bool first = !primed; done < nsteps; ++done, first = false)
+    if ((rc = launch_step(c, cur, first, done == nsteps - 1)) != PN_OK) return rc;
   c->cur = cur;
   return PN_OK;
 }
