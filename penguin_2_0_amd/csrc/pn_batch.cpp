@@ -94,9 +94,8 @@ int build_order_x(pn_batch* b, std::vector<int>& order, int& nslots) {
     const int nwin = f32_windows(c->g.imax, K), ngrp = (c->g.jmax + nc - 1) / nc;
     for (int l = 0; l < nwin; ++l) {
       const int lim = (l < nwin - 1) ? 64 * K : c->g.imax - real * (nwin - 1) + 2 * kNpad;
-      double passes = 1.0;
-      if (c->df.pack_tails && K == 4 && lim <= 21 * K) passes = 1.0 / 3.0;
-      else if (c->df.pack_tails && lim <= 32 * K) passes = 0.5;
+      // a short window runs several columns per wavefront pass (pencil_item)
+      const double passes = c->df.pack_tails && lim <= 32 * K ? 1.0 / (64 / ((lim + K - 1) / K)) : 1.0;
       const double cost = 0.3 * lim / (64.0 * K) + 0.7 * passes;
       for (int g = 0; g < ngrp; ++g) {
         items.push_back({d, l * ngrp + g, cost});

@@ -54,6 +54,8 @@ enum TabEntry {
   kTabRotPhS, kTabRotPhC,
   // EOS 3 (2-D): q_b = p_b / rho_b and q_b(s+1) - q_b(s)
   kTabQb, kTabDqb,
+  // reciprocals: of rho_b, p_b, the radial width and volume, the theta width and volume
+  kTabIrb, kTabIpb, kTabIdx0, kTabIdvol0, kTabIdz0, kTabIdvolZ,
   kTabEntries
 };
 constexpr int kTabOverhang = 256;   // >= the longest radial window
@@ -69,13 +71,14 @@ struct DevF32 {
   // are consecutive); stride tstride; its per-step rows are rewritten beside the others
   float* tabz;
   const double *rbg, *vbg;     // Sigma_b and v_bg per slot, FP64
-  const float *dy, *yvol;      // per column
+  const float* dy;             // per column
+  const float4* col;           // per column: dphi, its volume factor, and their reciprocals
   float2* trig;                // per column, per step: sin / cos of half the angle to the planet
   int nwin_x, nwin_y, nwin_z;  // windows of the variant in use
   int uniform_phi;             // every dphi equal: the azimuthal paraset is (1/2, -1/6, 1/6, 1/2, 1/2)
   int uniform_theta;           // every dtheta equal (3-D)
-  int pack_tails;              // radial / theta: a last window of at most 32 K cells runs two
-                               // columns per wavefront (same results, half the passes)
+  int pack_tails;              // radial / theta: a window of at most 32 K cells runs as many
+                               // columns per wavefront as fit (same results, fewer passes)
 };
 
 constexpr int kNumF32Variants = 4;

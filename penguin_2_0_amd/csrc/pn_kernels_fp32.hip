@@ -20,16 +20,14 @@ namespace pn {
 // Occupancy.  A SIMD's 512 VGPRs per lane hold eight waves of at most 64 VGPRs, six of 80,
 // five of 96 and four of 128; amdgpu_waves_per_eu asks the allocator to fit a count, spilling
 // what does not fit to scratch.
-// - LDS-staged pencils: the allocator left alone settles them at 99-122 (four waves).  A
-//   workgroup of four waves puts one on each SIMD, so a fifth wave per SIMD is a fifth
-//   workgroup per CU, which the LDS must hold too; for those shapes the kernels ask for five
-//   (pencil_waves).  It costs a few spills per pencil (radial sweep 1024 x 3072: two) and took
-//   that sweep from 75.1 to 73.3 us.  Workgroups of eight or sixteen waves gain nothing short
-//   of six or eight waves per SIMD, so they ask for nothing.
-// - Azimuthal windows of 128 cells: 66 VGPRs for a 2-D isothermal disk (seven waves; eight at
-//   64 for four spills) and 86 for the batch (five waves; six at 80 for six spills).  Longer
-//   windows and the 3-D and EOS 3 forms spill tens of values at the next step down, so they
-//   keep what the allocator gives (a minimum of one wave asks for nothing).
+// - LDS-staged pencils: the allocator left alone settles them at 99-136 (three or four waves).
+//   A workgroup of four waves puts one on each SIMD, so a fifth wave per SIMD is a fifth
+//   workgroup per CU, which the LDS must hold too; the kernels ask for as many as that allows
+//   (pencil_waves).  A 2-D isothermal pencil fits 96 without a spill.
+// - Azimuthal windows of 128 cells: eight waves (64 VGPRs, three spills) for a 2-D isothermal
+//   disk, six (80) in the batch; of 256 cells: four waves (128).  The EOS 3 forms spill tens of
+//   values at the next step down, so they keep what the allocator gives (a minimum of one wave
+//   asks for nothing).
 #define PN_WAVES(n) __attribute__((amdgpu_waves_per_eu(n, 8)))
 
 namespace {
@@ -147,24 +145,24 @@ struct XTile {
   float red[W];
 };
 
-// waves per SIMD a pencil kernel asks for: five where a fifth workgroup of four waves fits the
-// CU's 160 KiB of LDS, else no request; none for K = 3 either (three cells per lane spill
-// under the 96 registers of five waves and the 128 of four; unconstrained they take 165, three
-// waves per SIMD, without spilling)
+// waves per SIMD a pencil kernel asks for: as many, up to five, as workgroups of four waves fit
+// the CU's 160 KiB of LDS; no request for larger workgroups, nor for K = 3 (unconstrained it
+// takes 165 registers, three waves per SIMD, without spilling)
 template <int K, int W, int Q, int NF>
 constexpr int pencil_waves() {
-  if (K == 3) return 1;
-  return (W == 4 && 5 * sizeof(XTile<K, W, Q, NF>) <= 160 * 1024) ? 5 : 1;
+  constexpr size_t lds = sizeof(XTile<K, W, Q, NF>);
+  if (K == 3 || W != 4) return 1;
+  return 5 * lds <= 160 * 1024 ? 5 : 4 * lds <= 160 * 1024 ? 4 : 1;
 }
 
 // one work item: window l of the pencils of row `row` (radial: theta row k; theta: ring i),
 // column group grp.  Workgroup-uniform; starts with a barrier so that a workgroup can run
-// items back to back on the same LDS.  With CFL, returns in thread 0 the largest CFL term of
+// items back to back on the same LDS.  With cfl (theta), returns in thread 0 the largest CFL term of
 // the cells it stored (the last sweep of a 3-D step).
-template <int K, int W, int Q, int G, int VISC, bool CFL, bool ADIA = false, bool BARY = false>
+template <int K, int W, int Q, int G, int VISC, bool ADIA = false, bool BARY = false>
 __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, const DevParams& prm,
                                              const StepScalars* __restrict__ ss, int src, int grp, int l, int row,
-                                             XTile<K, W, Q, (G == kGeoRcyl && !ADIA ? 3 : 4)>& T) {
+                                             bool cfl, XTile<K, W, Q, (G == kGeoRcyl && !ADIA ? 3 : 4)>& T) {
   constexpr int NF = (G == kGeoRcyl && !ADIA) ? 3 : 4;
   constexpr int WIN = 64 * K, REAL = WIN - 2 * kNpad, NC = W * Q;
   constexpr bool TH = (G == kGeoTheta);
@@ -224,24 +222,26 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
   // theta: the theta-major table, whose slots run along the pencil (reads past the window
   // land on the next ring's slots or the overhang: finite values no kept cell depends on)
   const unsigned tbytes = 4u * (unsigned)kTabEntries * (unsigned)f.tstride;
-  // A window of at most SL K cells (a short last window, or a whole short pencil) runs
-  // NSEG = 64 / SL columns per wavefront pass, one in each run of SL lanes (lanes past the
-  // last run idle); every stage indexes cells within its own window (cell_in<SL>), so each
-  // column's result is the one-column pass's.  Column group gi = the NSEG columns
-  // gi NSEG + seg; wave wv takes groups wv QP .. wv QP + QP - 1; a column past the
-  // workgroup's NC reads column NC - 1 and stores nothing.
-  auto pencils = [&](auto sl_tag) {
-    constexpr int SL = decltype(sl_tag)::value, NSEG = 64 / SL;
-    constexpr int NG = (NC + NSEG - 1) / NSEG, QP = (NG + W - 1) / W;
-    const int seg = lane / SL, ll = lane % SL;
-    const TabLane<K> tx{Buf(TH ? f.tabz : f.tab, tbytes),
-                        4u * (unsigned)((TH ? (REAL * l - kNpad + g.k0) + g.sk * (row + kNpad) : s0) + K * ll),
-                        f.tstride};
-  for (int qq = 0; qq < QP; ++qq) {
-    const int gi = wv * QP + qq;
-    if (gi >= NG || jb + gi * NSEG >= jmax) break;   // wave-uniform
-    const int qv = gi * NSEG + seg;
-    const bool mine = seg < NSEG && qv < NC;   // this lane's column is one of the workgroup's
+  // A window of few cells (a short last window, or a whole short pencil) runs nseg = 64 / sl
+  // columns per wavefront pass, one in each run of sl = ceil(lim / K) lanes (lanes past the last
+  // run idle); every stage indexes cells within its own window (from c0), so each column's
+  // result is the one-column pass's.  Column group gi = the nseg columns gi nseg + seg; wave wv
+  // takes groups wv qp .. wv qp + qp - 1; a column past the workgroup's NC reads column NC - 1
+  // and stores nothing.
+  int sl = 64, nseg = 1;
+  if (f.pack_tails && lim <= 32 * K) {
+    sl = (lim + K - 1) / K;
+    nseg = 64 / sl;
+  }
+  const int ngp = (NC + nseg - 1) / nseg, qp = (ngp + W - 1) / W;
+  const int seg = nseg == 1 ? 0 : lane / sl, c0 = K * (lane - seg * sl);
+  const TabLane<K> tx{Buf(TH ? f.tabz : f.tab, tbytes),
+                      4u * (unsigned)((TH ? (REAL * l - kNpad + g.k0) + g.sk * (row + kNpad) : s0) + c0), f.tstride};
+  for (int qq = 0; qq < qp; ++qq) {
+    const int gi = wv * qp + qq;
+    if (gi >= ngp || jb + gi * nseg >= jmax) break;   // wave-uniform
+    const int qv = gi * nseg + seg;
+    const bool mine = seg < nseg && qv < NC;   // this lane's column is one of the workgroup's
     const int q = mine ? qv : NC - 1;
     // a column past jmax (the last group) computes on column jmax - 1's copies and is never
     // stored
@@ -283,10 +283,10 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
     Wp.ts = splat<float, K>(tr.x);
     Wp.tc = splat<float, K>(tr.y);
     const C<float, K> rc = tx.get(kTabRc);
-    const C<float, K> f0 = lds_k<K>(&tile[0][q][K * ll]), f1 = lds_k<K>(&tile[1][q][K * ll]),
-                      f2 = lds_k<K>(&tile[2][q][K * ll]);
+    const C<float, K> f0 = lds_k<K>(&tile[0][q][c0]), f1 = lds_k<K>(&tile[1][q][c0]),
+                      f2 = lds_k<K>(&tile[2][q][c0]);
     C<float, K> f3;
-    if constexpr (NF == 4) f3 = lds_k<K>(&tile[3][q][K * ll]);
+    if constexpr (NF == 4) f3 = lds_k<K>(&tile[3][q][c0]);
     Wp.r = f0;
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -304,7 +304,7 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
     }
     Para<float, K> P0;
     if constexpr (TH) {
-      P0 = f.uniform_theta ? paraset_uniform<K>() : paraset<float, K, SL>(0, lim, Wp.dx0);
+      P0 = f.uniform_theta ? paraset_uniform<K>() : paraset_f32<K>(Wp.dx0);
     } else {
       P0.c0 = tx.get(kTabP0);
       P0.c1 = tx.get(kTabP1);
@@ -312,13 +312,13 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
       P0.c3 = tx.get(kTabP3);
       P0.c4 = tx.get(kTabP4);
     }
-    ppmlr_pert<K, G, (G == kGeoRcyl ? 2 : 3), TabLane<K>, ADIA, SL, BARY>(Wp, tx, P0, lim, dt, 0.0f, pl, prm.plnt > 0,
+    ppmlr_pert<K, G, (G == kGeoRcyl ? 2 : 3), TabLane<K>, ADIA, BARY>(Wp, tx, P0, c0, lim, dt, 0.0f, pl, prm.plnt > 0,
                                                                      prm.flat != 0, sqrt_gam, 0.0f, false,
                                                                      (float)prm.gam);
     if (VISC == 1 || (VISC == 2 && prm.visc)) {
-      if constexpr (G == kGeoRcyl) visc_r_pert<K, SL>(Wp, tx, lim, dt);
-      else if constexpr (G == kGeoRsph) visc_r_pert<K, SL, true>(Wp, tx, lim, dt);
-      else visc_z_pert<K, SL>(Wp, tx, lim, dt, (float)prm.vis_nu);
+      if constexpr (G == kGeoRcyl) visc_r_pert<K>(Wp, tx, c0, lim, dt);
+      else if constexpr (G == kGeoRsph) visc_r_pert<K, true>(Wp, tx, c0, lim, dt);
+      else visc_z_pert<K>(Wp, tx, c0, lim, dt, (float)prm.vis_nu);
     }
     const C<float, K> irc = tx.get(kTabIrc);
     C<float, K> ixc;
@@ -328,7 +328,7 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
     // product (r v) (1/r) would scale it by the table's fixed r (1/r) - 1 every step)
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = K * ll + h;
+      const int c = c0 + h;
       if (mine && c >= kNpad && c < lim - kNpad) {   // only this lane's run touches column q
         tile[0][q][c] = Wp.r[h];
         if constexpr (TH) {
@@ -349,18 +349,6 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
       }
     }
   }
-  };
-  // workgroup-uniform choice: three windows of 21 lanes (K = 4: a 64-cell theta pencil with
-  // its halos, 76 cells), two of 32, or one
-  bool three = false;
-  if constexpr (K == 4) three = f.pack_tails && lim <= 21 * K;
-  if (three) {
-    if constexpr (K == 4) pencils(std::integral_constant<int, 21>{});
-  } else if (f.pack_tails && lim <= 32 * K) {
-    pencils(std::integral_constant<int, 32>{});
-  } else {
-    pencils(std::integral_constant<int, 64>{});
-  }
   __syncthreads();
   float m = 0.0f;
   const double FrRot = ss->FrRot;
@@ -376,7 +364,7 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
       const unsigned o = 4u * (unsigned)(sl * jmax + j);
 #pragma unroll
       for (int fi = 0; fi < NF; ++fi) fout[fi].put(tile[fi][q][c], o);
-      if constexpr (CFL) {
+      if (TH && cfl) {
         // the next step's CFL term of this cell (timestep.cu:12-108), isothermal c_s
         const float* T = f.tab + sl;
         const long ts = f.tstride;
@@ -389,7 +377,7 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
       }
     }
   }
-  if constexpr (CFL) {
+  if (TH && cfl) {
     m = wave_maxf(m);
     if (lane == 0) T.red[wv] = m;
     __syncthreads();
@@ -408,7 +396,7 @@ __global__ __launch_bounds__(64 * W) PN_WAVES((pencil_waves<K, W, Q, ADIA ? 4 : 
   const int bid = xcd_swizzle(blockIdx.x, gridDim.x);
   const int grp = bid % ngrp, l = bid / ngrp;
   if (l >= f.nwin_x) return;   // workgroup-uniform, before any barrier
-  pencil_item<K, W, Q, kGeoRcyl, VISC, false, ADIA, BARY>(g, f, prm, ss, src, grp, l, 0, T);
+  pencil_item<K, W, Q, kGeoRcyl, VISC, ADIA, BARY>(g, f, prm, ss, src, grp, l, 0, false, T);
 }
 
 // 3-D: the spherical radial sweep (item = theta row k, radial window, column group) and the
@@ -426,12 +414,8 @@ __global__ __launch_bounds__(64 * W) PN_WAVES((pencil_waves<K, W, Q, 4>())) void
   const int grp = bid % ngrp, rest = bid / ngrp;
   const int l = rest % nwin, row = rest / nwin;
   if (row >= nrow) return;   // workgroup-uniform, before any barrier
-  if (do_cfl) {
-    const float m = pencil_item<K, W, Q, G, VISC, true, false, BARY>(g, f, prm, ss, src, grp, l, row, T);
-    if (threadIdx.x == 0) cflp[blockIdx.x] = (double)m;
-  } else {
-    pencil_item<K, W, Q, G, VISC, false, false, BARY>(g, f, prm, ss, src, grp, l, row, T);
-  }
+  const float m = pencil_item<K, W, Q, G, VISC, false, BARY>(g, f, prm, ss, src, grp, l, row, do_cfl != 0, T);
+  if (do_cfl && threadIdx.x == 0) cflp[blockIdx.x] = (double)m;
 }
 
 // the disk owning work item it: base[d] <= it < base[d + 1] (ndisk small; base in device memory)
@@ -448,20 +432,14 @@ __device__ __forceinline__ int disk_of(const int* __restrict__ base, int ndisk, 
 // many disks, persistent: workgroup b runs items t = b, b + G, ... (G = gridDim, a multiple
 // of 8), each mapped through the XCD permutation so that one XCD walks a contiguous run of
 // items (neighbouring column groups share L2 lines).  base: ndisk + 1 item offsets.
-// The batch's radial kernel also keeps its item's disk lookup in scalar registers: asked for
-// five waves per SIMD it spilled 24 VGPRs to scratch and 60 SGPRs to VGPR lanes (each a VALU
-// lane write or read), at four it spills nothing and ran 7 % faster on the 48-disk sweep
-// (0.428 -> 0.397 ms per launch, same box; six waves: 0.428).
-template <int W>
-constexpr int batch_pencil_waves() {
-  return W == 4 ? 4 : 1;
-}
+// The batch's radial kernel keeps its item's disk lookup in scalar registers besides the pencil's
+// state; five waves per SIMD (96 registers) ran 84 us on twelve disks against 90 at four.
 
 // order: nslots (disk, item) pairs, the item of slot t for the workgroup that takes it
 // (slot t runs on XCD t % 8; the host lays each XCD's share out by decreasing cost, disk -1
 // marks an empty slot)
 template <int K, int W, int Q, bool BARY, bool ADIA>
-__global__ __launch_bounds__(64 * W) PN_WAVES(ADIA ? 1 : batch_pencil_waves<W>()) void k_sweep_x_f32_batch(const DiskDev* __restrict__ dd,
+__global__ __launch_bounds__(64 * W) PN_WAVES((pencil_waves<K, W, Q, ADIA ? 4 : 3>())) void k_sweep_x_f32_batch(const DiskDev* __restrict__ dd,
                                                               const DevF32* __restrict__ dfs,
                                                               const int* __restrict__ order, int nslots, int src) {
   __shared__ XTile<K, W, Q, ADIA ? 4 : 3> T;
@@ -471,8 +449,8 @@ __global__ __launch_bounds__(64 * W) PN_WAVES(ADIA ? 1 : batch_pencil_waves<W>()
     const DevGrid g = dd[d].g;
     const int ngrp = (g.jmax + W * Q - 1) / (W * Q);
     const int local = order[2 * t + 1];
-    pencil_item<K, W, Q, kGeoRcyl, 2, false, ADIA, BARY>(g, dfs[d], dd[d].p, dd[d].ss, src, local % ngrp, local / ngrp,
-                                                        0, T);
+    pencil_item<K, W, Q, kGeoRcyl, 2, ADIA, BARY>(g, dfs[d], dd[d].p, dd[d].ss, src, local % ngrp, local / ngrp, 0,
+                                                  false, T);
   }
 }
 
@@ -514,7 +492,7 @@ __device__ __forceinline__ float y_pencil(const DevGrid& g, const DevF32& f, con
   const long base = (long)s * jmax;
   const unsigned rb4 = 4u * (unsigned)jmax;
   const Buf bfr(f.f[src][0] + base, rb4), bfu(f.f[src][1] + base, rb4), bfv(f.f[src][2] + base, rb4);
-  const Buf btrig(f.trig, 2u * rb4), bdy(f.dy, rb4), byv(f.yvol, rb4);
+  const Buf btrig(f.trig, 2u * rb4), bdy(f.dy, rb4), bcol(f.col, 4u * rb4);
 
   WinP<K> W;
   unsigned jd[K];   // byte offset of the cell's data column
@@ -533,8 +511,11 @@ __device__ __forceinline__ float y_pencil(const DevGrid& g, const DevF32& f, con
     const float2 tr = btrig.f2(2u * o0);
     W.ts[h] = tr.x;
     W.tc[h] = tr.y;
-    W.dx0[h] = bdy.f(o0);
-    W.dvol0[h] = byv.f(o0) * rc;
+    const float4 col = bcol.f4(4u * o0);
+    W.dx0[h] = col.x;
+    W.dvol0[h] = col.y * rc;
+    W.idx0[h] = col.z;
+    W.iyv[h] = col.w;
     W.xa0[h] = 0.0f;
     W.rad[h] = rc;
     W.vrot[h] = vrot;
@@ -560,11 +541,11 @@ __device__ __forceinline__ float y_pencil(const DevGrid& g, const DevF32& f, con
     if constexpr (ADIA) W.q[h] = Buf(f.f[src][3] + base, rb4).f(o);
   }
   const float sqrt_gam = sqrtf((float)prm.gam);
-  const Para<float, K> P0 = f.uniform_phi ? paraset_uniform<K>() : paraset(0, lim, W.dx0);
-  ppmlr_pert<K, kGeoPhi, NDIM, TabLane<K>, ADIA, 64, BARY>(W, TabLane<K>{}, P0, lim, dt, wres, pl, prm.plnt > 0,
+  const Para<float, K> P0 = f.uniform_phi ? paraset_uniform<K>() : paraset_f32<K>(W.dx0);
+  ppmlr_pert<K, kGeoPhi, NDIM, TabLane<K>, ADIA, BARY>(W, TabLane<K>{}, P0, K * lane, lim, dt, wres, pl, prm.plnt > 0,
                                                            prm.flat != 0, sqrt_gam, rsph, f.uniform_phi != 0,
                                                            (float)prm.gam);
-  if (VISC == 1 || (VISC == 2 && prm.visc)) visc_p_pert<K, NDIM == 3>(W, lim, dt, T[kTabNu * ts], rc);
+  if (VISC == 1 || (VISC == 2 && prm.visc)) visc_p_pert<K, NDIM == 3>(W, K * lane, lim, dt, T[kTabNu * ts], rc);
 
   const Buf dr(f.f[src ^ 1][0] + base, rb4), du(f.f[src ^ 1][1] + base, rb4), dv(f.f[src ^ 1][2] + base, rb4);
   const float csnd = sqrt_gam * cs;
@@ -594,7 +575,7 @@ __device__ __forceinline__ float y_pencil(const DevGrid& g, const DevF32& f, con
 // one wavefront per (ring, window); with do_cfl each workgroup writes the maximum CFL term
 // of its waves to cflp[workgroup] (2-D)
 template <int K, int WPB, int VISC, int NDIM, bool ADIA, bool BARY>
-__global__ __launch_bounds__(64 * WPB) PN_WAVES((K == 2 && NDIM == 2 && !ADIA) ? 8 : 1) void k_sweep_y_f32(DevGrid g, DevF32 f, DevParams prm,
+__global__ __launch_bounds__(64 * WPB) PN_WAVES(ADIA ? 1 : K == 4 ? 4 : NDIM == 2 ? 8 : 1) void k_sweep_y_f32(DevGrid g, DevF32 f, DevParams prm,
                                                           const StepScalars* __restrict__ ss, double* cflp, int src,
                                                           int do_cfl) {
   __shared__ float shm[WPB];
@@ -617,7 +598,7 @@ __global__ __launch_bounds__(64 * WPB) PN_WAVES((K == 2 && NDIM == 2 && !ADIA) ?
 // many disks, persistent (as k_sweep_x_f32_batch): item = one workgroup's WPB waves of one
 // disk; each item writes its CFL partial to its disk's cflp[item - base[d]]
 template <int K, int WPB, bool BARY, bool ADIA>
-__global__ __launch_bounds__(64 * WPB) PN_WAVES((K == 2 && !ADIA) ? 6 : 1) void k_sweep_y_f32_batch(const DiskDev* __restrict__ dd,
+__global__ __launch_bounds__(64 * WPB) PN_WAVES(ADIA ? 1 : K == 4 ? 4 : 6) void k_sweep_y_f32_batch(const DiskDev* __restrict__ dd,
                                                               const DevF32* __restrict__ dfs,
                                                               const int* __restrict__ base, int ndisk, int src) {
   __shared__ float shm[WPB];
@@ -898,9 +879,7 @@ hipError_t sweep_x_k(const LaunchCtx& c, const DevF32& f0, int src) {
   // others run without them
   auto go = [&](auto bary) {
     constexpr bool B = decltype(bary)::value;
-    // EOS 3: a viscous disk runs its own instantiation (the viscosity updates velocities only)
-    if (c.p.eos == 3 && c.p.visc) k_sweep_x_f32<K, W, Q, 1, true, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, src);
-    else if (c.p.eos == 3) k_sweep_x_f32<K, W, Q, 0, true, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, src);
+    if (c.p.eos == 3) k_sweep_x_f32<K, W, Q, 2, true, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, src);
     else k_sweep_x_f32<K, W, Q, 2, false, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, src);
   };
   if (c.p.bary) go(std::true_type{});
@@ -922,10 +901,8 @@ hipError_t sweep_y_k(const LaunchCtx& c, const DevF32& f0, int src, int do_cfl) 
       k_sweep_y_f32<K, WPB, 1, 3, false, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, c.cflp, src, 0);
     else if (c.g.ndim == 3)
       k_sweep_y_f32<K, WPB, 0, 3, false, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, c.cflp, src, 0);
-    else if (c.p.eos == 3 && c.p.visc)
-      k_sweep_y_f32<K, WPB, 1, 2, true, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, c.cflp, src, do_cfl);
     else if (c.p.eos == 3)
-      k_sweep_y_f32<K, WPB, 0, 2, true, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, c.cflp, src, do_cfl);
+      k_sweep_y_f32<K, WPB, 2, 2, true, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, c.cflp, src, do_cfl);
     else k_sweep_y_f32<K, WPB, 2, 2, false, B><<<grid, block, 0, c.stream>>>(c.g, f, c.p, c.ss, c.cflp, src, do_cfl);
   };
   if (c.p.bary) go(std::true_type{});

@@ -102,26 +102,13 @@ __device__ __forceinline__ C<T, K> next2(const C<T, K>& x) {
 }
 
 __device__ __forceinline__ int cell_of(int K, int h) { return K * (int)(threadIdx.x & 63) + h; }
-// the cell index within a window when a wavefront holds 64 / SL windows side by side, SL
-// lanes each (SL = 64: one window per wavefront, cell_of; lanes past the last whole window
-// count from 0 again and store nothing).  Stencils reach across the seam between two windows
-// exactly as they reach past a window's last cell: every stage's index range keeps such
-// values out of the cells a window stores.
-template <int SL>
-__device__ __forceinline__ int cell_in(int K, int h) { return K * (int)((threadIdx.x & 63) % SL) + h; }
 
 // the limited slope of parabola.cu:87-96: sign(t1) min(|t1|, 2 |da_l|, 2 |da_r|), zero at an
 // extremum: a minimum of magnitudes and the sign by copysign, the values of the reference's
 // compare chain (a minimum and a sign change round nothing, doubling is exact)
-template <typename T>
-__device__ __forceinline__ T limited_slope(T t1, T da_l, T da_r) {
-  if constexpr (sizeof(T) == 4) {
-    t1 = copysignf(fminf(fminf(fabsf(t1), 2.0f * fabsf(da_l)), 2.0f * fabsf(da_r)), t1);
-  } else {
-    t1 = copysign(fmin(fabs(t1), T(2.0) * fmin(fabs(da_l), fabs(da_r))), t1);
-  }
-  if (da_l * da_r < T(0.0)) t1 = T(0.0);
-  return t1;
+__device__ __forceinline__ double limited_slope(double t1, double da_l, double da_r) {
+  t1 = copysign(fmin(fabs(t1), 2.0 * fmin(fabs(da_l), fabs(da_r))), t1);
+  return da_l * da_r < 0.0 ? 0.0 : t1;
 }
 template <typename T>
 __device__ __forceinline__ T max3(T A, T B, T Cc) {   // simple_func.cu:16-28
@@ -372,7 +359,7 @@ struct Para {
 };
 
 // paraset (parabola.cu:138-176) on the index range [nmin, nmaxp)
-template <typename T, int K, int SL = 64>
+template <typename T, int K>
 __device__ __forceinline__ Para<T, K> paraset(int nmin, int nmaxp, const C<T, K>& dx) {
   Para<T, K> P;
   C<T, K> dxp = next1(dx);
@@ -389,7 +376,7 @@ __device__ __forceinline__ Para<T, K> paraset(int nmin, int nmaxp, const C<T, K>
   C<T, K> anm = prev1(an), anp = next1(an), bnm = prev1(bn), ainm = prev1(ain);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_in<SL>(K, h);
+    const int c = cell_of(K, h);
     T c0 = T(0), c1 = T(0), c2 = T(0), c3 = T(0), c4 = T(0);
     if (c >= nmin + 1 && c < nmaxp - 2) {
       T d = T(1.0) / (anm[h] + anp[h]);
@@ -478,7 +465,7 @@ __device__ __forceinline__ Parab<double, K> parabola(const C<double, K>& flat, c
   C<double, K> dal = prev1(dar);
 #pragma unroll
   for (int h = 0; h < K; ++h)
-    slope[h] = limited_slope<double>(P.c3[h] * dar[h] + P.c4[h] * dal[h], dal[h], dar[h]);
+    slope[h] = limited_slope(P.c3[h] * dar[h] + P.c4[h] * dal[h], dal[h], dar[h]);
   C<double, K> slp = next1(slope);
   C<double, K> ar;
 #pragma unroll

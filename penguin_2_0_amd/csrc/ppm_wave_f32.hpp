@@ -24,6 +24,14 @@
 // its grid at the per-ring residual rate (v_bg - res_v)/r - FrRot; that uniform part of the
 // grid motion is kept apart from the velocity-dependent part so the cell volumes and the
 // density fluxes never difference it.
+//
+// What bounds it: instruction issue.  With its states in registers or LDS a sweep keeps the
+// SIMDs' vector pipes 70 to 90 % busy, and a reciprocal, root or exponential holds one four times as
+// long as a product.  So the limiters are medians, fixed divisors come as table reciprocals,
+// ranges are not masked where a kept cell cannot see the difference, and the library logarithm
+// and the flattening run only in wavefronts that hold a cell in need of them.  1024 x 3072,
+// inviscid: radial sweep 70 -> 58 us, azimuthal 48 -> 39 (1536 x 4608 with EOS 3: 171 -> 146, 139 -> 116;
+// 128 x 384 x 32: 59, 34 and 69 -> 45, 27 and 60).
 #pragma once
 
 #include "pn_f32.hpp"
@@ -51,6 +59,10 @@ struct Buf {
   __device__ __forceinline__ float2 f2(unsigned off) const {
     const f32x2_t v = __builtin_bit_cast(f32x2_t, (i32x2_t)__builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
     return make_float2(v.x, v.y);
+  }
+  __device__ __forceinline__ float4 f4(unsigned off) const {
+    const f32x4_t v = __builtin_bit_cast(f32x4_t, (i32x4_t)__builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
+    return make_float4(v.x, v.y, v.z, v.w);
   }
   __device__ __forceinline__ void put(float v, unsigned off) const {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)off, 0, 0);
@@ -86,8 +98,8 @@ __device__ __forceinline__ float star_fr_rest(const PlanetF& p, float r, float c
 // sin / cos of (A + e)/2 from sin / cos of A/2 and a small e (|e| < ~0.5)
 __device__ __forceinline__ void rot_half(float s, float c, float e, float& so, float& co) {
   const float h = 0.5f * e, h2 = h * h;
-  const float sh = h * (1.0f - h2 * (1.0f / 6.0f) * (1.0f - h2 * (1.0f / 20.0f) * (1.0f - h2 * (1.0f / 42.0f))));
-  const float ch = 1.0f - h2 * 0.5f * (1.0f - h2 * (1.0f / 12.0f) * (1.0f - h2 * (1.0f / 30.0f)));
+  const float sh = h + h * h2 * (-1.0f / 6.0f + h2 * (1.0f / 120.0f - h2 * (1.0f / 5040.0f)));
+  const float ch = 1.0f + h2 * (-0.5f + h2 * (1.0f / 24.0f - h2 * (1.0f / 720.0f)));
   so = s * ch + c * sh;
   co = c * ch - s * sh;
 }
@@ -98,21 +110,20 @@ __device__ __forceinline__ float planet_fr(const PlanetF& p, float rad, float s,
   const float s2 = s * s;
   const float cosd = 1.0f - 2.0f * s2;
   const float dr = rad - p.x;
-  const float R2 = dr * dr + 4.0f * rad * p.x * s2 + p.rs2;
-  const float ri = __frsqrt_rn(R2);
-  float f = -p.m * (dr + 2.0f * p.x * s2) * (ri * ri * ri) - p.m * cosd * p.inv_x2;
+  const float t = 2.0f * p.x * s2;
+  const float ri = __frsqrt_rn((dr * dr + p.rs2) + 2.0f * rad * t);
+  float f = -p.m * ((dr + t) * (ri * ri * ri) + cosd * p.inv_x2);
   if constexpr (BARY) if (p.bary) f += p.m / (rad * rad) + star_fr_rest(p, rad, cosd);
   return f;
 }
 template <bool BARY = false>
 __device__ __forceinline__ float planet_fphi(const PlanetF& p, float rad, float s, float c) {
-  const float s2 = s * s;
-  const float sind = 2.0f * s * c;
+  // the factors of one ring first: they are formed once for all its cells
+  const float s2 = s * s, sc = s * c;
   const float dr = rad - p.x;
-  const float R2 = dr * dr + 4.0f * rad * p.x * s2 + p.rs2;
-  const float ri = __frsqrt_rn(R2);
-  float f = -p.m * p.x * sind * (ri * ri * ri) + p.m * sind * p.inv_x2;
-  if constexpr (BARY) if (p.bary) f += p.stm * p.stx * sind * star_ri3(p, rad, 1.0f - 2.0f * s2);
+  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (4.0f * rad * p.x) * s2);
+  float f = sc * ((2.0f * p.m * p.inv_x2) - (2.0f * p.m * p.x) * (ri * ri * ri));
+  if constexpr (BARY) if (p.bary) f += 2.0f * p.stm * p.stx * sc * star_ri3(p, rad, 1.0f - 2.0f * s2);
   return f;
 }
 
@@ -127,8 +138,8 @@ __device__ __forceinline__ float planet_fr_sph(const PlanetF& p, float r, float 
   const float cosd = 1.0f - 2.0f * s2;
   const float k = oms + 2.0f * st * s2;
   const float dr = r - p.x;
-  const float ri = __frsqrt_rn(dr * dr + 2.0f * r * p.x * k + p.rs2);
-  float f = -p.m * (dr + p.x * k) * (ri * ri * ri) - p.m * st * cosd * p.inv_x2;
+  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (2.0f * r * p.x) * k);
+  float f = -p.m * ((dr + p.x * k) * (ri * ri * ri) + st * cosd * p.inv_x2);
   if constexpr (BARY) if (p.bary) f += star_fr_rest(p, r, st * cosd);
   return f;
 }
@@ -138,8 +149,8 @@ __device__ __forceinline__ float planet_fphi_sph(const PlanetF& p, float r, floa
   const float sind = 2.0f * s * c;
   const float k = oms + 2.0f * st * s2;
   const float dr = r - p.x;
-  const float ri = __frsqrt_rn(dr * dr + 2.0f * r * p.x * k + p.rs2);
-  float f = -p.m * p.x * sind * (ri * ri * ri) + p.m * st * sind * p.inv_x2;
+  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (2.0f * r * p.x) * k);
+  float f = sind * ((p.m * st * p.inv_x2) - (p.m * p.x) * (ri * ri * ri));
   if constexpr (BARY) if (p.bary) f += p.stm * p.stx * sind * star_ri3(p, r, st * (1.0f - 2.0f * s2));
   return f;
 }
@@ -150,27 +161,63 @@ __device__ __forceinline__ float planet_fth_sph(const PlanetF& p, float r, float
   const float cosd = 1.0f - 2.0f * s2;
   const float k = oms + 2.0f * st * s2;
   const float dr = r - p.x;
-  const float ri = __frsqrt_rn(dr * dr + 2.0f * r * p.x * k + p.rs2);
-  float f = p.m * p.x * cosd * ct * (ri * ri * ri) - p.m * cosd * ct / st * p.inv_x2;
+  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (2.0f * r * p.x) * k);
+  float f = p.m * cosd * ct * (p.x * (ri * ri * ri) - p.inv_x2 / st);
   if constexpr (BARY) if (p.bary) f -= p.stm * p.stx * cosd * ct * star_ri3(p, r, st * cosd);
   return f;
 }
 
 // log(1 + x): 2 atanh(x / (2 + x)) as an odd series for |x| < 1/4, else the library log.
-// Deviations that large are rare (next to a planet), so the library branch is taken only by
-// wavefronts that hold one; elsewhere it costs a compare and a scalar branch.
-__device__ __forceinline__ float log1p_acc(float x) {
+// Deviations that large are rare (next to a planet), so the library is called only by wavefronts
+// that hold one in a cell whose interface is used (wide, wave-uniform, from wave_any over the
+// arguments; a window's end lanes divide by the zeros shifted in past it and must not ask).  The
+// value depends on this lane's x alone: a cell's bits are the same in any company.
+__device__ __forceinline__ float log1p_acc(float x, bool wide) {
   const float z = x / (2.0f + x), z2 = z * z;
-  float s = 2.0f * z * (1.0f + z2 * (1.0f / 3.0f + z2 * (1.0f / 5.0f + z2 * (1.0f / 7.0f + z2 * (1.0f / 9.0f)))));
-  if (wave_any(!(fabsf(x) < 0.25f))) s = fabsf(x) < 0.25f ? s : __logf(1.0f + x);
+  float s = z * (2.0f + z2 * (2.0f / 3.0f + z2 * (2.0f / 5.0f + z2 * (2.0f / 7.0f + z2 * (2.0f / 9.0f)))));
+  if (wide) s = fabsf(x) < 0.25f ? s : __logf(1.0f + x);
   return s;
 }
-// exp(y) - 1: Taylor series to y^7 for |y| < 1/4, else the library exp (branch as above)
-__device__ __forceinline__ float expm1_acc(float y) {
+// exp(y) - 1: Taylor series to y^7 for |y| < 1/4, else the library exp (switch as above)
+__device__ __forceinline__ float expm1_acc(float y, bool wide) {
   float s =
       y * (1.0f + y * (0.5f + y * (1.0f / 6.0f + y * (1.0f / 24.0f + y * (1.0f / 120.0f + y * (1.0f / 720.0f + y * (1.0f / 5040.0f)))))));
-  if (wave_any(!(fabsf(y) < 0.25f))) s = fabsf(y) < 0.25f ? s : __expf(y) - 1.0f;
+  if (wide) s = fabsf(y) < 0.25f ? s : __expf(y) - 1.0f;
   return s;
+}
+// the median of 0, a and b: the smaller in magnitude where the signs agree, else 0
+__device__ __forceinline__ float med0(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 0.0f); }
+__device__ __forceinline__ float max4(float a, float b, float c, float d) {
+  return fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d)));
+}
+
+// paraset (CW84 eq. 1.6) in every cell: coefficients outside the
+// reference's index ranges (parabola.cu:138-176) reach no parabola that a kept cell reads.
+template <int K>
+__device__ __forceinline__ Para<float, K> paraset_f32(const C<float, K>& dx) {
+  Para<float, K> P;
+  C<float, K> dxp = next1(dx), an, ain, bn, bi, cc, ci;
+#pragma unroll
+  for (int h = 0; h < K; ++h) {
+    an[h] = dx[h] + dxp[h];
+    bn[h] = an[h] + dx[h];
+    cc[h] = an[h] + dxp[h];
+    ain[h] = 1.0f / an[h];
+    bi[h] = 1.0f / bn[h];
+    ci[h] = 1.0f / cc[h];
+  }
+  C<float, K> anm = prev1(an), anp = next1(an), bnm = prev1(bn), ainm = prev1(ain);
+#pragma unroll
+  for (int h = 0; h < K; ++h) {
+    const float d = 1.0f / (anm[h] + anp[h]), e = dx[h] / (anm[h] + dxp[h]);
+    const float wb = d * anm[h] * bi[h], wc = d * anp[h] * ci[h];
+    P.c0[h] = dx[h] * ain[h] * (1.0f + 2.0f * dxp[h] * (wb - wc));
+    P.c1[h] = -dx[h] * wb;
+    P.c2[h] = dxp[h] * wc;
+    P.c3[h] = e * bnm[h] * ain[h];
+    P.c4[h] = e * cc[h] * ainm[h];
+  }
+  return P;
 }
 
 // paraset of a uniform grid (CW84 eq. 1.6 with equal widths): constants
@@ -190,54 +237,56 @@ __device__ __forceinline__ Para<float, K> paraset_uniform() {
 // unused).  The edges are carried as offsets from the cell's own value (the right edge
 // c0 da_r + c1 slope(c+1) + c2 slope, the left edge the left neighbour's right edge in this
 // frame), so the flattening, the extremum and overshoot tests, the jump and the curvature
-// never subtract two values of the cell's size; the algebra is the reference's.  Outputs:
-// al = left edge - x, da, a6, and the jumps dl = X(c) - X(c-1), dr = X(c+1) - X(c) in this
-// cell's frame.  A cell outside [nmin+2, nmaxp-2) returns the plain parabola's zero edge
-// (al = -x, da = a6 = 0).
+// never subtract two values of the cell's size.  Both limiters are medians: the slope is the
+// smallest in magnitude of s, 2 dl and 2 dr if their signs agree, else 0 (parabola.cu:26-40);
+// of the edges' offsets r and l, zero if they share a sign (an extremum), the overshoot tests
+// d^2 < -+3 d (r + l), d = r - l, read |l| > 2 |r| and |r| > 2 |l|.  Outputs: al = left edge
+// - x, ar = right edge - x, da = ar - al, s = ar + al = -a6/3, and the jumps dl = X(c) - X(c-1),
+// dr = X(c+1) - X(c) in this cell's frame.  Cells whose stencil leaves the window, or outside
+// the reference's ranges, hold values that no kept cell reads.  flat: 1 - the flattening,
+// applied where shock (wave-uniform) says that the wavefront has any.
 template <int K>
 struct ParabR {
-  C<float, K> al, da, a6, dl, dr;
+  C<float, K> al, ar, da, s, dl, dr;
 };
 
-template <int K, int SL = 64, bool BG = true>
-__device__ __forceinline__ ParabR<K> parabola_rel(int nmin, int nmaxp, const C<float, K>& flat,
-                                                  const C<float, K>& val, const C<float, K>& dbg,
-                                                  const Para<float, K>& P) {
-  C<float, K> vm = prev1(val), vp = next1(val), dbm;
-  if constexpr (BG) dbm = prev1(dbg);
+template <int K, bool BG = true>
+__device__ __forceinline__ ParabR<K> parabola_rel(const C<float, K>& gfl, bool shock, const C<float, K>& val,
+                                                  const C<float, K>& dbg, const Para<float, K>& P) {
+  C<float, K> vp = next1(val);
   ParabR<K> o;
   C<float, K> slope;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     const float a = val[h];
     o.dr[h] = BG ? (vp[h] - a) + dbg[h] : vp[h] - a;
-    o.dl[h] = BG ? (a - vm[h]) + dbm[h] : a - vm[h];
-    slope[h] = limited_slope<float>(P.c3[h] * o.dr[h] + P.c4[h] * o.dl[h], o.dl[h], o.dr[h]);
   }
-  C<float, K> slp = next1(slope);
-  C<float, K> ar;   // right edge - x
-#pragma unroll
-  for (int h = 0; h < K; ++h) ar[h] = P.c0[h] * o.dr[h] + P.c1[h] * slp[h] + P.c2[h] * slope[h];
-  C<float, K> arm = prev1(ar);
+  o.dl = prev1(o.dr);   // the same difference, seen from the next cell
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_in<SL>(K, h);
-    const float g = 1.0f - flat[h];
-    float r = g * ar[h];                 // flattened right edge - x
-    float l = g * (arm[h] - o.dl[h]);    // flattened left edge - x
-    const float d = r - l;
-    const float t2 = d * d;
-    const float t1 = -3.0f * d * (r + l);   // (ar - la) 6 (x - (ar + la)/2)
-    if (r * l >= 0.0f) {                 // (ar - x)(x - la) <= 0: an extremum
-      r = 0.0f;
-      l = 0.0f;
+    const float s = P.c3[h] * o.dr[h] + P.c4[h] * o.dl[h];
+    slope[h] = med0(med0(s, 2.0f * o.dl[h]), 2.0f * o.dr[h]);
+  }
+  C<float, K> slp = next1(slope);
+#pragma unroll
+  for (int h = 0; h < K; ++h) o.ar[h] = P.c0[h] * o.dr[h] + P.c1[h] * slp[h] + P.c2[h] * slope[h];
+  C<float, K> arm = prev1(o.ar);
+#pragma unroll
+  for (int h = 0; h < K; ++h) o.al[h] = arm[h] - o.dl[h];
+  if (shock) {
+#pragma unroll
+    for (int h = 0; h < K; ++h) {
+      o.ar[h] *= gfl[h];
+      o.al[h] *= gfl[h];
     }
-    if (t2 < t1) l = -2.0f * r;          // la = 3 x - 2 ar
-    if (t2 < -t1) r = -2.0f * l;         // ar = 3 x - 2 la
-    const bool in = (c >= nmin + 2 && c < nmaxp - 2);
-    o.da[h] = in ? r - l : 0.0f;
-    o.a6[h] = in ? -3.0f * (r + l) : 0.0f;
-    o.al[h] = in ? l : -val[h];
+  }
+#pragma unroll
+  for (int h = 0; h < K; ++h) {
+    const float r = med0(o.ar[h], -2.0f * o.al[h]), l = med0(o.al[h], -2.0f * o.ar[h]);
+    o.ar[h] = r;
+    o.al[h] = l;
+    o.da[h] = r - l;
+    o.s[h] = r + l;
   }
   return o;
 }
@@ -262,6 +311,7 @@ struct WinP {
   // vrot (azimuthal sweep) or rs / rcs (radial and theta sweeps: sin / cos of the planet's
   // drift against the slot in half a step, halved) for the planet's azimuth over the step
   C<float, K> rad, xa0, dx0, dvol0, vrot, ts, tc, sth, oms, rs, rcs;
+  C<float, K> idx0, iyv;   // azimuthal sweep: 1/dx0 and rad/dvol0
 };
 
 // the per-slot table entries of this lane's K cells, entry-major (entry e of slot s at
@@ -299,24 +349,6 @@ struct TabLane {
   }
 };
 
-// the same for cells `step` slots apart (the theta sweep: one theta row of slots); c0 = this
-// lane's first cell of the window, reads past cell cmax (the window's last) repeat it
-template <int K>
-struct TabLaneS {
-  const float* __restrict__ p;
-  int stride, base, step, c0, cmax;
-  __device__ __forceinline__ C<float, K> get(int e) const {
-    const float* q = p + (long)e * stride + base;
-    C<float, K> o;
-#pragma unroll
-    for (int h = 0; h < K; ++h) {
-      const int c = c0 + h;
-      o[h] = q[(long)step * (c < cmax ? c : cmax)];
-    }
-    return o;
-  }
-};
-
 // the half angle (s, c) turned by the slot's half-step rotation (rs, rc), and by twice that
 // (a full step)
 __device__ __forceinline__ void rot_by(float s, float c, float rs, float rc, float& so, float& co) {
@@ -330,8 +362,8 @@ __device__ __forceinline__ void rot_by2(float s, float c, float rs, float rc, fl
 // cos(a + d) - cos(a) from sin a, cos a and a small d (|d| < ~0.3), without cancellation
 __device__ __forceinline__ float dcos(float sa, float ca, float d) {
   const float d2 = d * d;
-  const float sd = d * (1.0f - d2 * (1.0f / 6.0f) * (1.0f - d2 * (1.0f / 20.0f)));
-  const float omc = 0.5f * d2 * (1.0f - d2 * (1.0f / 12.0f) * (1.0f - d2 * (1.0f / 30.0f)));
+  const float sd = d + d * d2 * (-1.0f / 6.0f + d2 * (1.0f / 120.0f));
+  const float omc = d2 * (0.5f + d2 * (-1.0f / 24.0f + d2 * (1.0f / 720.0f)));
   return -sa * sd - ca * omc;
 }
 
@@ -339,8 +371,8 @@ __device__ __forceinline__ float dcos(float sa, float ca, float d) {
 __device__ __forceinline__ void rot_theta(float st, float ct, float oms, float e, float& so, float& co,
                                           float& omso) {
   const float e2 = e * e;
-  const float se = e * (1.0f - e2 * (1.0f / 6.0f) * (1.0f - e2 * (1.0f / 20.0f)));
-  const float omc = 0.5f * e2 * (1.0f - e2 * (1.0f / 12.0f) * (1.0f - e2 * (1.0f / 30.0f)));
+  const float se = e + e * e2 * (-1.0f / 6.0f + e2 * (1.0f / 120.0f));
+  const float omc = e2 * (0.5f + e2 * (-1.0f / 24.0f + e2 * (1.0f / 720.0f)));
   so = st * (1.0f - omc) + ct * se;
   co = ct * (1.0f - omc) - st * se;
   omso = oms + st * omc - ct * se;
@@ -348,20 +380,22 @@ __device__ __forceinline__ void rot_theta(float st, float ct, float oms, float e
 
 // The window update.  G: sweep geometry; NDIM: 2 or 3 (the azimuthal sweep carries w and uses
 // the spherical planet terms in 3-D); phi_rows: the azimuthal sweep's W.rs / W.rcs hold the
-// rotation from a column's left edge over half a step (uniform azimuthal grid).  tx: the per-slot table of this lane's cells (TabLane
-// or TabLaneS; radial and theta sweeps read their balance terms where they are used).  P0: paraset of the
+// rotation from a column's left edge over half a step (uniform azimuthal grid).  tx: the per-slot table of this lane's cells
+// (radial and theta sweeps read their balance terms where they are used).  P0: paraset of the
 // Eulerian grid (its values outside the window's paraset ranges never reach a parabola the
-// sweep keeps).  wres: the azimuthal grid's uniform angular rate.  rsph: the spherical
+// sweep keeps).  c0: this lane's first cell of its window (a wavefront may hold several windows
+// side by side: stencils reach across the seam between two as they reach past a window's last
+// cell, and every stage's index range keeps such values out of the cells a window stores).
+// wres: the azimuthal grid's uniform angular rate.  rsph: the spherical
 // radius of an azimuthal 3-D ring.  On return cells [6, nmax-6) hold the update.
-template <int K, int G, int NDIM, class Tab, bool ADIA = false, int SL = 64, bool BARY = false>
-__device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para<float, K>& P0, int nmax,
+template <int K, int G, int NDIM, class Tab, bool ADIA = false, bool BARY = false>
+__device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para<float, K>& P0, int c0, int nmax,
                                            float dt, float wres, const PlanetF& pl, bool planet, bool flat_on,
                                            float sqrt_gam, float rsph = 0.0f, bool phi_rows = false,
                                            float gam = 1.0f) {
   constexpr bool RAD = (G == kGeoRcyl || G == kGeoRsph);
   static_assert(!ADIA || (NDIM == 2 && (G == kGeoRcyl || G == kGeoPhi)), "EOS 3 is built for 2-D disks");
   const float hdt = 0.5f * dt;
-  const float fourthd = 1.3333333333333333f;
   const float smallr = 1.0e-15f;
   // EOS 3 carries q = p / rho as its deviation dq from q_b; the pressure deviation is
   // p - p_b = rho_b dq + q_b drho + drho dq (p_b = rho_b q_b)
@@ -372,7 +406,8 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   }
 
   // ---- flatten (flatten.cu:7-40), on absolute pressure (relative-jump thresholds)
-  C<float, K> flat = splat<float, K>(0.0f);
+  C<float, K> gfl = splat<float, K>(1.0f);   // 1 - the flattening
+  bool shocked = false;
   if (flat_on) {
     C<float, K> pabs;
 #pragma unroll
@@ -380,27 +415,35 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       if constexpr (ADIA) pabs[h] = W.pb[h] + dpc[h];
       else pabs[h] = W.pb[h] + W.r[h] * W.cs2[h];
     }
-    C<float, K> pm1 = prev1(pabs), pp1 = next1(pabs), pm2 = prev2(pabs), pp2 = next2(pabs);
+    C<float, K> pm1 = prev1(pabs), pp1 = next1(pabs);
     C<float, K> um1 = prev1(W.u), up1 = next1(W.u);
-    C<float, K> steep;
+    // the jump test as a product; most wavefronts hold no shock and skip the rest
+    C<bool, K> shock;
+    bool any = false;
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      // evaluated in every lane and selected (no divergent branch around it)
-      const int c = cell_in<SL>(K, h);
-      const float dp1 = pp1[h] - pm1[h];
-      float dp2 = pp2[h] - pm2[h];
-      dp2 = (fabsf(dp2) < 1.0e-15f) ? 1.0e-15f : dp2;
-      const float ddp = fabsf(dp1) / fminf(pp1[h], pm1[h]);
-      const bool shock = (c >= 2 && c < nmax - 2) && ddp > 0.33f && !(um1[h] < up1[h]);
-      const float st = fmaxf(0.0f, (dp1 / dp2 - 0.75f) * 5.0f);
-      steep[h] = shock ? st : 0.0f;
+      const int c = c0 + h;
+      const float m = fminf(pp1[h], pm1[h]);
+      shock[h] = (c >= 2 && c < nmax - 2) && m >= 0.0f && fabsf(pp1[h] - pm1[h]) > 0.33f * m && !(um1[h] < up1[h]);
+      any = any || shock[h];
     }
-    C<float, K> sm = prev1(steep), sp = next1(steep);
+    shocked = wave_any(any);
+    if (shocked) {
+      C<float, K> pm2 = prev2(pabs), pp2 = next2(pabs), steep;
 #pragma unroll
-    for (int h = 0; h < K; ++h) {
-      const int c = cell_in<SL>(K, h);
-      const float fl = fminf(0.5f, fmaxf(sm[h], fmaxf(steep[h], sp[h])));
-      flat[h] = (c >= 2 && c < nmax - 2) ? fl : 0.0f;
+      for (int h = 0; h < K; ++h) {
+        float dp2 = pp2[h] - pm2[h];
+        dp2 = (fabsf(dp2) < 1.0e-15f) ? 1.0e-15f : dp2;
+        const float st = fmaxf(0.0f, ((pp1[h] - pm1[h]) / dp2 - 0.75f) * 5.0f);
+        steep[h] = shock[h] ? st : 0.0f;
+      }
+      C<float, K> sm = prev1(steep), sp = next1(steep);
+#pragma unroll
+      for (int h = 0; h < K; ++h) {
+        const int c = c0 + h;
+        const float fl = fminf(0.5f, fmaxf(sm[h], fmaxf(steep[h], sp[h])));
+        gfl[h] = (c >= 2 && c < nmax - 2) ? 1.0f - fl : 1.0f;
+      }
     }
   }
 
@@ -471,24 +514,43 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       fhalf[h] = hdt * f;
     }
   }
-  C<float, K> csn, csfac;
+  // reciprocals of the cell's fixed numbers: table entries, or along phi the columns' and once per ring
+  C<float, K> idx0, irb, ipb, irad;
+  if constexpr (!RAD) {
+#pragma unroll
+    for (int h = 0; h < K; ++h) irad[h] = 1.0f / W.rad[h];
+  }
+  if constexpr (G == kGeoPhi) {
+#pragma unroll
+    for (int h = 0; h < K; ++h) {
+      idx0[h] = W.idx0[h];
+      irb[h] = 1.0f / W.rb[h];
+      ipb[h] = 1.0f / W.pb[h];
+    }
+  } else {
+    idx0 = tx.get(G == kGeoTheta ? kTabIdz0 : kTabIdx0);
+    irb = tx.get(kTabIrb);
+    ipb = tx.get(kTabIpb);
+  }
+  C<float, K> csn, csfac;   // csfac: 3 (1 - (4/3) csn), for s = -a6/3
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     // sqrt(gam p / rho) = sqrt(gam) c_s for the isothermal closure, sqrt(gam q) for EOS 3
     float s;
-    if constexpr (ADIA) s = hdt * sqrtf(gam * (W.qb[h] + W.q[h])) / W.dx0[h];
-    else s = hdt * sqrt_gam * W.cs[h] / W.dx0[h];
-    if constexpr (G == kGeoPhi || G == kGeoTheta) s = s / W.rad[h];
+    if constexpr (ADIA) s = hdt * sqrtf(gam * (W.qb[h] + W.q[h]));
+    else s = hdt * sqrt_gam * W.cs[h];
+    if constexpr (G == kGeoPhi || G == kGeoTheta) s = s * irad[h];
+    s = s * idx0[h];
     csn[h] = s;
-    csfac[h] = 1.0f - fourthd * s;
+    csfac[h] = 3.0f - 4.0f * s;
   }
   // edge averages of the traced parabolae (states.cu:45-68), in the cell's frame: the
   // cell's value x plus the average's offset from it
   auto edges = [&](const ParabR<K>& q, const C<float, K>& x, C<float, K>& re, C<float, K>& le) {
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      re[h] = x[h] + (q.al[h] + q.da[h] - csn[h] * (q.da[h] - csfac[h] * q.a6[h]));
-      le[h] = x[h] + (q.al[h] + csn[h] * (q.da[h] + csfac[h] * q.a6[h]));
+      re[h] = x[h] + (q.ar[h] - csn[h] * (q.da[h] + csfac[h] * q.s[h]));
+      le[h] = x[h] + (q.al[h] + csn[h] * (q.da[h] - csfac[h] * q.s[h]));
     }
   };
   // interface c: left state = right edge of cell c-1, right state = left edge of cell c, as
@@ -502,33 +564,33 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       else pp[h] = W.r[h] * W.cs2[h];
     }
     // along a ring p_b is one constant
-    edges(parabola_rel<K, SL, G != kGeoPhi>(0, nmax, flat, pp, W.dpb, P0), pp, re, le);
+    edges(parabola_rel<K, G != kGeoPhi>(gfl, shocked, pp, W.dpb, P0), pp, re, le);
     C<float, K> q;
 #pragma unroll
-    for (int h = 0; h < K; ++h) q[h] = re[h] / W.pb[h];
-    C<float, K> qm = prev1(q), pbm = prev1(W.pb), dpbm = prev1(W.dpb);
+    for (int h = 0; h < K; ++h) q[h] = re[h] * ipb[h];
+    C<float, K> qm = prev1(q), ipbm = prev1(ipb), dpbm = prev1(W.dpb);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       epl[h] = qm[h];
-      epr[h] = (le[h] + dpbm[h]) / pbm[h];
+      epr[h] = (le[h] + dpbm[h]) * ipbm[h];
     }
   }
   {
     C<float, K> re, le;
-    edges(parabola_rel<K, SL, G != kGeoPhi>(0, nmax, flat, W.r, W.drb, P0), W.r, re, le);
+    edges(parabola_rel<K, G != kGeoPhi>(gfl, shocked, W.r, W.drb, P0), W.r, re, le);
     C<float, K> q;
 #pragma unroll
-    for (int h = 0; h < K; ++h) q[h] = re[h] / W.rb[h];
-    C<float, K> qm = prev1(q), rbm = prev1(W.rb), drbm = prev1(W.drb);
+    for (int h = 0; h < K; ++h) q[h] = re[h] * irb[h];
+    C<float, K> qm = prev1(q), irbm = prev1(irb), drbm = prev1(W.drb);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       erl[h] = qm[h];
-      err[h] = (le[h] + drbm[h]) / rbm[h];
+      err[h] = (le[h] + drbm[h]) * irbm[h];
     }
   }
   {
     C<float, K> re, le;
-    edges(parabola_rel<K, SL, false>(0, nmax, flat, W.u, W.u, P0), W.u, re, le);
+    edges(parabola_rel<K, false>(gfl, shocked, W.u, W.u, P0), W.u, re, le);
     C<float, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -544,28 +606,34 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   if constexpr (ADIA) {
     // gamma-law interface (riemann.cu:55-71, EOS 2's solver): the two-rarefaction estimate
     // of p*, then u* from each side's shock or rarefaction curve.  Every quantity is taken
-    // relative to the background of cell c-1 (p_b, rho_b, c0^2 = gam q_b): a_s = c_s / c0,
-    // N / (2 c0) = (a_l + a_r)/2 - (gam-1)(ur-ul)/(4 c0), D / (2 c0 p_b^-z) =
+    // relative to the background of cell c-1 (p_b, rho_b, a0^2 = gam q_b): a_s = c_s / a0,
+    // N / (2 a0) = (a_l + a_r)/2 - (gam-1)(ur-ul)/(4 a0), D / (2 a0 p_b^-z) =
     // (a_l (1+epl)^-z + a_r (1+epr)^-z)/2, p* / p_b = (N / D)^(1/z) with every factor formed
     // as 1 + (a small number)
     const float z = 0.5f * (gam - 1.0f) / gam, iz = 1.0f / z, gm1 = gam - 1.0f, gp1 = gam + 1.0f;
     const C<float, K> qbm = prev1(W.qb);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const float lpl = log1p_acc(epl[h]), lpr = log1p_acc(epr[h]);
-      const float lrl = log1p_acc(erl[h]), lrr = log1p_acc(err[h]);
-      const float c0 = sqrtf(gam * qbm[h]);
+      const int c = c0 + h;
+      const bool used = c >= 3 && c < nmax - 2;
+      // jumps below 0.2 keep every argument of the states' logs and exps (z < 1/2) below 1/4
+      const bool w1 = wave_any(used && !(max4(epl[h], epr[h], erl[h], err[h]) < 0.2f));
+      const float lpl = log1p_acc(epl[h], w1), lpr = log1p_acc(epr[h], w1);
+      const float lrl = log1p_acc(erl[h], w1), lrr = log1p_acc(err[h], w1);
+      const float a0 = sqrtf(gam * qbm[h]);
       const float hl = 0.5f * (lpl - lrl), hr = 0.5f * (lpr - lrr);   // log(a_l), log(a_r)
-      const float al1 = expm1_acc(hl), ar1 = expm1_acc(hr);
-      const float nm1 = 0.5f * (al1 + ar1) - 0.25f * gm1 * (ur[h] - ul[h]) / c0;
-      const float dm1 = 0.5f * (expm1_acc(hl - z * lpl) + expm1_acc(hr - z * lpr));
-      const float lm = iz * (log1p_acc(nm1) - log1p_acc(dm1));   // log(p* / p_b)
-      const float e_ = expm1_acc(lm);
+      const float al1 = expm1_acc(hl, w1), ar1 = expm1_acc(hr, w1);
+      const float nm1 = 0.5f * (al1 + ar1) - 0.25f * gm1 * (ur[h] - ul[h]) / a0;
+      const float dm1 = 0.5f * (expm1_acc(hl - z * lpl, w1) + expm1_acc(hr - z * lpr, w1));
+      const bool w2 = wave_any(used && !(fmaxf(fabsf(nm1), fabsf(dm1)) < 0.25f));
+      const float lm = iz * (log1p_acc(nm1, w2) - log1p_acc(dm1, w2));   // log(p* / p_b)
+      const bool w3 = w1 || wave_any(used && !(fabsf(lm) < 0.25f));
+      const float e_ = expm1_acc(lm, w3);
       float t1, t2;   // right and left wave terms of u* (riemann.cu:64-70)
       if (e_ > epr[h]) t1 = (e_ - epr[h]) * sqrtf(2.0f * qbm[h] / ((1.0f + err[h]) * (gp1 * (1.0f + e_) + gm1 * (1.0f + epr[h]))));
-      else t1 = 2.0f * c0 * (1.0f + ar1) * expm1_acc(z * (lm - lpr)) / gm1;
+      else t1 = 2.0f * a0 * (1.0f + ar1) * expm1_acc(z * (lm - lpr), w3) / gm1;
       if (e_ > epl[h]) t2 = (e_ - epl[h]) * sqrtf(2.0f * qbm[h] / ((1.0f + erl[h]) * (gp1 * (1.0f + e_) + gm1 * (1.0f + epl[h]))));
-      else t2 = 2.0f * c0 * (1.0f + al1) * expm1_acc(z * (lm - lpl)) / gm1;
+      else t2 = 2.0f * a0 * (1.0f + al1) * expm1_acc(z * (lm - lpl), w3) / gm1;
       em[h] = e_;
       umid[h] = 0.5f * (ur[h] + ul[h]) + 0.5f * (t1 - t2);
     }
@@ -573,12 +641,17 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     C<float, K> csm = prev1(W.cs);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const float lpl = log1p_acc(epl[h]), lpr = log1p_acc(epr[h]);
       // t1 only scales small differences (of velocity and of log pressure), so its plain
-      // FP32 relative accuracy suffices: no logs of the density states
-      const float t1 = 0.5f * csm[h] * (sqrtf((1.0f + epl[h]) / (1.0f + erl[h])) + sqrtf((1.0f + epr[h]) / (1.0f + err[h])));
+      // FP32 relative accuracy suffices: no logs of the density states, sqrt(a/b) = a rsqrt(a b)
+      const float pl1 = 1.0f + epl[h], pr1 = 1.0f + epr[h];
+      const float t1 = 0.5f * csm[h] * (pl1 * __frsqrt_rn(pl1 + pl1 * erl[h]) + pr1 * __frsqrt_rn(pr1 + pr1 * err[h]));
       const float t2 = -0.5f * (ur[h] - ul[h]) / t1;
-      em[h] = expm1_acc(0.5f * (lpl + lpr) + t2);
+      const int c = c0 + h;
+      const bool used = c >= 3 && c < nmax - 2;
+      const bool w = wave_any(used && !(fmaxf(fabsf(epl[h]), fabsf(epr[h])) < 0.25f));
+      const float lpl = log1p_acc(epl[h], w), lpr = log1p_acc(epr[h], w);
+      const float y = 0.5f * (lpl + lpr) + t2;
+      em[h] = expm1_acc(y, wave_any(used && !(fabsf(y) < 0.25f)));
       umid[h] = ul[h] - t1 * (0.5f * (lpr - lpl) + t2);
     }
   } else {
@@ -587,39 +660,43 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     // c_s^2 times the density states, so eps_p = eps_rho and t1 = c_s exactly
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const float lrl = log1p_acc(erl[h]), lrr = log1p_acc(err[h]);
       const float t1 = W.cs[h];
-      const float t2 = -0.5f * (ur[h] - ul[h]) / t1;
-      em[h] = expm1_acc(0.5f * (lrl + lrr) + t2);
+      const float t2 = (-0.5f / t1) * (ur[h] - ul[h]);
+      const int c = c0 + h;
+      const bool used = c >= 3 && c < nmax - 2;
+      const bool w = wave_any(used && !(fmaxf(fabsf(erl[h]), fabsf(err[h])) < 0.25f));
+      const float lrl = log1p_acc(erl[h], w), lrr = log1p_acc(err[h], w);
+      const float y = 0.5f * (lrl + lrr) + t2;
+      em[h] = expm1_acc(y, wave_any(used && !(fabsf(y) < 0.25f)));
       umid[h] = ul[h] - t1 * (0.5f * (lrr - lrl) + t2);
     }
   }
 
   // ---- evolve (evolve.cu:3-166): edges as displacements from the Eulerian edges.  The
-  // reference moves edges [3, nmax-2) and cells [3, nmax-3).
-  C<float, K> smv, dlt;
+  // reference moves edges [3, nmax-2) and cells [3, nmax-3); here every one moves: what a kept
+  // cell reads lies inside those ranges (edges 3 to nmax-3, cells 3 to nmax-4).
+  C<float, K> sx, dltx;
   const float Wd = (G == kGeoPhi) ? dt * wres : 0.0f;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_in<SL>(K, h);
-    const bool mv = (c >= 3 && c < nmax - 2);
     float s;
     if constexpr (RAD) s = dt * umid[h];
-    else s = dt * umid[h] / W.rad[h];
-    smv[h] = mv ? s : 0.0f;
-    dlt[h] = mv ? s + Wd : 0.0f;
+    else s = dt * irad[h] * umid[h];
+    sx[h] = s;
+    dltx[h] = s + Wd;
   }
-  C<float, K> Dl, dltx, sx;
+  C<float, K> Dl;
   {
-    C<float, K> sp = next1(smv);
+    C<float, K> sp = next1(sx);
 #pragma unroll
-    for (int h = 0; h < K; ++h) {
-      const int c = cell_in<SL>(K, h);
-      const bool in = (c >= 3 && c < nmax - 3);
-      Dl[h] = in ? sp[h] - smv[h] : 0.0f;   // dxl - dx0, free of the uniform motion
-      dltx[h] = in ? dlt[h] : 0.0f;          // the left edge of a moved cell
-      sx[h] = in ? smv[h] : 0.0f;
-    }
+    for (int h = 0; h < K; ++h) Dl[h] = sp[h] - sx[h];   // dxl - dx0, free of the uniform motion
+  }
+  C<float, K> idvol0;
+  if constexpr (G == kGeoPhi) {
+#pragma unroll
+    for (int h = 0; h < K; ++h) idvol0[h] = irad[h] * W.iyv[h];
+  } else {
+    idvol0 = tx.get(G == kGeoTheta ? kTabIdvolZ : kTabIdvol0);
   }
   C<float, K> rL;   // Lagrangian density deviation
   C<float, K> szl, czl;   // theta sweep: sin / cos of the left edge
@@ -644,8 +721,6 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       }
 #pragma unroll
       for (int h = 0; h < K; ++h) {
-        const int c = cell_in<SL>(K, h);
-        const bool in = (c >= 3 && c < nmax - 3);
         const float ixc = tixc[h];
         const float ixc3 = ixc * ixc * ixc;
         const float rho = W.rb[h] + W.r[h];
@@ -690,8 +765,9 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
           V0 = 0.5f * (x0 * x0 + xa0p[h] * xa0p[h]);
           dV = 0.5f * (d * (x0 + d * (1.0f / 3.0f)) + dp_ * (xa0p[h] + dp_ * (1.0f / 3.0f)));
         }
-        const float acc = res_bg[h] + q1 + 0.5f * fdiff + abg[h] * (W.r[h] / rho) -
-                          (dpbm[h] * dV + dp * (V0 + dV)) / (rho * W.dvol0[h]);
+        const float irho = 1.0f / rho, im = irho * idvol0[h];
+        const float acc = res_bg[h] + q1 + 0.5f * fdiff + abg[h] * (W.r[h] * irho) -
+                          (dpbm[h] * dV + dp * (V0 + dV)) * im;
         // Lagrangian volume change in offset form
         float ddv;
         if constexpr (G == kGeoRcyl) {
@@ -704,7 +780,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
                 w0 * D * D + D * D * D * (1.0f / 3.0f);
         }
         const float dvol = W.dvol0[h] + ddv;
-        rL[h] = in ? W.r[h] - rho * ddv / dvol : W.r[h];   // (r dvol0 - rho_b ddv) / dvol
+        rL[h] = W.r[h] - rho * ddv / dvol;   // (r dvol0 - rho_b ddv) / dvol
         if constexpr (ADIA) {
           // EOS 3 (the line evolve.cu:146 leaves commented out): e = eps + u^2/2 gains
           // -dt/dm (F_r - F_l) + dt (u f1 + u' f2)/2, eps' = e - u'^2/2.  With u' = u + du and
@@ -713,11 +789,11 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
           //   eps' - eps = -dt/dm ((F_r - F_l) - (u + du/2) dp A) + dt du (f2 - f1) / 4
           const float du = dt * acc;
           const float dpA = dpbm[h] * V0 + (dpbm[h] * dV + dp * (V0 + dV));
-          const float de = -dt / (rho * W.dvol0[h]) * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpA) +
+          const float de = -dt * im * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpA) +
                            0.25f * dt * du * f21;
-          if (in) W.q[h] += (gam - 1.0f) * de;
+          W.q[h] += (gam - 1.0f) * de;
         }
-        if (in) W.u[h] = W.u[h] + dt * acc;
+        W.u[h] = W.u[h] + dt * acc;
       }
     } else if constexpr (G == kGeoPhi) {
       // EOS 3: the pressure work through the left edge, u* p* (unit area factor)
@@ -729,8 +805,6 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       }
 #pragma unroll
       for (int h = 0; h < K; ++h) {
-        const int c = cell_in<SL>(K, h);
-        const bool in = (c >= 3 && c < nmax - 3);
         float f = 0.0f, f21 = 0.0f;
         if (planet) {
           const float off = dltx[h] + 0.5f * Dl[h] + dt * (W.vrot[h] - pl.vy);
@@ -747,17 +821,18 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
         }
         const float rho = W.rb[h] + W.r[h];
         const float dpm = W.pb[h] * (emp[h] - em[h]);   // p_b is uniform along the ring
-        const float un = W.u[h] + (0.5f * dt * f - dt * dpm / (rho * W.dvol0[h]));
+        const float im = idvol0[h] / rho;
+        const float un = W.u[h] + (0.5f * dt * f - dt * dpm * im);
         const float ddv = Dl[h] * W.rad[h];
         const float dvol = W.dvol0[h] + ddv;
-        rL[h] = in ? W.r[h] - rho * ddv / dvol : W.r[h];   // (r dvol0 - rho_b ddv) / dvol
+        rL[h] = W.r[h] - rho * ddv / dvol;   // (r dvol0 - rho_b ddv) / dvol
         if constexpr (ADIA) {   // as in the radial sweep, with unit area factors
           const float du = un - W.u[h];
-          const float de = -dt / (rho * W.dvol0[h]) * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpm) +
+          const float de = -dt * im * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpm) +
                            0.25f * dt * du * f21;
-          if (in) W.q[h] += (gam - 1.0f) * de;
+          W.q[h] += (gam - 1.0f) * de;
         }
-        if (in) W.u[h] = un;
+        W.u[h] = un;
       }
     } else {
       // theta: centrifugal theta component L^2 G(theta), G = cos / (r sin)^3, minus the
@@ -776,8 +851,6 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       C<float, K> vfdp = next1(vfd);
 #pragma unroll
       for (int h = 0; h < K; ++h) {
-        const int c = cell_in<SL>(K, h);
-        const bool in = (c >= 3 && c < nmax - 3);
         const float rho = W.rb[h] + W.r[h];
         const float dl = W.w[h];
         const float qq = dl * (2.0f * W.Lb[h] + dl);
@@ -796,13 +869,14 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
         const float dp = W.pb[h] * emp[h] - pbm[h] * em[h];
         const float V0 = 0.5f * (szl[h] + szlp[h]);
         const float dV = 0.5f * (vfd[h] + vfdp[h]);
-        const float acc = res_bg[h] + qq * Gc[h] + 0.25f * fdiff + abg[h] * (W.r[h] / rho) -
-                          (dpbm[h] * dV + dp * (V0 + dV)) / (rho * W.dvol0[h]);
+        const float irho = 1.0f / rho;
+        const float acc = res_bg[h] + qq * Gc[h] + 0.25f * fdiff + abg[h] * (W.r[h] * irho) -
+                          (dpbm[h] * dV + dp * (V0 + dV)) * (irho * idvol0[h]);
         // dvol = r (cos(x0 + d) - cos(x1 + d + D)) with x1 the right edge
         const float ddv = W.rad[h] * (dcos(szl[h], czl[h], dltx[h]) - dcos(szr[h], czr[h], dltx[h] + Dl[h]));
         const float dvol = W.dvol0[h] + ddv;
-        rL[h] = in ? W.r[h] - rho * ddv / dvol : W.r[h];   // (r dvol0 - rho_b ddv) / dvol
-        if (in) W.u[h] = W.u[h] + dt * acc;
+        rL[h] = W.r[h] - rho * ddv / dvol;   // (r dvol0 - rho_b ddv) / dvol
+        W.u[h] = W.u[h] + dt * acc;
       }
     }
   }
@@ -811,8 +885,9 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   C<float, K> dxl;
 #pragma unroll
   for (int h = 0; h < K; ++h) dxl[h] = W.dx0[h] + Dl[h];
-  Para<float, K> P1 = paraset<float, K, SL>(3, nmax - 3, dxl);
-  C<float, K> dxf, dxf2, lvol, delC;
+  const Para<float, K> P1 = paraset_f32<K>(dxl);
+  C<float, K> dxf, dxf2, lvol;
+  C<bool, K> fwd;   // the edge moves forward: it sweeps the left neighbour
   C<float, K> dxm = prev1(dxl);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
@@ -821,32 +896,26 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     else if constexpr (G == kGeoRsph) lvol[h] = d * (W.xa0[h] * (W.xa0[h] + d) + d * d * (1.0f / 3.0f));
     else if constexpr (G == kGeoPhi) lvol[h] = d * W.rad[h];
     else lvol[h] = -W.rad[h] * dcos(szl[h], czl[h], d);
-    delC[h] = (d >= 0.0f) ? 1.0f : 0.0f;
-    float e;
-    if (d >= 0.0f) {
-      e = 0.5f * d / dxm[h];
-      dxf2[h] = 1.0f - fourthd * e;
-    } else {
-      e = 0.5f * d / dxl[h];
-      dxf2[h] = 1.0f + fourthd * e;
-    }
+    fwd[h] = d >= 0.0f;
+    const float e = 0.5f * d / (fwd[h] ? dxm[h] : dxl[h]);
     dxf[h] = e;
+    dxf2[h] = 3.0f - 4.0f * fabsf(e);   // either way the edge moves
   }
   // average over the swept region of the left edge (remap.cu:59-90) minus the cell's own
   // value: from the left neighbour's parabola (its offset from X(c-1), then the jump
   // X(c) - X(c-1) in this frame) or from this cell's own
   auto face = [&](const ParabR<K>& Q, C<float, K>& out) {
-    C<float, K> alm = prev1(Q.al), dam = prev1(Q.da), a6m = prev1(Q.a6);
+    C<float, K> arm = prev1(Q.ar), dam = prev1(Q.da), sm = prev1(Q.s);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      if (delC[h] != 0.0f) out[h] = (alm[h] + dam[h] - dxf[h] * (dam[h] - dxf2[h] * a6m[h])) - Q.dl[h];
-      else out[h] = Q.al[h] - dxf[h] * (Q.da[h] + dxf2[h] * Q.a6[h]);
+      if (fwd[h]) out[h] = (arm[h] - Q.dl[h]) - dxf[h] * (dam[h] + dxf2[h] * sm[h]);
+      else out[h] = Q.al[h] - dxf[h] * (Q.da[h] - dxf2[h] * Q.s[h]);
     }
   };
   C<float, K> invm, fr;
   {
     C<float, K> fv, frd;
-    face(parabola_rel<K, SL, G != kGeoPhi>(3, nmax - 3, flat, rL, W.drb, P1), fv);
+    face(parabola_rel<K, G != kGeoPhi>(gfl, shocked, rL, W.drb, P1), fv);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       fv[h] = rL[h] + fv[h];   // the face's deviation from rho_b of this cell
@@ -856,16 +925,17 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       } else {
         // rho_b times the uniform displacement is the same at every edge: it carries no
         // mass difference, so the density update leaves it out
-        frd[h] = W.rb[h] * (W.rad[h] * sx[h]) + fv[h] * lvol[h];
-        fr[h] = frd[h] + W.rb[h] * (W.rad[h] * (dltx[h] - sx[h]));
+        const float mr = W.rb[h] * W.rad[h];
+        frd[h] = mr * sx[h] + fv[h] * lvol[h];
+        fr[h] = frd[h] + mr * Wd;
       }
     }
     C<float, K> frp = next1(frd);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_in<SL>(K, h);
-      const float rn = W.r[h] + (frd[h] - frp[h]) / W.dvol0[h];
-      invm[h] = 1.0f / (fmaxf(W.rb[h] + rn, smallr) * W.dvol0[h]);
+      const int c = c0 + h;
+      const float rn = W.r[h] + (frd[h] - frp[h]) * idvol0[h];
+      invm[h] = idvol0[h] / fmaxf(W.rb[h] + rn, smallr);
       W.r[h] = (c >= 6 && c < nmax - 6) ? rn : rL[h];
     }
   }
@@ -883,18 +953,18 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     C<float, K> rlp = next1(rl);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const int c = cell_in<SL>(K, h);
+      const int c = c0 + h;
       // the right face relative to this cell's X: (face(c+1) - X(c+1)) + (X(c+1) + dbg - X)
       const float rr = rlp[h] + Q.dr[h];
       if (c >= 6 && c < nmax - 6) X[h] = X[h] + (rl[h] * fr[h] - rr * frp[h]) * invm[h];
     }
   };
-  auto remap_plain = [&](C<float, K>& X) { remap_inc(X, parabola_rel<K, SL, false>(3, nmax - 3, flat, X, X, P1)); };
+  auto remap_plain = [&](C<float, K>& X) { remap_inc(X, parabola_rel<K, false>(gfl, shocked, X, X, P1)); };
   // deviations from a background that varies along the sweep (l - L_b; EOS 3's q - q_b):
   // fluxes relative to the cell's own background; the right edge's face comes from the next
   // cell's frame, b(c+1) = b(c) + dbg
   auto remap_bg = [&](C<float, K>& X, const C<float, K>& dbg) {
-    remap_inc(X, parabola_rel<K, SL, true>(3, nmax - 3, flat, X, dbg, P1));
+    remap_inc(X, parabola_rel<K, true>(gfl, shocked, X, dbg, P1));
   };
   remap_plain(W.u);
   if constexpr (RAD) remap_bg(W.v, W.dLb);
@@ -915,8 +985,8 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
 // the cell widths: the left edges of c-1, c, c+1 sit at 0, dx(c-1), dx(c-1) + dx(c)).
 // l_new = l + dt R ddv / rho leaves L_b in place: dl += dt R ddv / rho.  SPH (3-D spherical
 // r): also w = r v_theta, whose background is zero.
-template <int K, int SL = 64, bool SPH = false>
-__device__ __forceinline__ void visc_r_pert(WinP<K>& W, const TabLane<K>& tx, int lim, float dt) {
+template <int K, bool SPH = false>
+__device__ __forceinline__ void visc_r_pert(WinP<K>& W, const TabLane<K>& tx, int c0, int lim, float dt) {
   const C<float, K> nu = tx.get(kTabNu), dnb = tx.get(kTabDnb), d1ob = tx.get(kTabD1Ob), d2ob = tx.get(kTabD2Ob),
                     irc = tx.get(kTabIrc), rcyl = tx.get(kTabRc);
   C<float, K> np_, om;
@@ -934,7 +1004,7 @@ __device__ __forceinline__ void visc_r_pert(WinP<K>& W, const TabLane<K>& tx, in
   }
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_in<SL>(K, h);
+    const int c = c0 + h;
     const float x2 = wm[h], x3 = wm[h] + W.dx0[h], R = rcyl[h];
     const float rho = W.rb[h] + W.r[h], n = nu[h] * rho;
     float dn, d1, d2, e1, e2;
@@ -964,7 +1034,7 @@ __device__ __forceinline__ void visc_r_pert(WinP<K>& W, const TabLane<K>& tx, in
 // uniform along the ring, so only deviations enter the derivatives.  The coordinates are
 // arc lengths along the ring, the left edges times R = r_cyl (ppm.cu:277-278).
 template <int K, bool W3 = false>
-__device__ __forceinline__ void visc_p_pert(WinP<K>& W, int lim, float dt, float nu, float R) {
+__device__ __forceinline__ void visc_p_pert(WinP<K>& W, int c0, int lim, float dt, float nu, float R) {
   C<float, K> np_, wx;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
@@ -981,7 +1051,7 @@ __device__ __forceinline__ void visc_p_pert(WinP<K>& W, int lim, float dt, float
   }
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_of(K, h);
+    const int c = c0 + h;
     const float x2 = wm[h], x3 = wm[h] + wx[h];
     const float rho = W.rb[h] + W.r[h], n = nu * rho;
     float dn, d1, d2;
@@ -1009,8 +1079,8 @@ __device__ __forceinline__ void visc_p_pert(WinP<K>& W, int lim, float dt, float
 // rho_b and v_bg vary along theta: their derivatives come from the table (FP64 rounded once),
 // the deviations' from the cell widths.  v_phi is carried as l - L_b = r_cyl (v_phi - v_bg):
 // the update adds dt r_cyl ddv / rho to it.
-template <int K, int SL = 64>
-__device__ __forceinline__ void visc_z_pert(WinP<K>& W, const TabLane<K>& tx, int lim, float dt, float vis_nu) {
+template <int K>
+__device__ __forceinline__ void visc_z_pert(WinP<K>& W, const TabLane<K>& tx, int c0, int lim, float dt, float vis_nu) {
   const C<float, K> dnb = tx.get(kTabDnbZ), d1vb = tx.get(kTabD1VZ), d2vb = tx.get(kTabD2VZ), irc = tx.get(kTabIrc),
                     rcyl = tx.get(kTabRc);
   C<float, K> np_, dv, wx;
@@ -1025,7 +1095,7 @@ __device__ __forceinline__ void visc_z_pert(WinP<K>& W, const TabLane<K>& tx, in
               vm = prev1(dv), vp = next1(dv);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_in<SL>(K, h);
+    const int c = c0 + h;
     const float x2 = wm[h], x3 = wm[h] + wx[h];
     const float rho = W.rb[h] + W.r[h], n = vis_nu * rho;
     float dn, d1, d2;
