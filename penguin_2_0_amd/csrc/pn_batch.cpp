@@ -200,8 +200,8 @@ bool all_fused(const pn_batch* b) {
 // one step of every disk: the CFL pass of each disk whose planet moves or which has damping
 // zones, the batched pre-step, each disk's radial ghost copies, the batched sweeps, each
 // damped disk's damping, the batched post-step,
-// then each moving planet's time, drift, disk forces (modes 8 / 9 from its FP32 state) and
-// closing kick -- the order pn_run gives a single disk (damping is ring-uniform, so it commutes
+// then each moving planet's damping and disk forces (modes 8 / 9 from its FP32 state), time, drift
+// and closing kick -- the order pn_run gives a single disk (damping is ring-uniform, so it commutes
 // with the roll that the post-step does for a moving planet's disk).  With every CFL fused, a step
 // that is not its run's first starts from the tables its predecessor left and one that is not its
 // last ends in the mid-step (post-step and next pre-step).
@@ -222,7 +222,7 @@ int launch_batch_step(pn_batch* b, int cur, bool first, bool last) {
   if (e == hipSuccess) e = f32_sweep_x_batch(b->stream, b->dd, b->dfs, b->order_x, b->nslot_x, b->var_x, cur, b->grid_x, any_bary(b), any_adia(b));
   if (e == hipSuccess) e = f32_sweep_y_batch(b->stream, b->dd, b->dfs, b->base_y, n, b->var_y, cur ^ 1, b->grid_y, any_bary(b), any_adia(b));
   for (pn_ctx* c : b->disks) {
-    if (!c->P.kill_flag || e != hipSuccess) continue;
+    if (!c->P.kill_flag || c->P.plnt_flag == 2 || e != hipSuccess) continue;
     e = f32_damp(on_batch(b, c), c->df, cur);
   }
   if (e == hipSuccess) {
@@ -231,7 +231,7 @@ int launch_batch_step(pn_batch* b, int cur, bool first, bool last) {
   }
   for (pn_ctx* c : b->disks) {
     if (c->P.plnt_flag != 2 || e != hipSuccess) continue;
-    e = launch_planet_after_sweep(on_batch(b, c), cur, &c->df);
+    e = launch_planet_after_sweep(on_batch(b, c), cur, &c->df, false);
   }
   if (e != hipSuccess) return bfail(b, PN_ERR_HIP, "batched step: %s", hipGetErrorString(e));
   return PN_OK;

@@ -63,6 +63,7 @@ struct DevGrid {
   int *rot_j, *inc_j;
   const double *y, *dy, *yc, *yvol;
   const pn_symdisk* val;
+  const double2* rpow;   // 2-D, a planet that feels the disk: x^-p_alpha and x^-3/2 per slot
   // FP64 contexts (null on the FP32 path): the slot table, in 3-D its theta-major copy (slot
   // (ir, kz) at kz + sk ir, so that a theta pencil's slots are consecutive), per column cos / sin
   // of the angle from the planet, and paraset of a uniform azimuthal grid
@@ -89,6 +90,7 @@ struct StepScalars {
   double FrRot;
   double simtime;
   pn_body planet;
+  pn_body moved;      // a planet that feels the disk: the planet after this step's drift
   double cfl_max;     // max signal speed / width behind the last dt
   double red[4];      // reduction results (mass, modes 8 / 9)
   int64_t ncycle;

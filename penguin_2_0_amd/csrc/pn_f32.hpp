@@ -140,6 +140,8 @@ hipError_t f32_reduce(const LaunchCtx& c, const DevF32& f, int src, int mode, do
 hipError_t f32_totals(const LaunchCtx& c, const DevF32& f, int src, double* out2);
 // azimuthal mean of field (0 Sigma, 1 P, 2 v_r, 3 v_phi, 4 v_theta) per interior ring into out
 hipError_t f32_ring_means(const LaunchCtx& c, const DevF32& f, int src, int field, double* out);
+// nb pairs of partial sums of the disk's pull on the planet at ss->moved, and the damping zones
+hipError_t f32_planet_torque(const LaunchCtx& c, const DevF32& f, int src, bool roll, int nb);
 // damping zones at the radial edges with ss->dt (the FP64 path's launch_damp on the FP32 state)
 hipError_t f32_damp(const LaunchCtx& c, const DevF32& f, int src);
 // radial boundary codes other than 3 (the FP64 path's launch_fill_ghosts on the FP32 state);

@@ -4,6 +4,7 @@
 
 #include "pn_f32.hpp"
 #include "pn_launch.hpp"
+#include "pn_torque.hpp"
 #include "ppm_wave.hpp"
 
 namespace pn {
@@ -52,10 +53,7 @@ __global__ void k_rotate(DevGrid g) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= g.imax * g.kmax) return;
   const int s = slot_of(g, n % g.imax, n / g.imax);
-  int j = g.rot_j[s] + g.inc_j[s];
-  if (j < 0) j += g.jmax;
-  if (j >= g.jmax) j -= g.jmax;
-  g.rot_j[s] = j;
+  g.rot_j[s] = rolled(g, s);
 }
 
 // set_boundx (boundary.cu:86-206) on the FP64 state of buffer src: each radial ghost cell
@@ -289,25 +287,47 @@ __device__ __forceinline__ void neumaier_add(double& s, double& c, double x) {
 
 constexpr int kSumThreads = 256;
 
-// Neumaier sum of nb partials (stride st) into out, in a fixed order: thread t sums
-// partials t, t + 256, ...; thread 0 then adds the 256 running sums and their
-// compensations in thread order
+// (s, c) += (s2, c2): compensated sums merged
+__device__ __forceinline__ void neumaier_merge(double& s, double& c, double s2, double c2) {
+  neumaier_add(s, c, s2);
+  c += c2;
+}
+
+// the workgroup's compensated sums added up in a fixed order, a tree over the lanes and then the
+// waves (one serial pass over 256 sums took 8 us); the result is valid in thread 0.  sh: two
+// doubles per wave, free again after the caller's next barrier.
+__device__ __forceinline__ double block_sum(double s, double c, double* sh) {
+  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  for (int off = 32; off > 0; off >>= 1) {
+    const double s2 = __shfl_down(s, off), c2 = __shfl_down(c, off);
+    neumaier_merge(s, c, s2, c2);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[2 * w] = s;
+    sh[2 * w + 1] = c;
+  }
+  __syncthreads();
+  if (w == 0) {
+    const bool in = threadIdx.x < (unsigned)nw;
+    s = in ? sh[2 * threadIdx.x] : 0.0;
+    c = in ? sh[2 * threadIdx.x + 1] : 0.0;
+    for (int off = 8; off > 0; off >>= 1) {   // at most 16 waves
+      const double s2 = __shfl_down(s, off), c2 = __shfl_down(c, off);
+      neumaier_merge(s, c, s2, c2);
+    }
+  }
+  return s + c;
+}
+
+// compensated sums of nb partials (stride st) into out, in a fixed order: thread t sums
+// partials t, t + 256, ...; then block_sum
 __global__ __launch_bounds__(kSumThreads) void k_sum_partials(const double* partials, int nb, int st, double* out) {
-  __shared__ double sh_s[kSumThreads], sh_c[kSumThreads];
+  __shared__ double sh[2 * (kSumThreads / 64)];
   for (int q = 0; q < st; ++q) {
     double s = 0.0, c = 0.0;
     for (int b = threadIdx.x; b < nb; b += kSumThreads) neumaier_add(s, c, partials[(long)b * st + q]);
-    sh_s[threadIdx.x] = s;
-    sh_c[threadIdx.x] = c;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double S = 0.0, Cc = 0.0;
-      for (int t = 0; t < kSumThreads; ++t) {
-        neumaier_add(S, Cc, sh_s[t]);
-        Cc += sh_c[t];
-      }
-      out[q] = S + Cc;
-    }
+    s = block_sum(s, c, sh);
+    if (threadIdx.x == 0) out[q] = s;
     __syncthreads();
   }
 }
@@ -349,19 +369,12 @@ __device__ void land_close(StepScalars* ss, double dt) {
   }
 }
 
-// after the sweeps: time advance, drift, forces and the closing half kick
-// (main.cu:378-387, planet.cu:54-93).  red[1], red[2] hold the mode 8 / 9 reductions
-// when the planet moves.
-__global__ void k_planet_drift(DevParams prm, StepScalars* ss) {
-  if (threadIdx.x != 0) return;
-  const double dt = ss->dt;
-  ss->simtime += dt;
-  ss->ncycle += 1;
-  pn_body& b = ss->planet;
+// the planet's drift over a step (main.cu:378, planet.cu:54-70)
+__device__ __forceinline__ void planet_drift(const DevParams& prm, double dt, double FrRot, pn_body& b) {
   const double old_rad = b.x;
   b.x += dt * b.vx;
   b.y += dt * b.vy;
-  b.vy = ((b.vy + ss->FrRot) * old_rad * old_rad / b.x / b.x) - ss->FrRot;
+  b.vy = ((b.vy + FrRot) * old_rad * old_rad / b.x / b.x) - FrRot;
   if (b.y < 0.0) b.y += kTwoPi;
   if (b.y >= kTwoPi) b.y -= kTwoPi;
   // get_h(x) = sqrt(c_s^2 x^3); the host computed rs for the current x, so it is only
@@ -369,25 +382,12 @@ __global__ void k_planet_drift(DevParams prm, StepScalars* ss) {
   if (b.x != old_rad) b.rs = prm.rs_fac * sqrt(cs2_of(prm, b.x) * b.x * b.x * b.x);
 }
 
-__global__ void k_planet_forces_kick(DevParams prm, StepScalars* ss, int do_kick) {
-  if (threadIdx.x != 0) return;
-  pn_body& b = ss->planet;
-  b.m = set_M_p(prm, ss->simtime);
-  if (prm.plnt == 2) {
-    b.fx = kSigma0 * ss->red[1] / b.m - 1.0 / b.x / b.x + b.x * ((b.vy + ss->FrRot) * (b.vy + ss->FrRot));
-    b.fy = kSigma0 * ss->red[2] / b.m;
-  } else {
-    b.fx = -1.0 / b.x / b.x + b.x * ((b.vy + ss->FrRot) * (b.vy + ss->FrRot));
-    b.fy = 0.0;
-  }
-  if (do_kick) {
-    const double dt = 0.5 * ss->dt;
-    b.vx += dt * b.fx;
-    b.vy += ss->FrRot + dt * b.fy / b.x / b.x;
-    ss->FrRot = (prm.frrot == 1) ? b.vy : 0.0;
-    b.vy -= ss->FrRot;
-    land_close(ss, ss->dt);   // the end of the step
-  }
+// half a kick from b's forces: velocities only, and the frame's rate that follows the planet
+__device__ __forceinline__ void half_kick(const DevParams& prm, StepScalars* ss, double hdt, double FrRot, pn_body& b) {
+  b.vx += hdt * b.fx;
+  b.vy += FrRot + hdt * b.fy / b.x / b.x;
+  ss->FrRot = (prm.frrot == 1) ? b.vy : 0.0;
+  b.vy -= ss->FrRot;
 }
 
 constexpr int kStepThreads = 1024;
@@ -546,14 +546,7 @@ __device__ __forceinline__ void pre_step_body(DevGrid g, const DevParams& prm, S
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0 && prm.plnt > 0) {
-    const double hdt = 0.5 * dt;
-    pn_body& b = ss->planet;
-    b.vx += hdt * b.fx;
-    b.vy += FrRot + hdt * b.fy / b.x / b.x;
-    ss->FrRot = (prm.frrot == 1) ? b.vy : 0.0;
-    b.vy -= ss->FrRot;
-  }
+  if (threadIdx.x == 0 && prm.plnt > 0) half_kick(prm, ss, 0.5 * dt, FrRot, ss->planet);
   if ((tab || g.tab) && rings) {
     __syncthreads();
     const double vy = ss->planet.vy;
@@ -562,6 +555,10 @@ __device__ __forceinline__ void pre_step_body(DevGrid g, const DevParams& prm, S
       if (tab) rot_rows_slot(g, vy, tab, tabz, tstride, dt, s);
       else turn_rows_slot(g, vy, dt, s);
     }
+  }
+  if (threadIdx.x == 0 && prm.plnt == 2) {   // where the disk's pull will be taken
+    ss->moved = ss->planet;
+    planet_drift(prm, dt, ss->FrRot, ss->moved);
   }
 }
 
@@ -596,10 +593,7 @@ __device__ __forceinline__ void roll_rings(DevGrid g) {
   const int nring = g.imax * g.kmax;
   for (int n = threadIdx.x; n < nring; n += blockDim.x) {
     const int s = slot_of(g, n % g.imax, n / g.imax);
-    int j = g.rot_j[s] + g.inc_j[s];
-    if (j < 0) j += g.jmax;
-    if (j >= g.jmax) j -= g.jmax;
-    g.rot_j[s] = j;
+    g.rot_j[s] = rolled(g, s);
   }
 }
 
@@ -615,21 +609,11 @@ __device__ __forceinline__ void post_step_body(DevGrid g, const DevParams& prm, 
   ss->ncycle += 1;
   if (prm.plnt > 0) {
     pn_body& b = ss->planet;
-    const double old_rad = b.x;
-    b.x += dt * b.vx;
-    b.y += dt * b.vy;
-    b.vy = ((b.vy + ss->FrRot) * old_rad * old_rad / b.x / b.x) - ss->FrRot;
-    if (b.y < 0.0) b.y += kTwoPi;
-    if (b.y >= kTwoPi) b.y -= kTwoPi;
-    if (b.x != old_rad) b.rs = prm.rs_fac * sqrt(cs2_of(prm, b.x) * b.x * b.x * b.x);
+    planet_drift(prm, dt, ss->FrRot, b);
     b.m = set_M_p(prm, ss->simtime);
     b.fx = -1.0 / b.x / b.x + b.x * ((b.vy + ss->FrRot) * (b.vy + ss->FrRot));
     b.fy = 0.0;
-    const double hdt = 0.5 * dt;
-    b.vx += hdt * b.fx;
-    b.vy += ss->FrRot + hdt * b.fy / b.x / b.x;
-    ss->FrRot = (prm.frrot == 1) ? b.vy : 0.0;
-    b.vy -= ss->FrRot;
+    half_kick(prm, ss, 0.5 * dt, ss->FrRot, b);
   }
   land_close(ss, dt);
   if (ncfl > 0) finalize_dt(prm, ss, mx);
@@ -661,12 +645,7 @@ __global__ __launch_bounds__(256) void k_mid_rings(DevGrid g, DevParams prm, con
   if (s >= g.sr * g.sk) return;
   if (prm.fargo > 0) {
     const int i = s % g.sr - kNpad, k = s / g.sr - g.k0;
-    if (i >= 0 && i < g.imax && k >= 0 && k < g.kmax) {
-      int j = g.rot_j[s] + g.inc_j[s];
-      if (j < 0) j += g.jmax;
-      if (j >= g.jmax) j -= g.jmax;
-      g.rot_j[s] = j;
-    }
+    if (i >= 0 && i < g.imax && k >= 0 && k < g.kmax) g.rot_j[s] = rolled(g, s);
   }
   ring_slot(g, prm, ss->dt, ss->fr_shift, ss->planet.vy, tab, tabz, tstride, s);
 }
@@ -683,6 +662,54 @@ __global__ __launch_bounds__(256) void k_max_chunks(const double* __restrict__ i
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) out[blockIdx.x] = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
+}
+
+// The end of a step for a planet that feels the disk, in one workgroup: the roll of every ring
+// (roll), the disk's pull from nb pairs of partials (none in 3-D, where the reference takes it as
+// zero), time, drift (already in ss->moved), forces and closing half kick.
+__global__ __launch_bounds__(kStepThreads) void k_planet_finish(DevGrid g, DevParams prm, StepScalars* ss,
+                                                                const double* __restrict__ partials, int nb, int roll) {
+  __shared__ double sh8[2 * (kStepThreads / 64)], sh9[2 * (kStepThreads / 64)];
+  if (roll) roll_rings(g);
+  double s8 = 0.0, c8 = 0.0, s9 = 0.0, c9 = 0.0;
+  for (int b = threadIdx.x; b < nb; b += kStepThreads) {
+    neumaier_add(s8, c8, partials[2 * b]);
+    neumaier_add(s9, c9, partials[2 * b + 1]);
+  }
+  s8 = block_sum(s8, c8, sh8);
+  s9 = block_sum(s9, c9, sh9);
+  if (threadIdx.x != 0) return;
+  ss->red[1] = s8;
+  ss->red[2] = s9;
+  const double dt = ss->dt;
+  ss->simtime += dt;
+  ss->ncycle += 1;
+  pn_body b = ss->moved;
+  b.m = set_M_p(prm, ss->simtime);
+  b.fx = kSigma0 * s8 / b.m - 1.0 / b.x / b.x + b.x * ((b.vy + ss->FrRot) * (b.vy + ss->FrRot));
+  b.fy = kSigma0 * s9 / b.m;
+  half_kick(prm, ss, 0.5 * dt, ss->FrRot, b);
+  ss->planet = b;
+  land_close(ss, dt);
+}
+
+// the disk's pull on a moving planet from the FP64 state, and its damping zones
+__global__ __launch_bounds__(256) void k_planet_torque(DevGrid g, DevParams prm, const StepScalars* __restrict__ ss,
+                                                       int src, int roll, double* partials) {
+  planet_torque(g, prm, ss, roll, partials, [&](int, int n, long a, double k) {
+    double r = g.f[src][FR][a];
+    if (k != 0.0) {
+      const pn_symdisk V = g.val[n];
+      r += k * (V.r - r);
+      g.f[src][FR][a] = r;
+      double* F[kNField] = {nullptr, g.f[src][FP], g.f[src][FU], g.f[src][FV], g.f[src][FW]};
+      F[FP][a] += k * (V.p - F[FP][a]);
+      F[FU][a] += k * (V.u - F[FU][a]);
+      F[FV][a] += k * (V.v - F[FV][a]);
+      F[FW][a] += k * (-F[FW][a]);
+    }
+    return r;
+  });
 }
 
 // one workgroup per disk of a batch; a planet that moves takes only the roll here, its time,
@@ -907,15 +934,25 @@ hipError_t launch_sum_partials(const LaunchCtx& c, int nb, int stride, double* o
   return hipGetLastError();
 }
 
-hipError_t launch_planet_after_sweep(const LaunchCtx& c, int src, const DevF32* f32) {
-  k_planet_drift<<<1, 64, 0, c.stream>>>(c.p, c.ss);
-  if (c.p.plnt == 2) {
-    hipError_t e = f32 ? f32_reduce(c, *f32, src, 8, 0.0, 1) : launch_reduce(c, src, 8, 0.0, 1);
+hipError_t launch_planet_after_sweep(const LaunchCtx& c, int src, const DevF32* f32, bool roll) {
+  roll = roll && c.p.fargo > 0;
+  // a disk of many rings rolls them over the whole grid, first
+  if (roll && split_rings(c.g)) {
+    hipError_t e = launch_rotate(c);
     if (e != hipSuccess) return e;
-    e = f32 ? f32_reduce(c, *f32, src, 9, 0.0, 2) : launch_reduce(c, src, 9, 0.0, 2);
-    if (e != hipSuccess) return e;
+    roll = false;
   }
-  k_planet_forces_kick<<<1, 64, 0, c.stream>>>(c.p, c.ss, 1);
+  int nb = 0;
+  hipError_t e = hipSuccess;
+  if (c.p.ndim == 2) {
+    nb = torque_blocks(c.g);
+    if (f32) e = f32_planet_torque(c, *f32, src, roll, nb);
+    else k_planet_torque<<<nb, 256, 0, c.stream>>>(c.g, c.p, c.ss, src, roll, c.partials);
+  } else if (c.p.kill) {
+    e = f32 ? f32_damp(c, *f32, src) : launch_damp(c, src);
+  }
+  if (e != hipSuccess) return e;
+  k_planet_finish<<<1, kStepThreads, 0, c.stream>>>(c.g, c.p, c.ss, c.partials, nb, roll);
   return hipGetLastError();
 }
 

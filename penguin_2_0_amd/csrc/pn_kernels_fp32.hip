@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "pn_f32.hpp"
+#include "pn_torque.hpp"
 #include "ppm_wave_f32.hpp"
 
 namespace pn {
@@ -737,21 +738,10 @@ __global__ void k_fill_ghosts_f32(DevGrid g, DevF32 f, DevParams prm, int src) {
   if ((g.ndim == 3 && code != 4) || prm.eos == 3) f.f[src][3][ag] = f.f[src][3][as];
 }
 
-__global__ void k_damp_f32(DevGrid g, DevF32 f, DevParams prm, const StepScalars* __restrict__ ss, int src) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= g.jmax) return;
-  const int n = blockIdx.y;   // ring i + imax k
-  const int s = slot_of(g, n % g.imax, n / g.imax);
-  const double d_kill = 0.5 * prm.sc_h;
-  const double inner = prm.xmin + d_kill, outer = prm.xmax - d_kill;
-  const double r = g.xc[s];
-  double k;
-  if (r < inner) k = (inner - r) / d_kill;
-  else if (r > outer) k = (r - outer) / d_kill;
-  else return;
-  k *= ss->dt * pow(r, -1.5);
+// damping of cell a of ring n by the fraction k
+__device__ __forceinline__ void damp_cell(const DevGrid& g, const DevF32& f, const DevParams& prm, int src, int n,
+                                          long a, double k) {
   const pn_symdisk V = g.val[n];
-  const long a = (long)s * g.jmax + j;
   float* const F0 = f.f[src][0];
   float* const F1 = f.f[src][1];
   float* const F2 = f.f[src][2];
@@ -770,6 +760,31 @@ __global__ void k_damp_f32(DevGrid g, DevF32 f, DevParams prm, const StepScalars
       F3[a] = (float)(p1 / rho1 - qb);
     }
   }
+}
+
+__global__ void k_damp_f32(DevGrid g, DevF32 f, DevParams prm, const StepScalars* __restrict__ ss, int src) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= g.jmax) return;
+  const int n = blockIdx.y;   // ring i + imax k
+  const int s = slot_of(g, n % g.imax, n / g.imax);
+  const double d_kill = 0.5 * prm.sc_h;
+  const double inner = prm.xmin + d_kill, outer = prm.xmax - d_kill;
+  const double r = g.xc[s];
+  double k;
+  if (r < inner) k = (inner - r) / d_kill;
+  else if (r > outer) k = (r - outer) / d_kill;
+  else return;
+  damp_cell(g, f, prm, src, n, (long)s * g.jmax + j, k * (ss->dt * pow(r, -1.5)));
+}
+
+// the disk's pull on a moving planet from the FP32 state, in FP64 with the background added back
+__global__ __launch_bounds__(256) void k_planet_torque_f32(DevGrid g, DevF32 f, DevParams prm,
+                                                           const StepScalars* __restrict__ ss, int src, int roll,
+                                                           double* partials) {
+  planet_torque(g, prm, ss, roll, partials, [&](int s, int n, long a, double k) {
+    if (k != 0.0) damp_cell(g, f, prm, src, n, a, k);
+    return f.rbg[s] + (double)f.f[src][0][a];
+  });
 }
 
 __global__ __launch_bounds__(256) void k_totals_f32(DevGrid g, DevF32 f, int src, double* partials) {
@@ -1108,6 +1123,12 @@ hipError_t f32_reduce(const LaunchCtx& c, const DevF32& f, int src, int mode, do
   const int nb = red_blocks(c.g);
   k_reduce_f32<<<nb, 256, 0, c.stream>>>(c.g, f, c.p, c.ss, src, mode, exclude, c.partials);
   return launch_sum_partials(c, nb, 1, &c.ss->red[slot]);
+}
+
+hipError_t f32_planet_torque(const LaunchCtx& c, const DevF32& f, int src, bool roll, int nb) {
+  if (2 * nb > kMaxPartials) return hipErrorInvalidValue;
+  k_planet_torque_f32<<<nb, 256, 0, c.stream>>>(c.g, f, c.p, c.ss, src, roll, c.partials);
+  return hipGetLastError();
 }
 
 hipError_t f32_damp(const LaunchCtx& c, const DevF32& f, int src) {

@@ -54,10 +54,11 @@ hipError_t launch_reduce(const LaunchCtx& c, int src, int mode, double exclude, 
 hipError_t launch_totals(const LaunchCtx& c, int src, double* out2);  // out2: device, mass and angmom
 // azimuthal mean of FP64 field `field` of every interior ring (out: device, imax kmax doubles)
 hipError_t launch_ring_means(const LaunchCtx& c, int src, int field, double* out);
-// simtime, drift, the disk's forces on the planet (modes 8 / 9; from the FP32 state when f32 is
-// given), closing half kick
+// the end of a step whose planet feels the disk: damping zones, the disk's forces on the planet
+// (modes 8 / 9; from the FP32 state when f32 is given), the integer roll if it is still to come
+// (roll), simtime, drift, closing half kick
 struct DevF32;
-hipError_t launch_planet_after_sweep(const LaunchCtx& c, int src, const DevF32* f32 = nullptr);
+hipError_t launch_planet_after_sweep(const LaunchCtx& c, int src, const DevF32* f32, bool roll);
 hipError_t launch_dt_finalize(const LaunchCtx& c, int n);           // dt = min(1.1 dt, courant / max of n cflp)
 hipError_t launch_sum_partials(const LaunchCtx& c, int nb, int stride, double* out);
 // radial ghost rings of buffer src from the interior under the boundary codes (FP64 state;

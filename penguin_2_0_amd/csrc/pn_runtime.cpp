@@ -207,15 +207,15 @@ int launch_step(pn_ctx* c, int& cur, bool first, bool last) {
   float* tabz = is_f32(c) ? c->df.tabz : nullptr;
   if (!fused || first) PN_LAUNCH(c, "pre step", launch_pre_step(L, ncfl, trig, tab, tabz, c->df.tstride));
   const bool post = c->P.plnt_flag < 2;
-  if ((rc = launch_sweeps(c, cur, fused ? 1 : 0, false, !post)) != PN_OK) return rc;
+  if ((rc = launch_sweeps(c, cur, fused ? 1 : 0, false, false)) != PN_OK) return rc;
   if (fused && !last) {
     PN_LAUNCH(c, "mid step", launch_mid_step(L, fused_partials(c), trig, tab, tabz, c->df.tstride));
     return PN_OK;
   }
   // damping zones: ring-uniform relaxation, which commutes with the integer roll
-  if (c->P.kill_flag) PN_LAUNCH(c, "damp", is_f32(c) ? f32_damp(L, c->df, cur) : launch_damp(L, cur));
+  if (c->P.kill_flag && post) PN_LAUNCH(c, "damp", is_f32(c) ? f32_damp(L, c->df, cur) : launch_damp(L, cur));
   if (post) PN_LAUNCH(c, "post step", launch_post_step(L, fused ? fused_partials(c) : 0));
-  else PN_LAUNCH(c, "planet update", launch_planet_after_sweep(L, cur, is_f32(c) ? &c->df : nullptr));
+  else PN_LAUNCH(c, "planet update", launch_planet_after_sweep(L, cur, is_f32(c) ? &c->df : nullptr, true));
   return PN_OK;
 }
 
@@ -575,6 +575,9 @@ int pn_create(const pn_grid* g, const pn_params* p, int precision, pn_ctx** out)
   for (double** t : col_tabs)
     if (r2 == PN_OK) r2 = dalloc(c, t, g->jmax);
   if (r2 == PN_OK) r2 = dalloc(c, &val, static_cast<size_t>(g->imax) * g->kmax);
+  double2* rpow = nullptr;
+  if (r2 == PN_OK && p->ndim == 2 && p->plnt_flag == 2) r2 = dalloc(c, &rpow, nslot);
+  d.rpow = rpow;
   if (r2 == PN_OK) r2 = dalloc(c, &c->ss, 1);
   if (r2 == PN_OK) r2 = dalloc(c, &c->partials, kMaxPartials);
   if (r2 == PN_OK) r2 = dalloc(c, &c->out2, 2);
@@ -1084,6 +1087,11 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
   PN_HIP(c, up(d.yc, c->h_yc.data(), J * sizeof(double)));
   PN_HIP(c, up(d.yvol, c->h_yvol.data(), J * sizeof(double)));
   PN_HIP(c, up(d.val, val, nring * sizeof(pn_symdisk)));
+  std::vector<double2> rpow;
+  if (d.rpow) {
+    for (long s = 0; s < nslot; ++s) rpow.push_back(make_double2(std::pow(sxc[s], -c->P.p_alpha), std::pow(sxc[s], -1.5)));
+    PN_HIP(c, up(d.rpow, rpow.data(), nslot * sizeof(double2)));
+  }
   rc = sync(c);
   if (rc != PN_OK) return rc;
   if (d.tabz) PN_LAUNCH(c, "theta table", fp64_tab_theta(lctx(c)));
