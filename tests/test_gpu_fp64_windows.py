@@ -104,3 +104,14 @@ def test_coarse_rings_and_large_jumps():
     p = configs.disk2d(20, 24, q=1.0e-3)
     got, ref = run_pair(abi.PnGrid(20, 24, 1), p, 5, noise=0.5)
     close(got, ref, "ruv", 1.0e-11, 1.0e-8, "jumps")
+
+
+# jumps within the interface's series (1/8), on both sides of it in one wavefront, and far past it;
+# bars of test_gpu_parity_flags.py's 10 steps of these closures
+@pytest.mark.parametrize("eos", [2, 3])
+@pytest.mark.parametrize("noise", [0.02, 0.15, 0.5])
+def test_gamma_law_jumps(eos, noise):
+    print("case: gamma-law jumps, eos", eos, "noise", noise, flush=True)
+    p = configs.disk2d(50, 90, q=1.0e-3, eos=eos, gam=1.4, init_p_iso=1)
+    got, ref = run_pair(abi.PnGrid(50, 90, 1), p, 5, noise=noise)
+    close(got, ref, "rpuv", 1.0e-10, 1.0e-8, f"eos {eos}")
