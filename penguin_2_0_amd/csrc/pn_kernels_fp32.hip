@@ -40,12 +40,6 @@ __device__ __forceinline__ int xcd_swizzle(int bid, int nblk) {
   return x * q + (x < rem ? x : rem) + idx;
 }
 
-__device__ __forceinline__ int wrapj(int j, int jmax) {
-  if (j < 0) j += jmax;
-  if (j >= jmax) j -= jmax;
-  return j;
-}
-
 template <int K>
 __device__ __forceinline__ int win_len_k(int len, int nwin, int l) {
   constexpr int WIN = 64 * K, REAL = WIN - 2 * kNpad;
@@ -142,7 +136,8 @@ template <int K, int W, int Q, int NF>
 struct XTile {
   static constexpr int WIN = 64 * K, NC = W * Q, LD = WIN + 2;
   float tile[NF][NC][LD];   // [field][column][cell]; LD even keeps K-float reads aligned
-  int srot[WIN];            // rot_j of the window's slots
+  int2 row[WIN];            // of the window's slots: rot_j, and the byte offset of lab column 0's datum
+                            // were it not wrapped, 4 (slot jmax - rot_j)
   float red[W];
 };
 
@@ -179,8 +174,11 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
   const int step = TH ? g.sr : 1;   // slots between neighbouring cells of the pencil
   const int qs = threadIdx.x % NC, cs = threadIdx.x / NC;
   const int jl = jb + qs;
-  __syncthreads();   // the previous item's stores have read srot and the tile
-  for (int c = threadIdx.x; c < WIN; c += 64 * W) T.srot[c] = g.rot_j[s0 + step * (c < lim ? c : lim - 1)];
+  __syncthreads();   // the previous item's stores have read row and the tile
+  for (int c = threadIdx.x; c < WIN; c += 64 * W) {
+    const int s = s0 + step * (c < lim ? c : lim - 1), rot = g.rot_j[s];
+    T.row[c] = make_int2(rot, 4 * (s * jmax - rot));
+  }
   __syncthreads();
   // the fields as buffer views with 32-bit byte offsets (a state buffer is below 2 GiB)
   const unsigned fbytes = 4u * (unsigned)(g.sr * g.sk) * (unsigned)jmax;
@@ -200,8 +198,9 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
 #pragma unroll
     for (int it = 0; it < CH; ++it) {
       const int c = cs + CSTEP * (i0 + it);
-      const unsigned o =
-          4u * (unsigned)((s0 + step * (c < lim ? c : lim - 1)) * jmax + wrapj(jlc - T.srot[c], jmax));
+      // rot_j in [0, jmax): one wrap at most
+      const int2 row = T.row[c];
+      const unsigned o = (unsigned)row.y + 4u * (unsigned)jlc + (jlc < row.x ? 4u * (unsigned)jmax : 0u);
 #pragma unroll
       for (int fi = 0; fi < NF; ++fi) v[it][fi] = fin[fi].f(o);
     }
@@ -360,13 +359,14 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
   for (int it = 0; it < NIT; ++it) {
     const int q = qs, c = cs + CSTEP * it;
     if (jl < jmax && c >= kNpad && c < lim - kNpad) {
-      const int sl = s0 + step * c;
-      const int j = wrapj(jl - T.srot[c], jmax);
-      const unsigned o = 4u * (unsigned)(sl * jmax + j);
+      const int2 row = T.row[c];
+      const bool wrap = jl < row.x;
+      const unsigned o = (unsigned)row.y + 4u * (unsigned)jl + (wrap ? 4u * (unsigned)jmax : 0u);
 #pragma unroll
       for (int fi = 0; fi < NF; ++fi) fout[fi].put(tile[fi][q][c], o);
       if (TH && cfl) {
         // the next step's CFL term of this cell (timestep.cu:12-108), isothermal c_s
+        const int sl = s0 + step * c, j = jl - row.x + (wrap ? jmax : 0);
         const float* T = f.tab + sl;
         const long ts = f.tstride;
         const float csnd = sqrt_gam * T[kTabCs * ts];
