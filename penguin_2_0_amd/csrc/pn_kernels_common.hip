@@ -403,7 +403,10 @@ __device__ double block_max_partials(const double* __restrict__ cflp, int n, dou
   m = wave_max(m);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x < 64) m = wave_max(threadIdx.x < (int)(blockDim.x >> 6) ? sh[threadIdx.x] : 0.0);
+  if (threadIdx.x < 64) {
+    m = threadIdx.x < (blockDim.x >> 6) ? sh[threadIdx.x] : 0.0;
+    for (int off = 8; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));   // at most 16 waves
+  }
   return m;
 }
 
@@ -442,17 +445,21 @@ __global__ void k_index_shift(DevGrid g, DevParams prm, const StepScalars* __res
 }
 
 // the per-step rotation rows of the FP32 table for slot s (ghost slots keep res_v = 0):
-// sin / cos of dt (res_v / r_cyl - v_y) / 4 with the planet velocity the sweeps will read
+// sin / cos of dt (res_v / r_cyl - v_y) / 4 with the planet velocity the sweeps will read.  By the
+// short series, four library calls in a row were a seventh of the step kernel (128 x 384: k_mid_step
+// 6.2 -> 5.4 us).
 // (3-D: also into the theta-major copy tabz, where slot (ir, kz) sits at kz + sk ir)
 __device__ __forceinline__ void rot_rows_slot(const DevGrid& g, double vy, float* tab, float* tabz, int tstride,
                                               double dt, int s) {
   const double h = 0.25 * dt * (g.res_v[s] / g.radc[s] - vy);
-  const float sh = (float)sin(h), ch = (float)cos(h);
+  double sn, cs;
+  sincos_small(h, sn, cs);
+  const float sh = (float)sn, ch = (float)cs;
   tab[(long)kTabRotS * tstride + s] = sh;
   tab[(long)kTabRotC * tstride + s] = ch;
-  const double hp = h - 0.25 * g.dy[0];
-  tab[(long)kTabRotPhS * tstride + s] = (float)sin(hp);
-  tab[(long)kTabRotPhC * tstride + s] = (float)cos(hp);
+  sincos_small(h - 0.25 * g.dy[0], sn, cs);
+  tab[(long)kTabRotPhS * tstride + s] = (float)sn;
+  tab[(long)kTabRotPhC * tstride + s] = (float)cs;
   if (tabz) {
     const long sz = s / g.sr + (long)g.sk * (s % g.sr);
     tabz[(long)kTabRotS * tstride + sz] = sh;
@@ -471,7 +478,7 @@ __device__ __forceinline__ void turn_rows_slot(const DevGrid& g, double vy, doub
     return;
   }
   double sn, cs;
-  sincos(0.5 * dt * (vrot - vy), &sn, &cs);
+  sincos_small(0.5 * dt * (vrot - vy), sn, cs);
   g.tab[kT64RotC * g.tstride + s] = cs;
   g.tab[kT64RotS * g.tstride + s] = sn;
 }
@@ -536,8 +543,9 @@ __device__ __forceinline__ void pre_step_body(DevGrid g, const DevParams& prm, S
     const double py = s_py;
     for (int j = threadIdx.x; j < g.jmax; j += blockDim.x) {
       if (trig) {
-        const double a = 0.5 * (g.yc[j] - py);
-        trig[j] = make_float2((float)sin(a), (float)cos(a));
+        double sn, cs;
+        sincos(0.5 * (g.yc[j] - py), &sn, &cs);
+        trig[j] = make_float2((float)sn, (float)cs);
       } else {
         double sn, cs;
         sincos(g.yc[j] - py, &sn, &cs);
