@@ -496,20 +496,6 @@ __device__ __forceinline__ Parab<double, K> parabola(const C<double, K>& flat, c
   return o;
 }
 
-// derivs (viscosity.cu:2-19): first and second derivative of a quadratic through the
-// left-edge coordinates of cells c-1, c, c+1
-template <typename T>
-__device__ __forceinline__ void derivs(T xm, T x0, T xp, T um, T u0, T up, T& first, T& second) {
-  T x2 = x0 - xm;
-  T x3 = xp - xm;
-  T h2 = (u0 - um) / x2;
-  T h3 = (up - um) / x3;
-  T A = (h3 - h2) / (x3 - x2);
-  T B = (x3 * h2 - x2 * h3) / (x3 - x2);
-  second = T(2.0) * A;
-  first = second * x2 + B;
-}
-
 // Window state and per-cell geometry.
 template <int K>
 struct Win {
