@@ -54,8 +54,6 @@ enum TabEntry {
   kTabRotPhS, kTabRotPhC,
   // EOS 3 (2-D): q_b = p_b / rho_b and q_b(s+1) - q_b(s)
   kTabQb, kTabDqb,
-  // reciprocals: of rho_b, p_b, the radial width and volume, the theta width and volume
-  kTabIrb, kTabIpb, kTabIdx0, kTabIdvol0, kTabIdz0, kTabIdvolZ,
   kTabEntries
 };
 constexpr int kTabOverhang = 256;   // >= the longest radial window
@@ -71,8 +69,7 @@ struct DevF32 {
   // are consecutive); stride tstride; its per-step rows are rewritten beside the others
   float* tabz;
   const double *rbg, *vbg;     // Sigma_b and v_bg per slot, FP64
-  const float* dy;             // per column
-  const float4* col;           // per column: dphi, its volume factor, and their reciprocals
+  const float *dy, *yvol;      // per column
   float2* trig;                // per column, per step: sin / cos of half the angle to the planet
   int nwin_x, nwin_y, nwin_z;  // windows of the variant in use
   int uniform_phi;             // every dphi equal: the azimuthal paraset is (1/2, -1/6, 1/6, 1/2, 1/2)

@@ -445,19 +445,17 @@ __global__ void k_index_shift(DevGrid g, DevParams prm, const StepScalars* __res
 }
 
 // the per-step rotation rows of the FP32 table for slot s (ghost slots keep res_v = 0):
-// sin / cos of dt (res_v / r_cyl - v_y) / 4 with the planet velocity the sweeps will read.  By the
-// short series, four library calls in a row were a seventh of the step kernel (128 x 384: k_mid_step
-// 6.2 -> 5.4 us).
+// sin / cos of dt (res_v / r_cyl - v_y) / 4 with the planet velocity the sweeps will read
 // (3-D: also into the theta-major copy tabz, where slot (ir, kz) sits at kz + sk ir)
 __device__ __forceinline__ void rot_rows_slot(const DevGrid& g, double vy, float* tab, float* tabz, int tstride,
                                               double dt, int s) {
   const double h = 0.25 * dt * (g.res_v[s] / g.radc[s] - vy);
   double sn, cs;
-  sincos_small(h, sn, cs);
+  sincos(h, &sn, &cs);
   const float sh = (float)sn, ch = (float)cs;
   tab[(long)kTabRotS * tstride + s] = sh;
   tab[(long)kTabRotC * tstride + s] = ch;
-  sincos_small(h - 0.25 * g.dy[0], sn, cs);
+  sincos(h - 0.25 * g.dy[0], &sn, &cs);
   tab[(long)kTabRotPhS * tstride + s] = (float)sn;
   tab[(long)kTabRotPhC * tstride + s] = (float)cs;
   if (tabz) {

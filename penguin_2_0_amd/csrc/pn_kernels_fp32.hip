@@ -21,14 +21,14 @@ namespace pn {
 // Occupancy.  A SIMD's 512 VGPRs per lane hold eight waves of at most 64 VGPRs, six of 80,
 // five of 96 and four of 128; amdgpu_waves_per_eu asks the allocator to fit a count, spilling
 // what does not fit to scratch.
-// - LDS-staged pencils: the allocator left alone settles them at 99-136 (three or four waves).
-//   A workgroup of four waves puts one on each SIMD, so a fifth wave per SIMD is a fifth
+// - LDS-staged pencils: the allocator left alone settles them at 104-117 (four waves).  A
+//   workgroup of four waves puts one on each SIMD, so a fifth wave per SIMD is a fifth
 //   workgroup per CU, which the LDS must hold too; the kernels ask for as many as that allows
-//   (pencil_waves).  A 2-D isothermal pencil fits 96 without a spill.
-// - Azimuthal windows of 128 cells: eight waves (64 VGPRs, three spills) for a 2-D isothermal
-//   disk, six (80) in the batch; of 256 cells: four waves (128).  The EOS 3 forms spill tens of
-//   values at the next step down, so they keep what the allocator gives (a minimum of one wave
-//   asks for nothing).
+//   (pencil_waves), for five to seventeen spilled registers a pencil.
+// - Azimuthal windows of 128 cells: eight waves (64 VGPRs, five spills) for a 2-D isothermal
+//   disk, six (80, two spills) in the batch; of 256 cells: four waves (128).  The EOS 3 forms
+//   spill tens of values at the next step down, so they keep what the allocator gives (a minimum
+//   of one wave asks for nothing).
 #define PN_WAVES(n) __attribute__((amdgpu_waves_per_eu(n, 8)))
 
 namespace {
@@ -149,6 +149,15 @@ constexpr int pencil_waves() {
   constexpr size_t lds = sizeof(XTile<K, W, Q, NF>);
   if (K == 3 || W != 4) return 1;
   return 5 * lds <= 160 * 1024 ? 5 : 4 * lds <= 160 * 1024 ? 4 : 1;
+}
+
+// An angular momentum back to a velocity as an increment: v + (l - r v) / r with r v formed as on
+// the way in, so a cell whose l did not change keeps v exactly (the product (r v) (1/r) would scale
+// it by the table's fixed r (1/r) - 1 every step).  That holds for a lane's first cell; the
+// others take r v exact in an FMA, as they did when the compiler chose (rot_fixed has the reason).
+__device__ __forceinline__ float velocity_of(int h, float l, float r, float v, float ir) {
+  if (h > 0) return v + __builtin_fmaf(-r, v, l) * ir;
+  return v + (l - rounded(r * v)) * ir;
 }
 
 // one work item: window l of the pencils of row `row` (radial: theta row k; theta: ring i),
@@ -304,7 +313,7 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
     }
     Para<float, K> P0;
     if constexpr (TH) {
-      P0 = f.uniform_theta ? paraset_uniform<K>() : paraset_f32<K>(Wp.dx0);
+      P0 = f.uniform_theta ? paraset_uniform<K>() : paraset<float, K>(c0, 0, lim, Wp.dx0);
     } else {
       P0.c0 = tx.get(kTabP0);
       P0.c1 = tx.get(kTabP1);
@@ -312,7 +321,7 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
       P0.c3 = tx.get(kTabP3);
       P0.c4 = tx.get(kTabP4);
     }
-    ppmlr_pert<K, G, (G == kGeoRcyl ? 2 : 3), TabLane<K>, ADIA, BARY>(Wp, tx, P0, c0, lim, dt, 0.0f, pl, prm.plnt > 0,
+    ppmlr_pert<K, G, (G == kGeoRcyl ? 2 : 3), TabLane<K>, ADIA, BARY, VISC == 0>(Wp, tx, P0, c0, lim, dt, 0.0f, pl, prm.plnt > 0,
                                                                      prm.flat != 0, sqrt_gam, 0.0f, false,
                                                                      (float)prm.gam);
     if (VISC == 1 || (VISC == 2 && prm.visc)) {
@@ -323,9 +332,6 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
     const C<float, K> irc = tx.get(kTabIrc);
     C<float, K> ixc;
     if constexpr (G == kGeoRsph) ixc = tx.get(kTabIxc);
-    // angular momenta back to velocities as increments: v_new = v + (l_new - r v) / r with
-    // r v formed as on the way in, so a cell whose l did not change keeps v exactly (the
-    // product (r v) (1/r) would scale it by the table's fixed r (1/r) - 1 every step)
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       const int c = c0 + h;
@@ -335,14 +341,14 @@ __device__ __forceinline__ float pencil_item(const DevGrid& g, const DevF32& f, 
           tile[3][q][c] = Wp.u[h];
           tile[1][q][c] = Wp.v[h];
           const float v0 = tile[2][q][c];
-          tile[2][q][c] = v0 + (Wp.w[h] - rc[h] * v0) * irc[h];
+          tile[2][q][c] = velocity_of(h, Wp.w[h], rc[h], v0, irc[h]);
         } else {
           tile[1][q][c] = Wp.u[h];
           const float v0 = tile[2][q][c];
-          tile[2][q][c] = v0 + (Wp.v[h] - rc[h] * v0) * irc[h];
+          tile[2][q][c] = velocity_of(h, Wp.v[h], rc[h], v0, irc[h]);
           if constexpr (G == kGeoRsph) {
             const float w0 = tile[3][q][c];
-            tile[3][q][c] = w0 + (Wp.w[h] - Wp.rad[h] * w0) * ixc[h];
+            tile[3][q][c] = velocity_of(h, Wp.w[h], Wp.rad[h], w0, ixc[h]);
           }
           if constexpr (ADIA) tile[3][q][c] = Wp.q[h];
         }
@@ -434,7 +440,8 @@ __device__ __forceinline__ int disk_of(const int* __restrict__ base, int ndisk, 
 // of 8), each mapped through the XCD permutation so that one XCD walks a contiguous run of
 // items (neighbouring column groups share L2 lines).  base: ndisk + 1 item offsets.
 // The batch's radial kernel keeps its item's disk lookup in scalar registers besides the pencil's
-// state; five waves per SIMD (96 registers) ran 84 us on twelve disks against 90 at four.
+// state: five waves per SIMD (96 registers, nine spills) run a step of 48 disks in 684 us against 697
+// at four, of twelve in 195 against 201.
 
 // order: nslots (disk, item) pairs, the item of slot t for the workgroup that takes it
 // (slot t runs on XCD t % 8; the host lays each XCD's share out by decreasing cost, disk -1
@@ -493,7 +500,7 @@ __device__ __forceinline__ float y_pencil(const DevGrid& g, const DevF32& f, con
   const long base = (long)s * jmax;
   const unsigned rb4 = 4u * (unsigned)jmax;
   const Buf bfr(f.f[src][0] + base, rb4), bfu(f.f[src][1] + base, rb4), bfv(f.f[src][2] + base, rb4);
-  const Buf btrig(f.trig, 2u * rb4), bdy(f.dy, rb4), bcol(f.col, 4u * rb4);
+  const Buf btrig(f.trig, 2u * rb4), bdy(f.dy, rb4), byv(f.yvol, rb4);
 
   WinP<K> W;
   unsigned jd[K];   // byte offset of the cell's data column
@@ -512,11 +519,8 @@ __device__ __forceinline__ float y_pencil(const DevGrid& g, const DevF32& f, con
     const float2 tr = btrig.f2(2u * o0);
     W.ts[h] = tr.x;
     W.tc[h] = tr.y;
-    const float4 col = bcol.f4(4u * o0);
-    W.dx0[h] = col.x;
-    W.dvol0[h] = col.y * rc;
-    W.idx0[h] = col.z;
-    W.iyv[h] = col.w;
+    W.dx0[h] = bdy.f(o0);
+    W.dvol0[h] = byv.f(o0) * rc;
     W.xa0[h] = 0.0f;
     W.rad[h] = rc;
     W.vrot[h] = vrot;
@@ -542,7 +546,7 @@ __device__ __forceinline__ float y_pencil(const DevGrid& g, const DevF32& f, con
     if constexpr (ADIA) W.q[h] = Buf(f.f[src][3] + base, rb4).f(o);
   }
   const float sqrt_gam = sqrtf((float)prm.gam);
-  const Para<float, K> P0 = f.uniform_phi ? paraset_uniform<K>() : paraset_f32<K>(W.dx0);
+  const Para<float, K> P0 = f.uniform_phi ? paraset_uniform<K>() : paraset<float, K>(K * lane, 0, lim, W.dx0);
   ppmlr_pert<K, kGeoPhi, NDIM, TabLane<K>, ADIA, BARY>(W, TabLane<K>{}, P0, K * lane, lim, dt, wres, pl, prm.plnt > 0,
                                                            prm.flat != 0, sqrt_gam, rsph, f.uniform_phi != 0,
                                                            (float)prm.gam);

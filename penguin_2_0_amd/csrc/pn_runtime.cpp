@@ -603,8 +603,7 @@ int pn_create(const pn_grid* g, const pn_params* p, int precision, pn_ctx** out)
     }
   }
   if (precision == PN_FP32) {
-    float* fdy;
-    float4* fcol;
+    float *fdy, *fyvol;
     double *rbg, *vbg;
     c->df.tstride = static_cast<int>((nslot + kTabOverhang + 3) / 4 * 4);
     if (r2 == PN_OK) r2 = dalloc(c, &c->df.tab, static_cast<size_t>(kTabEntries) * c->df.tstride);
@@ -612,13 +611,13 @@ int pn_create(const pn_grid* g, const pn_params* p, int precision, pn_ctx** out)
     if (r2 == PN_OK) r2 = dalloc(c, &rbg, nslot);
     if (r2 == PN_OK) r2 = dalloc(c, &vbg, nslot);
     if (r2 == PN_OK) r2 = dalloc(c, &fdy, g->jmax);
-    if (r2 == PN_OK) r2 = dalloc(c, &fcol, g->jmax);
+    if (r2 == PN_OK) r2 = dalloc(c, &fyvol, g->jmax);
     if (r2 == PN_OK) r2 = dalloc(c, &c->df.trig, g->jmax);
     if (r2 == PN_OK) {
       c->df.rbg = rbg;
       c->df.vbg = vbg;
       c->df.dy = fdy;
-      c->df.col = fcol;
+      c->df.yvol = fyvol;
     }
   }
   if (r2 != PN_OK) {
@@ -923,10 +922,6 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
       q[kTabRotPhS] = std::sin(-0.25 * c->h_dy[0]);
       q[kTabRotPhC] = std::cos(-0.25 * c->h_dy[0]);
       q[kTabDvol0] = sxvol[s];
-      q[kTabIrb] = 1.0 / rbg[s];
-      q[kTabIpb] = 1.0 / pb[s];
-      q[kTabIdx0] = 1.0 / w0;
-      q[kTabIdvol0] = 1.0 / sxvol[s];
       q[kTabQb] = qbg[s];
       q[kTabDqb] = hn ? qbg[s + 1] - qbg[s] : 0.0;
       q[kTabRc] = sradc[s];
@@ -985,8 +980,6 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
         q[kTabZa0] = za;
         q[kTabDz0] = sdz[s];
         q[kTabDvolZ] = dvz;
-        q[kTabIdz0] = 1.0 / sdz[s];
-        q[kTabIdvolZ] = 1.0 / dvz;
         q[kTabSzl] = sa;
         q[kTabCzl] = ca;
         q[kTabSzr] = sb;
@@ -1028,12 +1021,10 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
           for (long o = nslot; o < ts; ++o) tab[e * ts + o] = static_cast<float>(q[e]);
       }
     }
-    std::vector<float> t_dy(J);
-    std::vector<float4> t_col(J);
+    std::vector<float> t_dy(J), t_yvol(J);
     for (int j = 0; j < J; ++j) {
       t_dy[j] = static_cast<float>(c->h_dy[j]);
-      t_col[j] = make_float4(t_dy[j], static_cast<float>(c->h_yvol[j]), static_cast<float>(1.0 / c->h_dy[j]),
-                             static_cast<float>(1.0 / c->h_yvol[j]));
+      t_yvol[j] = static_cast<float>(c->h_yvol[j]);
     }
     PN_HIP(c, hipMemcpyAsync(c->df.tab, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice, st));
     std::vector<float> tabz;
@@ -1047,7 +1038,7 @@ int pn_load_rings(pn_ctx* c, const void* rings, size_t rings_bytes, const void* 
       PN_HIP(c, hipMemcpyAsync(c->df.tabz, tabz.data(), tabz.size() * sizeof(float), hipMemcpyHostToDevice, st));
     }
     PN_HIP(c, hipMemcpyAsync(const_cast<float*>(c->df.dy), t_dy.data(), J * sizeof(float), hipMemcpyHostToDevice, st));
-    PN_HIP(c, hipMemcpyAsync(const_cast<float4*>(c->df.col), t_col.data(), J * sizeof(float4), hipMemcpyHostToDevice, st));
+    PN_HIP(c, hipMemcpyAsync(const_cast<float*>(c->df.yvol), t_yvol.data(), J * sizeof(float), hipMemcpyHostToDevice, st));
     PN_HIP(c, hipMemcpyAsync(const_cast<double*>(c->df.rbg), c->h_rbg.data(), nslot * sizeof(double), hipMemcpyHostToDevice, st));
     PN_HIP(c, hipMemcpyAsync(const_cast<double*>(c->df.vbg), bvbg.data(), nslot * sizeof(double), hipMemcpyHostToDevice, st));
     c->df.nwin_x = f32_windows(I, kF32VariantsX[c->var_x][0]);

@@ -101,8 +101,6 @@ __device__ __forceinline__ C<T, K> next2(const C<T, K>& x) {
   }
 }
 
-__device__ __forceinline__ int cell_of(int K, int h) { return K * (int)(threadIdx.x & 63) + h; }
-
 // the limited slope of parabola.cu:87-96: sign(t1) min(|t1|, 2 |da_l|, 2 |da_r|), zero at an
 // extremum: a minimum of magnitudes and the sign by copysign, the values of the reference's
 // compare chain (a minimum and a sign change round nothing, doubling is exact)
@@ -358,9 +356,9 @@ struct Para {
   C<T, K> c0, c1, c2, c3, c4;
 };
 
-// paraset (parabola.cu:138-176) on the index range [nmin, nmaxp)
+// paraset (parabola.cu:138-176) on the index range [nmin, nmaxp); c0 = this lane's first cell
 template <typename T, int K>
-__device__ __forceinline__ Para<T, K> paraset(int nmin, int nmaxp, const C<T, K>& dx) {
+__device__ __forceinline__ Para<T, K> paraset(int c0, int nmin, int nmaxp, const C<T, K>& dx) {
   Para<T, K> P;
   C<T, K> dxp = next1(dx);
   C<T, K> an, ain, bn, bi, cc, ci;
@@ -376,11 +374,11 @@ __device__ __forceinline__ Para<T, K> paraset(int nmin, int nmaxp, const C<T, K>
   C<T, K> anm = prev1(an), anp = next1(an), bnm = prev1(bn), ainm = prev1(ain);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const int c = cell_of(K, h);
-    T c0 = T(0), c1 = T(0), c2 = T(0), c3 = T(0), c4 = T(0);
+    const int c = c0 + h;
+    T k0 = T(0), c1 = T(0), c2 = T(0), c3 = T(0), c4 = T(0);
     if (c >= nmin + 1 && c < nmaxp - 2) {
       T d = T(1.0) / (anm[h] + anp[h]);
-      c0 = dx[h] * ain[h] * (T(1.0) + T(2.0) * d * dxp[h] * (anm[h] * bi[h] - anp[h] * ci[h]));
+      k0 = dx[h] * ain[h] * (T(1.0) + T(2.0) * d * dxp[h] * (anm[h] * bi[h] - anp[h] * ci[h]));
       c1 = -d * dx[h] * anm[h] * bi[h];
       c2 = d * dxp[h] * anp[h] * ci[h];
     }
@@ -389,7 +387,7 @@ __device__ __forceinline__ Para<T, K> paraset(int nmin, int nmaxp, const C<T, K>
       c3 = d * bnm[h] * ain[h];
       c4 = d * cc[h] * ainm[h];
     }
-    P.c0[h] = c0; P.c1[h] = c1; P.c2[h] = c2; P.c3[h] = c3; P.c4[h] = c4;
+    P.c0[h] = k0; P.c1[h] = c1; P.c2[h] = c2; P.c3[h] = c3; P.c4[h] = c4;
   }
   return P;
 }
@@ -575,7 +573,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const
       P0.c3 = splat<T, K>(ring.p0[3]);
       P0.c4 = splat<T, K>(ring.p0[4]);
     } else {
-      P0 = paraset<T, K>(0, nmax, W.dx0);
+      P0 = paraset<T, K>(c0, 0, nmax, W.dx0);
     }
     irad = splat<T, K>(ring.irad);
 #pragma unroll

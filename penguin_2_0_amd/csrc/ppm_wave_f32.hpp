@@ -27,11 +27,13 @@
 //
 // What bounds it: instruction issue.  With its states in registers or LDS a sweep keeps the
 // SIMDs' vector pipes 70 to 90 % busy, and a reciprocal, root or exponential holds one four times as
-// long as a product.  So the limiters are medians, fixed divisors come as table reciprocals,
-// ranges are not masked where a kept cell cannot see the difference, and the library logarithm
-// and the flattening run only in wavefronts that hold a cell in need of them.  1024 x 3072,
-// inviscid: radial sweep 70 -> 58 us, azimuthal 48 -> 39 (1536 x 4608 with EOS 3: 171 -> 146, 139 -> 116;
-// 128 x 384 x 32: 59, 34 and 69 -> 45, 27 and 60).
+// long as a product; the library logarithm and the flattening run only in wavefronts that hold a
+// cell in need of them.  Cheaper arithmetic was tried and taken back: reciprocals of rho_b, p_b, the
+// widths and volumes from the table, limiters as medians and shared viscosity reciprocals ran the
+// sweeps 17 to 20 % faster (1024 x 3072: 61 -> 51 us radial, 41 -> 34 azimuthal), but a table's
+// reciprocal repeats its own rounding step after step: after 1000 steps of that disk L1 of Sigma
+// against FP64 had grown from 4.4e-9 to 4.9e-9 and the drift of the mass from 8.5e-8 of itself off
+// FP64's to 4.1e-7.
 #pragma once
 
 #include "pn_f32.hpp"
@@ -59,10 +61,6 @@ struct Buf {
   __device__ __forceinline__ float2 f2(unsigned off) const {
     const f32x2_t v = __builtin_bit_cast(f32x2_t, (i32x2_t)__builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
     return make_float2(v.x, v.y);
-  }
-  __device__ __forceinline__ float4 f4(unsigned off) const {
-    const f32x4_t v = __builtin_bit_cast(f32x4_t, (i32x4_t)__builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
-    return make_float4(v.x, v.y, v.z, v.w);
   }
   __device__ __forceinline__ void put(float v, unsigned off) const {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)off, 0, 0);
@@ -98,8 +96,8 @@ __device__ __forceinline__ float star_fr_rest(const PlanetF& p, float r, float c
 // sin / cos of (A + e)/2 from sin / cos of A/2 and a small e (|e| < ~0.5)
 __device__ __forceinline__ void rot_half(float s, float c, float e, float& so, float& co) {
   const float h = 0.5f * e, h2 = h * h;
-  const float sh = h + h * h2 * (-1.0f / 6.0f + h2 * (1.0f / 120.0f - h2 * (1.0f / 5040.0f)));
-  const float ch = 1.0f + h2 * (-0.5f + h2 * (1.0f / 24.0f - h2 * (1.0f / 720.0f)));
+  const float sh = h * (1.0f - h2 * (1.0f / 6.0f) * (1.0f - h2 * (1.0f / 20.0f) * (1.0f - h2 * (1.0f / 42.0f))));
+  const float ch = 1.0f - h2 * 0.5f * (1.0f - h2 * (1.0f / 12.0f) * (1.0f - h2 * (1.0f / 30.0f)));
   so = s * ch + c * sh;
   co = c * ch - s * sh;
 }
@@ -110,20 +108,21 @@ __device__ __forceinline__ float planet_fr(const PlanetF& p, float rad, float s,
   const float s2 = s * s;
   const float cosd = 1.0f - 2.0f * s2;
   const float dr = rad - p.x;
-  const float t = 2.0f * p.x * s2;
-  const float ri = __frsqrt_rn((dr * dr + p.rs2) + 2.0f * rad * t);
-  float f = -p.m * ((dr + t) * (ri * ri * ri) + cosd * p.inv_x2);
+  const float R2 = dr * dr + 4.0f * rad * p.x * s2 + p.rs2;
+  const float ri = __frsqrt_rn(R2);
+  float f = -p.m * (dr + 2.0f * p.x * s2) * (ri * ri * ri) - p.m * cosd * p.inv_x2;
   if constexpr (BARY) if (p.bary) f += p.m / (rad * rad) + star_fr_rest(p, rad, cosd);
   return f;
 }
 template <bool BARY = false>
 __device__ __forceinline__ float planet_fphi(const PlanetF& p, float rad, float s, float c) {
-  // the factors of one ring first: they are formed once for all its cells
-  const float s2 = s * s, sc = s * c;
+  const float s2 = s * s;
+  const float sind = 2.0f * s * c;
   const float dr = rad - p.x;
-  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (4.0f * rad * p.x) * s2);
-  float f = sc * ((2.0f * p.m * p.inv_x2) - (2.0f * p.m * p.x) * (ri * ri * ri));
-  if constexpr (BARY) if (p.bary) f += 2.0f * p.stm * p.stx * sc * star_ri3(p, rad, 1.0f - 2.0f * s2);
+  const float R2 = dr * dr + 4.0f * rad * p.x * s2 + p.rs2;
+  const float ri = __frsqrt_rn(R2);
+  float f = -p.m * p.x * sind * (ri * ri * ri) + p.m * sind * p.inv_x2;
+  if constexpr (BARY) if (p.bary) f += p.stm * p.stx * sind * star_ri3(p, rad, 1.0f - 2.0f * s2);
   return f;
 }
 
@@ -138,8 +137,8 @@ __device__ __forceinline__ float planet_fr_sph(const PlanetF& p, float r, float 
   const float cosd = 1.0f - 2.0f * s2;
   const float k = oms + 2.0f * st * s2;
   const float dr = r - p.x;
-  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (2.0f * r * p.x) * k);
-  float f = -p.m * ((dr + p.x * k) * (ri * ri * ri) + st * cosd * p.inv_x2);
+  const float ri = __frsqrt_rn(dr * dr + 2.0f * r * p.x * k + p.rs2);
+  float f = -p.m * (dr + p.x * k) * (ri * ri * ri) - p.m * st * cosd * p.inv_x2;
   if constexpr (BARY) if (p.bary) f += star_fr_rest(p, r, st * cosd);
   return f;
 }
@@ -149,8 +148,8 @@ __device__ __forceinline__ float planet_fphi_sph(const PlanetF& p, float r, floa
   const float sind = 2.0f * s * c;
   const float k = oms + 2.0f * st * s2;
   const float dr = r - p.x;
-  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (2.0f * r * p.x) * k);
-  float f = sind * ((p.m * st * p.inv_x2) - (p.m * p.x) * (ri * ri * ri));
+  const float ri = __frsqrt_rn(dr * dr + 2.0f * r * p.x * k + p.rs2);
+  float f = -p.m * p.x * sind * (ri * ri * ri) + p.m * st * sind * p.inv_x2;
   if constexpr (BARY) if (p.bary) f += p.stm * p.stx * sind * star_ri3(p, r, st * (1.0f - 2.0f * s2));
   return f;
 }
@@ -161,8 +160,8 @@ __device__ __forceinline__ float planet_fth_sph(const PlanetF& p, float r, float
   const float cosd = 1.0f - 2.0f * s2;
   const float k = oms + 2.0f * st * s2;
   const float dr = r - p.x;
-  const float ri = __frsqrt_rn((dr * dr + p.rs2) + (2.0f * r * p.x) * k);
-  float f = p.m * cosd * ct * (p.x * (ri * ri * ri) - p.inv_x2 / st);
+  const float ri = __frsqrt_rn(dr * dr + 2.0f * r * p.x * k + p.rs2);
+  float f = p.m * p.x * cosd * ct * (ri * ri * ri) - p.m * cosd * ct / st * p.inv_x2;
   if constexpr (BARY) if (p.bary) f -= p.stm * p.stx * cosd * ct * star_ri3(p, r, st * cosd);
   return f;
 }
@@ -174,7 +173,7 @@ __device__ __forceinline__ float planet_fth_sph(const PlanetF& p, float r, float
 // value depends on this lane's x alone: a cell's bits are the same in any company.
 __device__ __forceinline__ float log1p_acc(float x, bool wide) {
   const float z = x / (2.0f + x), z2 = z * z;
-  float s = z * (2.0f + z2 * (2.0f / 3.0f + z2 * (2.0f / 5.0f + z2 * (2.0f / 7.0f + z2 * (2.0f / 9.0f)))));
+  float s = 2.0f * z * (1.0f + z2 * (1.0f / 3.0f + z2 * (1.0f / 5.0f + z2 * (1.0f / 7.0f + z2 * (1.0f / 9.0f)))));
   if (wide) s = fabsf(x) < 0.25f ? s : __logf(1.0f + x);
   return s;
 }
@@ -185,39 +184,30 @@ __device__ __forceinline__ float expm1_acc(float y, bool wide) {
   if (wide) s = fabsf(y) < 0.25f ? s : __expf(y) - 1.0f;
   return s;
 }
-// the median of 0, a and b: the smaller in magnitude where the signs agree, else 0
-__device__ __forceinline__ float med0(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 0.0f); }
-__device__ __forceinline__ float max4(float a, float b, float c, float d) {
-  return fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d)));
+// a / b with one correction of the quotient
+__device__ __forceinline__ float quot_f32(float a, float b) {
+  const float y = 1.0f / b, q = a * y;
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+}
+// the limited slope of ppm_wave.hpp with one v_min3 and the sign by copysign
+__device__ __forceinline__ float limited_slope(float t1, float da_l, float da_r) {
+  t1 = copysignf(fminf(fminf(fabsf(t1), 2.0f * fabsf(da_l)), 2.0f * fabsf(da_r)), t1);
+  if (da_l * da_r < 0.0f) t1 = 0.0f;
+  return t1;
 }
 
-// paraset (CW84 eq. 1.6) in every cell: coefficients outside the
-// reference's index ranges (parabola.cu:138-176) reach no parabola that a kept cell reads.
-template <int K>
-__device__ __forceinline__ Para<float, K> paraset_f32(const C<float, K>& dx) {
-  Para<float, K> P;
-  C<float, K> dxp = next1(dx), an, ain, bn, bi, cc, ci;
-#pragma unroll
-  for (int h = 0; h < K; ++h) {
-    an[h] = dx[h] + dxp[h];
-    bn[h] = an[h] + dx[h];
-    cc[h] = an[h] + dxp[h];
-    ain[h] = 1.0f / an[h];
-    bi[h] = 1.0f / bn[h];
-    ci[h] = 1.0f / cc[h];
-  }
-  C<float, K> anm = prev1(an), anp = next1(an), bnm = prev1(bn), ainm = prev1(ain);
-#pragma unroll
-  for (int h = 0; h < K; ++h) {
-    const float d = 1.0f / (anm[h] + anp[h]), e = dx[h] / (anm[h] + dxp[h]);
-    const float wb = d * anm[h] * bi[h], wc = d * anp[h] * ci[h];
-    P.c0[h] = dx[h] * ain[h] * (1.0f + 2.0f * dxp[h] * (wb - wc));
-    P.c1[h] = -dx[h] * wb;
-    P.c2[h] = dxp[h] * wc;
-    P.c3[h] = e * bnm[h] * ain[h];
-    P.c4[h] = e * cc[h] * ainm[h];
-  }
-  return P;
+// first and second derivative at x0 of the quadratic through (xm, um), (x0, u0), (xp, up)
+// (viscosity.cu:2-19)
+__device__ __forceinline__ void derivs(float xm, float x0, float xp, float um, float u0, float up, float& first,
+                                       float& second) {
+  const float x2 = x0 - xm;
+  const float x3 = xp - xm;
+  const float h2 = (u0 - um) / x2;
+  const float h3 = (up - um) / x3;
+  const float A = (h3 - h2) / (x3 - x2);
+  const float B = (x3 * h2 - x2 * h3) / (x3 - x2);
+  second = 2.0f * A;
+  first = second * x2 + B;
 }
 
 // paraset of a uniform grid (CW84 eq. 1.6 with equal widths): constants
@@ -237,56 +227,55 @@ __device__ __forceinline__ Para<float, K> paraset_uniform() {
 // unused).  The edges are carried as offsets from the cell's own value (the right edge
 // c0 da_r + c1 slope(c+1) + c2 slope, the left edge the left neighbour's right edge in this
 // frame), so the flattening, the extremum and overshoot tests, the jump and the curvature
-// never subtract two values of the cell's size.  Both limiters are medians: the slope is the
-// smallest in magnitude of s, 2 dl and 2 dr if their signs agree, else 0 (parabola.cu:26-40);
-// of the edges' offsets r and l, zero if they share a sign (an extremum), the overshoot tests
-// d^2 < -+3 d (r + l), d = r - l, read |l| > 2 |r| and |r| > 2 |l|.  Outputs: al = left edge
-// - x, ar = right edge - x, da = ar - al, s = ar + al = -a6/3, and the jumps dl = X(c) - X(c-1),
-// dr = X(c+1) - X(c) in this cell's frame.  Cells whose stencil leaves the window, or outside
-// the reference's ranges, hold values that no kept cell reads.  flat: 1 - the flattening,
-// applied where shock (wave-uniform) says that the wavefront has any.
+// never subtract two values of the cell's size; the algebra is the reference's.  Outputs:
+// al = left edge - x, (EDGE) ar = right edge - x, da, a6, and the jumps dl = X(c) - X(c-1), dr = X(c+1) - X(c) in this
+// cell's frame.  A cell outside [nmin+2, nmaxp-2) returns the plain parabola's zero edge
+// (al = ar = -x, da = a6 = 0).
 template <int K>
 struct ParabR {
-  C<float, K> al, ar, da, s, dl, dr;
+  C<float, K> al, ar, da, a6, dl, dr;
 };
 
-template <int K, bool BG = true>
-__device__ __forceinline__ ParabR<K> parabola_rel(const C<float, K>& gfl, bool shock, const C<float, K>& val,
-                                                  const C<float, K>& dbg, const Para<float, K>& P) {
-  C<float, K> vp = next1(val);
+template <int K, bool BG = true, bool EDGE = false>
+__device__ __forceinline__ ParabR<K> parabola_rel(int c0, int nmin, int nmaxp, const C<float, K>& flat,
+                                                  const C<float, K>& val, const C<float, K>& dbg,
+                                                  const Para<float, K>& P) {
+  C<float, K> vm = prev1(val), vp = next1(val), dbm;
+  if constexpr (BG) dbm = prev1(dbg);
   ParabR<K> o;
   C<float, K> slope;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     const float a = val[h];
     o.dr[h] = BG ? (vp[h] - a) + dbg[h] : vp[h] - a;
-  }
-  o.dl = prev1(o.dr);   // the same difference, seen from the next cell
-#pragma unroll
-  for (int h = 0; h < K; ++h) {
-    const float s = P.c3[h] * o.dr[h] + P.c4[h] * o.dl[h];
-    slope[h] = med0(med0(s, 2.0f * o.dl[h]), 2.0f * o.dr[h]);
+    o.dl[h] = BG ? (a - vm[h]) + dbm[h] : a - vm[h];
+    slope[h] = limited_slope(P.c3[h] * o.dr[h] + P.c4[h] * o.dl[h], o.dl[h], o.dr[h]);
   }
   C<float, K> slp = next1(slope);
+  C<float, K> ar;   // right edge - x
 #pragma unroll
-  for (int h = 0; h < K; ++h) o.ar[h] = P.c0[h] * o.dr[h] + P.c1[h] * slp[h] + P.c2[h] * slope[h];
-  C<float, K> arm = prev1(o.ar);
-#pragma unroll
-  for (int h = 0; h < K; ++h) o.al[h] = arm[h] - o.dl[h];
-  if (shock) {
-#pragma unroll
-    for (int h = 0; h < K; ++h) {
-      o.ar[h] *= gfl[h];
-      o.al[h] *= gfl[h];
-    }
-  }
+  for (int h = 0; h < K; ++h) ar[h] = P.c0[h] * o.dr[h] + P.c1[h] * slp[h] + P.c2[h] * slope[h];
+  C<float, K> arm = prev1(ar);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
-    const float r = med0(o.ar[h], -2.0f * o.al[h]), l = med0(o.al[h], -2.0f * o.ar[h]);
-    o.ar[h] = r;
-    o.al[h] = l;
-    o.da[h] = r - l;
-    o.s[h] = r + l;
+    const int c = c0 + h;
+    const float g = 1.0f - flat[h];
+    float r = g * ar[h];                 // flattened right edge - x
+    float l = g * (arm[h] - o.dl[h]);    // flattened left edge - x
+    const float d = r - l;
+    const float t2 = d * d;
+    const float t1 = -3.0f * d * (r + l);   // (ar - la) 6 (x - (ar + la)/2)
+    if (r * l >= 0.0f) {                 // (ar - x)(x - la) <= 0: an extremum
+      r = 0.0f;
+      l = 0.0f;
+    }
+    if (t2 < t1) l = -2.0f * r;          // la = 3 x - 2 ar
+    if (t2 < -t1) r = -2.0f * l;         // ar = 3 x - 2 la
+    const bool in = (c >= nmin + 2 && c < nmaxp - 2);
+    o.da[h] = in ? r - l : 0.0f;
+    o.a6[h] = in ? -3.0f * (r + l) : 0.0f;
+    o.al[h] = in ? l : -val[h];
+    if constexpr (EDGE) o.ar[h] = in ? r : -val[h];
   }
   return o;
 }
@@ -311,7 +300,6 @@ struct WinP {
   // vrot (azimuthal sweep) or rs / rcs (radial and theta sweeps: sin / cos of the planet's
   // drift against the slot in half a step, halved) for the planet's azimuth over the step
   C<float, K> rad, xa0, dx0, dvol0, vrot, ts, tc, sth, oms, rs, rcs;
-  C<float, K> idx0, iyv;   // azimuthal sweep: 1/dx0 and rad/dvol0
 };
 
 // the per-slot table entries of this lane's K cells, entry-major (entry e of slot s at
@@ -355,15 +343,31 @@ __device__ __forceinline__ void rot_by(float s, float c, float rs, float rc, flo
   so = s * rc + c * rs;
   co = c * rc - s * rs;
 }
-__device__ __forceinline__ void rot_by2(float s, float c, float rs, float rc, float& so, float& co) {
-  rot_by(s, c, 2.0f * rs * rc, 1.0f - 2.0f * rs * rs, so, co);
+// the same for the radial and theta sweeps, with the product that rounds written out (ALT: the
+// other one of each pair, in the full turn of the isothermal cylindrical sweep).  Of two
+// products the compiler contracts either, and chooses anew when code around them changes: a disk
+// whose course amplifies roundings then runs elsewhere.  Here and below (velocity_of, the
+// density and last updates) the choice is therefore part of the source.
+template <bool ALT = false>
+__device__ __forceinline__ void rot_fixed(float s, float c, float rs, float rc, float& so, float& co) {
+  so = ALT ? __builtin_fmaf(c, rs, s * rc) : __builtin_fmaf(s, rc, c * rs);
+  co = ALT ? __builtin_fmaf(-s, rs, c * rc) : __builtin_fmaf(c, rc, -(s * rs));
+}
+template <bool ALT = false>
+__device__ __forceinline__ void rot_fixed2(float s, float c, float rs, float rc, float& so, float& co) {
+  rot_fixed<ALT>(s, c, 2.0f * rs * rc, 1.0f - 2.0f * rs * rs, so, co);
+}
+// a product that rounds by itself (no contraction into what it feeds)
+__device__ __forceinline__ float rounded(float x) {
+  asm("" : "+v"(x));
+  return x;
 }
 
 // cos(a + d) - cos(a) from sin a, cos a and a small d (|d| < ~0.3), without cancellation
 __device__ __forceinline__ float dcos(float sa, float ca, float d) {
   const float d2 = d * d;
-  const float sd = d + d * d2 * (-1.0f / 6.0f + d2 * (1.0f / 120.0f));
-  const float omc = d2 * (0.5f + d2 * (-1.0f / 24.0f + d2 * (1.0f / 720.0f)));
+  const float sd = d * (1.0f - d2 * (1.0f / 6.0f) * (1.0f - d2 * (1.0f / 20.0f)));
+  const float omc = 0.5f * d2 * (1.0f - d2 * (1.0f / 12.0f) * (1.0f - d2 * (1.0f / 30.0f)));
   return -sa * sd - ca * omc;
 }
 
@@ -371,8 +375,8 @@ __device__ __forceinline__ float dcos(float sa, float ca, float d) {
 __device__ __forceinline__ void rot_theta(float st, float ct, float oms, float e, float& so, float& co,
                                           float& omso) {
   const float e2 = e * e;
-  const float se = e + e * e2 * (-1.0f / 6.0f + e2 * (1.0f / 120.0f));
-  const float omc = e2 * (0.5f + e2 * (-1.0f / 24.0f + e2 * (1.0f / 720.0f)));
+  const float se = e * (1.0f - e2 * (1.0f / 6.0f) * (1.0f - e2 * (1.0f / 20.0f)));
+  const float omc = 0.5f * e2 * (1.0f - e2 * (1.0f / 12.0f) * (1.0f - e2 * (1.0f / 30.0f)));
   so = st * (1.0f - omc) + ct * se;
   co = ct * (1.0f - omc) - st * se;
   omso = oms + st * omc - ct * se;
@@ -385,10 +389,9 @@ __device__ __forceinline__ void rot_theta(float st, float ct, float oms, float e
 // Eulerian grid (its values outside the window's paraset ranges never reach a parabola the
 // sweep keeps).  c0: this lane's first cell of its window (a wavefront may hold several windows
 // side by side: stencils reach across the seam between two as they reach past a window's last
-// cell, and every stage's index range keeps such values out of the cells a window stores).
-// wres: the azimuthal grid's uniform angular rate.  rsph: the spherical
-// radius of an azimuthal 3-D ring.  On return cells [6, nmax-6) hold the update.
-template <int K, int G, int NDIM, class Tab, bool ADIA = false, bool BARY = false>
+// cell, and every stage's index range keeps such values out of the cells a window stores).  wres: the azimuthal grid's uniform angular rate.  rsph: the spherical
+// radius of an azimuthal 3-D ring.  ENDS: no viscosity follows (3-D).  On return cells [6, nmax-6) hold the update.
+template <int K, int G, int NDIM, class Tab, bool ADIA = false, bool BARY = false, bool ENDS = false>
 __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para<float, K>& P0, int c0, int nmax,
                                            float dt, float wres, const PlanetF& pl, bool planet, bool flat_on,
                                            float sqrt_gam, float rsph = 0.0f, bool phi_rows = false,
@@ -396,6 +399,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   constexpr bool RAD = (G == kGeoRcyl || G == kGeoRsph);
   static_assert(!ADIA || (NDIM == 2 && (G == kGeoRcyl || G == kGeoPhi)), "EOS 3 is built for 2-D disks");
   const float hdt = 0.5f * dt;
+  const float fourthd = 1.3333333333333333f;
   const float smallr = 1.0e-15f;
   // EOS 3 carries q = p / rho as its deviation dq from q_b; the pressure deviation is
   // p - p_b = rho_b dq + q_b drho + drho dq (p_b = rho_b q_b)
@@ -406,8 +410,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   }
 
   // ---- flatten (flatten.cu:7-40), on absolute pressure (relative-jump thresholds)
-  C<float, K> gfl = splat<float, K>(1.0f);   // 1 - the flattening
-  bool shocked = false;
+  C<float, K> flat = splat<float, K>(0.0f);
   if (flat_on) {
     C<float, K> pabs;
 #pragma unroll
@@ -417,32 +420,34 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     }
     C<float, K> pm1 = prev1(pabs), pp1 = next1(pabs);
     C<float, K> um1 = prev1(W.u), up1 = next1(W.u);
-    // the jump test as a product; most wavefronts hold no shock and skip the rest
-    C<bool, K> shock;
-    bool any = false;
+    // most wavefronts hold no jump near the threshold and skip the rest (the product lies below
+    // every quotient that passes the test)
+    bool near = false;
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       const int c = c0 + h;
-      const float m = fminf(pp1[h], pm1[h]);
-      shock[h] = (c >= 2 && c < nmax - 2) && m >= 0.0f && fabsf(pp1[h] - pm1[h]) > 0.33f * m && !(um1[h] < up1[h]);
-      any = any || shock[h];
+      near = near || ((c >= 2 && c < nmax - 2) && fabsf(pp1[h] - pm1[h]) > 0.3299f * fminf(pp1[h], pm1[h]) &&
+                      !(um1[h] < up1[h]));
     }
-    shocked = wave_any(any);
-    if (shocked) {
+    if (wave_any(near)) {
       C<float, K> pm2 = prev2(pabs), pp2 = next2(pabs), steep;
 #pragma unroll
       for (int h = 0; h < K; ++h) {
+        const int c = c0 + h;
+        const float dp1 = pp1[h] - pm1[h];
         float dp2 = pp2[h] - pm2[h];
         dp2 = (fabsf(dp2) < 1.0e-15f) ? 1.0e-15f : dp2;
-        const float st = fmaxf(0.0f, ((pp1[h] - pm1[h]) / dp2 - 0.75f) * 5.0f);
-        steep[h] = shock[h] ? st : 0.0f;
+        const float ddp = fabsf(dp1) / fminf(pp1[h], pm1[h]);
+        const bool shock = (c >= 2 && c < nmax - 2) && ddp > 0.33f && !(um1[h] < up1[h]);
+        const float st = fmaxf(0.0f, (dp1 / dp2 - 0.75f) * 5.0f);
+        steep[h] = shock ? st : 0.0f;
       }
       C<float, K> sm = prev1(steep), sp = next1(steep);
 #pragma unroll
       for (int h = 0; h < K; ++h) {
         const int c = c0 + h;
         const float fl = fminf(0.5f, fmaxf(sm[h], fmaxf(steep[h], sp[h])));
-        gfl[h] = (c >= 2 && c < nmax - 2) ? 1.0f - fl : 1.0f;
+        flat[h] = (c >= 2 && c < nmax - 2) ? fl : 0.0f;
       }
     }
   }
@@ -468,7 +473,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       }
       if (planet) {
         float s, c;
-        rot_by(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, c);
+        rot_fixed(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, c);
         if constexpr (G == kGeoRcyl) {
           f += planet_fr<BARY>(pl, W.xa0[h], s, c);
         } else {
@@ -508,53 +513,38 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       float f = ffb[h] + dlf * (2.0f * Lf[h] + dlf) * Gf[h];
       if (planet) {
         float s, c;
-        rot_by(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, c);
+        rot_fixed(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, c);
         f += planet_fth_sph<BARY>(pl, W.rad[h], szl[h], czl[h], 1.0f - szl[h], s, c);
       }
       fhalf[h] = hdt * f;
     }
   }
-  // reciprocals of the cell's fixed numbers: table entries, or along phi the columns' and once per ring
-  C<float, K> idx0, irb, ipb, irad;
-  if constexpr (!RAD) {
-#pragma unroll
-    for (int h = 0; h < K; ++h) irad[h] = 1.0f / W.rad[h];
-  }
-  if constexpr (G == kGeoPhi) {
-#pragma unroll
-    for (int h = 0; h < K; ++h) {
-      idx0[h] = W.idx0[h];
-      irb[h] = 1.0f / W.rb[h];
-      ipb[h] = 1.0f / W.pb[h];
-    }
-  } else {
-    idx0 = tx.get(G == kGeoTheta ? kTabIdz0 : kTabIdx0);
-    irb = tx.get(kTabIrb);
-    ipb = tx.get(kTabIpb);
-  }
-  C<float, K> csn, csfac;   // csfac: 3 (1 - (4/3) csn), for s = -a6/3
+  C<float, K> csn, csfac;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     // sqrt(gam p / rho) = sqrt(gam) c_s for the isothermal closure, sqrt(gam q) for EOS 3
     float s;
-    if constexpr (ADIA) s = hdt * sqrtf(gam * (W.qb[h] + W.q[h]));
-    else s = hdt * sqrt_gam * W.cs[h];
-    if constexpr (G == kGeoPhi || G == kGeoTheta) s = s * irad[h];
-    s = s * idx0[h];
+    if constexpr (ADIA) s = hdt * sqrtf(gam * (W.qb[h] + W.q[h])) / W.dx0[h];
+    else s = hdt * sqrt_gam * W.cs[h] / W.dx0[h];
+    if constexpr (G == kGeoPhi || G == kGeoTheta) s = s / W.rad[h];
     csn[h] = s;
-    csfac[h] = 3.0f - 4.0f * s;
+    csfac[h] = 1.0f - fourthd * s;
   }
   // edge averages of the traced parabolae (states.cu:45-68), in the cell's frame: the
   // cell's value x plus the average's offset from it
   auto edges = [&](const ParabR<K>& q, const C<float, K>& x, C<float, K>& re, C<float, K>& le) {
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      re[h] = x[h] + (q.ar[h] - csn[h] * (q.da[h] + csfac[h] * q.s[h]));
-      le[h] = x[h] + (q.al[h] + csn[h] * (q.da[h] - csfac[h] * q.s[h]));
+      if constexpr (ADIA) re[h] = x[h] + (q.ar[h] - csn[h] * (q.da[h] - csfac[h] * q.a6[h]));
+      else re[h] = x[h] + (q.al[h] + q.da[h] - csn[h] * (q.da[h] - csfac[h] * q.a6[h]));
+      le[h] = x[h] + (q.al[h] + csn[h] * (q.da[h] + csfac[h] * q.a6[h]));
     }
   };
   // interface c: left state = right edge of cell c-1, right state = left edge of cell c, as
-  // relative jumps against the backgrounds of cell c-1
+  // relative jumps against the backgrounds of cell c-1.  EOS 3 forms u* from differences of the
+  // jumps' logarithms, so it corrects their quotients and takes the right edge's offset as it is
+  // (al + da, the isothermal form, rounds it again); L1 against FP64 after 150 steps of 192 x 576: Sigma 2.1 ->
+  // 2.0e-9, p 2.4 -> 2.3e-9.
   C<float, K> epl, epr, erl, err, ul, ur;
   if constexpr (G != kGeoPhi || ADIA) {
     C<float, K> pp, re, le;
@@ -564,33 +554,41 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       else pp[h] = W.r[h] * W.cs2[h];
     }
     // along a ring p_b is one constant
-    edges(parabola_rel<K, G != kGeoPhi>(gfl, shocked, pp, W.dpb, P0), pp, re, le);
+    edges(parabola_rel<K, G != kGeoPhi, ADIA>(c0, 0, nmax, flat, pp, W.dpb, P0), pp, re, le);
     C<float, K> q;
 #pragma unroll
-    for (int h = 0; h < K; ++h) q[h] = re[h] * ipb[h];
-    C<float, K> qm = prev1(q), ipbm = prev1(ipb), dpbm = prev1(W.dpb);
+    for (int h = 0; h < K; ++h) {
+      if constexpr (ADIA) q[h] = quot_f32(re[h], W.pb[h]);
+      else q[h] = re[h] / W.pb[h];
+    }
+    C<float, K> qm = prev1(q), pbm = prev1(W.pb), dpbm = prev1(W.dpb);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       epl[h] = qm[h];
-      epr[h] = (le[h] + dpbm[h]) * ipbm[h];
+      if constexpr (ADIA) epr[h] = quot_f32(le[h] + dpbm[h], pbm[h]);
+      else epr[h] = (le[h] + dpbm[h]) / pbm[h];
     }
   }
   {
     C<float, K> re, le;
-    edges(parabola_rel<K, G != kGeoPhi>(gfl, shocked, W.r, W.drb, P0), W.r, re, le);
+    edges(parabola_rel<K, G != kGeoPhi, ADIA>(c0, 0, nmax, flat, W.r, W.drb, P0), W.r, re, le);
     C<float, K> q;
 #pragma unroll
-    for (int h = 0; h < K; ++h) q[h] = re[h] * irb[h];
-    C<float, K> qm = prev1(q), irbm = prev1(irb), drbm = prev1(W.drb);
+    for (int h = 0; h < K; ++h) {
+      if constexpr (ADIA) q[h] = quot_f32(re[h], W.rb[h]);
+      else q[h] = re[h] / W.rb[h];
+    }
+    C<float, K> qm = prev1(q), rbm = prev1(W.rb), drbm = prev1(W.drb);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       erl[h] = qm[h];
-      err[h] = (le[h] + drbm[h]) * irbm[h];
+      if constexpr (ADIA) err[h] = quot_f32(le[h] + drbm[h], rbm[h]);
+      else err[h] = (le[h] + drbm[h]) / rbm[h];
     }
   }
   {
     C<float, K> re, le;
-    edges(parabola_rel<K, false>(gfl, shocked, W.u, W.u, P0), W.u, re, le);
+    edges(parabola_rel<K, false, ADIA>(c0, 0, nmax, flat, W.u, W.u, P0), W.u, re, le);
     C<float, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -616,24 +614,22 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     for (int h = 0; h < K; ++h) {
       const int c = c0 + h;
       const bool used = c >= 3 && c < nmax - 2;
-      // jumps below 0.2 keep every argument of the states' logs and exps (z < 1/2) below 1/4
-      const bool w1 = wave_any(used && !(max4(epl[h], epr[h], erl[h], err[h]) < 0.2f));
-      const float lpl = log1p_acc(epl[h], w1), lpr = log1p_acc(epr[h], w1);
-      const float lrl = log1p_acc(erl[h], w1), lrr = log1p_acc(err[h], w1);
+      auto log1p_of = [&](float x) { return log1p_acc(x, wave_any(used && !(fabsf(x) < 0.25f))); };
+      auto expm1_of = [&](float y) { return expm1_acc(y, wave_any(used && !(fabsf(y) < 0.25f))); };
+      const float lpl = log1p_of(epl[h]), lpr = log1p_of(epr[h]);
+      const float lrl = log1p_of(erl[h]), lrr = log1p_of(err[h]);
       const float a0 = sqrtf(gam * qbm[h]);
       const float hl = 0.5f * (lpl - lrl), hr = 0.5f * (lpr - lrr);   // log(a_l), log(a_r)
-      const float al1 = expm1_acc(hl, w1), ar1 = expm1_acc(hr, w1);
+      const float al1 = expm1_of(hl), ar1 = expm1_of(hr);
       const float nm1 = 0.5f * (al1 + ar1) - 0.25f * gm1 * (ur[h] - ul[h]) / a0;
-      const float dm1 = 0.5f * (expm1_acc(hl - z * lpl, w1) + expm1_acc(hr - z * lpr, w1));
-      const bool w2 = wave_any(used && !(fmaxf(fabsf(nm1), fabsf(dm1)) < 0.25f));
-      const float lm = iz * (log1p_acc(nm1, w2) - log1p_acc(dm1, w2));   // log(p* / p_b)
-      const bool w3 = w1 || wave_any(used && !(fabsf(lm) < 0.25f));
-      const float e_ = expm1_acc(lm, w3);
+      const float dm1 = 0.5f * (expm1_of(hl - z * lpl) + expm1_of(hr - z * lpr));
+      const float lm = iz * (log1p_of(nm1) - log1p_of(dm1));   // log(p* / p_b)
+      const float e_ = expm1_of(lm);
       float t1, t2;   // right and left wave terms of u* (riemann.cu:64-70)
       if (e_ > epr[h]) t1 = (e_ - epr[h]) * sqrtf(2.0f * qbm[h] / ((1.0f + err[h]) * (gp1 * (1.0f + e_) + gm1 * (1.0f + epr[h]))));
-      else t1 = 2.0f * a0 * (1.0f + ar1) * expm1_acc(z * (lm - lpr), w3) / gm1;
+      else t1 = 2.0f * a0 * (1.0f + ar1) * expm1_of(z * (lm - lpr)) / gm1;
       if (e_ > epl[h]) t2 = (e_ - epl[h]) * sqrtf(2.0f * qbm[h] / ((1.0f + erl[h]) * (gp1 * (1.0f + e_) + gm1 * (1.0f + epl[h]))));
-      else t2 = 2.0f * a0 * (1.0f + al1) * expm1_acc(z * (lm - lpl), w3) / gm1;
+      else t2 = 2.0f * a0 * (1.0f + al1) * expm1_of(z * (lm - lpl)) / gm1;
       em[h] = e_;
       umid[h] = 0.5f * (ur[h] + ul[h]) + 0.5f * (t1 - t2);
     }
@@ -641,15 +637,14 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     C<float, K> csm = prev1(W.cs);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      // t1 only scales small differences (of velocity and of log pressure), so its plain
-      // FP32 relative accuracy suffices: no logs of the density states, sqrt(a/b) = a rsqrt(a b)
-      const float pl1 = 1.0f + epl[h], pr1 = 1.0f + epr[h];
-      const float t1 = 0.5f * csm[h] * (pl1 * __frsqrt_rn(pl1 + pl1 * erl[h]) + pr1 * __frsqrt_rn(pr1 + pr1 * err[h]));
-      const float t2 = -0.5f * (ur[h] - ul[h]) / t1;
       const int c = c0 + h;
       const bool used = c >= 3 && c < nmax - 2;
       const bool w = wave_any(used && !(fmaxf(fabsf(epl[h]), fabsf(epr[h])) < 0.25f));
       const float lpl = log1p_acc(epl[h], w), lpr = log1p_acc(epr[h], w);
+      // t1 only scales small differences (of velocity and of log pressure), so its plain
+      // FP32 relative accuracy suffices: no logs of the density states
+      const float t1 = 0.5f * csm[h] * (sqrtf((1.0f + epl[h]) / (1.0f + erl[h])) + sqrtf((1.0f + epr[h]) / (1.0f + err[h])));
+      const float t2 = -0.5f * (ur[h] - ul[h]) / t1;
       const float y = 0.5f * (lpl + lpr) + t2;
       em[h] = expm1_acc(y, wave_any(used && !(fabsf(y) < 0.25f)));
       umid[h] = ul[h] - t1 * (0.5f * (lpr - lpl) + t2);
@@ -660,12 +655,12 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     // c_s^2 times the density states, so eps_p = eps_rho and t1 = c_s exactly
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      const float t1 = W.cs[h];
-      const float t2 = (-0.5f / t1) * (ur[h] - ul[h]);
       const int c = c0 + h;
       const bool used = c >= 3 && c < nmax - 2;
       const bool w = wave_any(used && !(fmaxf(fabsf(erl[h]), fabsf(err[h])) < 0.25f));
       const float lrl = log1p_acc(erl[h], w), lrr = log1p_acc(err[h], w);
+      const float t1 = W.cs[h];
+      const float t2 = -0.5f * (ur[h] - ul[h]) / t1;
       const float y = 0.5f * (lrl + lrr) + t2;
       em[h] = expm1_acc(y, wave_any(used && !(fabsf(y) < 0.25f)));
       umid[h] = ul[h] - t1 * (0.5f * (lrr - lrl) + t2);
@@ -673,30 +668,30 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   }
 
   // ---- evolve (evolve.cu:3-166): edges as displacements from the Eulerian edges.  The
-  // reference moves edges [3, nmax-2) and cells [3, nmax-3); here every one moves: what a kept
-  // cell reads lies inside those ranges (edges 3 to nmax-3, cells 3 to nmax-4).
-  C<float, K> sx, dltx;
+  // reference moves edges [3, nmax-2) and cells [3, nmax-3).
+  C<float, K> smv, dlt;
   const float Wd = (G == kGeoPhi) ? dt * wres : 0.0f;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
+    const int c = c0 + h;
+    const bool mv = (c >= 3 && c < nmax - 2);
     float s;
     if constexpr (RAD) s = dt * umid[h];
-    else s = dt * irad[h] * umid[h];
-    sx[h] = s;
-    dltx[h] = s + Wd;
+    else s = dt * umid[h] / W.rad[h];
+    smv[h] = mv ? s : 0.0f;
+    dlt[h] = mv ? s + Wd : 0.0f;
   }
-  C<float, K> Dl;
+  C<float, K> Dl, dltx, sx;
   {
-    C<float, K> sp = next1(sx);
+    C<float, K> sp = next1(smv);
 #pragma unroll
-    for (int h = 0; h < K; ++h) Dl[h] = sp[h] - sx[h];   // dxl - dx0, free of the uniform motion
-  }
-  C<float, K> idvol0;
-  if constexpr (G == kGeoPhi) {
-#pragma unroll
-    for (int h = 0; h < K; ++h) idvol0[h] = irad[h] * W.iyv[h];
-  } else {
-    idvol0 = tx.get(G == kGeoTheta ? kTabIdvolZ : kTabIdvol0);
+    for (int h = 0; h < K; ++h) {
+      const int c = c0 + h;
+      const bool in = (c >= 3 && c < nmax - 3);
+      Dl[h] = in ? sp[h] - smv[h] : 0.0f;   // dxl - dx0, free of the uniform motion
+      dltx[h] = in ? dlt[h] : 0.0f;          // the left edge of a moved cell
+      sx[h] = in ? smv[h] : 0.0f;
+    }
   }
   C<float, K> rL;   // Lagrangian density deviation
   C<float, K> szl, czl;   // theta sweep: sin / cos of the left edge
@@ -721,6 +716,8 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       }
 #pragma unroll
       for (int h = 0; h < K; ++h) {
+        const int c = c0 + h;
+        const bool in = (c >= 3 && c < nmax - 3);
         const float ixc = tixc[h];
         const float ixc3 = ixc * ixc * ixc;
         const float rho = W.rb[h] + W.r[h];
@@ -740,7 +737,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
         float f21 = fdiff;   // force at the moved centre - at the centre (EOS 3)
         if (planet) {
           float s, cc;
-          rot_by2(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, cc);
+          rot_fixed2<G == kGeoRcyl && !ADIA>(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, cc);
           if constexpr (G == kGeoRcyl) {
             const float p1 = planet_fr<BARY>(pl, W.rad[h], W.ts[h], W.tc[h]), p2 = planet_fr<BARY>(pl, W.rad[h] + dxc, s, cc);
             fdiff += p1 + p2;
@@ -765,9 +762,8 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
           V0 = 0.5f * (x0 * x0 + xa0p[h] * xa0p[h]);
           dV = 0.5f * (d * (x0 + d * (1.0f / 3.0f)) + dp_ * (xa0p[h] + dp_ * (1.0f / 3.0f)));
         }
-        const float irho = 1.0f / rho, im = irho * idvol0[h];
-        const float acc = res_bg[h] + q1 + 0.5f * fdiff + abg[h] * (W.r[h] * irho) -
-                          (dpbm[h] * dV + dp * (V0 + dV)) * im;
+        const float acc = res_bg[h] + q1 + 0.5f * fdiff + abg[h] * (W.r[h] / rho) -
+                          (dpbm[h] * dV + dp * (V0 + dV)) / (rho * W.dvol0[h]);
         // Lagrangian volume change in offset form
         float ddv;
         if constexpr (G == kGeoRcyl) {
@@ -780,7 +776,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
                 w0 * D * D + D * D * D * (1.0f / 3.0f);
         }
         const float dvol = W.dvol0[h] + ddv;
-        rL[h] = W.r[h] - rho * ddv / dvol;   // (r dvol0 - rho_b ddv) / dvol
+        rL[h] = in ? W.r[h] - rho * ddv / dvol : W.r[h];   // (r dvol0 - rho_b ddv) / dvol
         if constexpr (ADIA) {
           // EOS 3 (the line evolve.cu:146 leaves commented out): e = eps + u^2/2 gains
           // -dt/dm (F_r - F_l) + dt (u f1 + u' f2)/2, eps' = e - u'^2/2.  With u' = u + du and
@@ -789,11 +785,11 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
           //   eps' - eps = -dt/dm ((F_r - F_l) - (u + du/2) dp A) + dt du (f2 - f1) / 4
           const float du = dt * acc;
           const float dpA = dpbm[h] * V0 + (dpbm[h] * dV + dp * (V0 + dV));
-          const float de = -dt * im * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpA) +
+          const float de = -dt / (rho * W.dvol0[h]) * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpA) +
                            0.25f * dt * du * f21;
-          W.q[h] += (gam - 1.0f) * de;
+          if (in) W.q[h] += (gam - 1.0f) * de;
         }
-        W.u[h] = W.u[h] + dt * acc;
+        if (in) W.u[h] = W.u[h] + dt * acc;
       }
     } else if constexpr (G == kGeoPhi) {
       // EOS 3: the pressure work through the left edge, u* p* (unit area factor)
@@ -805,6 +801,8 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       }
 #pragma unroll
       for (int h = 0; h < K; ++h) {
+        const int c = c0 + h;
+        const bool in = (c >= 3 && c < nmax - 3);
         float f = 0.0f, f21 = 0.0f;
         if (planet) {
           const float off = dltx[h] + 0.5f * Dl[h] + dt * (W.vrot[h] - pl.vy);
@@ -821,18 +819,17 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
         }
         const float rho = W.rb[h] + W.r[h];
         const float dpm = W.pb[h] * (emp[h] - em[h]);   // p_b is uniform along the ring
-        const float im = idvol0[h] / rho;
-        const float un = W.u[h] + (0.5f * dt * f - dt * dpm * im);
+        const float un = W.u[h] + (0.5f * dt * f - dt * dpm / (rho * W.dvol0[h]));
         const float ddv = Dl[h] * W.rad[h];
         const float dvol = W.dvol0[h] + ddv;
-        rL[h] = W.r[h] - rho * ddv / dvol;   // (r dvol0 - rho_b ddv) / dvol
+        rL[h] = in ? W.r[h] - rho * ddv / dvol : W.r[h];   // (r dvol0 - rho_b ddv) / dvol
         if constexpr (ADIA) {   // as in the radial sweep, with unit area factors
           const float du = un - W.u[h];
-          const float de = -dt * im * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpm) +
+          const float de = -dt / (rho * W.dvol0[h]) * ((Flp[h] - Fl[h]) - (W.u[h] + 0.5f * du) * dpm) +
                            0.25f * dt * du * f21;
-          W.q[h] += (gam - 1.0f) * de;
+          if (in) W.q[h] += (gam - 1.0f) * de;
         }
-        W.u[h] = un;
+        if (in) W.u[h] = un;
       }
     } else {
       // theta: centrifugal theta component L^2 G(theta), G = cos / (r sin)^3, minus the
@@ -851,6 +848,8 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       C<float, K> vfdp = next1(vfd);
 #pragma unroll
       for (int h = 0; h < K; ++h) {
+        const int c = c0 + h;
+        const bool in = (c >= 3 && c < nmax - 3);
         const float rho = W.rb[h] + W.r[h];
         const float dl = W.w[h];
         const float qq = dl * (2.0f * W.Lb[h] + dl);
@@ -861,7 +860,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
         float fdiff = L2 * e * (2.0f * G1[h] + e * G2[h]);
         if (planet) {
           float s, cc, so, co, omso;
-          rot_by2(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, cc);
+          rot_fixed2(W.ts[h], W.tc[h], W.rs[h], W.rcs[h], s, cc);
           rot_theta(W.sth[h], cth[h], W.oms[h], e, so, co, omso);
           fdiff += 2.0f * (planet_fth_sph<BARY>(pl, W.rad[h], W.sth[h], cth[h], W.oms[h], W.ts[h], W.tc[h]) +
                            planet_fth_sph<BARY>(pl, W.rad[h], so, co, omso, s, cc));
@@ -869,14 +868,13 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
         const float dp = W.pb[h] * emp[h] - pbm[h] * em[h];
         const float V0 = 0.5f * (szl[h] + szlp[h]);
         const float dV = 0.5f * (vfd[h] + vfdp[h]);
-        const float irho = 1.0f / rho;
-        const float acc = res_bg[h] + qq * Gc[h] + 0.25f * fdiff + abg[h] * (W.r[h] * irho) -
-                          (dpbm[h] * dV + dp * (V0 + dV)) * (irho * idvol0[h]);
+        const float acc = res_bg[h] + qq * Gc[h] + 0.25f * fdiff + abg[h] * (W.r[h] / rho) -
+                          (dpbm[h] * dV + dp * (V0 + dV)) / (rho * W.dvol0[h]);
         // dvol = r (cos(x0 + d) - cos(x1 + d + D)) with x1 the right edge
         const float ddv = W.rad[h] * (dcos(szl[h], czl[h], dltx[h]) - dcos(szr[h], czr[h], dltx[h] + Dl[h]));
         const float dvol = W.dvol0[h] + ddv;
-        rL[h] = W.r[h] - rho * ddv / dvol;   // (r dvol0 - rho_b ddv) / dvol
-        W.u[h] = W.u[h] + dt * acc;
+        rL[h] = in ? W.r[h] - rho * ddv / dvol : W.r[h];   // (r dvol0 - rho_b ddv) / dvol
+        if (in) W.u[h] = W.u[h] + dt * acc;
       }
     }
   }
@@ -885,9 +883,8 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   C<float, K> dxl;
 #pragma unroll
   for (int h = 0; h < K; ++h) dxl[h] = W.dx0[h] + Dl[h];
-  const Para<float, K> P1 = paraset_f32<K>(dxl);
-  C<float, K> dxf, dxf2, lvol;
-  C<bool, K> fwd;   // the edge moves forward: it sweeps the left neighbour
+  Para<float, K> P1 = paraset<float, K>(c0, 3, nmax - 3, dxl);
+  C<float, K> dxf, dxf2, lvol, delC;
   C<float, K> dxm = prev1(dxl);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
@@ -896,26 +893,36 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
     else if constexpr (G == kGeoRsph) lvol[h] = d * (W.xa0[h] * (W.xa0[h] + d) + d * d * (1.0f / 3.0f));
     else if constexpr (G == kGeoPhi) lvol[h] = d * W.rad[h];
     else lvol[h] = -W.rad[h] * dcos(szl[h], czl[h], d);
-    fwd[h] = d >= 0.0f;
-    const float e = 0.5f * d / (fwd[h] ? dxm[h] : dxl[h]);
+    delC[h] = (d >= 0.0f) ? 1.0f : 0.0f;
+    float e;
+    if (d >= 0.0f) {
+      e = 0.5f * d / dxm[h];
+      dxf2[h] = 1.0f - fourthd * e;
+    } else {
+      e = 0.5f * d / dxl[h];
+      dxf2[h] = 1.0f + fourthd * e;
+    }
     dxf[h] = e;
-    dxf2[h] = 3.0f - 4.0f * fabsf(e);   // either way the edge moves
   }
   // average over the swept region of the left edge (remap.cu:59-90) minus the cell's own
   // value: from the left neighbour's parabola (its offset from X(c-1), then the jump
   // X(c) - X(c-1) in this frame) or from this cell's own
   auto face = [&](const ParabR<K>& Q, C<float, K>& out) {
-    C<float, K> arm = prev1(Q.ar), dam = prev1(Q.da), sm = prev1(Q.s);
+    C<float, K> alm = prev1(Q.al), dam = prev1(Q.da), a6m = prev1(Q.a6), arm;
+    if constexpr (ADIA) arm = prev1(Q.ar);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
-      if (fwd[h]) out[h] = (arm[h] - Q.dl[h]) - dxf[h] * (dam[h] + dxf2[h] * sm[h]);
-      else out[h] = Q.al[h] - dxf[h] * (Q.da[h] - dxf2[h] * Q.s[h]);
+      if (delC[h] != 0.0f) {
+        if constexpr (ADIA) out[h] = (arm[h] - Q.dl[h]) - dxf[h] * (dam[h] - dxf2[h] * a6m[h]);
+        else out[h] = (alm[h] + dam[h] - dxf[h] * (dam[h] - dxf2[h] * a6m[h])) - Q.dl[h];
+      }
+      else out[h] = Q.al[h] - dxf[h] * (Q.da[h] + dxf2[h] * Q.a6[h]);
     }
   };
   C<float, K> invm, fr;
   {
     C<float, K> fv, frd;
-    face(parabola_rel<K, G != kGeoPhi>(gfl, shocked, rL, W.drb, P1), fv);
+    face(parabola_rel<K, G != kGeoPhi, ADIA>(c0, 3, nmax - 3, flat, rL, W.drb, P1), fv);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       fv[h] = rL[h] + fv[h];   // the face's deviation from rho_b of this cell
@@ -925,17 +932,23 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       } else {
         // rho_b times the uniform displacement is the same at every edge: it carries no
         // mass difference, so the density update leaves it out
-        const float mr = W.rb[h] * W.rad[h];
-        frd[h] = mr * sx[h] + fv[h] * lvol[h];
-        fr[h] = frd[h] + mr * Wd;
+        frd[h] = W.rb[h] * (W.rad[h] * sx[h]) + fv[h] * lvol[h];
+        fr[h] = frd[h] + W.rb[h] * (W.rad[h] * (dltx[h] - sx[h]));
       }
     }
     C<float, K> frp = next1(frd);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
       const int c = c0 + h;
-      const float rn = W.r[h] + (frd[h] - frp[h]) * idvol0[h];
-      invm[h] = idvol0[h] / fmaxf(W.rb[h] + rn, smallr);
+      // the difference of two faces' masses, one of the products exact in the FMA: the next face's
+      // where this lane holds it
+      float dm = frd[h] - frp[h];
+      if constexpr (G != kGeoPhi) {
+        if (h + 1 < K) dm = __builtin_fmaf(-(W.rb[h + 1] + fv[h + 1]), lvol[h + 1], frd[h]);
+        else dm = __builtin_fmaf(W.rb[h] + fv[h], lvol[h], -frp[h]);
+      }
+      const float rn = W.r[h] + dm / W.dvol0[h];
+      invm[h] = 1.0f / (fmaxf(W.rb[h] + rn, smallr) * W.dvol0[h]);
       W.r[h] = (c >= 6 && c < nmax - 6) ? rn : rL[h];
     }
   }
@@ -947,7 +960,7 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
   // (X m + ...) / m_new rounds X m / m_new away from X by up to an ulp of X, the same ulp
   // step after step in a steady flow, a drift of 1e-4 of X over 1000 steps.
   C<float, K> frp = next1(fr);
-  auto remap_inc = [&](C<float, K>& X, const ParabR<K>& Q) {
+  auto remap_inc = [&](C<float, K>& X, const ParabR<K>& Q, bool split = false) {
     C<float, K> rl;
     face(Q, rl);
     C<float, K> rlp = next1(rl);
@@ -956,39 +969,31 @@ __device__ __forceinline__ void ppmlr_pert(WinP<K>& W, const Tab& tx, const Para
       const int c = c0 + h;
       // the right face relative to this cell's X: (face(c+1) - X(c+1)) + (X(c+1) + dbg - X)
       const float rr = rlp[h] + Q.dr[h];
-      if (c >= 6 && c < nmax - 6) X[h] = X[h] + (rl[h] * fr[h] - rr * frp[h]) * invm[h];
+      if (c >= 6 && c < nmax - 6) {
+        const float inc = (rl[h] * fr[h] - rr * frp[h]) * invm[h];
+        X[h] = X[h] + (split && h == 0 ? rounded(inc) : inc);
+      }
     }
   };
-  auto remap_plain = [&](C<float, K>& X) { remap_inc(X, parabola_rel<K, false>(gfl, shocked, X, X, P1)); };
+  auto remap_plain = [&](C<float, K>& X, bool split = false) {
+    remap_inc(X, parabola_rel<K, false, ADIA>(c0, 3, nmax - 3, flat, X, X, P1), split);
+  };
   // deviations from a background that varies along the sweep (l - L_b; EOS 3's q - q_b):
   // fluxes relative to the cell's own background; the right edge's face comes from the next
   // cell's frame, b(c+1) = b(c) + dbg
-  auto remap_bg = [&](C<float, K>& X, const C<float, K>& dbg) {
-    remap_inc(X, parabola_rel<K, true>(gfl, shocked, X, dbg, P1));
+  auto remap_bg = [&](C<float, K>& X, const C<float, K>& dbg, bool split = false) {
+    remap_inc(X, parabola_rel<K, true, ADIA>(c0, 3, nmax - 3, flat, X, dbg, P1), split);
   };
   remap_plain(W.u);
   if constexpr (RAD) remap_bg(W.v, W.dLb);
   else remap_plain(W.v);
-  if constexpr (G == kGeoRsph || (G == kGeoPhi && NDIM == 3)) remap_plain(W.w);
-  if constexpr (G == kGeoTheta) remap_bg(W.w, W.dLb);
+  if constexpr (G == kGeoRsph || (G == kGeoPhi && NDIM == 3)) remap_plain(W.w, G == kGeoRsph && ENDS);
+  if constexpr (G == kGeoTheta) remap_bg(W.w, W.dLb, ENDS);
   // EOS 3: q = p / rho, mass-weighted (remap.cu:171-176); q_b is uniform along a ring
   if constexpr (ADIA) {
     if constexpr (G == kGeoPhi) remap_plain(W.q);
     else remap_bg(W.q, W.dqb);
   }
-}
-
-// first and second derivative at x2 of the quadratic through (0, um), (x2, u0), (x3, up)
-// (viscosity.cu:2-19), u = um + B x + A x^2: h2 = B + A x2, so u'(x2) = h2 + A x2.  i2, i3, i32:
-// 1/x2, 1/x3, 1/(x3 - x2), for all of a cell's fields; x2 and x3 - x2 are cell widths (radial and
-// theta: reciprocals from the table; along phi an own one per cell, since 1/dphi kept through the
-// sweep costs a spill).  Twelve viscous disks: radial 81.5 -> 79.9 us, azimuthal 64.2 -> 62.7.
-__device__ __forceinline__ void derivs_f32(float x2, float i2, float i3, float i32, float um, float u0, float up,
-                                           float& first, float& second) {
-  const float h2 = (u0 - um) * i2, h3 = (up - um) * i3;
-  const float A = (h3 - h2) * i32;
-  second = 2.0f * A;
-  first = h2 + A * x2;
 }
 
 // Explicit viscosity after the radial remap (device_viscosity_r, viscosity.cu:370-421) on
@@ -1001,14 +1006,14 @@ __device__ __forceinline__ void derivs_f32(float x2, float i2, float i3, float i
 template <int K, bool SPH = false>
 __device__ __forceinline__ void visc_r_pert(WinP<K>& W, const TabLane<K>& tx, int c0, int lim, float dt) {
   const C<float, K> nu = tx.get(kTabNu), dnb = tx.get(kTabDnb), d1ob = tx.get(kTabD1Ob), d2ob = tx.get(kTabD2Ob),
-                    irc = tx.get(kTabIrc), rcyl = tx.get(kTabRc), idx0 = tx.get(kTabIdx0);
+                    irc = tx.get(kTabIrc), rcyl = tx.get(kTabRc);
   C<float, K> np_, om;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     np_[h] = nu[h] * W.r[h];
     om[h] = W.v[h] * (irc[h] * irc[h]);
   }
-  C<float, K> wm = prev1(W.dx0), iwm = prev1(idx0);
+  C<float, K> wm = prev1(W.dx0);
   C<float, K> nm = prev1(np_), npp = next1(np_), um = prev1(W.u), up = next1(W.u), omm = prev1(om), omp = next1(om);
   C<float, K> tm, tp;
   if constexpr (SPH) {
@@ -1018,27 +1023,26 @@ __device__ __forceinline__ void visc_r_pert(WinP<K>& W, const TabLane<K>& tx, in
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     const int c = c0 + h;
-    const float x2 = wm[h], i2 = iwm[h], i3 = 1.0f / (wm[h] + W.dx0[h]), i32 = idx0[h], R = rcyl[h], iR = irc[h];
+    const float x2 = wm[h], x3 = wm[h] + W.dx0[h], R = rcyl[h];
     const float rho = W.rb[h] + W.r[h], n = nu[h] * rho;
     float dn, d1, d2, e1, e2;
-    derivs_f32(x2, i2, i3, i32, nm[h], np_[h], npp[h], dn, d2);
+    derivs(0.0f, x2, x3, nm[h], np_[h], npp[h], dn, d2);
     dn += dnb[h];
-    derivs_f32(x2, i2, i3, i32, um[h], W.u[h], up[h], d1, d2);
-    const float ddu = 2.0f * (n * (d2 + (d1 - W.u[h] * iR) * iR) + dn * d1);
-    derivs_f32(x2, i2, i3, i32, omm[h], om[h], omp[h], e1, e2);
+    derivs(0.0f, x2, x3, um[h], W.u[h], up[h], d1, d2);
+    const float ddu = 2.0f * n * d2 + 2.0f * dn * d1 + 2.0f * n * d1 / R - 2.0f * n * W.u[h] / R / R;
+    derivs(0.0f, x2, x3, omm[h], om[h], omp[h], e1, e2);
     e1 += d1ob[h];
     e2 += d2ob[h];
-    const float ddv = R * (n * e2 + dn * e1) + 3.0f * n * e1;
+    const float ddv = R * n * e2 + R * dn * e1 + 3.0f * n * e1;
     float ddw = 0.0f;
     if constexpr (SPH) {
-      derivs_f32(x2, i2, i3, i32, tm[h], W.w[h], tp[h], d1, d2);
-      ddw = n * (d2 + d1 * iR) + dn * d1;
+      derivs(0.0f, x2, x3, tm[h], W.w[h], tp[h], d1, d2);
+      ddw = n * d2 + dn * d1 + n * d1 / R;
     }
     if (c >= kNpad && c < lim - kNpad) {
-      const float f = dt / rho;
-      W.u[h] = W.u[h] + f * ddu;
-      W.v[h] = W.v[h] + f * R * ddv;
-      if constexpr (SPH) W.w[h] = W.w[h] + f * ddw;
+      W.u[h] = W.u[h] + dt * ddu / rho;
+      W.v[h] = W.v[h] + dt * R * ddv / rho;
+      if constexpr (SPH) W.w[h] = W.w[h] + dt * ddw / rho;
     }
   }
 }
@@ -1049,14 +1053,13 @@ __device__ __forceinline__ void visc_r_pert(WinP<K>& W, const TabLane<K>& tx, in
 // arc lengths along the ring, the left edges times R = r_cyl (ppm.cu:277-278).
 template <int K, bool W3 = false>
 __device__ __forceinline__ void visc_p_pert(WinP<K>& W, int c0, int lim, float dt, float nu, float R) {
-  C<float, K> np_, wx, iwx;
+  C<float, K> np_, wx;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     np_[h] = nu * W.r[h];
     wx[h] = W.dx0[h] * R;
-    iwx[h] = 1.0f / wx[h];
   }
-  C<float, K> wm = prev1(wx), iwm = prev1(iwx);
+  C<float, K> wm = prev1(wx);
   C<float, K> nm = prev1(np_), npp = next1(np_);
   C<float, K> vm = prev1(W.u), vp = next1(W.u), rm = prev1(W.v), rp = next1(W.v);
   C<float, K> tm, tp;
@@ -1067,24 +1070,23 @@ __device__ __forceinline__ void visc_p_pert(WinP<K>& W, int c0, int lim, float d
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     const int c = c0 + h;
-    const float x2 = wm[h], i2 = iwm[h], i3 = 1.0f / (wm[h] + wx[h]), i32 = iwx[h];
+    const float x2 = wm[h], x3 = wm[h] + wx[h];
     const float rho = W.rb[h] + W.r[h], n = nu * rho;
     float dn, d1, d2;
-    derivs_f32(x2, i2, i3, i32, nm[h], np_[h], npp[h], dn, d2);
-    derivs_f32(x2, i2, i3, i32, vm[h], W.u[h], vp[h], d1, d2);
-    const float ddv = 2.0f * (n * d2 + dn * d1);
-    derivs_f32(x2, i2, i3, i32, rm[h], W.v[h], rp[h], d1, d2);
+    derivs(0.0f, x2, x3, nm[h], np_[h], npp[h], dn, d2);
+    derivs(0.0f, x2, x3, vm[h], W.u[h], vp[h], d1, d2);
+    const float ddv = 2.0f * n * d2 + 2.0f * dn * d1;
+    derivs(0.0f, x2, x3, rm[h], W.v[h], rp[h], d1, d2);
     const float ddu = n * d2 + dn * d1;
     float ddw = 0.0f;
     if constexpr (W3) {
-      derivs_f32(x2, i2, i3, i32, tm[h], W.w[h], tp[h], d1, d2);
+      derivs(0.0f, x2, x3, tm[h], W.w[h], tp[h], d1, d2);
       ddw = n * d2 + dn * d1;
     }
     if (c >= kNpad && c < lim - kNpad) {
-      const float f = dt / rho;
-      W.u[h] = W.u[h] + f * ddv;
-      W.v[h] = W.v[h] + f * ddu;
-      if constexpr (W3) W.w[h] = W.w[h] + f * ddw;
+      W.u[h] = W.u[h] + dt * ddv / rho;
+      W.v[h] = W.v[h] + dt * ddu / rho;
+      if constexpr (W3) W.w[h] = W.w[h] + dt * ddw / rho;
     }
   }
 }
@@ -1098,37 +1100,35 @@ __device__ __forceinline__ void visc_p_pert(WinP<K>& W, int c0, int lim, float d
 template <int K>
 __device__ __forceinline__ void visc_z_pert(WinP<K>& W, const TabLane<K>& tx, int c0, int lim, float dt, float vis_nu) {
   const C<float, K> dnb = tx.get(kTabDnbZ), d1vb = tx.get(kTabD1VZ), d2vb = tx.get(kTabD2VZ), irc = tx.get(kTabIrc),
-                    rcyl = tx.get(kTabRc), idz = tx.get(kTabIdz0), ir = tx.get(kTabIxc);
-  C<float, K> np_, dv, wx, iwx;
+                    rcyl = tx.get(kTabRc);
+  C<float, K> np_, dv, wx;
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     np_[h] = vis_nu * W.r[h];
     dv[h] = W.w[h] * irc[h];   // v_phi - v_bg
     wx[h] = W.dx0[h] * W.rad[h];
-    iwx[h] = idz[h] * ir[h];
   }
-  C<float, K> wm = prev1(wx), iwm = prev1(iwx);
+  C<float, K> wm = prev1(wx);
   C<float, K> nm = prev1(np_), npp = next1(np_), tm = prev1(W.u), tp = next1(W.u), rm = prev1(W.v), rp = next1(W.v),
               vm = prev1(dv), vp = next1(dv);
 #pragma unroll
   for (int h = 0; h < K; ++h) {
     const int c = c0 + h;
-    const float x2 = wm[h], i2 = iwm[h], i3 = 1.0f / (wm[h] + wx[h]), i32 = iwx[h];
+    const float x2 = wm[h], x3 = wm[h] + wx[h];
     const float rho = W.rb[h] + W.r[h], n = vis_nu * rho;
     float dn, d1, d2;
-    derivs_f32(x2, i2, i3, i32, nm[h], np_[h], npp[h], dn, d2);
+    derivs(0.0f, x2, x3, nm[h], np_[h], npp[h], dn, d2);
     dn += dnb[h];
-    derivs_f32(x2, i2, i3, i32, tm[h], W.u[h], tp[h], d1, d2);
-    const float ddt = 2.0f * (n * d2 + dn * d1);
-    derivs_f32(x2, i2, i3, i32, rm[h], W.v[h], rp[h], d1, d2);
+    derivs(0.0f, x2, x3, tm[h], W.u[h], tp[h], d1, d2);
+    const float ddt = 2.0f * n * d2 + 2.0f * dn * d1;
+    derivs(0.0f, x2, x3, rm[h], W.v[h], rp[h], d1, d2);
     const float ddr = n * d2 + dn * d1;
-    derivs_f32(x2, i2, i3, i32, vm[h], dv[h], vp[h], d1, d2);
+    derivs(0.0f, x2, x3, vm[h], dv[h], vp[h], d1, d2);
     const float ddv = n * (d2 + d2vb[h]) + dn * (d1 + d1vb[h]);
     if (c >= kNpad && c < lim - kNpad) {
-      const float f = dt / rho;
-      W.u[h] = W.u[h] + f * ddt;
-      W.v[h] = W.v[h] + f * ddr;
-      W.w[h] = W.w[h] + f * rcyl[h] * ddv;
+      W.u[h] = W.u[h] + dt * ddt / rho;
+      W.v[h] = W.v[h] + dt * ddr / rho;
+      W.w[h] = W.w[h] + dt * rcyl[h] * ddv / rho;
     }
   }
 }
