@@ -452,8 +452,9 @@ struct Parab {
 // parabola (parabola.cu:70-136), valid on [nmin+2, nmaxp-2) for coefficients valid on the
 // reference's ranges of [nmin, nmaxp); outside it holds values no kept cell reads.  omf = 1 -
 // flat.  The differences come once per interface (da_l of a cell is da_r of the one before it,
-// the same subtraction); everything else is the reference's, operation for operation.
-template <int K>
+// the same subtraction); everything else is the reference's, operation for operation, but for the
+// flattened edges, whose product rounds apart only with EX.
+template <int K, bool EX>
 __device__ __forceinline__ Parab<double, K> parabola(const C<double, K>& flat, const C<double, K>& omf,
                                                      const C<double, K>& val, const Para<double, K>& P) {
   C<double, K> vp = next1(val);
@@ -475,8 +476,8 @@ __device__ __forceinline__ Parab<double, K> parabola(const C<double, K>& flat, c
   for (int h = 0; h < K; ++h) {
     const double a = val[h];
     double t1 = flat[h] * a;
-    double arr = __builtin_fma(omf[h], ar[h], t1);
-    double la = __builtin_fma(omf[h], alv[h], t1);
+    double arr = EX ? t1 + omf[h] * ar[h] : __builtin_fma(omf[h], ar[h], t1);
+    double la = EX ? t1 + omf[h] * alv[h] : __builtin_fma(omf[h], alv[h], t1);
     t1 = arr - la;
     const double t2 = t1 * t1;
     t1 = t1 * (6.0 * (a - 0.5 * (arr + la)));
@@ -681,7 +682,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const
   C<T, K> Spl, Spr, Srl, Srr, Sul, Sur;
   {
     C<T, K> re, le;
-    traced(parabola(flat, omf, W.p, P0), re, le);
+    traced(parabola<K, EX>(flat, omf, W.p, P0), re, le);
     C<T, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -691,7 +692,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const
   }
   {
     C<T, K> re, le;
-    traced(parabola(flat, omf, W.r, P0), re, le);
+    traced(parabola<K, EX>(flat, omf, W.r, P0), re, le);
     C<T, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -701,7 +702,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const
   }
   {
     C<T, K> re, le;
-    traced(parabola(flat, omf, W.u, P0), re, le);
+    traced(parabola<K, EX>(flat, omf, W.u, P0), re, le);
     C<T, K> rem = prev1(re);
 #pragma unroll
     for (int h = 0; h < K; ++h) {
@@ -1038,7 +1039,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const
   };
   C<T, K> mass, invm;
   {
-    Parab<T, K> Q = parabola(flat, omf, W.r, P1);
+    Parab<T, K> Q = parabola<K, EX>(flat, omf, W.r, P1);
     C<T, K> fv;
     face(Q, fv);
 #pragma unroll
@@ -1055,7 +1056,7 @@ __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const
     }
   }
   auto remap_field = [&](C<T, K>& X) {
-    Parab<T, K> Q = parabola(flat, omf, X, P1);
+    Parab<T, K> Q = parabola<K, EX>(flat, omf, X, P1);
     C<T, K> fl;
     face(Q, fl);
 #pragma unroll
