@@ -38,6 +38,7 @@ struct pn_ctx {
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   int cur = 0;                      // buffer holding the state
   bool loaded = false;
+  bool frame_moves = false;         // this run's FrRot changes inside a step (frame_moves())
   // host copies of the per-ring values the device never changes (for packing)
   std::vector<double> h_x, h_dx, h_xc, h_xvol, h_z, h_dz, h_zc, h_zvol, h_vbg, h_rbg, h_cs2, h_qbg;
   std::vector<double> h_y, h_dy, h_yc, h_yvol;

@@ -87,10 +87,24 @@ int nwin(int len) { return (len + kReal - 1) / kReal; }
 
 bool is_f32(const pn_ctx* c) { return c->precision == PN_FP32; }
 
-// the next dt from the last sweep's epilogue: FrRot cannot change inside a step (it does when the
-// planet moves under the disk's torque) and nothing after the sweeps changes the state the CFL
-// reads (damping does)
-bool fused_cfl(const pn_ctx* c) { return c->P.plnt_flag < 2 && !c->P.kill_flag; }
+// Does a frame that follows the planet (frrot_flag 1) change its rate over a step?  Not while the
+// planet stays on an exact circle, where the kicks and the drift return what they took: no
+// velocity in the frame, no force, and the drift's products cancel.  A caller's planet with a
+// radial velocity, or a radius whose orbit does not close to the last bit, moves it.
+bool frame_moves(const pn_params& P, const pn_body& b, double FrRot) {
+  if (P.plnt_flag == 0 || P.frrot_flag != 1) return false;
+  const bool still = b.vx == 0.0 && b.vy == 0.0 && b.fx == 0.0 && b.fy == 0.0 &&
+                     FrRot * b.x * b.x / b.x / b.x == FrRot && -1.0 / b.x / b.x + b.x * (FrRot * FrRot) == 0.0;
+  return !still;
+}
+
+// the next dt from the last sweep's epilogue, which knows the FrRot of its step: FrRot must be the
+// same after the step and nothing after the sweeps may change the state the CFL reads (damping
+// does).  A planet under the disk's torque moves the frame, and in FP64 any planet that does
+// (frame_moves); FP32 takes such a step's dt with the rate its sweeps saw.
+bool fused_cfl(const pn_ctx* c) {
+  return c->P.plnt_flag < 2 && !c->P.kill_flag && (is_f32(c) || !c->frame_moves);
+}
 
 // the FP32 radial sweep of the context's geometry
 hipError_t f32_x(const pn_ctx* c, const LaunchCtx& L, int variant, int src) {
@@ -1591,6 +1605,11 @@ int pn_run(pn_ctx* c, int nsteps, int graph, pn_run_state* st) {
   h.land = st->land ? 1 : 0;
   h.event = 0;
   if ((rc = upload_scalars(c, h)) != PN_OK) return rc;
+  const bool moves = frame_moves(c->P, st->planet, st->FrRot);
+  if (moves != c->frame_moves) {
+    drop_graphs(c);   // their steps take dt the other way
+    c->frame_moves = moves;
+  }
   const bool fused = fused_cfl(c);
   // with the CFL taken in the sweep epilogue, dt of the first step comes from the state
   if (fused && nsteps > 0 && (rc = launch_cfl_any(c, c->cur)) != PN_OK) return rc;
