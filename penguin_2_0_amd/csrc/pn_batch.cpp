@@ -35,7 +35,9 @@ struct pn_batch {
   int nslot_x = 0;
   int* base_y = nullptr;     // device, ndisk + 1 azimuthal item offsets
   hipGraphExec_t gexec = nullptr;
-  int gexec_cur = 0;          // the buffer the captured step reads (it returns there)
+  // what the captured step was made from: the buffer it reads (and returns to), the radial slots
+  // and the grids of its launches
+  int gexec_cur = 0, gexec_nslot = 0, gexec_gx = 0, gexec_gy = 0;
 };
 
 namespace {
@@ -246,8 +248,11 @@ int batch_steps(pn_batch* b, int cur, int nsteps, int graph) {
   const bool replay = graph && nsteps > 1;
   if (replay) {
     // the captured step names its buffer; a disk moved to the other one since (for example by
-    // pn_sweep_axis on pn_batch_disk) needs a step captured from there
-    if (b->gexec && b->gexec_cur != cur) drop_graph(b);
+    // pn_sweep_axis on pn_batch_disk) needs a step captured from there.  It holds the counts of the
+    // radial order too, which changes with each disk's packing (pn_set_packing on pn_batch_disk)
+    if (b->gexec && (b->gexec_cur != cur || b->gexec_nslot != b->nslot_x || b->gexec_gx != b->grid_x ||
+                     b->gexec_gy != b->grid_y))
+      drop_graph(b);
     if (!b->gexec) {
       hipGraph_t gr;
       PB_HIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
@@ -259,6 +264,9 @@ int batch_steps(pn_batch* b, int cur, int nsteps, int graph) {
       hipGraphDestroy(gr);
       if (e != hipSuccess) return bfail(b, PN_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
       b->gexec_cur = cur;
+      b->gexec_nslot = b->nslot_x;
+      b->gexec_gx = b->grid_x;
+      b->gexec_gy = b->grid_y;
     }
     if (fused) PB_HIP(b, launch_pre_step_batch(b->stream, b->dd, ndisk(b)));
     for (; done < (fused ? nsteps - 1 : nsteps); ++done) PB_HIP(b, hipGraphLaunch(b->gexec, b->stream));
