@@ -145,11 +145,11 @@ __device__ __forceinline__ double rsq64(double x) {
   const double e = __builtin_fma(-(x * y), y, 1.0);
   return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
 }
-// sqrt(x) correctly rounded, x > 0 and normal
+// sqrt(x) correctly rounded, x zero or normal and positive
 __device__ __forceinline__ double sqrt64_rn(double x) {
   const double y = rsq64(x);
   const double g = x * y;
-  return __builtin_fma(__builtin_fma(-g, g, x), 0.5 * y, g);
+  return x == 0.0 ? x : __builtin_fma(__builtin_fma(-g, g, x), 0.5 * y, g);
 }
 // exp(t) for |t| < 1/8: 1 + (t + t^2 / 2 + ... + t^10 / 10!); the one rounding that matters is
 // the last addition's
@@ -548,7 +548,9 @@ __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const
         T dp2 = pp2[h] - pm2[h];
         if (fabs(dp2) < smallp) dp2 = smallp;
         const T lo = fmin(pp1[h], pm1[h]);
-        bool shock = div64(fabs(dp1), lo, rcp64(lo)) > T(0.33);
+        // a jump from no pressure at all (an infinite quotient, NaN here) is a shock; without a jump
+        // the steepness below is 0 either way
+        bool shock = !(div64(fabs(dp1), lo, rcp64(lo)) <= T(0.33));
         if (um1[h] < up1[h]) shock = false;
         if (shock) s = fmax(T(0.0), (dp1 / dp2 - T(0.75)) * T(5.0));
       }
