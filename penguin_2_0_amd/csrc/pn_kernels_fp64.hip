@@ -67,12 +67,13 @@ __device__ __forceinline__ double cfl_term(double v, double cs, double width, do
   const double a = fabs(v) + cs;
   return fmax(div64(a, width, y), 0.5 * (a * y));
 }
-// sqrt(gam p / r) of the CFL, rounded as written; zero and infinity as the library functions have them
+// sqrt(gam p / r) of the CFL, rounded as written; anything but an ordinary positive quotient by the
+// library's root (a negative pressure gives NaN, which the maximum passes over)
 __device__ __forceinline__ double cfl_sound(double gp, double r) {
   const double y = rcp64(r);
   const double c2 = fmax(div64(gp, r, y), 0.5 * (gp * y));
   const double s = sqrt64_rn(c2);
-  return c2 > 0.0 && c2 < 1.0e300 ? s : c2;
+  return c2 > 0.0 && c2 < 1.0e300 ? s : sqrt(c2);
 }
 __device__ __forceinline__ double wave_max(double v) {
   for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
