@@ -10,9 +10,13 @@ namespace pn {
 // columns of one work item (a run of one ring)
 constexpr int kTorqueCols = 256;
 
-// rot_j of slot s after the step's integer roll (rotate_rings, ppm.cu:309-322)
+// rot_j of slot s after the step's integer roll (rotate_rings, ppm.cu:309-322).  A shift of more
+// than a turn (a cold or coarse disk's step, or a loaded record's inc_j) rolls by what is left of
+// it: every address of the ring is formed from rot_j in [0, jmax).
 __device__ __forceinline__ int rolled(const DevGrid& g, int s) {
-  int j = g.rot_j[s] + g.inc_j[s];
+  int inc = g.inc_j[s];
+  if (inc >= g.jmax || inc <= -g.jmax) inc %= g.jmax;
+  int j = g.rot_j[s] + inc;
   if (j < 0) j += g.jmax;
   if (j >= g.jmax) j -= g.jmax;
   return j;
