@@ -2,8 +2,8 @@
 //
 // Method: the reference's ppmlr (ppmlr.cu:2-56) -- flatten, states (paraset, parabola,
 // characteristic averages, interface force), Riemann solve, Lagrangian evolve, PPM remap --
-// followed by the explicit viscosity (viscosity.cu:370-472).  Same operands in the same
-// order per cell, so the FP64 instantiation reproduces the reference arithmetic.
+// followed by the explicit viscosity (viscosity.cu:370-472).  The statements are the reference's; which
+// of them round as it writes them and which carry an ulp of their own is said at ppmlr_wave.
 //
 // Execution model (not the reference's): one 64-lane wavefront owns a whole window, each
 // lane K consecutive cells (cell c = K*lane + h).  Every stencil access is to the cell
@@ -118,10 +118,11 @@ __device__ __forceinline__ T max3(T A, T B, T Cc) {   // simple_func.cu:16-28
 // FP64 divisions, roots, exp and log of the windows.  A sweep divides by the same few numbers
 // over and over (a radius three times in a row, a cell's density, the Lagrangian volume), and
 // the compiler's division is 11 instructions each time.  Here a reciprocal is formed once and
-// each quotient by it takes three: q = a y, r = a - q b (exact in an FMA), q + r y, which is the
-// correctly rounded a / b for any y within an ulp of 1 / b (Markstein 1990), so the result
-// keeps the bits of the division.  For finite, normal operands; a zero or non-finite divisor
-// gives NaN where a division gives an infinity.
+// each quotient by it takes three: q = a y, r = a - q b (exact in an FMA), q + r y (Markstein 1990).
+// With y within an ulp of 1 / b the sum lies within 2^-51 ulp of a / b before its one rounding, so
+// it is the division's result unless a / b lies that close to the middle between two numbers (one
+// quotient in 2^50; a divisor 2 - 2^-52 has such ones).  For finite, normal operands; a zero or
+// non-finite divisor gives NaN where a division gives an infinity.
 
 // 1 / b to an ulp: the hardware estimate (2^-24 or better) and one cubic step
 __device__ __forceinline__ double rcp64(double b) {
@@ -129,12 +130,12 @@ __device__ __forceinline__ double rcp64(double b) {
   const double e = __builtin_fma(-b, y, 1.0);
   return __builtin_fma(y, __builtin_fma(e, e, e), y);
 }
-// 1 / b correctly rounded, from y = rcp64(b)
+// 1 / b rounded as the division (as above), from y = rcp64(b)
 __device__ __forceinline__ double rcp64_rn(double b) {
   const double y = rcp64(b);
   return __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
 }
-// a / b correctly rounded, y = 1 / b to an ulp
+// a / b rounded as the division (as above), y = 1 / b to an ulp
 __device__ __forceinline__ double div64(double a, double b, double y) {
   const double q = a * y;
   return __builtin_fma(__builtin_fma(-q, b, a), y, q);
@@ -145,7 +146,8 @@ __device__ __forceinline__ double rsq64(double x) {
   const double e = __builtin_fma(-(x * y), y, 1.0);
   return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
 }
-// sqrt(x) correctly rounded, x zero or normal and positive
+// sqrt(x) rounded as the root but for values within 2^-49 ulp of a middle, x zero or normal and
+// positive
 __device__ __forceinline__ double sqrt64_rn(double x) {
   const double y = rsq64(x);
   const double g = x * y;
@@ -514,10 +516,12 @@ struct Ring64 {
 
 // One PPMLR update of the window (ppmlr.cu:2-56).  c0 = this lane's first cell, nmax = window
 // length, drift = vrot - v_y (azimuthal sweep).  On return the cells [6, nmax-6) hold the
-// updated r, u, v, w (and p for EOS 1, 2).  What is kept of the reference's arithmetic bit for
-// bit and what is not: in 3-D everything.  In 2-D every value that a stored field is built from
-// rounds as the reference's does; the planet's pull, the logarithm and exponential of the
-// interface and the Lagrangian interpolation coefficients carry an ulp of their own.
+// updated r, u, v, w (and p for EOS 1, 2).  What is kept of the reference's rounding: in 3-D every
+// operation's (quotients and roots as said at div64).  In 2-D the states, the star's and the
+// centrifugal force, the Lagrangian step and the mass update round as written; the planet's pull, the
+// interface's logarithm, exponential and powers (EOS 0, 2, 3), the Lagrangian interpolation
+// coefficients, the flattened edges, the average over a swept face and the viscous increment carry an
+// ulp of their own (1e-12 to 2e-11 of a field after some ten steps).
 template <int K, class CF>
 __device__ __forceinline__ void ppmlr_wave(Win<K>& W, const TabLane64& tx, const Ring64& ring, int c0, int nmax,
                                            double dt, double FrRot, const Planet& pl, const RunFlags& rf, double gam) {
