@@ -268,15 +268,15 @@ int pn_set_variants(pn_ctx* ctx, int var_x, int var_y);
 /* The variants in use (after tuning or pinning; 0 for FP64 contexts). */
 int pn_get_variants(const pn_ctx* ctx, int* var_x, int* var_y);
 /* The 3-D FP32 theta sweep's own shape: var_z 0..3 as var_x (what pn_set_variants sets it
- * to), or 4 = (3, 4, 2), 192-cell windows, which run two theta pencils of up to 84 cells with
- * their halos per wavefront (refused with PN_ERR_ARG for a viscous disk, which keeps 128-cell
+ * to), or 4 = (3, 4, 2), 192-cell windows, where a theta pencil of up to 84 layers shares its
+ * wavefront with at least one other (refused with PN_ERR_ARG for a viscous disk, which keeps 128-cell
  * theta windows).  pn_tune picks it apart from the radial shape.  0 for FP64 and 2-D
  * contexts. */
 int pn_set_variant_z(pn_ctx* ctx, int var_z);
 int pn_get_variant_z(const pn_ctx* ctx, int* var_z);
 /* FP32 radial and theta sweeps: on (1, the default) the last window of a pencil, when it
- * holds at most 32 K cells (K cells per lane), runs two lab columns per wavefront, one in
- * each half; off (0) it runs one, like every other window.  The results are the same either
+ * holds at most 32 K cells (K cells per lane), runs as many lab columns per wavefront as fit,
+ * each on its own run of lanes; off (0) it runs one, like every other window.  The results are the same either
  * way; the switch exists to show that.  A batch's disks follow their own contexts' setting
  * (pn_batch_disk).  No counterpart in the reference. */
 int pn_set_packing(pn_ctx* ctx, int on);

@@ -356,7 +356,7 @@ class Context:
         return v.value
 
     def set_packing(self, on: bool):
-        """Two short last radial / theta windows per wavefront (pn_set_packing)."""
+        """As many short last radial / theta windows per wavefront as fit (pn_set_packing)."""
         self._chk(self.lib.pn_set_packing(self.h, 1 if on else 0), "pn_set_packing")
 
     def totals_noalloc(self) -> tuple[float, float]:

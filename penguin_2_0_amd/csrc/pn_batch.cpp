@@ -80,10 +80,10 @@ bool any_adia(const pn_batch* b) { return b->disks[0]->P.eos == 3; }
 // XCD t % 8.  Each XCD gets a contiguous run of the disks' items (neighbouring column groups
 // share L2 lines) of an equal share of the estimated cost, laid out by decreasing cost (a
 // stable sort, so equal items keep their neighbours): every XCD's last, partial round then
-// holds its cheapest items -- last windows short enough to run two columns per wavefront pass
+// holds its cheapest items -- last windows short enough to run several columns per wavefront pass
 // -- instead of a random mix, whose most expensive workgroup would set the launch's length.
 // Cost of a window item: 0.3 for the staging (scaled by the window's cells) and 0.7 for the
-// pencil passes (halved when the window runs two columns per pass, a third for three).
+// pencil passes (a half when the window runs two columns per pass, a third for three, and so on).
 int build_order_x(pn_batch* b, std::vector<int>& order, int& nslots) {
   const int K = kF32VariantsX[b->var_x][0];
   const int nc = kF32VariantsX[b->var_x][1] * kF32VariantsX[b->var_x][2];

@@ -31,8 +31,9 @@ struct pn_ctx {
   double* ringbuf = nullptr;        // device, one double per interior ring (ring means)
   hipStream_t stream = nullptr;
   std::vector<void*> allocs;
-  // pinned staging of pn_store_rings: two pieces of the fields and the FARGO state (made on the
-  // first picture, at most 8 MiB or two rings beside 24 bytes a slot)
+  // pinned staging of pn_load_rings and pn_store_rings: two pieces of the fields and the FARGO state
+  // (made on the first load, at most 8 MiB or two rings beside 24 bytes a slot; freed with the
+  // context, so a batch holds one per disk)
   void* stage = nullptr;
   bool stage_pinned = false;
   hipEvent_t stage_ev[2] = {nullptr, nullptr};

@@ -83,7 +83,7 @@ constexpr int kNumF32Variants = 4;
 // stages a window of W*Q columns through LDS
 extern const int kF32VariantsX[kNumF32Variants][3];
 // theta sweep: kF32VariantsX, plus (3, 4, 2): 192-cell windows, which hold two theta pencils of
-// 64 cells with their halos per wavefront (76 cells each)
+// 64 layers with their halos per wavefront (76 cells each), or more shorter ones
 constexpr int kNumF32VariantsZ = 5;
 extern const int kF32VariantsZ[kNumF32VariantsZ][3];
 // azimuthal sweep: (cells per lane K, waves per workgroup W)
