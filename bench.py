@@ -127,7 +127,8 @@ def roofline_entry(kernel: str, variant: int, kernel_ms: float, bytes_per_launch
          "traffic_over_algorithmic": traffic / bytes_per_launch if traffic else None, "kernels_ms": km,
          "copy_measured_gbs": copy_gbs, "frac_of_copy": achieved / copy_gbs}
     if "sq_insts_valu" in prof:
-        # what bounds the sweeps: VALU issue, against one instruction per CU per clock
+        # what bounds the sweeps: VALU issue, against one instruction per CU per clock (a yardstick:
+        # some issue beside others, and EOS 3's sweeps pass it)
         ips = prof["sq_insts_valu"] / (kernel_ms * 1e-3)
         r["valu"] = {"insts_per_launch": prof["sq_insts_valu"], "achieved_insts_per_s": ips,
                      "peak_insts_per_s": VALU_PEAK_INSTS, "frac": ips / VALU_PEAK_INSTS}

@@ -632,7 +632,7 @@ __global__ __launch_bounds__(kStepThreads) void k_post_step(DevGrid g, DevParams
 
 // The end of one step and the beginning of the next in one workgroup, for a step whose dt comes
 // from its last sweep's CFL: between two steps a disk then launches this alone, where the two
-// bodies apart cost two launches (128 x 384, FP32: 29.6 -> 23.0 us a step with the longer graphs).
+// bodies apart cost two launches (128 x 384, FP32: 29.3 -> 23.1 us a step with the longer graphs).
 // Every thread rolls and shifts the same rings in both bodies, so between them only thread 0's
 // scalars have to be seen.
 __global__ __launch_bounds__(kStepThreads) void k_mid_step(DevGrid g, DevParams prm, StepScalars* ss,

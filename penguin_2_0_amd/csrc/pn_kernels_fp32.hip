@@ -143,7 +143,7 @@ struct XTile {
 
 // waves per SIMD a pencil kernel asks for: as many, up to five, as workgroups of four waves fit
 // the CU's 160 KiB of LDS; no request for larger workgroups, nor for K = 3 (unconstrained it
-// takes 165 registers, three waves per SIMD, without spilling)
+// takes 157 to 159 registers, three waves per SIMD, without spilling)
 template <int K, int W, int Q, int NF>
 constexpr int pencil_waves() {
   constexpr size_t lds = sizeof(XTile<K, W, Q, NF>);

@@ -11,8 +11,9 @@
 // the angle to the planet is turned from a per-column cosine and sine instead of taken anew at
 // three times: 1024 x 3072, inviscid, 5347 -> 2516 static VALU instructions a radial pass.  With the
 // radial and theta sweeps staged through LDS and short windows packed two to a wavefront (below):
-//   1024 x 3072 radial 208 -> 125 us, azimuthal 189 -> 108 us; 256 x 768 radial 30.6 -> 13.5 us;
-//   96 x 288 x 32, whose sweeps keep every bit, r / phi / theta 110 / 83 / 345 -> 68 / 61 / 97 us.
+//   1024 x 3072 radial 197 -> 113 us, azimuthal 189 -> 114 us; 256 x 768 radial 29.2 -> 13.4 us;
+//   96 x 288 x 32, whose sweeps round every operation as written, r / phi / theta 97 / 78 / 342 ->
+//   58 / 56 / 101 us (timed back to back; the azimuthal ones carry the next step's CFL since).
 #include "pn_launch.hpp"
 #include "ppm_wave.hpp"
 

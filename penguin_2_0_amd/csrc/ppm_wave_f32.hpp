@@ -25,12 +25,12 @@
 // grid motion is kept apart from the velocity-dependent part so the cell volumes and the
 // density fluxes never difference it.
 //
-// What bounds it: instruction issue.  With its states in registers or LDS a sweep keeps the
-// SIMDs' vector pipes 70 to 90 % busy, and a reciprocal, root or exponential holds one four times as
-// long as a product; the library logarithm and the flattening run only in wavefronts that hold a
-// cell in need of them.  Cheaper arithmetic was tried and taken back: reciprocals of rho_b, p_b, the
-// widths and volumes from the table, limiters as medians and shared viscosity reciprocals ran the
-// sweeps 17 to 20 % faster (1024 x 3072: 61 -> 51 us radial, 41 -> 34 azimuthal), but a table's
+// What bounds it: instruction issue.  With its states in registers or LDS a sweep issues 0.77 to
+// 0.96 vector instructions per CU and clock (up to 1.2 with EOS 3), and a reciprocal, root or
+// exponential holds its pipe four times as long as a product; the library logarithm and the
+// flattening run only in wavefronts that hold a cell in need of them.  Cheaper arithmetic was tried
+// and taken back: reciprocals of rho_b, p_b, the widths and volumes from the table, limiters as
+// medians and shared viscosity reciprocals ran the sweeps 17 to 20 % faster (1024 x 3072: 61 -> 51 us radial, 41 -> 34 azimuthal), but a table's
 // reciprocal repeats its own rounding step after step: after 1000 steps of that disk L1 of Sigma
 // against FP64 had grown from 4.4e-9 to 4.9e-9 and the drift of the mass from 8.5e-8 of itself off
 // FP64's to 4.1e-7.
